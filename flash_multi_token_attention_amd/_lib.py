@@ -79,6 +79,8 @@ _SIGNATURES = {
     "convattn_headmix_bwd_workspace_bytes": (C.c_size_t, [_HD]),
     "convattn_headmix_bwd_dq_dw": (C.c_int, [_HD] + [_P] * 12),
     "convattn_headmix_bwd_dkdv": (C.c_int, [_HD] + [_P] * 12),
+    "convattn_headmix_bwd_fused_workspace_bytes": (C.c_size_t, [_HD]),
+    "convattn_headmix_bwd_fused": (C.c_int, [_HD, C.c_int] + [_P] * 14),
 }
 EXPORTS = tuple(_SIGNATURES)
 

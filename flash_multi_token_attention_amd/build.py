@@ -42,6 +42,7 @@ UNITS = [
     ("bwd_dq_rows.hip", "bwd_dq_rows", []),
     ("decode_stream.hip", "decode_stream", []),
     ("headmix_attn.hip", "headmix_attn", []),
+    ("headmix_bwd.hip", "headmix_bwd", []),
 ]
 SOURCES = sorted({u[0] for u in UNITS})
 

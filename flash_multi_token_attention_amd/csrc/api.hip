@@ -496,4 +496,51 @@ int convattn_headmix_bwd_dkdv(const convattn_headmix_desc *desc, const void *q, 
                                  dk, dv, s);
 }
 
+// Scratch of the one-pass backward: D, LSE, dw partials, then the dS and the P blocks.
+struct HeadmixFusedWs {
+    size_t lse_off, part_off, ds_off, p_off, total;
+};
+static Problem headmix_problem(const convattn_headmix_desc *d) {
+    Problem p{};
+    p.B = d->B; p.H = d->H; p.Nq = p.Nk = d->N; p.d = d->d; p.c_q = p.c_k = 1;
+    p.scale = d->scale; p.causal = d->causal ? 1 : 0; p.n_splits = 1;
+    return p;
+}
+static HeadmixFusedWs headmix_fused_ws(const convattn_headmix_desc *d) {
+    const Problem p = headmix_problem(d);
+    const size_t stat = align256((size_t)d->B * d->H * d->N * sizeof(float)), ds = align256(chain_ds_bytes(p));
+    HeadmixFusedWs w;
+    w.lse_off = stat;
+    w.part_off = 2 * stat;
+    w.ds_off = w.part_off + align256((size_t)d->B * headmix_score_wgs(d->B, d->H, d->N, p.causal) * d->H * d->H * sizeof(float));
+    w.p_off = w.ds_off + ds;
+    w.total = w.p_off + ds;
+    return w;
+}
+
+size_t convattn_headmix_bwd_fused_workspace_bytes(const convattn_headmix_desc *desc) {
+    return headmix_check(desc) ? 0 : headmix_fused_ws(desc).total;
+}
+
+int convattn_headmix_bwd_fused(const convattn_headmix_desc *desc, int grad_dtype, const void *q, const void *k,
+                               const void *v, const float *w, const void *o, const void *d_o, const float *l,
+                               const float *m, void *workspace, void *dq, void *dk, void *dv, float *dw, void *stream) {
+    int rc = headmix_check(desc);
+    if (rc) return rc;
+    if (grad_dtype != CONVATTN_BF16 && grad_dtype != CONVATTN_F32) return CONVATTN_ERR_DTYPE;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(w); REQUIRE_PTR(o); REQUIRE_PTR(d_o);
+    REQUIRE_PTR(l); REQUIRE_PTR(m); REQUIRE_PTR(workspace);
+    if (dq || dw) { REQUIRE_PTR(dq); REQUIRE_PTR(dw); }
+    if (dk || dv || !dq) { REQUIRE_PTR(dk); REQUIRE_PTR(dv); }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const Problem p = headmix_problem(desc);
+    const HeadmixFusedWs ws = headmix_fused_ws(desc);
+    unsigned char *base = static_cast<unsigned char *>(workspace);
+    float *Dl = reinterpret_cast<float *>(base), *lse = reinterpret_cast<float *>(base + ws.lse_off);
+    rc = (int)bwd_preprocess(p, desc->in_dtype, desc->out_dtype, o, d_o, m, l, Dl, lse, s);
+    if (rc) return rc;
+    return (int)headmix_bwd_fused(p, grad_dtype, q, k, v, w, d_o, lse, Dl, base + ws.p_off, base + ws.ds_off,
+                                  reinterpret_cast<float *>(base + ws.part_off), dq, dk, dv, dw, s);
+}
+
 }  // extern "C"

@@ -1,0 +1,555 @@
+// One-pass backward of head-mixing attention (gfx950): dQ, dK, dV and the gradient of the mixing matrix.
+//
+//   S_h' = Q_h' K_h'^T,  Z_h = scale sum_h' w[h][h'] S_h',  P_h = exp(Z_h - LSE_h),  dP_h = dO_h V_h^T,
+//   dZ_h = P_h (dP_h - D_h),  dS_h' = scale sum_h w[h][h'] dZ_h,  dw[h][h'] = scale sum dZ_h S_h',
+//   dQ_h' = dS_h' K_h',  dK_h' = dS_h'^T Q_h',  dV_h = P_h^T dO_h.
+//
+// The head mix couples all heads of a (row, key) pair, the last three products couple all keys (or
+// rows) of a head.  Kept in one workgroup, their accumulators (2 H d floats per key) leave room for 16
+// keys only, and every byte of Q and dO is then loaded for 16 keys at a time.  So the pass is cut between
+// the two: headmix_scores_kernel computes P and dS once per (row, key) pair and writes them as bf16
+// blocks of 32 rows x 32 keys (the operand precision of the products that follow); dQ = dS K is
+// the product kernel of the window backward (bwd_dq_rows.hip, same block layout) and
+// headmix_dkdv_kernel takes dV = P^T dO and dK = dS^T Q from one walk over the blocks of 128 keys.
+#include "mfma_common.hpp"
+
+namespace convattn {
+namespace {
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// Workgroup barrier for data that is exchanged through LDS: waits for this wave's LDS operations, not for the
+// global loads it has issued ahead.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+constexpr int SC_WAVES = 8;
+constexpr int SC_BLK = kChainRows * kChainKeys;   // elements of a P / dS block
+
+// Tile of the score kernel: 512 (row, key) pairs of all heads per step, 64 pairs per wave.
+//   RB = 2: 32 rows x 16 keys (16 heads);  RB = 1: 16 rows x 32 keys (32 heads: the resident row fragments
+//   of 32 heads take the registers of 16 heads' 32 rows).
+template <int H, int D> struct ScoreTile {
+    static constexpr int RB = H == 16 ? 2 : 1;
+    static constexpr int R = 16 * RB, KT = 512 / R, KB = KT / 16, NQ = KT / 4;
+    static constexpr int RW = R / SC_WAVES;                 // rows of a wave in the mixing phase
+    static constexpr int SWZ = RB == 2 ? 2 : 1;             // see slot()
+    static constexpr int HS = R * KT + 4;                   // floats per head (+4: 16 heads on 16 bank quads)
+    static constexpr int arr = H * HS;                      // floats of one array
+    static constexpr int NBUF = H == 16 ? 2 : 1;
+    static constexpr int HPW = H / SC_WAVES, HB = H / 16;
+    static constexpr int WST = H + 4;                       // floats per row of w in LDS
+    static constexpr int w_off = NBUF * 2 * arr, wt_off = w_off + H * WST, lds = (wt_off + H * WST) * 4;
+    // Four keys 4q .. 4q+3 of tile row `lr` sit at float lr * KT + 4 * slot: the XOR spreads both the score
+    // phase's writes (16 rows, one quad) and the mixing phase's reads (RW rows, all quads) over all banks.
+    __device__ static __forceinline__ int slot(int lr, int q) { return q ^ ((lr >> SWZ) & (NQ - 1)); }
+    // Query row of tile row lr: even rows of the 32-row block first, as the blocks are laid out
+    __device__ static __forceinline__ int row(int i0, int lr) {
+        return RB == 2 ? i0 + 2 * (lr & 15) + (lr >> 4) : i0 + 2 * (lr & 7) + (lr >> 3);
+    }
+};
+
+struct ScoreArgs {
+    int B, N, causal, n_rt32, n_kt, steps_per_wg, n_wg;
+    float scale;
+    const bf16_t *Q, *K, *V, *dO;
+    const float *W, *lse, *Dl;
+    bf16_t *P, *dS;      // blocks; P may be null (dQ and dW only)
+    float *dw_part;      // [B][n_wg][H][H], or null
+};
+
+// Workgroup `id` of the n_wg of a batch entry -> row tile and first key step of its chunk.  Chunks of the
+// same keys are neighbours, and neighbours run on the same XCD (workgroup ids go round robin over the eight),
+// so that the rows of K and V of a chunk come from one L2.
+template <int H, int D>
+__device__ __forceinline__ bool score_unit(const ScoreArgs &a, int &rt, int &s0, int &s_end) {
+    using T = ScoreTile<H, D>;
+    const int n_tiles = a.n_rt32 * (32 / T::R);
+    const int per = (a.n_wg + 7) / 8;
+    int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || id >= a.n_wg) return false;
+    const int all = a.n_rt32 * (32 / T::KT);
+    for (int c = 0;; ++c) {
+        s0 = c * a.steps_per_wg;
+        const int first = a.causal ? (s0 * T::KT / 32) * (32 / T::R) : 0;   // first row tile that sees the chunk
+        if (id < n_tiles - first) {
+            rt = n_tiles - 1 - id;
+            const int end = a.causal ? (rt * T::R / 32 + 1) * (32 / T::KT) : all;
+            s_end = min(s0 + a.steps_per_wg, end);
+            return true;
+        }
+        id -= n_tiles - first;
+    }
+}
+
+template <int H, int D>
+__global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs a) {
+    using T = ScoreTile<H, D>;
+    constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, HPW = T::HPW,
+                  HB = T::HB, KS = D / 32, NCH = HPW * KB;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    float *lds = reinterpret_cast<float *>(smem);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
+              n = lane & 15;
+    const int b = blockIdx.y;
+    int rt, s0, s_end;
+    if (!score_unit<H, D>(a, rt, s0, s_end)) return;
+    const int i0 = rt * R, N = a.N;
+    const size_t bo = (size_t)b * H * N * D;
+    const int h0 = wave * HPW;
+
+    // ---- resident: Q and dO fragments of this wave's heads ----
+    bf16x8 qf[HPW][RB][KS], of[HPW][RB][KS];
+#pragma unroll
+    for (int t = 0; t < HPW; ++t)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int row = min(T::row(i0, rb * 16 + n), N - 1);
+            const size_t o = bo + ((size_t)(h0 + t) * N + row) * D + 8 * g;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                qf[t][rb][ks] = *reinterpret_cast<const bf16x8 *>(a.Q + o + 32 * ks);
+                of[t][rb][ks] = *reinterpret_cast<const bf16x8 *>(a.dO + o + 32 * ks);
+            }
+        }
+    // ---- the mixing phase: lane (g, n) = heads 4g .. 4g+3 of each block of 16, tile row lr, keys 4q .. 4q+3 ----
+    const int lr = wave * RW + (n & (RW - 1)), q4 = n / RW;
+    const int row = T::row(i0, lr);
+    float lse2[HB][4], dl[HB][4];
+#pragma unroll
+    for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const size_t o = ((size_t)b * H + 16 * hb + 4 * g + r) * N + min(row, N - 1);
+            // (rows past the last: P = exp2(-1e30) = 0, so nothing of them is in dS, dV, dK or dw)
+            lse2[hb][r] = row < N ? a.lse[o] * kLog2e : 1e30f;
+            dl[hb][r] = a.Dl[o];
+        }
+    // w of the mix and its transpose, with the scales of the two products, in LDS (read as four k steps at a time:
+    // k slot g of step s is head 4g + s)
+    for (int i = tid; i < H * H; i += SC_WAVES * 64) {
+        const float w = a.W[i];
+        lds[T::w_off + (i / H) * T::WST + i % H] = w * (a.scale * kLog2e);
+        lds[T::wt_off + (i % H) * T::WST + i / H] = w * a.scale;
+    }
+    const float *wf_l = lds + T::w_off + n * T::WST + 4 * g, *wb_l = lds + T::wt_off + n * T::WST + 4 * g;
+    f32x4 acc_w[HB][HB];
+#pragma unroll
+    for (int x = 0; x < HB; ++x)
+#pragma unroll
+        for (int y = 0; y < HB; ++y) acc_w[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    // ---- score phase, in chunks of one head and 16 keys whose K and V rows are loaded two chunks ahead ----
+    bf16x8 kf[2][KS], vf[2][KS];
+    auto load_chunk = [&](int buf, int step, int c) {
+        const int t = c / KB, kb = c % KB;
+        const int key = min(step * KT + kb * 16 + n, N - 1);
+        const size_t o = bo + ((size_t)(h0 + t) * N + key) * D + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            kf[buf][ks] = *reinterpret_cast<const bf16x8 *>(a.K + o + 32 * ks);
+            vf[buf][ks] = *reinterpret_cast<const bf16x8 *>(a.V + o + 32 * ks);
+        }
+    };
+    auto score_chunk = [&](float *S, int buf, int c) {
+        const int t = c / KB, kb = c % KB;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                s = mfma_bf16(kf[buf][ks], qf[t][rb][ks], s);
+                dp = mfma_bf16(vf[buf][ks], of[t][rb][ks], dp);
+            }
+            float *dst = S + (h0 + t) * HS + (rb * 16 + n) * KT + 4 * T::slot(rb * 16 + n, 4 * kb + g);
+            *reinterpret_cast<f32x4 *>(dst) = s;
+            *reinterpret_cast<f32x4 *>(dst + T::arr) = dp;
+        }
+    };
+
+    // ---- mixing phase of one step ----
+    const int pos = lr * KT + 4 * T::slot(lr, q4);
+    // element of a block for this lane: [row parity][key half][row pair][16 keys]
+    const int brow = row & 31;
+    auto mix_step = [&](float *S, int step, auto masked_c) {
+        constexpr bool masked = decltype(masked_c)::value;
+        float *dP = S + T::arr;
+        const int j0 = step * KT;
+        f32x4 z[HB][4];
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) z[x][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int y = 0; y < HB; ++y) {
+            f32x4 wf[HB];
+#pragma unroll
+            for (int x = 0; x < HB; ++x) wf[x] = *reinterpret_cast<const f32x4 *>(wf_l + 16 * x * T::WST + 16 * y);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(S + (16 * y + 4 * g + s) * HS + pos);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
+            }
+        }
+        const int kt = j0 / 32;
+        const long long blk = chain_ds_block_off(a.causal != 0, a.n_rt32, kt) + i0 / 32 - chain_ds_first_rt(a.causal != 0, kt);
+        const long long per_head = chain_ds_block_off(a.causal != 0, a.n_rt32, a.n_kt);
+        const size_t out = ((size_t)b * H * per_head + blk) * SC_BLK +
+                           (((brow & 1) * 2 + ((j0 + 4 * q4) >> 4 & 1)) * 16 + (brow >> 1)) * 16 + ((4 * q4) & 15);
+#pragma unroll
+        for (int x = 0; x < HB; ++x) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float *dz = dP + (16 * x + 4 * g + r) * HS + pos;
+                f32x4 d = *reinterpret_cast<const f32x4 *>(dz);
+                bf16x4 pb;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    float p = fast_exp2(z[x][t][r] - lse2[x][r]);
+                    if constexpr (masked) {
+                        const int key = j0 + 4 * q4 + t;
+                        if (key >= N || (a.causal && key > row)) p = 0.f;
+                    }
+                    pb[t] = (bf16_t)p;
+                    d[t] = p * (d[t] - dl[x][r]);
+                    z[x][t][r] = d[t];
+                }
+                *reinterpret_cast<f32x4 *>(dz) = d;
+                if (a.P)
+                    __builtin_nontemporal_store(__builtin_bit_cast(u32x2, pb), reinterpret_cast<u32x2 *>(
+                        a.P + out + (size_t)(16 * x + 4 * g + r) * per_head * SC_BLK));
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < HB; ++x) {
+            f32x4 ds[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) ds[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int y = 0; y < HB; ++y) {
+                const f32x4 wb = *reinterpret_cast<const f32x4 *>(wb_l + 16 * x * T::WST + 16 * y);
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) ds[t] = mfma4(wb[s], z[y][t][s], ds[t]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                bf16x4 db;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) db[t] = (bf16_t)ds[t][r];
+                __builtin_nontemporal_store(__builtin_bit_cast(u32x2, db), reinterpret_cast<u32x2 *>(
+                    a.dS + out + (size_t)(16 * x + 4 * g + r) * per_head * SC_BLK));
+            }
+        }
+        // dw += dZ S^T over the wave's own 64 pairs: lane n = head of either operand
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < RW * NQ / 4; ++i) {
+            const int r2 = wave * RW + i / (NQ / 4), q = 4 * (i % (NQ / 4)) + g;
+            const int o = n * HS + r2 * KT + 4 * T::slot(r2, q);
+            f32x4 za[HB], sb[HB];
+#pragma unroll
+            for (int x = 0; x < HB; ++x) {
+                za[x] = *reinterpret_cast<const f32x4 *>(dP + 16 * x * HS + o);
+                sb[x] = *reinterpret_cast<const f32x4 *>(S + 16 * x * HS + o);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int x = 0; x < HB; ++x)
+#pragma unroll
+                    for (int y = 0; y < HB; ++y) acc_w[x][y] = mfma4(za[x][e], sb[y][e], acc_w[x][y]);
+        }
+    };
+    auto mix = [&](float *S, int step) {
+        // masks only where a key of the tile is past the tile's first row or past the last key
+        if ((a.causal && step * KT + KT - 1 > i0) || step * KT + KT > N) mix_step(S, step, std::true_type{});
+        else mix_step(S, step, std::false_type{});
+    };
+
+    load_chunk(0, s0, 0);
+    if constexpr (NCH > 1) load_chunk(1, s0, 1);
+    if constexpr (T::NBUF == 2) {
+        static_assert(NCH == 2, "two chunks per step");
+        score_chunk(lds, 0, 0);
+        load_chunk(0, min(s0 + 1, s_end - 1), 0);
+        score_chunk(lds, 1, 1);
+        load_chunk(1, min(s0 + 1, s_end - 1), 1);
+        lds_barrier();
+        for (int u = s0; u < s_end; ++u) {
+            float *cur = lds + ((u - s0) & 1) * 2 * T::arr, *nxt = lds + ((u - s0 + 1) & 1) * 2 * T::arr;
+            const bool more = u + 1 < s_end;
+            const int ahead = min(u + 2, s_end - 1);
+            if (more) {
+                score_chunk(nxt, 0, 0);
+                load_chunk(0, ahead, 0);
+            }
+            mix(cur, u);
+            if (more) {
+                score_chunk(nxt, 1, 1);
+                load_chunk(1, ahead, 1);
+            }
+            lds_barrier();
+        }
+    } else {
+        for (int u = s0; u < s_end; ++u) {
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) {
+                score_chunk(lds, c & 1, c);
+                if (c + 2 < NCH) load_chunk(c & 1, u, c + 2);
+                else load_chunk(c & 1, min(u + 1, s_end - 1), c + 2 - NCH);
+            }
+            lds_barrier();
+            mix(lds, u);
+            lds_barrier();
+        }
+    }
+
+    // ---- the workgroup's dw partial: the waves' accumulators added in wave order ----
+    if (a.dw_part) {
+        lds_barrier();
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
+#pragma unroll
+            for (int y = 0; y < HB; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) lds[(wave * H + 16 * x + 4 * g + r) * H + 16 * y + n] = acc_w[x][y][r];
+        lds_barrier();
+        const int per = (a.n_wg + 7) / 8;
+        const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+        float *part = a.dw_part + ((size_t)b * a.n_wg + id) * H * H;
+        for (int i = tid; i < H * H; i += SC_WAVES * 64) {
+            float s = 0.f;
+#pragma unroll
+            for (int w = 0; w < SC_WAVES; ++w) s += lds[w * H * H + i];
+            part[i] = s * a.scale;
+        }
+    }
+}
+
+// dw[h][h'] = sum of the partials in a fixed order: a workgroup takes 16 entries, 16 threads per entry each
+// add every 16th partial, the sixteen sums are added in order.
+__global__ __launch_bounds__(256) void headmix_dw_sum_kernel(int n_part, int hh, const float *__restrict__ part,
+                                                             float *__restrict__ dW) {
+    __shared__ float red[16][17];
+    const int e = threadIdx.x & 15, c = threadIdx.x >> 4, idx = blockIdx.x * 16 + e;
+    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
+    int q = c;
+    for (; q + 48 < n_part; q += 64) {
+        s0 += part[(size_t)q * hh + idx];
+        s1 += part[(size_t)(q + 16) * hh + idx];
+        s2 += part[(size_t)(q + 32) * hh + idx];
+        s3 += part[(size_t)(q + 48) * hh + idx];
+    }
+    for (; q < n_part; q += 16) s0 += part[(size_t)q * hh + idx];
+    red[c][e] = (s0 + s1) + (s2 + s3);
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s += red[i][threadIdx.x];
+        dW[blockIdx.x * 16 + threadIdx.x] = s;
+    }
+}
+
+// ------------------------------------------------------------------ dV = P^T dO, dK = dS^T Q
+// Workgroup = 4 waves = 128 keys of one (batch, head), wave = 32 keys (one block column); row tiles of 32.  Q and
+// dO rows and the wave's P and dS blocks pass through LDS, everything is read with transpose reads (the contraction
+// runs over the rows); k slots of a lane group: rows 8g, 8g+2, 8g+4, 8g+6, then the odd ones, which is how
+// the blocks keep them.  Loads are one row tile ahead in registers.
+constexpr int KV_WAVES = 4;
+template <int D> struct KvLds {
+    static constexpr int RST = D * 2 + 16;            // bytes per staged row
+    static constexpr int rows = 32 * RST;             // one matrix, [parity][16 row pairs]
+    static constexpr int blocks = KV_WAVES * 2 * SC_BLK * 2;
+    static constexpr int buf = 2 * rows + blocks;
+    static constexpr int total = 2 * buf;
+};
+
+template <int D, typename TO>
+__global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, int H, int N, int causal, int n_rt, int n_kt,
+                                                                     const bf16_t *__restrict__ Q,
+                                                                     const bf16_t *__restrict__ dO,
+                                                                     const bf16_t *__restrict__ Pws,
+                                                                     const bf16_t *__restrict__ dSws,
+                                                                     TO *__restrict__ dK, TO *__restrict__ dV) {
+    using Lds = KvLds<D>;
+    constexpr int DB = D / 16, CPR = D / 8, LD = 32 * CPR / (KV_WAVES * 64) > 0 ? 32 * CPR / (KV_WAVES * 64) : 1;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
+    const int h = blockIdx.x, b = blockIdx.y;
+    const int kt = blockIdx.z * KV_WAVES + wave;          // this wave's block column
+    const size_t bh = (size_t)b * H + h;
+    const bf16_t *Qb = Q + bh * N * D, *Ob = dO + bh * N * D;
+    const size_t wso = bh * (size_t)chain_ds_block_off(causal != 0, n_rt, n_kt) * SC_BLK;
+    const int kt_c = min(kt, n_rt - 1);                   // (N keys and N rows: n_rt columns exist)
+    const bool own = kt < n_rt;
+    const size_t col = wso + (size_t)(chain_ds_block_off(causal != 0, n_rt, kt_c) - chain_ds_first_rt(causal != 0, kt_c)) * SC_BLK;
+    const int rt0 = causal ? blockIdx.z * KV_WAVES : 0;
+
+    f32x4 acc_v[2][DB], acc_k[2][DB];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) acc_v[kb][db] = acc_k[kb][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    u32x4 qr[LD], orr[LD], pr[2], sr[2];
+    auto load = [&](int rt) {
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+            const int c = (tid + i * KV_WAVES * 64) % (32 * CPR), row = min(rt * 32 + c / CPR, N - 1), cc = c % CPR;
+            qr[i] = *reinterpret_cast<const u32x4 *>(Qb + (size_t)row * D + cc * 8);
+            orr[i] = *reinterpret_cast<const u32x4 *>(Ob + (size_t)row * D + cc * 8);
+        }
+        // (columns start at row tile kt under the causal mask: an earlier one is not read)
+        const size_t o = col + (size_t)max(rt, causal ? kt_c : 0) * SC_BLK + lane * 8;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            pr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(Pws + o + i * 512));
+            sr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(dSws + o + i * 512));
+        }
+    };
+    load(rt0);
+    for (int rt = rt0; rt < n_rt; ++rt) {
+        unsigned char *buf = smem + ((rt - rt0) & 1) * Lds::buf;
+        unsigned char *Ql = buf, *Ol = buf + Lds::rows, *Pl = buf + 2 * Lds::rows + wave * 2 * SC_BLK * 2, *Sl = Pl + SC_BLK * 2;
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+            const int c = tid + i * KV_WAVES * 64, row = c / CPR, cc = c % CPR;
+            if (c < 32 * CPR) {
+                // (rows past the last: copies of the last one, which P = dS = 0 takes out)
+                const int o = ((row & 1) * 16 + (row >> 1)) * Lds::RST + cc * 16;
+                *reinterpret_cast<u32x4 *>(Ql + o) = qr[i];
+                *reinterpret_cast<u32x4 *>(Ol + o) = orr[i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            *reinterpret_cast<u32x4 *>(Pl + lane * 16 + i * 1024) = pr[i];
+            *reinterpret_cast<u32x4 *>(Sl + lane * 16 + i * 1024) = sr[i];
+        }
+        lds_barrier();
+        if (rt + 1 < n_rt) load(rt + 1);
+        if (!own || (causal && rt < kt)) continue;
+        bf16x8 pf[2], sf[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            // block element [parity][key half kb][pair][16 keys]: pairs 4g .. 4g+3 of both parities
+            const bf16x4 pl = lds_read_tr4x16(Pl + kb * 512, 32, 4 * g, 0, n), ph = lds_read_tr4x16(Pl + 1024 + kb * 512, 32, 4 * g, 0, n);
+            const bf16x4 sl = lds_read_tr4x16(Sl + kb * 512, 32, 4 * g, 0, n), sh = lds_read_tr4x16(Sl + 1024 + kb * 512, 32, 4 * g, 0, n);
+            pf[kb] = __builtin_shufflevector(pl, ph, 0, 1, 2, 3, 4, 5, 6, 7);
+            sf[kb] = __builtin_shufflevector(sl, sh, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            const bf16x4 ol = lds_read_tr4x16(Ol, Lds::RST, 4 * g, db * 16, n), oh = lds_read_tr4x16(Ol + 16 * Lds::RST, Lds::RST, 4 * g, db * 16, n);
+            const bf16x4 ql = lds_read_tr4x16(Ql, Lds::RST, 4 * g, db * 16, n), qh = lds_read_tr4x16(Ql + 16 * Lds::RST, Lds::RST, 4 * g, db * 16, n);
+            const bf16x8 of = __builtin_shufflevector(ol, oh, 0, 1, 2, 3, 4, 5, 6, 7), qf = __builtin_shufflevector(ql, qh, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                // rows of the product = head-dim columns, so that a lane holds four consecutive ones of a key
+                acc_v[kb][db] = mfma_bf16(of, pf[kb], acc_v[kb][db]);
+                acc_k[kb][db] = mfma_bf16(qf, sf[kb], acc_k[kb][db]);
+            }
+        }
+    }
+    if (!own) return;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+        const int key = kt * 32 + kb * 16 + n;
+        if (key >= N) continue;
+        const size_t o = (bh * N + key) * D + 4 * g;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            if constexpr (sizeof(TO) == 2) {
+                bf16x4 v, k;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) { v[r] = (bf16_t)acc_v[kb][db][r]; k[r] = (bf16_t)acc_k[kb][db][r]; }
+                *reinterpret_cast<bf16x4 *>(dV + o + 16 * db) = v;
+                *reinterpret_cast<bf16x4 *>(dK + o + 16 * db) = k;
+            } else {
+                *reinterpret_cast<f32x4 *>(dV + o + 16 * db) = acc_v[kb][db];
+                *reinterpret_cast<f32x4 *>(dK + o + 16 * db) = acc_k[kb][db];
+            }
+        }
+    }
+}
+
+// Key steps per score workgroup and the workgroups of a batch entry.
+struct ScorePlan { int steps_per_wg, n_wg; };
+ScorePlan score_plan(int B, int H, int N, int causal) {
+    const int R = H == 16 ? 32 : 16, KT = 512 / R, n_rt32 = (N + 31) / 32, n_tiles = n_rt32 * (32 / R);
+    const int all = n_rt32 * (32 / KT);
+    const long long steps = causal ? (long long)n_tiles * (all + 32 / KT) / 2 : (long long)n_tiles * all;
+    // four workgroups per CU level out the tail of the launch; fewer than eight steps do not pay for a workgroup's
+    // resident fragments while there are CUs for longer ones, more than 64 gain nothing
+    long long per = steps * B / (256 * 4);
+    const int unit = 32 / KT;   // whole blocks of 32 keys
+    const long long least = steps * B / 256 >= 8 ? 8 : 2;
+    per = per < least ? least : per > 64 ? 64 : per;
+    ScorePlan p;
+    p.steps_per_wg = (int)((per + unit - 1) / unit) * unit;
+    p.n_wg = 0;
+    for (int s0 = 0; s0 < all; s0 += p.steps_per_wg) p.n_wg += n_tiles - (causal ? (s0 * KT / 32) * (32 / R) : 0);
+    return p;
+}
+
+template <int H, int D>
+hipError_t launch_scores(const ScoreArgs &a, hipStream_t s) {
+    constexpr int lds = ScoreTile<H, D>::lds;
+    static_assert(lds <= 160 * 1024 && SC_WAVES * H * H * 4 <= lds, "LDS budget");
+    hipError_t e = set_max_lds_once<headmix_scores_kernel<H, D>>(lds);
+    if (e != hipSuccess) return e;
+    headmix_scores_kernel<H, D><<<dim3((a.n_wg + 7) / 8 * 8, a.B), SC_WAVES * 64, lds, s>>>(a);
+    return hipGetLastError();
+}
+
+template <int D, typename TO>
+hipError_t launch_dkdv(const Problem &p, const void *q, const void *d_o, const bf16_t *P, const bf16_t *dS, void *dk, void *dv,
+                       hipStream_t s) {
+    constexpr int lds = KvLds<D>::total;
+    hipError_t e = set_max_lds_once<headmix_dkdv_kernel<D, TO>>(lds);
+    if (e != hipSuccess) return e;
+    headmix_dkdv_kernel<D, TO><<<dim3(p.H, p.B, (p.Nk + 127) / 128), KV_WAVES * 64, lds, s>>>(
+        p.B, p.H, p.Nk, p.causal, chain_row_tiles(p), chain_key_tiles(p), (const bf16_t *)q, (const bf16_t *)d_o, P, dS, (TO *)dk, (TO *)dv);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+int headmix_score_wgs(int B, int H, int N, int causal) { return score_plan(B, H, N, causal).n_wg; }
+
+hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,
+                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, float *dw_part,
+                             void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
+    const ScorePlan plan = score_plan(p.B, p.H, p.Nq, p.causal);
+    const bool want_kv = dk != nullptr;
+    const ScoreArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), plan.steps_per_wg, plan.n_wg, p.scale,
+                      (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)d_o, w, lse, Dl,
+                      want_kv ? (bf16_t *)P : nullptr, (bf16_t *)dS, dq ? dw_part : nullptr};
+    hipError_t e = hipErrorInvalidValue;
+    if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, s) : p.d == 64 ? launch_scores<16, 64>(a, s) : launch_scores<16, 128>(a, s);
+    if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, s) : p.d == 64 ? launch_scores<32, 64>(a, s) : launch_scores<32, 128>(a, s);
+    if (e != hipSuccess) return e;
+    if (want_kv) {
+#define CALL(DD) (grad_dt == CONVATTN_BF16 ? launch_dkdv<DD, bf16_t>(p, q, d_o, a.P, a.dS, dk, dv, s) \
+                                           : launch_dkdv<DD, float>(p, q, d_o, a.P, a.dS, dk, dv, s))
+        e = p.d == 32 ? CALL(32) : p.d == 64 ? CALL(64) : CALL(128);
+#undef CALL
+        if (e != hipSuccess) return e;
+    }
+    if (dq) {
+        e = mfma_dq_from_rows(p, grad_dt, k, dS, nullptr, dq, s);
+        if (e != hipSuccess) return e;
+        headmix_dw_sum_kernel<<<p.H * p.H / 16, 256, 0, s>>>(p.B * plan.n_wg, p.H * p.H, dw_part, dw);
+        e = hipGetLastError();
+    }
+    return e;
+}
+
+}  // namespace convattn

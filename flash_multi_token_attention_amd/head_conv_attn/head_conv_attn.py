@@ -8,7 +8,7 @@ import torch
 import torch.nn as nn
 from torch.autograd import Function
 
-from .ops import bwd_dkdv, bwd_dq_dw, forward
+from .ops import backward, bwd_dkdv, bwd_dq_dw, forward
 
 
 class HeadConvAttentionFunction(Function):
@@ -26,6 +26,12 @@ class HeadConvAttentionFunction(Function):
     def backward(ctx, grad_output):
         q, k, v, w, output, l, m = ctx.saved_tensors
         grad_q = grad_k = grad_v = grad_w = None
+        need_q, need_k, need_v, need_w = ctx.needs_input_grad[:4]
+        if (need_q or need_w) and (need_k or need_v):
+            lo = torch.bfloat16 if q.dtype == k.dtype == v.dtype == torch.bfloat16 else torch.float32
+            grad_q, grad_k, grad_v, grad_w = backward(q, k, v, w, output, grad_output, l, m, causal=ctx.causal,
+                                                      scale=ctx.scale, out_dtype=lo)
+            return (grad_q.to(q.dtype), grad_k.to(k.dtype), grad_v.to(v.dtype), grad_w.to(w.dtype), None, None)
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[3]:
             grad_q, grad_w = bwd_dq_dw(q, k, v, w, output, grad_output, l, m, causal=ctx.causal, scale=ctx.scale)
             grad_q, grad_w = grad_q.to(q.dtype), grad_w.to(w.dtype)

@@ -17,6 +17,7 @@ from typing import Optional, Tuple
 import torch
 
 from .. import _lib
+from ..conv_attn.ops import max_workspace_bytes
 
 
 def _ptr(t: torch.Tensor):
@@ -69,7 +70,11 @@ def forward(q, k, v, w, scale: float = 1.0, causal: bool = False) -> Tuple[torch
     return (o if out_dtype == q.dtype else o.to(q.dtype)), l, m
 
 
-def _backward(entry: str, q, k, v, w, o, do, l, m, causal: bool, scale: Optional[float]):
+def _backward(want_q: bool, want_kv: bool, q, k, v, w, o, do, l, m, causal: bool, scale: Optional[float],
+              grad_dtype: torch.dtype = torch.float32):
+    """(dQ, dW, dK, dV), None for those not wanted.  One pass over the scores with the probabilities and dS in the
+    workspace (bf16); above the workspace cap, or when the allocation fails, the kernels with O(N) scratch run instead
+    (fp32 gradients, converted here)."""
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
     qb, kb, vb, gb = _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v"), _bf16(do, "do")
@@ -79,27 +84,47 @@ def _backward(entry: str, q, k, v, w, o, do, l, m, causal: bool, scale: Optional
     desc = _desc(qb, wf, scale, causal, out_dtype)
     lf, mf = l.to(torch.float32).contiguous(), m.to(torch.float32).contiguous()
     lib = _lib.load()
-    ws = torch.empty(lib.convattn_headmix_bwd_workspace_bytes(C.byref(desc)), dtype=torch.uint8, device=q.device)
     B, H, N, d = qb.shape
-    if entry == "dq_dw":
-        g0 = torch.empty(B, H, N, d, dtype=torch.float32, device=q.device)
-        g1 = torch.empty(H, H, dtype=torch.float32, device=q.device)
-        fn = lib.convattn_headmix_bwd_dq_dw
-    else:
-        g0 = torch.empty(B, H, N, d, dtype=torch.float32, device=q.device)
-        g1 = torch.empty_like(g0)
-        fn = lib.convattn_headmix_bwd_dkdv
-    rc = fn(C.byref(desc), _ptr(qb), _ptr(kb), _ptr(vb), _ptr(wf), _ptr(ob), _ptr(gb), _ptr(lf), _ptr(mf), _ptr(ws),
-            _ptr(g0), _ptr(g1), _stream(q))
-    _lib.check(rc, "head_conv_attention_bwd_" + entry)
-    return g0, g1
+    ins = [_ptr(t) for t in (qb, kb, vb, wf, ob, gb, lf, mf)]
+    ws = None
+    nbytes = lib.convattn_headmix_bwd_fused_workspace_bytes(C.byref(desc))
+    if nbytes <= max_workspace_bytes():
+        try:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:
+            pass
+    gt = grad_dtype if ws is not None else torch.float32
+    dq = torch.empty(B, H, N, d, dtype=gt, device=q.device) if want_q else None
+    dw = torch.empty(H, H, dtype=torch.float32, device=q.device) if want_q else None
+    dk, dv = (torch.empty(B, H, N, d, dtype=gt, device=q.device) if want_kv else None for _ in range(2))
+    if ws is not None:
+        rc = lib.convattn_headmix_bwd_fused(C.byref(desc), _lib.BF16 if gt == torch.bfloat16 else _lib.F32, *ins, _ptr(ws),
+                                            *[_ptr(t) if t is not None else None for t in (dq, dk, dv, dw)], _stream(q))
+        _lib.check(rc, "head_conv_attention_bwd")
+        return dq, dw, dk, dv
+    ws = torch.empty(lib.convattn_headmix_bwd_workspace_bytes(C.byref(desc)), dtype=torch.uint8, device=q.device)
+    if want_q:
+        rc = lib.convattn_headmix_bwd_dq_dw(C.byref(desc), *ins, _ptr(ws), _ptr(dq), _ptr(dw), _stream(q))
+        _lib.check(rc, "head_conv_attention_bwd_dq_dw")
+    if want_kv:
+        rc = lib.convattn_headmix_bwd_dkdv(C.byref(desc), *ins, _ptr(ws), _ptr(dk), _ptr(dv), _stream(q))
+        _lib.check(rc, "head_conv_attention_bwd_dkdv")
+    return (None if dq is None else dq.to(grad_dtype)), dw, *(None if t is None else t.to(grad_dtype) for t in (dk, dv))
 
 
 def bwd_dq_dw(q, k, v, w, o, do, l, m, causal: bool = False, scale: Optional[float] = None):
     """(dQ [B,H,N,d], dW [H,H]), float32."""
-    return _backward("dq_dw", q, k, v, w, o, do, l, m, causal, scale)
+    return _backward(True, False, q, k, v, w, o, do, l, m, causal, scale)[:2]
 
 
 def bwd_dkdv(q, k, v, w, o, do, l, m, causal: bool = False, scale: Optional[float] = None):
     """(dK, dV) [B,H,N,d], float32."""
-    return _backward("dkdv", q, k, v, w, o, do, l, m, causal, scale)
+    return _backward(False, True, q, k, v, w, o, do, l, m, causal, scale)[2:]
+
+
+def backward(q, k, v, w, o, do, l, m, causal: bool = False, scale: Optional[float] = None,
+             out_dtype: torch.dtype = torch.float32):
+    """(dQ, dK, dV [B,H,N,d] in ``out_dtype``, bfloat16 or float32, dW [H,H] float32) from one pass: the results of
+    ``bwd_dq_dw`` and ``bwd_dkdv``."""
+    dq, dw, dk, dv = _backward(True, True, q, k, v, w, o, do, l, m, causal, scale, out_dtype)
+    return dq, dk, dv, dw

@@ -335,6 +335,17 @@ int convattn_headmix_bwd_dkdv(const convattn_headmix_desc *desc, const void *q, 
                               const float *w, const void *o, const void *d_o, const float *l, const float *m,
                               void *workspace, float *dk, float *dv, void *stream);
 
+/*
+ * All gradients from one pass over the scores: what the two entry points above compute, without computing the
+ * scores and the head mix twice.  grad_dtype: CONVATTN_BF16 or CONVATTN_F32, of dq, dk and dv (dw is fp32).
+ * dq and dw, or dk and dv, may be null together: then only the others are computed.  The workspace holds
+ * the probabilities and dS as bf16 (4 B H N^2 bytes, causal: half of it); the two entry points above need O(N).
+ */
+size_t convattn_headmix_bwd_fused_workspace_bytes(const convattn_headmix_desc *desc);
+int convattn_headmix_bwd_fused(const convattn_headmix_desc *desc, int grad_dtype, const void *q, const void *k,
+                               const void *v, const float *w, const void *o, const void *d_o, const float *l,
+                               const float *m, void *workspace, void *dq, void *dk, void *dv, float *dw, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
