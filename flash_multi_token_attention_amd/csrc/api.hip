@@ -496,9 +496,9 @@ int convattn_headmix_bwd_dkdv(const convattn_headmix_desc *desc, const void *q, 
                                  dk, dv, s);
 }
 
-// Scratch of the one-pass backward: D, LSE, dw partials, then the dS and the P blocks.
+// Scratch of the one-pass backward: D, LSE, dw partials, K and V in fragment order, the dS and the P blocks.
 struct HeadmixFusedWs {
-    size_t lse_off, part_off, ds_off, p_off, total;
+    size_t lse_off, part_off, kv_off, ds_off, p_off, total;
 };
 static Problem headmix_problem(const convattn_headmix_desc *d) {
     Problem p{};
@@ -512,7 +512,8 @@ static HeadmixFusedWs headmix_fused_ws(const convattn_headmix_desc *d) {
     HeadmixFusedWs w;
     w.lse_off = stat;
     w.part_off = 2 * stat;
-    w.ds_off = w.part_off + align256((size_t)d->B * headmix_score_wgs(d->B, d->H, d->N, p.causal) * d->H * d->H * sizeof(float));
+    w.kv_off = w.part_off + align256((size_t)d->B * headmix_score_wgs(d->B, d->H, d->N, p.causal) * d->H * d->H * sizeof(float));
+    w.ds_off = w.kv_off + 2 * align256(headmix_frag_bytes(p));
     w.p_off = w.ds_off + ds;
     w.total = w.p_off + ds;
     return w;
@@ -539,7 +540,7 @@ int convattn_headmix_bwd_fused(const convattn_headmix_desc *desc, int grad_dtype
     float *Dl = reinterpret_cast<float *>(base), *lse = reinterpret_cast<float *>(base + ws.lse_off);
     rc = (int)bwd_preprocess(p, desc->in_dtype, desc->out_dtype, o, d_o, m, l, Dl, lse, s);
     if (rc) return rc;
-    return (int)headmix_bwd_fused(p, grad_dtype, q, k, v, w, d_o, lse, Dl, base + ws.p_off, base + ws.ds_off,
+    return (int)headmix_bwd_fused(p, grad_dtype, q, k, v, w, d_o, lse, Dl, base + ws.p_off, base + ws.ds_off, base + ws.kv_off,
                                   reinterpret_cast<float *>(base + ws.part_off), dq, dk, dv, dw, s);
 }
 

@@ -32,7 +32,7 @@ template <int D, typename TO>
 __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_t *__restrict__ K,
                                                           const bf16_t *__restrict__ dS_ws,
                                                           const float *__restrict__ dc_scale, int n_kt,
-                                                          int n_rt, TO *__restrict__ dQ) {
+                                                          int n_rt, int heads_inner, TO *__restrict__ dQ) {
     using Lds = RowsLds<D>;
     constexpr int RST = Lds::RST;
     constexpr int DB = D / 16, CPR = D / 8;
@@ -49,7 +49,9 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
     const bool causal = p.causal != 0;
     const size_t bh = (size_t)b * p.H + h;
     const bf16_t *Kb = K + bh * p.Nk * D;
-    const bf16_t *ws = dS_ws + bh * (size_t)chain_ds_block_off(causal, n_rt, n_kt) * BLK;
+    const size_t n_blk = (size_t)chain_ds_block_off(causal, n_rt, n_kt);
+    const bf16_t *ws = dS_ws + (heads_inner ? b * n_blk * p.H + h : bh * n_blk) * BLK;
+    const int blk_step = heads_inner ? p.H * BLK : BLK;   // elements from block to block
 
     f32x4 acc[2][DB];
 #pragma unroll
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
                 // Raw: blocks that do not exist are cleared where the registers are used (a select here
                 // would wait for the load within this step)
                 sr[kp][ob] = __builtin_nontemporal_load(
-                    reinterpret_cast<const u32x4 *>(ws + blk * BLK + ((ob * 2 + (g >> 1)) * 16 + n) * 16 + 8 * (g & 1)));
+                    reinterpret_cast<const u32x4 *>(ws + blk * blk_step + ((ob * 2 + (g >> 1)) * 16 + n) * 16 + 8 * (g & 1)));
             }
         }
     };
@@ -156,29 +158,29 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
 
 template <int D, typename TO>
 hipError_t launch(const Problem &p, const void *k, const void *ds_ws, const float *dc_scale, void *dq,
-                  hipStream_t s) {
+                  hipStream_t s, int heads_inner) {
     auto kern = dq_rows_kernel<D, TO>;
     constexpr int lds = RowsLds<D>::total;
     dim3 grid(p.H, p.B, (p.Nq + BQ - 1) / BQ);
     kern<<<grid, NW * 64, lds, s>>>(p, (const bf16_t *)k, (const bf16_t *)ds_ws, dc_scale, chain_key_tiles(p),
-                                    chain_row_tiles(p), (TO *)dq);
+                                    chain_row_tiles(p), heads_inner, (TO *)dq);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t mfma_dq_from_rows(const Problem &p, int out_dt, const void *k, const void *ds_ws, const float *dc_scale,
-                           void *dq, hipStream_t s) {
+                           void *dq, hipStream_t s, bool heads_inner) {
     if (p.d == 128) {
-        if (out_dt == CONVATTN_BF16) return launch<128, bf16_t>(p, k, ds_ws, dc_scale, dq, s);
-        return launch<128, float>(p, k, ds_ws, dc_scale, dq, s);
+        if (out_dt == CONVATTN_BF16) return launch<128, bf16_t>(p, k, ds_ws, dc_scale, dq, s, heads_inner);
+        return launch<128, float>(p, k, ds_ws, dc_scale, dq, s, heads_inner);
     }
     if (p.d == 32) {
-        if (out_dt == CONVATTN_BF16) return launch<32, bf16_t>(p, k, ds_ws, dc_scale, dq, s);
-        return launch<32, float>(p, k, ds_ws, dc_scale, dq, s);
+        if (out_dt == CONVATTN_BF16) return launch<32, bf16_t>(p, k, ds_ws, dc_scale, dq, s, heads_inner);
+        return launch<32, float>(p, k, ds_ws, dc_scale, dq, s, heads_inner);
     }
-    if (out_dt == CONVATTN_BF16) return launch<64, bf16_t>(p, k, ds_ws, dc_scale, dq, s);
-    return launch<64, float>(p, k, ds_ws, dc_scale, dq, s);
+    if (out_dt == CONVATTN_BF16) return launch<64, bf16_t>(p, k, ds_ws, dc_scale, dq, s, heads_inner);
+    return launch<64, float>(p, k, ds_ws, dc_scale, dq, s, heads_inner);
 }
 
 }  // namespace convattn

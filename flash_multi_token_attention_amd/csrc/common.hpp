@@ -87,9 +87,10 @@ hipError_t headmix_bwd_dkdv(int B, int H, int N, int d, float scale, int causal,
                             float *dv, hipStream_t s);
 int headmix_row_tiles(int N);
 // one pass for all gradients (headmix_bwd.hip); p: B, H, Nq = Nk = N, d, scale, causal.  dk / dv or dq / dw may be null.
+size_t headmix_frag_bytes(const Problem &p);              // kv_frag holds two of these
 int headmix_score_wgs(int B, int H, int N, int causal);   // dw partials per batch entry
 hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,
-                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, float *dw_part,
+                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, void *kv_frag, float *dw_part,
                              void *dq, void *dk, void *dv, float *dw, hipStream_t s);
 
 }  // namespace convattn

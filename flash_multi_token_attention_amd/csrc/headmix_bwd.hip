@@ -38,8 +38,13 @@ template <int H, int D> struct ScoreTile {
     static constexpr int arr = H * HS;                      // floats of one array
     static constexpr int NBUF = H == 16 ? 2 : 1;
     static constexpr int HPW = H / SC_WAVES, HB = H / 16;
+    static constexpr bool STATS_LDS = H * D >= 2048;          // LSE and D of the tile rows: registers are short
     static constexpr int WST = H + 4;                       // floats per row of w in LDS
-    static constexpr int w_off = NBUF * 2 * arr, wt_off = w_off + H * WST, lds = (wt_off + H * WST) * 4;
+    static constexpr int w_off = NBUF * 2 * arr, wt_off = w_off + H * WST, 
+                         st_off = wt_off + H * WST,       // LSE and D of the tile's rows (32 heads: not in registers)
+                         lds = (st_off + (STATS_LDS ? 2 * R * WST : 0)) * 4;
+    // chunks of K and V rows in flight during the mixing phase, as far as the registers go
+    static constexpr int AHEAD = H == 32 && D == 128 ? 1 : 2;
     // Four keys 4q .. 4q+3 of tile row `lr` sit at float lr * KT + 4 * slot: the XOR spreads both the score
     // phase's writes (16 rows, one quad) and the mixing phase's reads (RW rows, all quads) over all banks.
     __device__ static __forceinline__ int slot(int lr, int q) { return q ^ ((lr >> SWZ) & (NQ - 1)); }
@@ -49,10 +54,29 @@ template <int H, int D> struct ScoreTile {
     }
 };
 
+// K and V of a launch in the order in which the score kernel's lanes read them: [batch, head][16 keys][k step][lane][8]
+// (lane 16g + n: key n, columns 32 ks + 8g ..), zeros past the last key.  Read straight from the rows, every
+// fragment load touches 16 rows with neighbouring lanes in different rows: 64 cache accesses per load instead of
+// 16, and the score kernel was bound by them (3.3 M of its 4.1 M clocks per CU at B4 H16 N4096 d128).  One copy of K and V
+// (0.06 ms there) is read N / 32 times.
+template <int D>
+__global__ __launch_bounds__(256) void headmix_frag_order_kernel(int N, int n_t16, const bf16_t *__restrict__ K,
+                                                                 const bf16_t *__restrict__ V, bf16_t *__restrict__ KF,
+                                                                 bf16_t *__restrict__ VF, size_t n_frag) {
+    const size_t f = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // one 1 KB fragment per wave
+    if (f >= n_frag) return;
+    constexpr int KS = D / 32;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const size_t bh = f / ((size_t)n_t16 * KS);
+    const int r = (int)(f - bh * n_t16 * KS), row = (r / KS) * 16 + n, col = (r % KS) * 32 + 8 * g;
+    *reinterpret_cast<u32x4 *>(KF + f * 512 + lane * 8) = load_row16<D>(K + bh * N * D, row, N, col);
+    *reinterpret_cast<u32x4 *>(VF + f * 512 + lane * 8) = load_row16<D>(V + bh * N * D, row, N, col);
+}
+
 struct ScoreArgs {
     int B, N, causal, n_rt32, n_kt, steps_per_wg, n_wg;
     float scale;
-    const bf16_t *Q, *K, *V, *dO;
+    const bf16_t *Q, *KF, *VF, *dO;   // KF, VF: fragment order
     const float *W, *lse, *Dl;
     bf16_t *P, *dS;      // blocks; P may be null (dQ and dW only)
     float *dw_part;      // [B][n_wg][H][H], or null
@@ -98,33 +122,63 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
     const size_t bo = (size_t)b * H * N * D;
     const int h0 = wave * HPW;
 
-    // ---- resident: Q and dO fragments of this wave's heads ----
+    // ---- resident: Q and dO fragments of this wave's heads (rows loaded whole, turned in the wave's share of the LDS) ----
     bf16x8 qf[HPW][RB][KS], of[HPW][RB][KS];
+    {
+        constexpr int CPR = D / 8, RST = D * 2 + 16, LD = R * CPR / 64;
+        static_assert(R * RST <= T::arr * 4 * 2 * T::NBUF / SC_WAVES, "room for one head's rows");
+        unsigned char *st = smem + wave * (T::arr * 4 * 2 * T::NBUF / SC_WAVES / 16 * 16);
+        auto turn = [&](const bf16_t *src, bf16x8 (&f)[RB][KS]) {
+            u32x4 raw[LD];
 #pragma unroll
-    for (int t = 0; t < HPW; ++t)
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const int row = min(T::row(i0, rb * 16 + n), N - 1);
-            const size_t o = bo + ((size_t)(h0 + t) * N + row) * D + 8 * g;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                qf[t][rb][ks] = *reinterpret_cast<const bf16x8 *>(a.Q + o + 32 * ks);
-                of[t][rb][ks] = *reinterpret_cast<const bf16x8 *>(a.dO + o + 32 * ks);
+            for (int i = 0; i < LD; ++i) {
+                const int c = lane + i * 64;
+                raw[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)min(i0 + c / CPR, N - 1) * D + (c % CPR) * 8);
             }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < LD; ++i) {
+                const int c = lane + i * 64;
+                *reinterpret_cast<u32x4 *>(st + (c / CPR) * RST + (c % CPR) * 16) = raw[i];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    f[rb][ks] = *reinterpret_cast<const bf16x8 *>(st + (T::row(0, rb * 16 + n)) * RST + ks * 64 + g * 16);
+        };
+#pragma unroll
+        for (int t = 0; t < HPW; ++t) {
+            turn(a.Q + bo + (size_t)(h0 + t) * N * D, qf[t]);
+            turn(a.dO + bo + (size_t)(h0 + t) * N * D, of[t]);
         }
+        lds_barrier();   // the score tiles go where the other waves' rows are
+    }
     // ---- the mixing phase: lane (g, n) = heads 4g .. 4g+3 of each block of 16, tile row lr, keys 4q .. 4q+3 ----
     const int lr = wave * RW + (n & (RW - 1)), q4 = n / RW;
     const int row = T::row(i0, lr);
-    float lse2[HB][4], dl[HB][4];
-#pragma unroll
-    for (int hb = 0; hb < HB; ++hb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const size_t o = ((size_t)b * H + 16 * hb + 4 * g + r) * N + min(row, N - 1);
-            // (rows past the last: P = exp2(-1e30) = 0, so nothing of them is in dS, dV, dK or dw)
-            lse2[hb][r] = row < N ? a.lse[o] * kLog2e : 1e30f;
-            dl[hb][r] = a.Dl[o];
+    // (rows past the last: P = exp2(-1e30) = 0, so nothing of them is in dS, dV, dK or dw)
+    float *st_l = lds + T::st_off;
+    f32x4 lse_r[HB], dl_r[HB];
+    if constexpr (T::STATS_LDS) {
+        for (int i = tid; i < R * H; i += SC_WAVES * 64) {
+            const int hh = i / R, lr2 = i % R, rr = T::row(i0, lr2);
+            const size_t o = ((size_t)b * H + hh) * N + min(rr, N - 1);
+            st_l[lr2 * T::WST + hh] = rr < N ? a.lse[o] * kLog2e : 1e30f;
+            st_l[(R + lr2) * T::WST + hh] = a.Dl[o];
         }
+    } else {
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const size_t o = ((size_t)b * H + 16 * hb + 4 * g + r) * N + min(row, N - 1);
+                lse_r[hb][r] = row < N ? a.lse[o] * kLog2e : 1e30f;
+                dl_r[hb][r] = a.Dl[o];
+            }
+    }
     // w of the mix and its transpose, with the scales of the two products, in LDS (read as four k steps at a time:
     // k slot g of step s is head 4g + s)
     for (int i = tid; i < H * H; i += SC_WAVES * 64) {
@@ -141,14 +195,15 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
 
     // ---- score phase, in chunks of one head and 16 keys whose K and V rows are loaded two chunks ahead ----
     bf16x8 kf[2][KS], vf[2][KS];
+    const int n_t16 = a.n_rt32 * 2;
     auto load_chunk = [&](int buf, int step, int c) {
         const int t = c / KB, kb = c % KB;
-        const int key = min(step * KT + kb * 16 + n, N - 1);
-        const size_t o = bo + ((size_t)(h0 + t) * N + key) * D + 8 * g;
+        const size_t o = (((size_t)b * H + h0 + t) * n_t16 + step * KB + kb) * KS * 512;
+        const bf16_t *kp = a.KF + o, *vp = a.VF + o;   // (the same in all lanes)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            kf[buf][ks] = *reinterpret_cast<const bf16x8 *>(a.K + o + 32 * ks);
-            vf[buf][ks] = *reinterpret_cast<const bf16x8 *>(a.V + o + 32 * ks);
+            kf[buf][ks] = *reinterpret_cast<const bf16x8 *>(kp + lane * 8 + ks * 512);
+            vf[buf][ks] = *reinterpret_cast<const bf16x8 *>(vp + lane * 8 + ks * 512);
         }
     };
     auto score_chunk = [&](float *S, int buf, int c) {
@@ -196,11 +251,18 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
         }
         const int kt = j0 / 32;
         const long long blk = chain_ds_block_off(a.causal != 0, a.n_rt32, kt) + i0 / 32 - chain_ds_first_rt(a.causal != 0, kt);
-        const long long per_head = chain_ds_block_off(a.causal != 0, a.n_rt32, a.n_kt);
-        const size_t out = ((size_t)b * H * per_head + blk) * SC_BLK +
-                           (((brow & 1) * 2 + ((j0 + 4 * q4) >> 4 & 1)) * 16 + (brow >> 1)) * 16 + ((4 * q4) & 15);
+        // blocks of all heads side by side: [batch][block][head][1024]
+        const long long n_blk = chain_ds_block_off(a.causal != 0, a.n_rt32, a.n_kt);
+        const size_t first = ((size_t)b * n_blk + blk) * H * SC_BLK;
+        bf16_t *p_out = a.P + first, *ds_out = a.dS + first;
+        const int out = (((brow & 1) * 2 + ((j0 + 4 * q4) >> 4 & 1)) * 16 + (brow >> 1)) * 16 + ((4 * q4) & 15) + 4 * g * SC_BLK;
 #pragma unroll
         for (int x = 0; x < HB; ++x) {
+            f32x4 lse2 = lse_r[x], dl = dl_r[x];
+            if constexpr (T::STATS_LDS) {
+                lse2 = *reinterpret_cast<const f32x4 *>(st_l + lr * T::WST + 16 * x + 4 * g);
+                dl = *reinterpret_cast<const f32x4 *>(st_l + (R + lr) * T::WST + 16 * x + 4 * g);
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float *dz = dP + (16 * x + 4 * g + r) * HS + pos;
@@ -208,19 +270,19 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
                 bf16x4 pb;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    float p = fast_exp2(z[x][t][r] - lse2[x][r]);
+                    float p = fast_exp2(z[x][t][r] - lse2[r]);
                     if constexpr (masked) {
                         const int key = j0 + 4 * q4 + t;
                         if (key >= N || (a.causal && key > row)) p = 0.f;
                     }
                     pb[t] = (bf16_t)p;
-                    d[t] = p * (d[t] - dl[x][r]);
+                    d[t] = p * (d[t] - dl[r]);
                     z[x][t][r] = d[t];
                 }
                 *reinterpret_cast<f32x4 *>(dz) = d;
                 if (a.P)
                     __builtin_nontemporal_store(__builtin_bit_cast(u32x2, pb), reinterpret_cast<u32x2 *>(
-                        a.P + out + (size_t)(16 * x + 4 * g + r) * per_head * SC_BLK));
+                        p_out + out + (16 * x + r) * SC_BLK));
             }
         }
 #pragma unroll
@@ -242,7 +304,7 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
 #pragma unroll
                 for (int t = 0; t < 4; ++t) db[t] = (bf16_t)ds[t][r];
                 __builtin_nontemporal_store(__builtin_bit_cast(u32x2, db), reinterpret_cast<u32x2 *>(
-                    a.dS + out + (size_t)(16 * x + 4 * g + r) * per_head * SC_BLK));
+                    ds_out + out + (16 * x + r) * SC_BLK));
             }
         }
         // dw += dZ S^T over the wave's own 64 pairs: lane n = head of either operand
@@ -273,7 +335,7 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
     };
 
     load_chunk(0, s0, 0);
-    if constexpr (NCH > 1) load_chunk(1, s0, 1);
+    if constexpr (T::AHEAD == 2) load_chunk(1, s0, 1);
     if constexpr (T::NBUF == 2) {
         static_assert(NCH == 2, "two chunks per step");
         score_chunk(lds, 0, 0);
@@ -300,10 +362,16 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
         for (int u = s0; u < s_end; ++u) {
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
-                score_chunk(lds, c & 1, c);
-                if (c + 2 < NCH) load_chunk(c & 1, u, c + 2);
-                else load_chunk(c & 1, min(u + 1, s_end - 1), c + 2 - NCH);
+                if constexpr (T::AHEAD == 1) {
+                    if (c + 1 < NCH) load_chunk((c + 1) & 1, u, c + 1);
+                    score_chunk(lds, c & 1, c);
+                } else {
+                    score_chunk(lds, c & 1, c);
+                    if (c + 2 < NCH) load_chunk(c & 1, u, c + 2);
+                    else load_chunk(c & 1, min(u + 1, s_end - 1), c + 2 - NCH);
+                }
             }
+            if constexpr (T::AHEAD == 1) load_chunk(0, min(u + 1, s_end - 1), 0);
             lds_barrier();
             mix(lds, u);
             lds_barrier();
@@ -386,10 +454,10 @@ __global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, i
     const int kt = blockIdx.z * KV_WAVES + wave;          // this wave's block column
     const size_t bh = (size_t)b * H + h;
     const bf16_t *Qb = Q + bh * N * D, *Ob = dO + bh * N * D;
-    const size_t wso = bh * (size_t)chain_ds_block_off(causal != 0, n_rt, n_kt) * SC_BLK;
+    const size_t wso = (size_t)b * chain_ds_block_off(causal != 0, n_rt, n_kt) * H + h;   // blocks lie [batch][block][head]
     const int kt_c = min(kt, n_rt - 1);                   // (N keys and N rows: n_rt columns exist)
     const bool own = kt < n_rt;
-    const size_t col = wso + (size_t)(chain_ds_block_off(causal != 0, n_rt, kt_c) - chain_ds_first_rt(causal != 0, kt_c)) * SC_BLK;
+    const size_t col = wso + (chain_ds_block_off(causal != 0, n_rt, kt_c) - chain_ds_first_rt(causal != 0, kt_c)) * H;
     const int rt0 = causal ? blockIdx.z * KV_WAVES : 0;
 
     f32x4 acc_v[2][DB], acc_k[2][DB];
@@ -407,7 +475,7 @@ __global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, i
             orr[i] = *reinterpret_cast<const u32x4 *>(Ob + (size_t)row * D + cc * 8);
         }
         // (columns start at row tile kt under the causal mask: an earlier one is not read)
-        const size_t o = col + (size_t)max(rt, causal ? kt_c : 0) * SC_BLK + lane * 8;
+        const size_t o = (col + (size_t)max(rt, causal ? kt_c : 0) * H) * SC_BLK + lane * 8;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             pr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(Pws + o + i * 512));
@@ -500,7 +568,10 @@ ScorePlan score_plan(int B, int H, int N, int causal) {
 }
 
 template <int H, int D>
-hipError_t launch_scores(const ScoreArgs &a, hipStream_t s) {
+hipError_t launch_scores(const ScoreArgs &a, const void *k, const void *v, hipStream_t s) {
+    const size_t n_frag = (size_t)a.B * H * a.n_rt32 * 2 * (D / 32);
+    headmix_frag_order_kernel<D><<<(unsigned)((n_frag + 3) / 4), 256, 0, s>>>(a.N, a.n_rt32 * 2, (const bf16_t *)k, (const bf16_t *)v,
+                                                                            (bf16_t *)a.KF, (bf16_t *)a.VF, n_frag);
     constexpr int lds = ScoreTile<H, D>::lds;
     static_assert(lds <= 160 * 1024 && SC_WAVES * H * H * 4 <= lds, "LDS budget");
     hipError_t e = set_max_lds_once<headmix_scores_kernel<H, D>>(lds);
@@ -522,19 +593,21 @@ hipError_t launch_dkdv(const Problem &p, const void *q, const void *d_o, const b
 
 }  // namespace
 
+// K (or V) in fragment order
+size_t headmix_frag_bytes(const Problem &p) { return (size_t)p.B * p.H * chain_row_tiles(p) * 32 * p.d * 2; }
 int headmix_score_wgs(int B, int H, int N, int causal) { return score_plan(B, H, N, causal).n_wg; }
 
 hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,
-                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, float *dw_part,
+                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, void *kv_frag, float *dw_part,
                              void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
     const ScorePlan plan = score_plan(p.B, p.H, p.Nq, p.causal);
     const bool want_kv = dk != nullptr;
     const ScoreArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), plan.steps_per_wg, plan.n_wg, p.scale,
-                      (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)d_o, w, lse, Dl,
+                      (const bf16_t *)q, (const bf16_t *)kv_frag, (const bf16_t *)kv_frag + headmix_frag_bytes(p) / 2, (const bf16_t *)d_o, w, lse, Dl,
                       want_kv ? (bf16_t *)P : nullptr, (bf16_t *)dS, dq ? dw_part : nullptr};
     hipError_t e = hipErrorInvalidValue;
-    if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, s) : p.d == 64 ? launch_scores<16, 64>(a, s) : launch_scores<16, 128>(a, s);
-    if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, s) : p.d == 64 ? launch_scores<32, 64>(a, s) : launch_scores<32, 128>(a, s);
+    if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, k, v, s) : p.d == 64 ? launch_scores<16, 64>(a, k, v, s) : launch_scores<16, 128>(a, k, v, s);
+    if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, k, v, s) : p.d == 64 ? launch_scores<32, 64>(a, k, v, s) : launch_scores<32, 128>(a, k, v, s);
     if (e != hipSuccess) return e;
     if (want_kv) {
 #define CALL(DD) (grad_dt == CONVATTN_BF16 ? launch_dkdv<DD, bf16_t>(p, q, d_o, a.P, a.dS, dk, dv, s) \
@@ -544,7 +617,7 @@ hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const
         if (e != hipSuccess) return e;
     }
     if (dq) {
-        e = mfma_dq_from_rows(p, grad_dt, k, dS, nullptr, dq, s);
+        e = mfma_dq_from_rows(p, grad_dt, k, dS, nullptr, dq, s, true);
         if (e != hipSuccess) return e;
         headmix_dw_sum_kernel<<<p.H * p.H / 16, 256, 0, s>>>(p.B * plan.n_wg, p.H * p.H, dw_part, dw);
         e = hipGetLastError();

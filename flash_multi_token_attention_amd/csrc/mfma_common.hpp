@@ -294,8 +294,9 @@ inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const v
     if (want == 2) return mfma_bwd_chain_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
     return mfma_bwd_chain_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
 }
+// heads_inner: the blocks lie [batch][block][head] (all heads of a block side by side) instead of [batch, head][block]
 hipError_t mfma_dq_from_rows(const Problem &p, int out_dt, const void *k, const void *ds_ws,
-                             const float *dc_scale, void *dq, hipStream_t s);
+                             const float *dc_scale, void *dq, hipStream_t s, bool heads_inner = false);
 
 // ---- decode as an HBM stream (decode_stream.hip) ----
 bool decode_stream_ok(const Problem &p, int in_dt, unsigned flags);
