@@ -76,6 +76,8 @@ _SIGNATURES = {
     "convattn_decode_noalloc": (C.c_int, [_D] + [_P] * 4 + [C.c_longlong] * 2 + [_P] * 4),
     "convattn_headmix_validate": (C.c_int, [_HD]),
     "convattn_headmix_fwd": (C.c_int, [_HD] + [_P] * 8),
+    "convattn_headmix_fwd_workspace_bytes": (C.c_size_t, [_HD]),
+    "convattn_headmix_fwd_ws": (C.c_int, [_HD] + [_P] * 9),
     "convattn_headmix_bwd_workspace_bytes": (C.c_size_t, [_HD]),
     "convattn_headmix_bwd_dq_dw": (C.c_int, [_HD] + [_P] * 12),
     "convattn_headmix_bwd_dkdv": (C.c_int, [_HD] + [_P] * 12),

@@ -42,7 +42,8 @@ UNITS = [
     ("bwd_dq_rows.hip", "bwd_dq_rows", []),
     ("decode_stream.hip", "decode_stream", []),
     ("headmix_attn.hip", "headmix_attn", []),
-    ("headmix_bwd.hip", "headmix_bwd", []),
+    ("headmix_probs.hip", "headmix_probs", []),
+    ("headmix_scores.hip", "headmix_scores", []),
 ]
 SOURCES = sorted({u[0] for u in UNITS})
 

@@ -519,6 +519,20 @@ static HeadmixFusedWs headmix_fused_ws(const convattn_headmix_desc *d) {
     return w;
 }
 
+size_t convattn_headmix_fwd_workspace_bytes(const convattn_headmix_desc *desc) {
+    return headmix_check(desc) ? 0 : headmix_fwd_workspace(headmix_problem(desc));
+}
+
+int convattn_headmix_fwd_ws(const convattn_headmix_desc *desc, const void *q, const void *k, const void *v,
+                            const float *w, void *workspace, void *o, float *l, float *m, void *stream) {
+    int rc = headmix_check(desc);
+    if (rc) return rc;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(w); REQUIRE_PTR(workspace);
+    REQUIRE_PTR(o); REQUIRE_PTR(l); REQUIRE_PTR(m);
+    return (int)headmix_fwd_blocks(headmix_problem(desc), desc->out_dtype, q, k, v, w, workspace, o, l, m,
+                                    static_cast<hipStream_t>(stream));
+}
+
 size_t convattn_headmix_bwd_fused_workspace_bytes(const convattn_headmix_desc *desc) {
     return headmix_check(desc) ? 0 : headmix_fused_ws(desc).total;
 }

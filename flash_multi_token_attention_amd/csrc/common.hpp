@@ -86,7 +86,11 @@ hipError_t headmix_bwd_dkdv(int B, int H, int N, int d, float scale, int causal,
                             const void *v, const float *w, const void *d_o, const float *lse, const float *Dl, float *dk,
                             float *dv, hipStream_t s);
 int headmix_row_tiles(int N);
-// one pass for all gradients (headmix_bwd.hip); p: B, H, Nq = Nk = N, d, scale, causal.  dk / dv or dq / dw may be null.
+// forward with the probabilities as blocks in the workspace (headmix_probs.hip)
+size_t headmix_fwd_workspace(const Problem &p);
+hipError_t headmix_fwd_blocks(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const float *w,
+                               void *ws, void *o, float *l, float *m, hipStream_t s);
+// one pass for all gradients (headmix_scores.hip); p: B, H, Nq = Nk = N, d, scale, causal.  dk / dv or dq / dw may be null.
 size_t headmix_frag_bytes(const Problem &p);              // kv_frag holds two of these
 int headmix_score_wgs(int B, int H, int N, int causal);   // dw partials per batch entry
 hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,

@@ -1,0 +1,135 @@
+// Pieces shared by the head-mixing kernels that work on tiles of (row, key) pairs of all heads
+// (headmix_probs.hip: forward, headmix_scores.hip: backward).
+//
+// A workgroup owns R query rows of all heads of a batch entry and walks KT keys per step, alternating between
+// "a wave takes heads" (products of rows, bf16 MFMA) and "a wave takes rows" (the head mix as a product over the head
+// index on the fp32 MFMA); the two meet in LDS arrays [head][tile row][key].  What the tiles leave
+// (probabilities, dS) goes to global memory as bf16 blocks of 32 rows x 32 keys in the layout of the
+// product kernels, [row parity][key half][row pair][16 keys], the blocks of all heads side by side:
+// [batch][block][head].
+#pragma once
+#include "mfma_common.hpp"
+
+namespace convattn {
+namespace headmix {
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// Workgroup barrier for data that is exchanged through LDS: waits for this wave's LDS operations, not for the
+// global loads it has issued ahead.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// the value of the lane ROR places on in the row of 16
+template <int ROR> __device__ __forceinline__ float row16_rot(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + ROR, 0xf, 0xf, true));
+}
+
+constexpr int kBlock = kChainRows * kChainKeys;   // elements of a block
+
+// H heads, WAVES waves, R rows; 64 pairs per wave in the mixing phase: lane n = RW rows x NQ quads of keys.
+template <int H_, int WAVES_, int R_> struct Tile {
+    static constexpr int H = H_, WAVES = WAVES_, R = R_, RB = R / 16, KT = WAVES * 64 / R, KB = KT / 16, NQ = KT / 4;
+    static constexpr int RW = R / WAVES, HPW = H / WAVES, HB = H / 16;
+    static_assert(RW * NQ == 16 && HPW >= 1 && (NQ == 4 || NQ == 8), "64 pairs per wave");
+    static constexpr int HS = R * KT + 4;                   // floats per head (+4: 16 heads on 16 bank quads)
+    static constexpr int arr = H * HS;                      // floats of one array
+    static constexpr int WST = H + 4;                       // floats per row of w in LDS
+    // Four keys 4q .. 4q+3 of tile row `lr` sit at float lr * KT + 4 * slot: the XOR spreads both the score
+    // phase's writes (16 rows, one quad) and the mixing phase's reads (RW rows, all quads) over all banks.
+    __device__ static __forceinline__ int slot(int lr, int q) { return q ^ ((lr >> (NQ == 4 ? 2 : 1)) & (NQ - 1)); }
+    // Query row of tile row lr: even rows of the 32-row block first, as the blocks are laid out
+    __device__ static __forceinline__ int row(int i0, int lr) {
+        return RB == 2 ? i0 + 2 * (lr & 15) + (lr >> 4) : i0 + 2 * (lr & 7) + (lr >> 3);
+    }
+};
+
+// Key steps per workgroup and the workgroups of a batch entry (chunks of key steps, row tiles within).
+struct Plan { int steps_per_wg, n_wg, n_chunks; };
+template <typename T> Plan make_plan(int B, int N, int causal, int wgs_per_cu, int least, int most) {
+    constexpr int unit = 32 / T::KT;   // whole blocks of 32 keys
+    const int n_rt32 = (N + 31) / 32, n_tiles = n_rt32 * (32 / T::R), all = n_rt32 * unit;
+    const long long steps = causal ? (long long)n_tiles * (all + unit) / 2 : (long long)n_tiles * all;
+    long long per = steps * B / (256 * wgs_per_cu);
+    per = per < least ? least : per > most ? most : per;
+    Plan p;
+    p.steps_per_wg = (int)((per + unit - 1) / unit) * unit;
+    p.n_chunks = (all + p.steps_per_wg - 1) / p.steps_per_wg;
+    p.n_wg = 0;
+    for (int c = 0; c < p.n_chunks; ++c) p.n_wg += n_tiles - (causal ? (c * p.steps_per_wg * T::KT / 32) * (32 / T::R) : 0);
+    return p;
+}
+// Workgroup `id` of the n_wg of a batch entry -> row tile, chunk and its key steps.  Tiles of one chunk are
+// neighbours, and neighbours run on the same XCD (workgroup ids go round robin over the eight), so that the rows
+// of K and V of a chunk come from one L2.
+template <typename T>
+__device__ __forceinline__ bool find_unit(int causal, int n_rt32, const Plan &pl, int &id, int &rt, int &chunk, int &s0, int &s_end) {
+    const int n_tiles = n_rt32 * (32 / T::R), per = (pl.n_wg + 7) / 8;
+    id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || id >= pl.n_wg) return false;
+    int i = id;
+    for (chunk = 0;; ++chunk) {
+        s0 = chunk * pl.steps_per_wg;
+        const int first = causal ? (s0 * T::KT / 32) * (32 / T::R) : 0;   // first row tile that sees the chunk
+        if (i < n_tiles - first) break;
+        i -= n_tiles - first;
+    }
+    rt = n_tiles - 1 - i;
+    s_end = min(s0 + pl.steps_per_wg, causal ? (rt * T::R / 32 + 1) * (32 / T::KT) : n_rt32 * (32 / T::KT));
+    return true;
+}
+
+// Row fragments (lane 16g + n: tile row 16 rb + n, columns 32 ks + 8g ..) of rows i0 .. i0+R-1 of a head: whole rows
+// loaded, turned in `st`, this wave's room of R * (2 D + 16) bytes in LDS.  Rows past the last: copies of it.
+template <typename T, int D>
+__device__ __forceinline__ void turn_rows(bf16x8 (&f)[T::RB][D / 32], const bf16_t *__restrict__ src, int i0, int N, unsigned char *st) {
+    constexpr int CPR = D / 8, RST = D * 2 + 16, LD = T::R * CPR / 64;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    u32x4 raw[LD];
+#pragma unroll
+    for (int i = 0; i < LD; ++i) {
+        const int c = lane + i * 64;
+        raw[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)min(i0 + c / CPR, N - 1) * D + (c % CPR) * 8);
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < LD; ++i) {
+        const int c = lane + i * 64;
+        *reinterpret_cast<u32x4 *>(st + (c / CPR) * RST + (c % CPR) * 16) = raw[i];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int rb = 0; rb < T::RB; ++rb)
+#pragma unroll
+        for (int ks = 0; ks < D / 32; ++ks)
+            f[rb][ks] = *reinterpret_cast<const bf16x8 *>(st + T::row(0, rb * 16 + n) * RST + ks * 64 + g * 16);
+}
+
+// Rows of a tensor in the order in which the score phases' lanes read them: [batch, head][16 rows][k step][lane][8]
+// (lane 16g + n: row n, columns 32 ks + 8g ..), zeros past the last row.  Read straight from the rows, a fragment
+// load has neighbouring lanes in different rows: 64 cache accesses instead of 16, and the backward's score kernel was
+// bound by them (3.3 M of its 4.1 M clocks per CU at B4 H16 N4096 d128).  One copy of K and V (0.04 ms there) is read
+// N / 32 times.  V may be null.
+template <int D>
+__global__ __launch_bounds__(256) void frag_order_kernel(int N, int n_t16, const bf16_t *__restrict__ K,
+                                                         const bf16_t *__restrict__ V, bf16_t *__restrict__ KF,
+                                                         bf16_t *__restrict__ VF, size_t n_frag) {
+    const size_t f = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // one 1 KB fragment per wave
+    if (f >= n_frag) return;
+    constexpr int KS = D / 32;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const size_t bh = f / ((size_t)n_t16 * KS);
+    const int r = (int)(f - bh * n_t16 * KS), row = (r / KS) * 16 + n, col = (r % KS) * 32 + 8 * g;
+    *reinterpret_cast<u32x4 *>(KF + f * 512 + lane * 8) = load_row16<D>(K + bh * N * D, row, N, col);
+    if (V) *reinterpret_cast<u32x4 *>(VF + f * 512 + lane * 8) = load_row16<D>(V + bh * N * D, row, N, col);
+}
+template <int D>
+void launch_frag_order(int BH, int N, const void *k, const void *v, const bf16_t *kf, const bf16_t *vf, hipStream_t s) {
+    const int n_t16 = (N + 31) / 32 * 2;
+    const size_t n_frag = (size_t)BH * n_t16 * (D / 32);
+    frag_order_kernel<D><<<(unsigned)((n_frag + 3) / 4), 256, 0, s>>>(N, n_t16, (const bf16_t *)k, (const bf16_t *)v, const_cast<bf16_t *>(kf),
+                                                                     const_cast<bf16_t *>(vf), n_frag);
+}
+
+}  // namespace headmix
+}  // namespace convattn

@@ -1,0 +1,417 @@
+// Forward of head-mixing attention (gfx950): O_h = softmax(scale sum_h' w[h][h'] Q_h' K_h'^T + causal mask) V_h.
+//
+// The head mix couples all heads of a (row, key) pair, the product with V all keys of a head.  In one workgroup, O of
+// all heads (H d floats per row) and the Q fragments leave the registers no room for anything to be loaded
+// ahead (measured at B4 H16 N4096 d128: 1.9 ms with 40 registers spilled, the 16-row form before it 1.8 ms).
+// So the pass is cut there: headmix_probs_kernel writes the probabilities as bf16 blocks (the operand precision of the
+// product), un-normalised, and headmix_pv_kernel multiplies them with V and divides by the row sums.
+//
+// Probabilities are exp2(z - ref) with one whole-number reference per (row, head): the largest score of the row's
+// first tile of keys, rounded up.  Every chunk of a row's keys derives the same reference from that tile, so that chunks
+// need no merging, and a row has no running maximum: bf16 and fp32 keep their relative precision over
+// 2^+-126, and only a score more than kSlack above the reference moves it (the workgroup then rescales what it has
+// written so far; exact, the factor being a power of two).
+#include "headmix_common.hpp"
+
+namespace convattn {
+namespace {
+
+using namespace headmix;
+
+constexpr float kSlack = 60.f;   // log2 units: sums of 2^60 terms times V stay far inside fp32 and bf16
+
+// 16 heads: 16 waves of 128 registers (one head each), 32 rows x 32 keys per step; 32 heads: 8 waves of 256
+// registers, 16 rows x 32 keys.  Two score buffers: the products of a step run under the mix of the step before it,
+// one barrier per step.
+template <int H, int D> struct ProbTile : Tile<H, H == 16 ? 16 : 8, H == 16 ? 32 : 16> {
+    using B = Tile<H, H == 16 ? 16 : 8, H == 16 ? 32 : 16>;
+    static constexpr int ROOM = B::R * (D * 2 + 16);        // a head's rows while they are turned
+    static constexpr int w_off = 2 * B::arr, used = (w_off + H * B::WST) * 4, lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
+};
+
+struct ProbArgs {
+    int B, N, causal, n_rt32, n_kt;
+    Plan plan;
+    float scale;
+    const bf16_t *Q, *KF;    // KF: fragment order
+    const float *W;
+    bf16_t *P;               // blocks
+    float *stats;            // [B][chunk][reference, largest score, sum, sum of the rounded][H][N]
+};
+
+template <int H, int D>
+__global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_kernel(ProbArgs a) {
+    using T = ProbTile<H, D>;
+    constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, HPW = T::HPW, HB = T::HB,
+                  KS = D / 32, NCH = HPW * KB;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    float *lds = reinterpret_cast<float *>(smem);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
+    const int b = blockIdx.y;
+    int id, rt, chunk, s0, s_end;
+    if (!find_unit<T>(a.causal, a.n_rt32, a.plan, id, rt, chunk, s0, s_end)) return;
+    const int i0 = rt * R, N = a.N, h0 = wave * HPW;
+
+    bf16x8 qf[HPW][RB][KS];
+    {
+#pragma unroll
+        for (int t = 0; t < HPW; ++t)
+            turn_rows<T, D>(qf[t], a.Q + ((size_t)b * H + h0 + t) * N * D, i0, N, smem + wave * T::ROOM);
+        lds_barrier();
+    }
+    for (int i = tid; i < H * H; i += T::WAVES * 64) lds[T::w_off + (i / H) * T::WST + i % H] = a.W[i] * (a.scale * kLog2e);
+    const float *wf_l = lds + T::w_off + n * T::WST + 4 * g;
+
+    // ---- score phase: chunks of one head and 16 keys, K rows two chunks ahead ----
+    bf16x8 kf[2][KS];
+    const int n_t16 = a.n_rt32 * 2;
+    auto load_chunk = [&](int step, int c) {
+        const bf16_t *kp = a.KF + (((size_t)b * H + h0 + c / KB) * n_t16 + step * KB + c % KB) * KS * 512;   // (uniform)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) kf[c & 1][ks] = *reinterpret_cast<const bf16x8 *>(kp + lane * 8 + ks * 512);
+    };
+    auto score_chunk = [&](float *S, int c) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) s = mfma_bf16(kf[c & 1][ks], qf[c / KB][rb][ks], s);
+            *reinterpret_cast<f32x4 *>(S + (h0 + c / KB) * HS + (rb * 16 + n) * KT + 4 * T::slot(rb * 16 + n, 4 * (c % KB) + g)) = s;
+        }
+    };
+    // all chunks of `step` into S, loading the first two of step `next`
+    auto scores = [&](float *S, int step, int next) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            score_chunk(S, c);
+            if (c + 2 < NCH) load_chunk(step, c + 2);
+            else load_chunk(next, c + 2 - NCH);
+        }
+    };
+
+    // ---- mixing phase: lane (g, n) = heads 16x + 4g .. +3, tile row lr, keys 4q4 .. 4q4+3 ----
+    const int lr = wave * RW + (n & (RW - 1)), q4 = n / RW, row = T::row(i0, lr), brow = row & 31;
+    const int pos = lr * KT + 4 * T::slot(lr, q4);
+    f32x4 ref[HB], top[HB], l_sum[HB], l_hat[HB];
+#pragma unroll
+    for (int x = 0; x < HB; ++x) {
+        l_sum[x] = l_hat[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        top[x] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
+    }
+    auto mix = [&](f32x4 (&z)[HB][4], const float *S, int step) {
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) z[x][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int y = 0; y < HB; ++y) {
+            f32x4 wf[HB];
+#pragma unroll
+            for (int x = 0; x < HB; ++x) wf[x] = *reinterpret_cast<const f32x4 *>(wf_l + 16 * x * T::WST + 16 * y);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(S + (16 * y + 4 * g + s) * HS + pos);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
+            }
+        }
+        // masks only where a key of the tile is past the tile's first row or past the last key
+        if ((a.causal && step * KT + KT - 1 > i0) || step * KT + KT > N) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int key = step * KT + 4 * q4 + t;
+                if (key >= N || (a.causal && key > row)) {
+#pragma unroll
+                    for (int x = 0; x < HB; ++x) z[x][t] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
+                }
+            }
+        }
+    };
+    auto row_max = [&](float v) {   // over the lanes of a row
+        v = fmaxf(v, row16_rot<8>(v));
+        v = fmaxf(v, row16_rot<4>(v));
+        if constexpr (RW == 2) v = fmaxf(v, row16_rot<2>(v));
+        return v;
+    };
+    const long long n_blk = chain_ds_block_off(a.causal != 0, a.n_rt32, a.n_kt);
+    auto block_of = [&](int step) {
+        const int kt = step * KT / 32;
+        return a.P + ((size_t)b * n_blk + chain_ds_block_off(a.causal != 0, a.n_rt32, kt) + i0 / 32 - chain_ds_first_rt(a.causal != 0, kt)) * H * kBlock;
+    };
+    const int out = (((brow & 1) * 2 + ((4 * q4) >> 4)) * 16 + (brow >> 1)) * 16 + ((4 * q4) & 15) + 4 * g * kBlock;
+    static_assert(KT == 32, "a step is a column of blocks");
+
+    auto probs = [&](const float *S, int step) {
+        f32x4 z[HB][4];
+        mix(z, S, step);
+        bool over = false;
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float m = fmaxf(fmaxf(z[x][0][r], z[x][1][r]), fmaxf(z[x][2][r], z[x][3][r]));
+                top[x][r] = fmaxf(top[x][r], m);
+                over |= m > ref[x][r] + kSlack;
+            }
+        if (__any(over)) {
+            // rare: move the references of the wave's rows; this wave wrote all of their probabilities itself, lane by lane
+#pragma unroll
+            for (int x = 0; x < HB; ++x)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float m_new = fmaxf(ref[x][r], ceilf(row_max(top[x][r])));
+                    const float f = fast_exp2(ref[x][r] - m_new);
+                    l_sum[x][r] *= f;
+                    l_hat[x][r] *= f;
+                    ref[x][r] = m_new;
+                    for (int e = s0; e < step; ++e) {
+                        bf16x4 *pp = reinterpret_cast<bf16x4 *>(block_of(e) + out + (16 * x + r) * kBlock);
+                        bf16x4 pb = *pp;
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) pb[t] = (bf16_t)((float)pb[t] * f);
+                        *pp = pb;
+                    }
+                }
+        }
+        bf16_t *p_out = block_of(step);
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                bf16x4 pb;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const float p = fast_exp2(z[x][t][r] - ref[x][r]);
+                    l_sum[x][r] += p;
+                    pb[t] = (bf16_t)p;
+                    l_hat[x][r] += (float)pb[t];
+                }
+                __builtin_nontemporal_store(__builtin_bit_cast(u32x2, pb), reinterpret_cast<u32x2 *>(p_out + out + (16 * x + r) * kBlock));
+            }
+    };
+
+    // ---- reference of every row from the first tile of keys (key 0 is visible to all rows) ----
+    float *buf0 = lds, *buf1 = lds + T::arr;
+    load_chunk(0, 0);
+    load_chunk(0, 1);
+    scores(buf1, 0, s0);
+    scores(buf0, s0, min(s0 + 1, s_end - 1));
+    lds_barrier();
+    {
+        f32x4 z[HB][4];
+        mix(z, buf1, 0);
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                ref[x][r] = ceilf(row_max(fmaxf(fmaxf(z[x][0][r], z[x][1][r]), fmaxf(z[x][2][r], z[x][3][r]))));
+    }
+    lds_barrier();
+    for (int u = s0; u < s_end; ++u) {
+        float *cur = (u - s0) & 1 ? buf1 : buf0, *nxt = (u - s0) & 1 ? buf0 : buf1;
+        if (u + 1 < s_end) scores(nxt, u + 1, min(u + 2, s_end - 1));
+        probs(cur, u);
+        lds_barrier();
+    }
+
+    float *st = a.stats + ((size_t)b * a.plan.n_chunks + chunk) * 4 * H * N;
+#pragma unroll
+    for (int x = 0; x < HB; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float l = l_sum[x][r], lh = l_hat[x][r];
+            l += row16_rot<8>(l); lh += row16_rot<8>(lh);
+            l += row16_rot<4>(l); lh += row16_rot<4>(lh);
+            if constexpr (RW == 2) { l += row16_rot<2>(l); lh += row16_rot<2>(lh); }
+            const float m = row_max(top[x][r]);
+            const size_t o = (size_t)(16 * x + 4 * g + r) * N + row, hn = (size_t)H * N;
+            if (q4 == 0 && row < N) {
+                st[o] = ref[x][r];
+                st[hn + o] = m;
+                st[2 * hn + o] = l;
+                st[3 * hn + o] = lh;
+            }
+        }
+}
+
+// O = P V / (sum of P): the product kernel of dQ = dS K (bwd_dq_rows.hip) with the row sums, L and M at the end.
+// Workgroup = 4 waves = 128 rows of one (batch, head), wave = 32 rows, steps of 64 keys; P blocks go straight
+// into the operand registers (non-temporal, two steps ahead), V passes through LDS.
+constexpr int PV_WAVES = 4, PV_ROWS = 128, PV_KEYS = 64;
+
+template <int D, typename TO>
+__global__ __launch_bounds__(PV_WAVES * 64) void headmix_pv_kernel(ProbArgs a, int H, int tile_keys, int tile_rows, const bf16_t *__restrict__ V,
+                                                                   TO *__restrict__ O, float *__restrict__ L, float *__restrict__ M) {
+    constexpr int RST = D * 2 + 16, DB = D / 16, CPR = D / 8, LD = PV_KEYS * CPR / (PV_WAVES * 64);
+    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * PV_KEYS * RST];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
+    const int h = blockIdx.x, b = blockIdx.y, qt = gridDim.z - 1 - blockIdx.z;   // longest (causal) tiles first
+    const int N = a.N, i0 = qt * PV_ROWS, rw = i0 + wave * 32, rt = rw / 32, n_rt = a.n_rt32;
+    const bool causal = a.causal != 0, row_ok = rt < n_rt;
+    const size_t bh = (size_t)b * H + h;
+    const bf16_t *Vb = V + bh * N * D;
+    const bf16_t *ws = a.P + ((size_t)b * chain_ds_block_off(causal, n_rt, a.n_kt) * H + h) * kBlock;
+
+    // ---- the rows' statistics over the chunks of their keys: lane n of block ob = row 2n + ob ----
+    const int chunk_keys = a.plan.steps_per_wg * tile_keys;
+    const int n_ch = causal ? min(min(rt, n_rt - 1) * 32 / chunk_keys + 1, a.plan.n_chunks) : a.plan.n_chunks;
+    float ref[2], inv[2];
+    bool moved = false;
+#pragma unroll
+    for (int ob = 0; ob < 2; ++ob) {
+        const int row = min(rw + 2 * n + ob, N - 1);
+        const size_t hn = (size_t)H * N;
+        const float *st = a.stats + (size_t)b * a.plan.n_chunks * 4 * hn + (size_t)h * N + row;
+        float r = st[0], m = st[hn], l = st[2 * hn], lh = st[3 * hn];
+        for (int c = 1; c < n_ch; ++c) {
+            const float *s = st + (size_t)c * 4 * hn;
+            const float rc = s[0], rn = fmaxf(r, rc), f0 = fast_exp2(r - rn), f1 = fast_exp2(rc - rn);
+            moved |= rc != r;
+            m = fmaxf(m, s[hn]);
+            l = l * f0 + s[2 * hn] * f1;
+            lh = lh * f0 + s[3 * hn] * f1;
+            r = rn;
+        }
+        ref[ob] = r;
+        inv[ob] = 1.f / lh;
+        if (g == 0 && rw + 2 * n + ob < N) {
+            M[bh * N + row] = m * (1.f / kLog2e);
+            L[bh * N + row] = l * fast_exp2(r - m);
+        }
+    }
+    moved = __any(moved);
+
+    f32x4 acc[2][DB];
+#pragma unroll
+    for (int ob = 0; ob < 2; ++ob)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) acc[ob][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int k_end = causal ? min(N, i0 + PV_ROWS) : N, n_steps = (k_end + PV_KEYS - 1) / PV_KEYS;
+    u32x4 vr[LD], pr_a[2][2], pr_b[2][2];
+    auto load_v = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+            const int c = tid + i * PV_WAVES * 64;
+            vr[i] = load_row16_clamped<D>(Vb, s * PV_KEYS + c / CPR, N, (c % CPR) * 8);
+        }
+    };
+    auto load_p = [&](int s, u32x4 (&pr)[2][2]) {
+#pragma unroll
+        for (int kp = 0; kp < 2; ++kp) {
+            const int kt = s * 2 + kp;
+            // (a block that does not exist: any block that does; the registers are cleared before their use)
+            const int rt_c = min(rt, n_rt - 1), kt_c = min(kt, causal ? rt_c : n_rt - 1);
+            const size_t blk = (size_t)chain_ds_block_off(causal, n_rt, kt_c) + rt_c - chain_ds_first_rt(causal, kt_c);
+#pragma unroll
+            for (int ob = 0; ob < 2; ++ob)
+                pr[kp][ob] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(
+                    ws + blk * H * kBlock + ((ob * 2 + (g >> 1)) * 16 + n) * 16 + 8 * (g & 1)));
+        }
+    };
+    auto run_step = [&](int s, u32x4 (&pr)[2][2]) {
+        unsigned char *Vs = smem + (s & 1) * PV_KEYS * RST;
+#pragma unroll
+        for (int i = 0; i < LD; ++i) {
+            const int c = tid + i * PV_WAVES * 64;
+            *reinterpret_cast<u32x4 *>(Vs + (c / CPR) * RST + (c % CPR) * 16) = zero_unless(s * PV_KEYS + c / CPR < N, vr[i]);
+        }
+        bf16x8 pf[2][2];
+#pragma unroll
+        for (int kp = 0; kp < 2; ++kp) {
+            const int kt = s * 2 + kp;
+            const bool ok = row_ok && kt < n_rt && (!causal || kt <= rt);
+#pragma unroll
+            for (int ob = 0; ob < 2; ++ob) pf[kp][ob] = __builtin_bit_cast(bf16x8, zero_unless(ok, pr[kp][ob]));
+            if (moved && ok) {   // rare: a chunk of some row has a reference of its own
+                const float *st = a.stats + ((size_t)b * a.plan.n_chunks + min(kt * 32 / chunk_keys, n_ch - 1)) * 4 * H * N + (size_t)h * N;
+#pragma unroll
+                for (int ob = 0; ob < 2; ++ob) {
+                    const float f = fast_exp2(st[min(rw + 2 * n + ob, N - 1)] - ref[ob]);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) pf[kp][ob][e] = (bf16_t)((float)pf[kp][ob][e] * f);
+                }
+            }
+        }
+        __syncthreads();
+        load_v(s + 1);
+        load_p(s + 2, pr);
+        if (causal && s * PV_KEYS > rw + 31) return;  // every key of the step is after the wave's rows
+#pragma unroll
+        for (int kp = 0; kp < 2; ++kp)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) {
+                const bf16x4 lo = lds_read_tr4x16(Vs, RST, kp * 32 + 8 * g, db * 16, n), hi = lds_read_tr4x16(Vs, RST, kp * 32 + 8 * g + 4, db * 16, n);
+                const bf16x8 vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int ob = 0; ob < 2; ++ob) acc[ob][db] = mfma_bf16(vf, pf[kp][ob], acc[ob][db]);
+            }
+    };
+    load_v(0);
+    load_p(0, pr_a);
+    load_p(1, pr_b);
+    for (int s = 0; s < n_steps; s += 2) {
+        run_step(s, pr_a);
+        if (s + 1 < n_steps) run_step(s + 1, pr_b);
+    }
+#pragma unroll
+    for (int ob = 0; ob < 2; ++ob) {
+        const int row = rw + 2 * n + ob;
+        if (row >= N) continue;
+        TO *o = O + (bh * N + row) * D + 4 * g;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+            const f32x4 v = acc[ob][db] * inv[ob];
+            if constexpr (sizeof(TO) == 2) {
+                bf16x4 ov;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ov[r] = (bf16_t)v[r];
+                *reinterpret_cast<bf16x4 *>(o + 16 * db) = ov;
+            } else {
+                *reinterpret_cast<f32x4 *>(o + 16 * db) = v;
+            }
+        }
+    }
+}
+
+// Four workgroups per CU level out the tail of the launch; a chunk repeats the first tile of its rows for the reference:
+// at least eight steps where there are enough workgroups without more.
+Plan prob_plan(const Problem &p) {
+    const long long all = (long long)((p.Nq + 31) / 32) * ((p.Nq + 31) / 32) * p.B / (p.causal ? 2 : 1) / 256;
+    const int least = all >= 16 ? 8 : all >= 4 ? 4 : 2;
+    return p.H == 16 ? make_plan<ProbTile<16, 32>>(p.B, p.Nq, p.causal, 4, least, 64) : make_plan<ProbTile<32, 32>>(p.B, p.Nq, p.causal, 4, least, 64);
+}
+
+template <int H, int D, typename TO>
+hipError_t launch(const Problem &p, const ProbArgs &a, const void *k, const void *v, void *o, float *l, float *m, hipStream_t s) {
+    using T = ProbTile<H, D>;
+    static_assert(T::lds <= 160 * 1024, "LDS budget");
+    launch_frag_order<D>(p.B * H, a.N, k, nullptr, a.KF, nullptr, s);
+    hipError_t e = set_max_lds_once<headmix_probs_kernel<H, D>>(T::lds);
+    if (e != hipSuccess) return e;
+    headmix_probs_kernel<H, D><<<dim3((a.plan.n_wg + 7) / 8 * 8, p.B), T::WAVES * 64, T::lds, s>>>(a);
+    headmix_pv_kernel<D, TO><<<dim3(H, p.B, (a.N + PV_ROWS - 1) / PV_ROWS), PV_WAVES * 64, 0, s>>>(a, H, T::KT, T::R, (const bf16_t *)v, (TO *)o, l, m);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// K in fragment order, statistics of the chunks, blocks
+static size_t prob_stats_bytes(const Problem &p) { return ((size_t)p.B * prob_plan(p).n_chunks * 4 * p.H * p.Nq * sizeof(float) + 255) / 256 * 256; }
+size_t headmix_fwd_workspace(const Problem &p) { return headmix_frag_bytes(p) + prob_stats_bytes(p) + chain_ds_bytes(p); }
+
+hipError_t headmix_fwd_blocks(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const float *w,
+                              void *ws, void *o, float *l, float *m, hipStream_t s) {
+    unsigned char *base = static_cast<unsigned char *>(ws);
+    const size_t fb = headmix_frag_bytes(p), sb = prob_stats_bytes(p);
+    const ProbArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), prob_plan(p), p.scale, (const bf16_t *)q,
+                     (const bf16_t *)base, w, (bf16_t *)(base + fb + sb), (float *)(base + fb)};
+#define CALL(HH, DD) (out_dt == CONVATTN_BF16 ? launch<HH, DD, bf16_t>(p, a, k, v, o, l, m, s) : launch<HH, DD, float>(p, a, k, v, o, l, m, s))
+    if (p.H == 16) return p.d == 32 ? CALL(16, 32) : p.d == 64 ? CALL(16, 64) : CALL(16, 128);
+    if (p.H == 32) return p.d == 32 ? CALL(32, 32) : p.d == 64 ? CALL(32, 64) : CALL(32, 128);
+#undef CALL
+    return hipErrorInvalidValue;
+}
+
+}  // namespace convattn

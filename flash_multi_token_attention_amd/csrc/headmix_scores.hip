@@ -11,70 +11,29 @@
 // blocks of 32 rows x 32 keys (the operand precision of the products that follow); dQ = dS K is
 // the product kernel of the window backward (bwd_dq_rows.hip, same block layout) and
 // headmix_dkdv_kernel takes dV = P^T dO and dK = dS^T Q from one walk over the blocks of 128 keys.
-#include "mfma_common.hpp"
+#include "headmix_common.hpp"
 
 namespace convattn {
 namespace {
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-// Workgroup barrier for data that is exchanged through LDS: waits for this wave's LDS operations, not for the
-// global loads it has issued ahead.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+using namespace headmix;
+constexpr int SC_BLK = kBlock;
 
-constexpr int SC_WAVES = 8;
-constexpr int SC_BLK = kChainRows * kChainKeys;   // elements of a P / dS block
-
-// Tile of the score kernel: 512 (row, key) pairs of all heads per step, 64 pairs per wave.
-//   RB = 2: 32 rows x 16 keys (16 heads);  RB = 1: 16 rows x 32 keys (32 heads: the resident row fragments
-//   of 32 heads take the registers of 16 heads' 32 rows).
-template <int H, int D> struct ScoreTile {
-    static constexpr int RB = H == 16 ? 2 : 1;
-    static constexpr int R = 16 * RB, KT = 512 / R, KB = KT / 16, NQ = KT / 4;
-    static constexpr int RW = R / SC_WAVES;                 // rows of a wave in the mixing phase
-    static constexpr int SWZ = RB == 2 ? 2 : 1;             // see slot()
-    static constexpr int HS = R * KT + 4;                   // floats per head (+4: 16 heads on 16 bank quads)
-    static constexpr int arr = H * HS;                      // floats of one array
+// 8 waves of 256 registers: 512 pairs per step, 32 rows x 16 keys with 16 heads, 16 rows x 32 keys with 32 (the
+// resident row fragments of 32 heads take the registers of 16 heads' 32 rows).
+template <int H, int D> struct ScoreTile : Tile<H, 8, H == 16 ? 32 : 16> {
+    using B = Tile<H, 8, H == 16 ? 32 : 16>;
     static constexpr int NBUF = H == 16 ? 2 : 1;
-    static constexpr int HPW = H / SC_WAVES, HB = H / 16;
     static constexpr bool STATS_LDS = H * D >= 2048;          // LSE and D of the tile rows: registers are short
-    static constexpr int WST = H + 4;                       // floats per row of w in LDS
-    static constexpr int w_off = NBUF * 2 * arr, wt_off = w_off + H * WST, 
-                         st_off = wt_off + H * WST,       // LSE and D of the tile's rows (32 heads: not in registers)
-                         lds = (st_off + (STATS_LDS ? 2 * R * WST : 0)) * 4;
+    static constexpr int w_off = NBUF * 2 * B::arr, wt_off = w_off + H * B::WST, st_off = wt_off + H * B::WST,
+                         lds = (st_off + (STATS_LDS ? 2 * B::R * B::WST : 0)) * 4;
     // chunks of K and V rows in flight during the mixing phase, as far as the registers go
     static constexpr int AHEAD = H == 32 && D == 128 ? 1 : 2;
-    // Four keys 4q .. 4q+3 of tile row `lr` sit at float lr * KT + 4 * slot: the XOR spreads both the score
-    // phase's writes (16 rows, one quad) and the mixing phase's reads (RW rows, all quads) over all banks.
-    __device__ static __forceinline__ int slot(int lr, int q) { return q ^ ((lr >> SWZ) & (NQ - 1)); }
-    // Query row of tile row lr: even rows of the 32-row block first, as the blocks are laid out
-    __device__ static __forceinline__ int row(int i0, int lr) {
-        return RB == 2 ? i0 + 2 * (lr & 15) + (lr >> 4) : i0 + 2 * (lr & 7) + (lr >> 3);
-    }
 };
 
-// K and V of a launch in the order in which the score kernel's lanes read them: [batch, head][16 keys][k step][lane][8]
-// (lane 16g + n: key n, columns 32 ks + 8g ..), zeros past the last key.  Read straight from the rows, every
-// fragment load touches 16 rows with neighbouring lanes in different rows: 64 cache accesses per load instead of
-// 16, and the score kernel was bound by them (3.3 M of its 4.1 M clocks per CU at B4 H16 N4096 d128).  One copy of K and V
-// (0.06 ms there) is read N / 32 times.
-template <int D>
-__global__ __launch_bounds__(256) void headmix_frag_order_kernel(int N, int n_t16, const bf16_t *__restrict__ K,
-                                                                 const bf16_t *__restrict__ V, bf16_t *__restrict__ KF,
-                                                                 bf16_t *__restrict__ VF, size_t n_frag) {
-    const size_t f = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // one 1 KB fragment per wave
-    if (f >= n_frag) return;
-    constexpr int KS = D / 32;
-    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const size_t bh = f / ((size_t)n_t16 * KS);
-    const int r = (int)(f - bh * n_t16 * KS), row = (r / KS) * 16 + n, col = (r % KS) * 32 + 8 * g;
-    *reinterpret_cast<u32x4 *>(KF + f * 512 + lane * 8) = load_row16<D>(K + bh * N * D, row, N, col);
-    *reinterpret_cast<u32x4 *>(VF + f * 512 + lane * 8) = load_row16<D>(V + bh * N * D, row, N, col);
-}
-
 struct ScoreArgs {
-    int B, N, causal, n_rt32, n_kt, steps_per_wg, n_wg;
+    int B, N, causal, n_rt32, n_kt;
+    Plan plan;
     float scale;
     const bf16_t *Q, *KF, *VF, *dO;   // KF, VF: fragment order
     const float *W, *lse, *Dl;
@@ -82,32 +41,8 @@ struct ScoreArgs {
     float *dw_part;      // [B][n_wg][H][H], or null
 };
 
-// Workgroup `id` of the n_wg of a batch entry -> row tile and first key step of its chunk.  Chunks of the
-// same keys are neighbours, and neighbours run on the same XCD (workgroup ids go round robin over the eight),
-// so that the rows of K and V of a chunk come from one L2.
 template <int H, int D>
-__device__ __forceinline__ bool score_unit(const ScoreArgs &a, int &rt, int &s0, int &s_end) {
-    using T = ScoreTile<H, D>;
-    const int n_tiles = a.n_rt32 * (32 / T::R);
-    const int per = (a.n_wg + 7) / 8;
-    int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || id >= a.n_wg) return false;
-    const int all = a.n_rt32 * (32 / T::KT);
-    for (int c = 0;; ++c) {
-        s0 = c * a.steps_per_wg;
-        const int first = a.causal ? (s0 * T::KT / 32) * (32 / T::R) : 0;   // first row tile that sees the chunk
-        if (id < n_tiles - first) {
-            rt = n_tiles - 1 - id;
-            const int end = a.causal ? (rt * T::R / 32 + 1) * (32 / T::KT) : all;
-            s_end = min(s0 + a.steps_per_wg, end);
-            return true;
-        }
-        id -= n_tiles - first;
-    }
-}
-
-template <int H, int D>
-__global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs a) {
+__global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_kernel(ScoreArgs a) {
     using T = ScoreTile<H, D>;
     constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, HPW = T::HPW,
                   HB = T::HB, KS = D / 32, NCH = HPW * KB;
@@ -116,8 +51,8 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
               n = lane & 15;
     const int b = blockIdx.y;
-    int rt, s0, s_end;
-    if (!score_unit<H, D>(a, rt, s0, s_end)) return;
+    int id, rt, chunk, s0, s_end;
+    if (!find_unit<T>(a.causal, a.n_rt32, a.plan, id, rt, chunk, s0, s_end)) return;
     const int i0 = rt * R, N = a.N;
     const size_t bo = (size_t)b * H * N * D;
     const int h0 = wave * HPW;
@@ -125,34 +60,12 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
     // ---- resident: Q and dO fragments of this wave's heads (rows loaded whole, turned in the wave's share of the LDS) ----
     bf16x8 qf[HPW][RB][KS], of[HPW][RB][KS];
     {
-        constexpr int CPR = D / 8, RST = D * 2 + 16, LD = R * CPR / 64;
-        static_assert(R * RST <= T::arr * 4 * 2 * T::NBUF / SC_WAVES, "room for one head's rows");
-        unsigned char *st = smem + wave * (T::arr * 4 * 2 * T::NBUF / SC_WAVES / 16 * 16);
-        auto turn = [&](const bf16_t *src, bf16x8 (&f)[RB][KS]) {
-            u32x4 raw[LD];
-#pragma unroll
-            for (int i = 0; i < LD; ++i) {
-                const int c = lane + i * 64;
-                raw[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)min(i0 + c / CPR, N - 1) * D + (c % CPR) * 8);
-            }
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int i = 0; i < LD; ++i) {
-                const int c = lane + i * 64;
-                *reinterpret_cast<u32x4 *>(st + (c / CPR) * RST + (c % CPR) * 16) = raw[i];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks)
-                    f[rb][ks] = *reinterpret_cast<const bf16x8 *>(st + (T::row(0, rb * 16 + n)) * RST + ks * 64 + g * 16);
-        };
+        constexpr int ROOM = T::NBUF * 2 * T::arr * 4 / T::WAVES / 16 * 16;
+        static_assert(R * (D * 2 + 16) <= ROOM, "room for one head's rows");
 #pragma unroll
         for (int t = 0; t < HPW; ++t) {
-            turn(a.Q + bo + (size_t)(h0 + t) * N * D, qf[t]);
-            turn(a.dO + bo + (size_t)(h0 + t) * N * D, of[t]);
+            turn_rows<T, D>(qf[t], a.Q + bo + (size_t)(h0 + t) * N * D, i0, N, smem + wave * ROOM);
+            turn_rows<T, D>(of[t], a.dO + bo + (size_t)(h0 + t) * N * D, i0, N, smem + wave * ROOM);
         }
         lds_barrier();   // the score tiles go where the other waves' rows are
     }
@@ -163,7 +76,7 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
     float *st_l = lds + T::st_off;
     f32x4 lse_r[HB], dl_r[HB];
     if constexpr (T::STATS_LDS) {
-        for (int i = tid; i < R * H; i += SC_WAVES * 64) {
+        for (int i = tid; i < R * H; i += T::WAVES * 64) {
             const int hh = i / R, lr2 = i % R, rr = T::row(i0, lr2);
             const size_t o = ((size_t)b * H + hh) * N + min(rr, N - 1);
             st_l[lr2 * T::WST + hh] = rr < N ? a.lse[o] * kLog2e : 1e30f;
@@ -181,7 +94,7 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
     }
     // w of the mix and its transpose, with the scales of the two products, in LDS (read as four k steps at a time:
     // k slot g of step s is head 4g + s)
-    for (int i = tid; i < H * H; i += SC_WAVES * 64) {
+    for (int i = tid; i < H * H; i += T::WAVES * 64) {
         const float w = a.W[i];
         lds[T::w_off + (i / H) * T::WST + i % H] = w * (a.scale * kLog2e);
         lds[T::wt_off + (i % H) * T::WST + i / H] = w * a.scale;
@@ -388,13 +301,11 @@ __global__ __launch_bounds__(SC_WAVES * 64) void headmix_scores_kernel(ScoreArgs
 #pragma unroll
                 for (int r = 0; r < 4; ++r) lds[(wave * H + 16 * x + 4 * g + r) * H + 16 * y + n] = acc_w[x][y][r];
         lds_barrier();
-        const int per = (a.n_wg + 7) / 8;
-        const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-        float *part = a.dw_part + ((size_t)b * a.n_wg + id) * H * H;
-        for (int i = tid; i < H * H; i += SC_WAVES * 64) {
+        float *part = a.dw_part + ((size_t)b * a.plan.n_wg + id) * H * H;
+        for (int i = tid; i < H * H; i += T::WAVES * 64) {
             float s = 0.f;
 #pragma unroll
-            for (int w = 0; w < SC_WAVES; ++w) s += lds[w * H * H + i];
+            for (int w = 0; w < T::WAVES; ++w) s += lds[w * H * H + i];
             part[i] = s * a.scale;
         }
     }
@@ -548,35 +459,22 @@ __global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, i
     }
 }
 
-// Key steps per score workgroup and the workgroups of a batch entry.
-struct ScorePlan { int steps_per_wg, n_wg; };
-ScorePlan score_plan(int B, int H, int N, int causal) {
-    const int R = H == 16 ? 32 : 16, KT = 512 / R, n_rt32 = (N + 31) / 32, n_tiles = n_rt32 * (32 / R);
-    const int all = n_rt32 * (32 / KT);
-    const long long steps = causal ? (long long)n_tiles * (all + 32 / KT) / 2 : (long long)n_tiles * all;
-    // four workgroups per CU level out the tail of the launch; fewer than eight steps do not pay for a workgroup's
-    // resident fragments while there are CUs for longer ones, more than 64 gain nothing
-    long long per = steps * B / (256 * 4);
-    const int unit = 32 / KT;   // whole blocks of 32 keys
-    const long long least = steps * B / 256 >= 8 ? 8 : 2;
-    per = per < least ? least : per > 64 ? 64 : per;
-    ScorePlan p;
-    p.steps_per_wg = (int)((per + unit - 1) / unit) * unit;
-    p.n_wg = 0;
-    for (int s0 = 0; s0 < all; s0 += p.steps_per_wg) p.n_wg += n_tiles - (causal ? (s0 * KT / 32) * (32 / R) : 0);
-    return p;
+// Four workgroups per CU level out the tail of the launch; fewer than eight steps do not pay for a workgroup's
+// resident fragments while there are CUs for longer ones, more than 64 gain nothing.
+Plan score_plan(int B, int H, int N, int causal) {
+    const long long all = (long long)((N + 31) / 32) * ((N + 31) / 32) * B / (causal ? 2 : 1);
+    const int least = all >= 2048 ? 8 : 2;
+    return H == 16 ? make_plan<ScoreTile<16, 32>>(B, N, causal, 4, least, 64) : make_plan<ScoreTile<32, 32>>(B, N, causal, 4, least, 64);
 }
 
 template <int H, int D>
 hipError_t launch_scores(const ScoreArgs &a, const void *k, const void *v, hipStream_t s) {
-    const size_t n_frag = (size_t)a.B * H * a.n_rt32 * 2 * (D / 32);
-    headmix_frag_order_kernel<D><<<(unsigned)((n_frag + 3) / 4), 256, 0, s>>>(a.N, a.n_rt32 * 2, (const bf16_t *)k, (const bf16_t *)v,
-                                                                            (bf16_t *)a.KF, (bf16_t *)a.VF, n_frag);
+    launch_frag_order<D>(a.B * H, a.N, k, v, a.KF, a.VF, s);
     constexpr int lds = ScoreTile<H, D>::lds;
-    static_assert(lds <= 160 * 1024 && SC_WAVES * H * H * 4 <= lds, "LDS budget");
+    static_assert(lds <= 160 * 1024 && ScoreTile<H, D>::WAVES * H * H * 4 <= lds, "LDS budget");
     hipError_t e = set_max_lds_once<headmix_scores_kernel<H, D>>(lds);
     if (e != hipSuccess) return e;
-    headmix_scores_kernel<H, D><<<dim3((a.n_wg + 7) / 8 * 8, a.B), SC_WAVES * 64, lds, s>>>(a);
+    headmix_scores_kernel<H, D><<<dim3((a.plan.n_wg + 7) / 8 * 8, a.B), ScoreTile<H, D>::WAVES * 64, lds, s>>>(a);
     return hipGetLastError();
 }
 
@@ -600,9 +498,9 @@ int headmix_score_wgs(int B, int H, int N, int causal) { return score_plan(B, H,
 hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,
                              const void *d_o, const float *lse, const float *Dl, void *P, void *dS, void *kv_frag, float *dw_part,
                              void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
-    const ScorePlan plan = score_plan(p.B, p.H, p.Nq, p.causal);
+    const Plan plan = score_plan(p.B, p.H, p.Nq, p.causal);
     const bool want_kv = dk != nullptr;
-    const ScoreArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), plan.steps_per_wg, plan.n_wg, p.scale,
+    const ScoreArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), plan, p.scale,
                       (const bf16_t *)q, (const bf16_t *)kv_frag, (const bf16_t *)kv_frag + headmix_frag_bytes(p) / 2, (const bf16_t *)d_o, w, lse, Dl,
                       want_kv ? (bf16_t *)P : nullptr, (bf16_t *)dS, dq ? dw_part : nullptr};
     hipError_t e = hipErrorInvalidValue;

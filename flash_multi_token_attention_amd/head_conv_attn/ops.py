@@ -52,6 +52,17 @@ def _desc(q: torch.Tensor, w: torch.Tensor, scale: float, causal: bool, out_dtyp
     return desc
 
 
+def _workspace(nbytes: int, device):
+    """A scratch buffer for bf16 score-sized blocks; None above the workspace cap or when it cannot be allocated (the
+    kernels that need none, or O(N), run then)."""
+    if nbytes > max_workspace_bytes():
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def forward(q, k, v, w, scale: float = 1.0, causal: bool = False) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """(O, L, M): O [B,H,N,d] in q's dtype, L = sum_j exp(Z - M) and M = max_j Z, float32 [B,H,N]."""
     out_dtype = torch.bfloat16 if q.dtype == torch.bfloat16 else torch.float32
@@ -64,8 +75,13 @@ def forward(q, k, v, w, scale: float = 1.0, causal: bool = False) -> Tuple[torch
     o = torch.empty(B, H, N, d, dtype=out_dtype, device=q.device)
     l = torch.empty(B, H, N, dtype=torch.float32, device=q.device)
     m = torch.empty_like(l)
-    rc = _lib.load().convattn_headmix_fwd(C.byref(desc), _ptr(qb), _ptr(kb), _ptr(vb), _ptr(wf), _ptr(o), _ptr(l),
-                                          _ptr(m), _stream(q))
+    lib = _lib.load()
+    ins = [_ptr(t) for t in (qb, kb, vb, wf)]
+    ws = _workspace(lib.convattn_headmix_fwd_workspace_bytes(C.byref(desc)), q.device)
+    if ws is not None:
+        rc = lib.convattn_headmix_fwd_ws(C.byref(desc), *ins, _ptr(ws), _ptr(o), _ptr(l), _ptr(m), _stream(q))
+    else:
+        rc = lib.convattn_headmix_fwd(C.byref(desc), *ins, _ptr(o), _ptr(l), _ptr(m), _stream(q))
     _lib.check(rc, "head_conv_attention_forward")
     return (o if out_dtype == q.dtype else o.to(q.dtype)), l, m
 
@@ -86,13 +102,7 @@ def _backward(want_q: bool, want_kv: bool, q, k, v, w, o, do, l, m, causal: bool
     lib = _lib.load()
     B, H, N, d = qb.shape
     ins = [_ptr(t) for t in (qb, kb, vb, wf, ob, gb, lf, mf)]
-    ws = None
-    nbytes = lib.convattn_headmix_bwd_fused_workspace_bytes(C.byref(desc))
-    if nbytes <= max_workspace_bytes():
-        try:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-        except torch.OutOfMemoryError:
-            pass
+    ws = _workspace(lib.convattn_headmix_bwd_fused_workspace_bytes(C.byref(desc)), q.device)
     gt = grad_dtype if ws is not None else torch.float32
     dq = torch.empty(B, H, N, d, dtype=gt, device=q.device) if want_q else None
     dw = torch.empty(H, H, dtype=torch.float32, device=q.device) if want_q else None

@@ -317,6 +317,14 @@ int convattn_headmix_validate(const convattn_headmix_desc *desc);
 int convattn_headmix_fwd(const convattn_headmix_desc *desc, const void *q, const void *k, const void *v,
                          const float *w, void *o, float *l, float *m, void *stream);
 
+/*
+ * The same with a scratch buffer (not initialised by the caller) that holds the probabilities as bf16 (2 B H N^2
+ * bytes, causal: half of it) between the kernel that mixes the heads and the product with V.
+ */
+size_t convattn_headmix_fwd_workspace_bytes(const convattn_headmix_desc *desc);
+int convattn_headmix_fwd_ws(const convattn_headmix_desc *desc, const void *q, const void *k, const void *v,
+                            const float *w, void *workspace, void *o, float *l, float *m, void *stream);
+
 /* Bytes of the scratch buffer the two backward entry points need (D and LSE of every row, the dW
  * partials of every row tile); its contents need not be initialised.  0 on a bad descriptor. */
 size_t convattn_headmix_bwd_workspace_bytes(const convattn_headmix_desc *desc);
