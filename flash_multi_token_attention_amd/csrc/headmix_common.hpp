@@ -24,6 +24,14 @@ template <int ROR> __device__ __forceinline__ float row16_rot(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + ROR, 0xf, 0xf, true));
 }
 
+// base (the same in all lanes) + a lane's byte offset: the form the loads and stores take with the base in scalar registers
+template <typename V> __device__ __forceinline__ const V *at(const bf16_t *base, unsigned off) {
+    return reinterpret_cast<const V *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename V> __device__ __forceinline__ V *at(bf16_t *base, unsigned off) {
+    return reinterpret_cast<V *>(reinterpret_cast<char *>(base) + off);
+}
+
 constexpr int kBlock = kChainRows * kChainKeys;   // elements of a block
 
 // H heads, WAVES waves, R rows; 64 pairs per wave in the mixing phase: lane n = RW rows x NQ quads of keys.

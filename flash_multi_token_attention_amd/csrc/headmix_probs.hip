@@ -42,7 +42,7 @@ struct ProbArgs {
 template <int H, int D>
 __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_kernel(ProbArgs a) {
     using T = ProbTile<H, D>;
-    constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, HPW = T::HPW, HB = T::HB,
+    constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, RW = T::RW, HS = T::HS, HPW = T::HPW, HB = T::HB,
                   KS = D / 32, NCH = HPW * KB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     float *lds = reinterpret_cast<float *>(smem);
@@ -211,8 +211,13 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     lds_barrier();
     for (int u = s0; u < s_end; ++u) {
         float *cur = (u - s0) & 1 ? buf1 : buf0, *nxt = (u - s0) & 1 ? buf0 : buf1;
-        if (u + 1 < s_end) scores(nxt, u + 1, min(u + 2, s_end - 1));
+        // (half of the waves take the scores of the next step first, half the mix of this one: one half's LDS and vector work
+        // runs under the other's products)
+        const bool first = wave < T::WAVES / 2, more = u + 1 < s_end;
+        const int ahead = min(u + 2, s_end - 1);
+        if (more && first) scores(nxt, u + 1, ahead);
         probs(cur, u);
+        if (more && !first) scores(nxt, u + 1, ahead);
         lds_barrier();
     }
 

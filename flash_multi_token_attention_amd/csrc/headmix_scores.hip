@@ -19,16 +19,20 @@ namespace {
 using namespace headmix;
 constexpr int SC_BLK = kBlock;
 
-// 8 waves of 256 registers: 512 pairs per step, 32 rows x 16 keys with 16 heads, 16 rows x 32 keys with 32 (the
-// resident row fragments of 32 heads take the registers of 16 heads' 32 rows).
+// 8 waves of 256 registers.  16 heads: 32 rows x 16 keys per step, two tile buffers; 32 heads: 16 rows x 32 keys, one.
 template <int H, int D> struct ScoreTile : Tile<H, 8, H == 16 ? 32 : 16> {
     using B = Tile<H, 8, H == 16 ? 32 : 16>;
-    static constexpr int NBUF = H == 16 ? 2 : 1;
-    static constexpr bool STATS_LDS = H * D >= 2048;          // LSE and D of the tile rows: registers are short
-    static constexpr int w_off = NBUF * 2 * B::arr, wt_off = w_off + H * B::WST, st_off = wt_off + H * B::WST,
-                         lds = (st_off + (STATS_LDS ? 2 * B::R * B::WST : 0)) * 4;
-    // chunks of K and V rows in flight during the mixing phase, as far as the registers go
-    static constexpr int AHEAD = H == 32 && D == 128 ? 1 : 2;
+    static constexpr int SPW = 2 * B::HPW;                  // heads of a wave in the score phase
+    static constexpr int ROOM = B::R * (D * 2 + 16);        // a head's rows while they are turned
+    // LDS per head: scores, then dP (then dZ in its place) at a distance that fits the instructions' offsets; +4 floats as in Tile
+    static constexpr int DP = B::R * B::KT, HS = 2 * DP + 4, NBUF = H == 16 ? 2 : 1;
+    static constexpr bool STATS_LDS = D >= 64;               // LSE and D of the tile rows: registers are short
+    static constexpr int w_off = NBUF * H * HS, wt_off = w_off + H * B::WST, st_off = wt_off + H * B::WST,
+                         used = (st_off + (STATS_LDS ? 2 * B::R * B::WST : 0)) * 4, lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
+    // chunks (one head, 16 keys) of K or V rows in registers, and how many of them stay in flight during the mixing phase
+    // (B4 H16 N4096 d128: 2 / 3 / 4 chunks 1.24 / 1.18 / 1.29 ms, the last with registers spilled; without the two orders of
+    // scores and mix 1.34)
+    static constexpr int RING = H == 16 ? (D == 128 ? 3 : 4) : 2, AHEAD = H == 16 ? RING : D == 128 ? 0 : 2;
 };
 
 struct ScoreArgs {
@@ -37,15 +41,15 @@ struct ScoreArgs {
     float scale;
     const bf16_t *Q, *KF, *VF, *dO;   // KF, VF: fragment order
     const float *W, *lse, *Dl;
-    bf16_t *P, *dS;      // blocks; P may be null (dQ and dW only)
+    bf16_t *P, *dS;      // blocks
     float *dw_part;      // [B][n_wg][H][H], or null
 };
 
 template <int H, int D>
 __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_kernel(ScoreArgs a) {
     using T = ScoreTile<H, D>;
-    constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, HPW = T::HPW,
-                  HB = T::HB, KS = D / 32, NCH = HPW * KB;
+    constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, DP = T::DP, SPW = T::SPW,
+                  HB = T::HB, KS = D / 32, NCH = SPW * KB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     float *lds = reinterpret_cast<float *>(smem);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
@@ -55,20 +59,15 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
     if (!find_unit<T>(a.causal, a.n_rt32, a.plan, id, rt, chunk, s0, s_end)) return;
     const int i0 = rt * R, N = a.N;
     const size_t bo = (size_t)b * H * N * D;
-    const int h0 = wave * HPW;
+    // score phase: the first half of the waves takes S = Q K^T, the second half dP = dO V^T, SPW heads each
+    const int mat = wave / (T::WAVES / 2), h0 = (wave - mat * (T::WAVES / 2)) * SPW;
 
-    // ---- resident: Q and dO fragments of this wave's heads (rows loaded whole, turned in the wave's share of the LDS) ----
-    bf16x8 qf[HPW][RB][KS], of[HPW][RB][KS];
-    {
-        constexpr int ROOM = T::NBUF * 2 * T::arr * 4 / T::WAVES / 16 * 16;
-        static_assert(R * (D * 2 + 16) <= ROOM, "room for one head's rows");
+    // ---- resident: Q or dO fragments of this wave's heads ----
+    bf16x8 qf[SPW][RB][KS];
 #pragma unroll
-        for (int t = 0; t < HPW; ++t) {
-            turn_rows<T, D>(qf[t], a.Q + bo + (size_t)(h0 + t) * N * D, i0, N, smem + wave * ROOM);
-            turn_rows<T, D>(of[t], a.dO + bo + (size_t)(h0 + t) * N * D, i0, N, smem + wave * ROOM);
-        }
-        lds_barrier();   // the score tiles go where the other waves' rows are
-    }
+    for (int t = 0; t < SPW; ++t)
+        turn_rows<T, D>(qf[t], (mat ? a.dO : a.Q) + bo + (size_t)(h0 + t) * N * D, i0, N, smem + wave * T::ROOM);
+    lds_barrier();   // the score tiles go where the other waves' rows are
     // ---- the mixing phase: lane (g, n) = heads 4g .. 4g+3 of each block of 16, tile row lr, keys 4q .. 4q+3 ----
     const int lr = wave * RW + (n & (RW - 1)), q4 = n / RW;
     const int row = T::row(i0, lr);
@@ -106,32 +105,23 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
 #pragma unroll
         for (int y = 0; y < HB; ++y) acc_w[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-    // ---- score phase, in chunks of one head and 16 keys whose K and V rows are loaded two chunks ahead ----
-    bf16x8 kf[2][KS], vf[2][KS];
+    // ---- score phase, in chunks of one head and 16 keys whose rows are loaded two chunks ahead ----
+    bf16x8 kf[T::RING][KS];
     const int n_t16 = a.n_rt32 * 2;
-    auto load_chunk = [&](int buf, int step, int c) {
-        const int t = c / KB, kb = c % KB;
-        const size_t o = (((size_t)b * H + h0 + t) * n_t16 + step * KB + kb) * KS * 512;
-        const bf16_t *kp = a.KF + o, *vp = a.VF + o;   // (the same in all lanes)
+    const bf16_t *frag = (mat ? a.VF : a.KF) + ((size_t)b * H + h0) * n_t16 * KS * 512;
+    auto load_chunk = [&](int step, int c) {
+        const bf16_t *kp = frag + ((size_t)(c / KB) * n_t16 + step * KB + c % KB) * KS * 512;   // (the same in all lanes)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            kf[buf][ks] = *reinterpret_cast<const bf16x8 *>(kp + lane * 8 + ks * 512);
-            vf[buf][ks] = *reinterpret_cast<const bf16x8 *>(vp + lane * 8 + ks * 512);
-        }
+        for (int ks = 0; ks < KS; ++ks) kf[c % T::RING][ks] = *at<bf16x8>(kp, (unsigned)lane * 16 + ks * 1024);
     };
-    auto score_chunk = [&](float *S, int buf, int c) {
+    auto score_chunk = [&](float *S, int c) {
         const int t = c / KB, kb = c % KB;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
+            f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                s = mfma_bf16(kf[buf][ks], qf[t][rb][ks], s);
-                dp = mfma_bf16(vf[buf][ks], of[t][rb][ks], dp);
-            }
-            float *dst = S + (h0 + t) * HS + (rb * 16 + n) * KT + 4 * T::slot(rb * 16 + n, 4 * kb + g);
-            *reinterpret_cast<f32x4 *>(dst) = s;
-            *reinterpret_cast<f32x4 *>(dst + T::arr) = dp;
+            for (int ks = 0; ks < KS; ++ks) s = mfma_bf16(kf[c % T::RING][ks], qf[t][rb][ks], s);
+            *reinterpret_cast<f32x4 *>(S + mat * DP + (h0 + t) * HS + (rb * 16 + n) * KT + 4 * T::slot(rb * 16 + n, 4 * kb + g)) = s;
         }
     };
 
@@ -139,9 +129,10 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
     const int pos = lr * KT + 4 * T::slot(lr, q4);
     // element of a block for this lane: [row parity][key half][row pair][16 keys]
     const int brow = row & 31;
-    auto mix_step = [&](float *S, int step, auto masked_c) {
-        constexpr bool masked = decltype(masked_c)::value;
-        float *dP = S + T::arr;
+    const unsigned out = 2 * ((((brow & 1) * 2 + (q4 >> 2)) * 16 + (brow >> 1)) * 16 + 4 * (q4 & 3) + 4 * g * SC_BLK);
+    const int key_max = a.causal ? min(row, N - 1) : N - 1;   // last key the row sees
+    auto mix = [&](float *S, int step) {
+        float *dP = S + DP;
         const int j0 = step * KT;
         f32x4 z[HB][4];
 #pragma unroll
@@ -162,13 +153,24 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                     for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
             }
         }
+        // masks only where a key of the tile is past the tile's first row or past the last key
+        if ((a.causal && j0 + KT - 1 > i0) || j0 + KT > N) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const bool dead = j0 + 4 * q4 + t > key_max;
+#pragma unroll
+                for (int x = 0; x < HB; ++x)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) z[x][t][r] = dead ? kNegInf : z[x][t][r];
+            }
+        }
         const int kt = j0 / 32;
         const long long blk = chain_ds_block_off(a.causal != 0, a.n_rt32, kt) + i0 / 32 - chain_ds_first_rt(a.causal != 0, kt);
         // blocks of all heads side by side: [batch][block][head][1024]
         const long long n_blk = chain_ds_block_off(a.causal != 0, a.n_rt32, a.n_kt);
         const size_t first = ((size_t)b * n_blk + blk) * H * SC_BLK;
-        bf16_t *p_out = a.P + first, *ds_out = a.dS + first;
-        const int out = (((brow & 1) * 2 + ((j0 + 4 * q4) >> 4 & 1)) * 16 + (brow >> 1)) * 16 + ((4 * q4) & 15) + 4 * g * SC_BLK;
+        const int half = KT == 16 ? (step & 1) * 256 : 0;    // steps of 16 keys: the second half of the block's keys
+        bf16_t *p_out = a.P + first + half, *ds_out = a.dS + first + half;
 #pragma unroll
         for (int x = 0; x < HB; ++x) {
             f32x4 lse2 = lse_r[x], dl = dl_r[x];
@@ -183,19 +185,13 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                 bf16x4 pb;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    float p = fast_exp2(z[x][t][r] - lse2[r]);
-                    if constexpr (masked) {
-                        const int key = j0 + 4 * q4 + t;
-                        if (key >= N || (a.causal && key > row)) p = 0.f;
-                    }
+                    const float p = fast_exp2(z[x][t][r] - lse2[r]);
                     pb[t] = (bf16_t)p;
                     d[t] = p * (d[t] - dl[r]);
                     z[x][t][r] = d[t];
                 }
                 *reinterpret_cast<f32x4 *>(dz) = d;
-                if (a.P)
-                    __builtin_nontemporal_store(__builtin_bit_cast(u32x2, pb), reinterpret_cast<u32x2 *>(
-                        p_out + out + (16 * x + r) * SC_BLK));
+                __builtin_nontemporal_store(__builtin_bit_cast(u32x2, pb), at<u32x2>(p_out, out + (16 * x + r) * SC_BLK * 2));
             }
         }
 #pragma unroll
@@ -216,8 +212,7 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                 bf16x4 db;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) db[t] = (bf16_t)ds[t][r];
-                __builtin_nontemporal_store(__builtin_bit_cast(u32x2, db), reinterpret_cast<u32x2 *>(
-                    ds_out + out + (16 * x + r) * SC_BLK));
+                __builtin_nontemporal_store(__builtin_bit_cast(u32x2, db), at<u32x2>(ds_out, out + (16 * x + r) * SC_BLK * 2));
             }
         }
         // dw += dZ S^T over the wave's own 64 pairs: lane n = head of either operand
@@ -225,8 +220,8 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int i = 0; i < RW * NQ / 4; ++i) {
-            const int r2 = wave * RW + i / (NQ / 4), q = 4 * (i % (NQ / 4)) + g;
-            const int o = n * HS + r2 * KT + 4 * T::slot(r2, q);
+            // (quads in the order in which they lie: the sum runs over all of them)
+            const int o = n * HS + wave * RW * KT + i * 16 + 4 * g;
             f32x4 za[HB], sb[HB];
 #pragma unroll
             for (int x = 0; x < HB; ++x) {
@@ -241,50 +236,37 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                     for (int y = 0; y < HB; ++y) acc_w[x][y] = mfma4(za[x][e], sb[y][e], acc_w[x][y]);
         }
     };
-    auto mix = [&](float *S, int step) {
-        // masks only where a key of the tile is past the tile's first row or past the last key
-        if ((a.causal && step * KT + KT - 1 > i0) || step * KT + KT > N) mix_step(S, step, std::true_type{});
-        else mix_step(S, step, std::false_type{});
-    };
 
-    load_chunk(0, s0, 0);
-    if constexpr (T::AHEAD == 2) load_chunk(1, s0, 1);
+    // the chunks of `step` into S; the first AHEAD ones of step `next` are loaded on the way
+    auto scores = [&](float *S, int step, int next) {
+#pragma unroll
+        for (int c = T::AHEAD; c < T::RING; ++c) load_chunk(step, c);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            score_chunk(S, c);
+            if (c + T::RING < NCH) load_chunk(step, c + T::RING);
+            else if (c + T::RING - NCH < T::AHEAD) load_chunk(next, c + T::RING - NCH);
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < T::AHEAD; ++c) load_chunk(s0, c);
     if constexpr (T::NBUF == 2) {
-        static_assert(NCH == 2, "two chunks per step");
-        score_chunk(lds, 0, 0);
-        load_chunk(0, min(s0 + 1, s_end - 1), 0);
-        score_chunk(lds, 1, 1);
-        load_chunk(1, min(s0 + 1, s_end - 1), 1);
+        // One barrier per step.  Of the two waves of a SIMD one takes the scores of the next step first, the other the mix of
+        // this one, so that one's LDS and vector work runs under the other's products.
+        scores(lds, s0, min(s0 + 1, s_end - 1));
         lds_barrier();
         for (int u = s0; u < s_end; ++u) {
-            float *cur = lds + ((u - s0) & 1) * 2 * T::arr, *nxt = lds + ((u - s0 + 1) & 1) * 2 * T::arr;
-            const bool more = u + 1 < s_end;
+            float *cur = lds + ((u - s0) & 1) * H * HS, *nxt = lds + ((u - s0 + 1) & 1) * H * HS;
+            const bool first = wave < T::WAVES / 2, more = u + 1 < s_end;
             const int ahead = min(u + 2, s_end - 1);
-            if (more) {
-                score_chunk(nxt, 0, 0);
-                load_chunk(0, ahead, 0);
-            }
+            if (more && first) scores(nxt, u + 1, ahead);
             mix(cur, u);
-            if (more) {
-                score_chunk(nxt, 1, 1);
-                load_chunk(1, ahead, 1);
-            }
+            if (more && !first) scores(nxt, u + 1, ahead);
             lds_barrier();
         }
     } else {
         for (int u = s0; u < s_end; ++u) {
-#pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                if constexpr (T::AHEAD == 1) {
-                    if (c + 1 < NCH) load_chunk((c + 1) & 1, u, c + 1);
-                    score_chunk(lds, c & 1, c);
-                } else {
-                    score_chunk(lds, c & 1, c);
-                    if (c + 2 < NCH) load_chunk(c & 1, u, c + 2);
-                    else load_chunk(c & 1, min(u + 1, s_end - 1), c + 2 - NCH);
-                }
-            }
-            if constexpr (T::AHEAD == 1) load_chunk(0, min(u + 1, s_end - 1), 0);
+            scores(lds, u, min(u + 1, s_end - 1));
             lds_barrier();
             mix(lds, u);
             lds_barrier();
@@ -502,7 +484,7 @@ hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const
     const bool want_kv = dk != nullptr;
     const ScoreArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), plan, p.scale,
                       (const bf16_t *)q, (const bf16_t *)kv_frag, (const bf16_t *)kv_frag + headmix_frag_bytes(p) / 2, (const bf16_t *)d_o, w, lse, Dl,
-                      want_kv ? (bf16_t *)P : nullptr, (bf16_t *)dS, dq ? dw_part : nullptr};
+                      (bf16_t *)P, (bf16_t *)dS, dq ? dw_part : nullptr};
     hipError_t e = hipErrorInvalidValue;
     if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, k, v, s) : p.d == 64 ? launch_scores<16, 64>(a, k, v, s) : launch_scores<16, 128>(a, k, v, s);
     if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, k, v, s) : p.d == 64 ? launch_scores<32, 64>(a, k, v, s) : launch_scores<32, 128>(a, k, v, s);
