@@ -87,6 +87,7 @@ _SIGNATURES = {
 EXPORTS = tuple(_SIGNATURES)
 
 _lib = None
+_host = None
 _lock = threading.Lock()
 
 
@@ -108,6 +109,24 @@ def load() -> C.CDLL:
                 fn.restype, fn.argtypes = res, args
             _lib = lib
     return _lib
+
+
+def host():
+    """The native host path (csrc/host.cpp) on top of the loaded library; raises if it has not been built."""
+    global _host
+    if _host is not None:
+        return _host
+    load()
+    with _lock:
+        if _host is None:
+            try:
+                from . import _host as h
+            except ImportError as e:
+                raise RuntimeError(f"the native host path (_host.so) cannot be loaded: {e}; build it with "
+                                   "`python -m flash_multi_token_attention_amd.build`") from e
+            h.init(LIB_PATH)
+            _host = h
+    return _host
 
 
 def strerror(code: int) -> str:

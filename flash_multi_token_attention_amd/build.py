@@ -1,9 +1,10 @@
 """Ahead-of-time build of the conv-attention HIP library for gfx950.
 
 ``python -m flash_multi_token_attention_amd.build`` (or ``setup.py build_ext``)
-compiles every source under ``csrc/`` with hipcc and links
-``libconvattn_hip.so`` next to this file.  hipcc cross-compiles, so no GPU is
-needed to build.
+compiles every HIP source under ``csrc/`` with hipcc and links
+``libconvattn_hip.so`` next to this file, and the native host path
+(``csrc/host.cpp``, no device code) with g++ against the installed torch into
+``_host.so``.  hipcc cross-compiles, so no GPU is needed to build.
 """
 from __future__ import annotations
 
@@ -19,6 +20,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 LIB_NAME = "libconvattn_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 
 # MFMA results in ordinary VGPRs (the 512-register dQ kernel otherwise copies every transient
 # accumulator out of the accumulation file).  Not for the dK/dV kernel: with its two tile loops
@@ -76,6 +78,24 @@ def _compile(cc: str, src: str, obj: str, extra) -> None:
         sys.stderr.write(err + "\n")
 
 
+def _compile_host() -> None:
+    import sysconfig
+    import torch
+    t = os.path.dirname(os.path.abspath(torch.__file__))
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           os.path.join(rocm, "include"), sysconfig.get_paths()["include"], INCLUDE]
+    tmp = HOST_PATH + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-DTORCH_EXTENSION_NAME=_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[a for i in inc for a in ("-isystem", i)], os.path.join(CSRC, "host.cpp"), "-o", tmp, "-L" + os.path.join(t, "lib"),
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-Wl,-rpath," + os.path.join(t, "lib")]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for host.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = True, extra_flags=()) -> str:
     """Compile all sources (always, even if the library exists) and link."""
     cc = hipcc()
@@ -85,7 +105,9 @@ def build(verbose: bool = True, extra_flags=()) -> str:
     for name, obj_name, unit_flags in UNITS:
         jobs.append((os.path.join(CSRC, name), os.path.join(obj_dir, obj_name + ".o"), unit_flags))
     with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
+        host = ex.submit(_compile_host)
         list(ex.map(lambda so: _compile(cc, so[0], so[1], [*so[2], *extra_flags]), jobs))
+        host.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", *[j[1] for j in jobs], "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -93,7 +115,7 @@ def build(verbose: bool = True, extra_flags=()) -> str:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB_PATH)
     if verbose:
-        print(f"built {LIB_PATH}")
+        print(f"built {LIB_PATH} and {HOST_PATH}")
     return LIB_PATH
 
 

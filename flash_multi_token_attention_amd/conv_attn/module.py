@@ -9,14 +9,52 @@ import math
 import torch
 import torch.nn as nn
 
+from .. import _lib
 from . import ops
+
+
+def _backward(Q, K, V, conv_kernel, M, L, O, dO, scale, pad_q, pad_k, causal, need_q, need_k, need_v, need_w):
+    """[dQ, dK, dV, dconv_kernel], None for those not wanted."""
+    D, LSE = ops.bwd_preprocess(O, dO, M, L)
+    args = (Q, K, V, dO, D, LSE, conv_kernel, scale, pad_q, pad_k, causal)
+    dQ = dW = dK = dV = None
+    if (need_q or need_w) and (need_k or need_v):
+        dQ, dK, dV, dW = ops.backward(*args, out_dtype=Q.dtype)
+        return [dQ, dK, dV, dW.to(conv_kernel.dtype)]
+    if need_q or need_w:
+        dQ, dW = ops.dq_backward(*args, out_dtype=Q.dtype)
+        dW = dW.to(conv_kernel.dtype)
+    if need_k or need_v:
+        dK, dV = ops.dkdv_backward(*args, out_dtype=Q.dtype)
+    return [dQ, dK, dV, dW]
+
+
+_native = None
+
+
+def _host():
+    global _native
+    if _native is None:
+        h = _lib.host()
+        h.set_slow_backward("window", _backward)
+        _native = h
+    return _native
 
 
 class FlashConvAttentionCUDAFunction(torch.autograd.Function):
     """O = conv_attention(Q, K, V, conv_kernel).  bf16 or fp32 inputs (fp32 runs
     the fp32-arithmetic kernels); O and the gradients come back in the input
     dtype, dconv_kernel in the dtype of ``conv_kernel``.  M, L, LSE and D stay
-    fp32 between forward and backward."""
+    fp32 between forward and backward.  ``apply`` runs the native host path (csrc/host.cpp) where it takes the
+    call; ``forward`` and ``backward`` below are what it does for everything else."""
+
+    @classmethod
+    def apply(cls, Q, K, V, conv_kernel, scale, pad_q, pad_k, causal):
+        if cls is FlashConvAttentionCUDAFunction and all(isinstance(t, torch.Tensor) for t in (Q, K, V, conv_kernel)):
+            O = _host().window_attention(Q, K, V, conv_kernel, scale, pad_q, pad_k, bool(causal))
+            if O is not None:
+                return O
+        return super().apply(Q, K, V, conv_kernel, scale, pad_q, pad_k, causal)
 
     @staticmethod
     def forward(ctx, Q, K, V, conv_kernel, scale, pad_q, pad_k, causal):
@@ -34,19 +72,8 @@ class FlashConvAttentionCUDAFunction(torch.autograd.Function):
     def backward(ctx, dO):
         Q, K, V, conv_kernel, M, L, O = ctx.saved_tensors
         dO = dO.to(Q.dtype).contiguous()
-        D, LSE = ops.bwd_preprocess(O, dO, M, L)
-        args = (Q, K, V, dO, D, LSE, conv_kernel, ctx.scale, ctx.pad_q, ctx.pad_k, ctx.causal)
-        need_q, need_k, need_v, need_w = ctx.needs_input_grad[:4]
-        dQ = dW = dK = dV = None
-        if (need_q or need_w) and (need_k or need_v):
-            dQ, dK, dV, dW = ops.backward(*args, out_dtype=Q.dtype)
-            return dQ, dK, dV, dW.to(conv_kernel.dtype), None, None, None, None
-        if need_q or need_w:
-            dQ, dW = ops.dq_backward(*args, out_dtype=Q.dtype)
-            dW = dW.to(conv_kernel.dtype)
-        if need_k or need_v:
-            dK, dV = ops.dkdv_backward(*args, out_dtype=Q.dtype)
-        return dQ, dK, dV, dW, None, None, None, None
+        return (*_backward(Q, K, V, conv_kernel, M, L, O, dO, ctx.scale, ctx.pad_q, ctx.pad_k, ctx.causal,
+                           *ctx.needs_input_grad[:4]), None, None, None, None)
 
 
 class ConvAttentionCUDA(nn.Module):

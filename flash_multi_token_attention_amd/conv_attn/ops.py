@@ -293,6 +293,12 @@ def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.
     K and V may be views ``cache[:, :, :Nk]`` of a cache allocated as [B,H,N_max,d] (same
     strides for both): they are read in place, where the reference's CHECK_CONTIGUOUS
     (conv_attn/kernels/fwd_inference_wrapper.cu:8,26-27) forces a copy per step."""
+    if workspace is None and not exact and all(isinstance(t, torch.Tensor) for t in (Q, K, V, conv_kernel)) and K.dim() == 4:
+        # the ordinary case in one native call; anything it does not take comes back as None and is checked below
+        r = _lib.host().decode_dense(Q, K, V, conv_kernel, k_splits or default_k_splits(Q.shape[0], Q.shape[1], K.shape[2]),
+                                     scale, bool(causal), out_dtype)
+        if r is not None:
+            return r[0], r[1], r[2], r[3:]
     _check_qkv(Q, K, V, kv_views=True)
     if K.stride() != V.stride():
         raise RuntimeError("K and V must have the same strides")
@@ -331,15 +337,31 @@ def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.
     return O, M, L, (O_part, M_part, L_part)
 
 
+def _kv_splits(B: int, H: int, H_kv: int, Nk: int, c_q: int) -> int:
+    """Default split count with shared KV heads: a workgroup takes 4 or 2 query heads of one KV head when the window has at
+    most 8 query taps."""
+    group = H // max(1, H_kv or H)
+    heads_per_wg = 1 if c_q > 8 else 4 if group % 4 == 0 else 2 if group % 2 == 0 else 1
+    return default_k_splits(B, H // heads_per_wg, Nk)
+
+
+def _decode_kv_native(Q, K, V, block_table, seq_lens, Nk, conv_kernel, k_splits, scale, causal, out_dtype, what):
+    """The ordinary case in one native call; None when the caller has to check (and raise or convert) itself."""
+    if not (isinstance(Q, torch.Tensor) and isinstance(K, torch.Tensor) and Q.dim() == 4 and K.dim() == 4 and conv_kernel.dim() == 3
+            and K.shape[1] > 0 and Q.shape[1] % K.shape[1] == 0):
+        return None
+    r = _lib.host().decode_kv(Q, K, V, block_table, seq_lens, Nk, conv_kernel,
+                              k_splits or _kv_splits(Q.shape[0], Q.shape[1], K.shape[1], Nk, conv_kernel.shape[1]),
+                              scale, bool(causal), out_dtype, what)
+    return r if r is None else (r[0], r[1], r[2], r[3:])
+
+
 def _decode_kv(Q, K, V, layout: "_lib.KvLayout", Nk: int, conv_kernel, k_splits, scale, causal, out_dtype, what: str):
     B, H, r, d = Q.shape
     c_q, c_k = conv_kernel.shape[1], conv_kernel.shape[2]
     W = _weights(conv_kernel, H, c_q - 1, (c_k - 1) // 2, Q.device)
     if not k_splits:
-        # a workgroup takes 4 or 2 query heads of one KV head when the window has at most 8 query taps
-        group = H // max(1, layout.H_kv or H)
-        heads_per_wg = 1 if c_q > 8 else 4 if group % 4 == 0 else 2 if group % 2 == 0 else 1
-        k_splits = default_k_splits(B, H // heads_per_wg, Nk)
+        k_splits = _kv_splits(B, H, layout.H_kv, Nk, c_q)
     if out_dtype not in _DT:
         raise RuntimeError("out_dtype must be bfloat16 or float32")
     desc = _lib.Desc(B, H, r, Nk, d, c_q, c_k, float(scale), int(bool(causal)), _DT[Q.dtype], _DT[out_dtype],
@@ -377,6 +399,10 @@ def decode_gqa(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=to
     h // (H // H_kv), the window weights stay per query head.  ``seq_lens`` (int32 [B] on the device,
     each 1..Nk) gives every batch entry its own number of keys.  -> (O [B,H,1,d], M, L, partials).
     bf16 only (the streaming decode kernel)."""
+    r = _decode_kv_native(Q, K, V, None, seq_lens, K.shape[2] if K.dim() == 4 else 0, conv_kernel, k_splits, scale, causal,
+                          out_dtype, "conv_attn.decode_gqa")
+    if r is not None:
+        return r
     for t, n in ((Q, "Q"), (K, "K"), (V, "V")):
         if t.dim() != 4:
             raise RuntimeError(f"{n} must be [batch, heads, seq_len, d_head]")
@@ -405,6 +431,10 @@ def decode_paged(Q, k_pool, v_pool, block_table, seq_lens, max_seq_len, conv_ker
     [B] on the device or None (then every entry has ``max_seq_len`` keys); ``max_seq_len`` is a host
     integer (no device synchronisation).  H may be a multiple of H_kv.
     -> (O [B,H,1,d], M, L, partials).  bf16 only (the streaming decode kernel)."""
+    r = _decode_kv_native(Q, k_pool, v_pool, block_table, seq_lens, int(max_seq_len), conv_kernel, k_splits, scale, causal,
+                          out_dtype, "conv_attn.decode_paged")
+    if r is not None:
+        return r
     if k_pool.dim() != 4 or k_pool.shape != v_pool.shape or not k_pool.is_contiguous() or not v_pool.is_contiguous():
         raise RuntimeError("k_pool and v_pool must be contiguous [n_pages, kv_heads, page_size, d_head] tensors of one shape")
     if Q.dim() != 4 or not Q.is_contiguous() or not Q.is_cuda or not k_pool.is_cuda:

@@ -30,9 +30,9 @@ template <int H, int D> struct ScoreTile : Tile<H, 8, H == 16 ? 32 : 16> {
     static constexpr int w_off = NBUF * H * HS, wt_off = w_off + H * B::WST, st_off = wt_off + H * B::WST,
                          used = (st_off + (STATS_LDS ? 2 * B::R * B::WST : 0)) * 4, lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
     // chunks (one head, 16 keys) of K or V rows in registers, and how many of them stay in flight during the mixing phase
-    // (B4 H16 N4096 d128: 2 / 3 / 4 chunks 1.24 / 1.18 / 1.29 ms, the last with registers spilled; without the two orders of
-    // scores and mix 1.34)
-    static constexpr int RING = H == 16 ? (D == 128 ? 3 : 4) : 2, AHEAD = H == 16 ? RING : D == 128 ? 0 : 2;
+    static constexpr int RING = H == 16 ? 4 : 2, AHEAD = H == 16 ? (D == 128 ? 2 : 4) : D == 128 ? 0 : 2;
+    // (B4 H16 N4096 d128: 2 / 3 / 4 chunks in flight 1.27 / 1.33 / 1.32 ms; without the two orders of scores and mix 1.34)
+    static_assert(SPW * B::KB % RING == 0, "a chunk's registers are the same in every step");
 };
 
 struct ScoreArgs {

@@ -8,10 +8,47 @@ import torch
 import torch.nn as nn
 from torch.autograd import Function
 
+from .. import _lib
 from .ops import backward, bwd_dkdv, bwd_dq_dw, forward
 
 
+def _backward(q, k, v, w, output, grad_output, l, m, causal, scale, want_q, want_kv):
+    """[dq, dk, dv, dw] in the dtypes of their tensors, None for those not wanted."""
+    gq = gk = gv = gw = None
+    if want_q and want_kv:
+        lo = torch.bfloat16 if q.dtype == k.dtype == v.dtype == torch.bfloat16 else torch.float32
+        gq, gk, gv, gw = backward(q, k, v, w, output, grad_output, l, m, causal=causal, scale=scale, out_dtype=lo)
+    elif want_q:
+        gq, gw = bwd_dq_dw(q, k, v, w, output, grad_output, l, m, causal=causal, scale=scale)
+    elif want_kv:
+        gk, gv = bwd_dkdv(q, k, v, w, output, grad_output, l, m, causal=causal, scale=scale)
+    return [None if g is None else g.to(t.dtype) for g, t in ((gq, q), (gk, k), (gv, v), (gw, w))]
+
+
+_native = None
+
+
+def _host():
+    global _native
+    if _native is None:
+        h = _lib.host()
+        h.set_slow_backward("mix", _backward)
+        _native = h
+    return _native
+
+
 class HeadConvAttentionFunction(Function):
+    """``apply`` runs the native host path (csrc/host.cpp) where it takes the call; ``forward`` and ``backward`` are
+    what it does for everything else."""
+
+    @classmethod
+    def apply(cls, q, k, v, w, causal=False, scale=None):
+        if cls is HeadConvAttentionFunction and all(isinstance(t, torch.Tensor) for t in (q, k, v, w)):
+            out = _host().mix_attention(q, k, v, w, bool(causal), 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale)
+            if out is not None:
+                return out
+        return super().apply(q, k, v, w, causal, scale)
+
     @staticmethod
     def forward(ctx, q, k, v, w, causal=False, scale=None):
         if scale is None:
@@ -25,20 +62,9 @@ class HeadConvAttentionFunction(Function):
     @staticmethod
     def backward(ctx, grad_output):
         q, k, v, w, output, l, m = ctx.saved_tensors
-        grad_q = grad_k = grad_v = grad_w = None
         need_q, need_k, need_v, need_w = ctx.needs_input_grad[:4]
-        if (need_q or need_w) and (need_k or need_v):
-            lo = torch.bfloat16 if q.dtype == k.dtype == v.dtype == torch.bfloat16 else torch.float32
-            grad_q, grad_k, grad_v, grad_w = backward(q, k, v, w, output, grad_output, l, m, causal=ctx.causal,
-                                                      scale=ctx.scale, out_dtype=lo)
-            return (grad_q.to(q.dtype), grad_k.to(k.dtype), grad_v.to(v.dtype), grad_w.to(w.dtype), None, None)
-        if ctx.needs_input_grad[0] or ctx.needs_input_grad[3]:
-            grad_q, grad_w = bwd_dq_dw(q, k, v, w, output, grad_output, l, m, causal=ctx.causal, scale=ctx.scale)
-            grad_q, grad_w = grad_q.to(q.dtype), grad_w.to(w.dtype)
-        if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
-            grad_k, grad_v = bwd_dkdv(q, k, v, w, output, grad_output, l, m, causal=ctx.causal, scale=ctx.scale)
-            grad_k, grad_v = grad_k.to(k.dtype), grad_v.to(v.dtype)
-        return grad_q, grad_k, grad_v, grad_w, None, None
+        return (*_backward(q, k, v, w, output, grad_output, l, m, ctx.causal, ctx.scale, need_q or need_w, need_k or need_v),
+                None, None)
 
 
 class HeadConvAttention(nn.Module):

@@ -28,7 +28,7 @@ setup(
     version="0.1.0",
     description="MI355X-native fused conv-attention (multi-token attention), drop-in for flash_multi_token_attention.conv_attn",
     packages=find_packages(include=["flash_multi_token_attention_amd*", "flash_multi_token_attention*"]),
-    package_data={"flash_multi_token_attention_amd": ["libconvattn_hip.so", "csrc/*"]},
+    package_data={"flash_multi_token_attention_amd": ["libconvattn_hip.so", "_host.so", "csrc/*"]},
     python_requires=">=3.8",
     install_requires=["torch"],
     cmdclass={"build_ext": build_ext, "build_py": build_py},
