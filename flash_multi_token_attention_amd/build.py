@@ -32,6 +32,7 @@ VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 UNITS = [
     ("api.hip", "api", []),
     ("generic_kernels.hip", "generic_kernels", []),
+    ("staged_fp32.hip", "staged_fp32", []),
     ("reduce_kernels.hip", "reduce_kernels", []),
     ("fwd_reg_mfma.hip", "fwd_reg_mfma", []),
     ("bwd_dq_mfma.hip", "bwd_dq_mfma", VGPR_FORM),

@@ -119,6 +119,32 @@ def kernel_path(Q, K, conv_kernel, causal=True, op="fwd", exact=False) -> str:
     return "mfma" if code == 1 else "fp32"
 
 
+def _staged_workspace(desc, op: int, device):
+    """Workspace of the fp32-arithmetic path's staged kernels; None when the call does not run them (bf16 matrix-core path, a
+    workspace above the cap or one that cannot be allocated: the kernels without score-sized scratch run then)."""
+    nbytes = _lib.load().convattn_staged_workspace_bytes(C.byref(desc), op)
+    if nbytes == 0 or nbytes > max_workspace_bytes():
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def _staged_backward(desc, Q, K, V, dO, D, L, W, out_dtype, want_q: bool, want_kv: bool, what: str):
+    """(dQ, dK, dV, dW), None for those not wanted, from the staged kernels; None when they do not run."""
+    ws = _staged_workspace(desc, _lib.OP_BWD, Q.device)
+    if ws is None:
+        return None
+    dQ = torch.empty(Q.shape, dtype=out_dtype, device=Q.device) if want_q else None
+    dW = torch.empty(W.shape, dtype=torch.float32, device=Q.device) if want_q else None
+    dK, dV = (torch.empty(t.shape, dtype=out_dtype, device=Q.device) if want_kv else None for t in (K, V))
+    rc = _lib.load().convattn_staged_bwd(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(dO), _ptr(D), _ptr(L), _ptr(W),
+                                         _ptr(dQ), _ptr(dK), _ptr(dV), _ptr(dW), _ptr(ws), _stream(Q))
+    _lib.check(rc, what)
+    return dQ, dK, dV, dW
+
+
 def forward(Q, K, V, conv_kernel, scale, pad_q, pad_k, causal, out_dtype=torch.float32,
             exact=False) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Training forward -> (O [B,H,N,d], M [B,H,N], L [B,H,N]); M is the row max of
@@ -130,8 +156,13 @@ def forward(Q, K, V, conv_kernel, scale, pad_q, pad_k, causal, out_dtype=torch.f
     O = torch.empty((B, H, Nq, d), dtype=out_dtype, device=Q.device)
     M = torch.empty((B, H, Nq), dtype=torch.float32, device=Q.device)
     L = torch.empty((B, H, Nq), dtype=torch.float32, device=Q.device)
-    rc = _lib.load().convattn_fwd(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), _ptr(O), _ptr(M),
-                                  _ptr(L), _stream(Q))
+    lib = _lib.load()
+    ws = _staged_workspace(desc, _lib.OP_FWD, Q.device)
+    if ws is not None:
+        rc = lib.convattn_staged_fwd(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), _ptr(ws), _ptr(O), _ptr(M), _ptr(L),
+                                     _stream(Q))
+    else:
+        rc = lib.convattn_fwd(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), _ptr(O), _ptr(M), _ptr(L), _stream(Q))
     _lib.check(rc, "conv_attn.forward")
     return O, M, L
 
@@ -176,6 +207,10 @@ def dq_backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
     W, D, L, desc = _bwd_common(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
                                 out_dtype, exact, low_memory)
     lib = _lib.load()
+    if not low_memory:
+        r = _staged_backward(desc, Q, K, V, dO, D, L, W, out_dtype, True, False, "conv_attn.dq_backward")
+        if r is not None:
+            return r[0], r[3]
     dQ = torch.empty(Q.shape, dtype=out_dtype, device=Q.device)
     nbytes = lib.convattn_dw_partial_bytes(C.byref(desc))
     if nbytes == 0:
@@ -207,6 +242,9 @@ def dkdv_backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
     """-> (dK, dV) [B,H,N,d]; same arguments as ``dq_backward``."""
     W, D, L, desc = _bwd_common(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
                                 out_dtype, exact)
+    r = _staged_backward(desc, Q, K, V, dO, D, L, W, out_dtype, False, True, "conv_attn.dkdv_backward")
+    if r is not None:
+        return r[1], r[2]
     dK = torch.empty(K.shape, dtype=out_dtype, device=Q.device)
     dV = torch.empty(V.shape, dtype=out_dtype, device=Q.device)
     rc = _lib.load().convattn_bwd_dkdv(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(dO), _ptr(D),
@@ -235,6 +273,9 @@ def backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
     W, D, L, desc = _bwd_common(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
                                 out_dtype, exact)
     lib = _lib.load()
+    r = _staged_backward(desc, Q, K, V, dO, D, L, W, out_dtype, True, True, "conv_attn.backward")
+    if r is not None:
+        return r
     nbytes = lib.convattn_bwd_fused_workspace_bytes(C.byref(desc))
     if nbytes == 0:
         _lib.check(lib.convattn_validate(C.byref(desc), _lib.OP_BWD), "conv_attn.backward")

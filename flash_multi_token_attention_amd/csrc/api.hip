@@ -306,6 +306,43 @@ int convattn_bwd_fused(const convattn_desc *desc, const void *q, const void *k, 
     return rc;
 }
 
+// fp32-arithmetic path with score-sized matrices in the caller's workspace
+static bool takes_staged(const convattn_desc *desc, int op, Problem *p) {
+    return (op == CONVATTN_OP_FWD || op == CONVATTN_OP_BWD) && validate(desc, op, p) == 0 && pick_path(desc, *p, op) != 1 && staged_ok(*p);
+}
+
+size_t convattn_staged_workspace_bytes(const convattn_desc *desc, int op) {
+    Problem p;
+    if (!takes_staged(desc, op, &p)) return 0;
+    return op == CONVATTN_OP_FWD ? staged_fwd_bytes(p) : staged_bwd_bytes(p);
+}
+
+int convattn_staged_fwd(const convattn_desc *desc, const void *q, const void *k, const void *v, const float *w, void *workspace,
+                        void *o, float *m, float *l, void *stream) {
+    Problem p;
+    int rc = validate(desc, CONVATTN_OP_FWD, &p);
+    if (rc) return rc;
+    if (!takes_staged(desc, CONVATTN_OP_FWD, &p)) return CONVATTN_ERR_SHAPE;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(w); REQUIRE_PTR(workspace);
+    REQUIRE_PTR(o); REQUIRE_PTR(m); REQUIRE_PTR(l);
+    return (int)staged_fwd(p, desc->in_dtype, desc->out_dtype, q, k, v, w, workspace, o, m, l, static_cast<hipStream_t>(stream));
+}
+
+int convattn_staged_bwd(const convattn_desc *desc, const void *q, const void *k, const void *v, const void *d_o, const float *D,
+                        const float *lse, const float *w, void *dq, void *dk, void *dv, float *dw, void *workspace,
+                        void *stream) {
+    Problem p;
+    int rc = validate(desc, CONVATTN_OP_BWD, &p);
+    if (rc) return rc;
+    if (!takes_staged(desc, CONVATTN_OP_BWD, &p)) return CONVATTN_ERR_SHAPE;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(d_o); REQUIRE_PTR(D); REQUIRE_PTR(lse); REQUIRE_PTR(w);
+    REQUIRE_PTR(workspace);
+    if (dq || dw) { REQUIRE_PTR(dq); REQUIRE_PTR(dw); }
+    if (dk || dv || !dq) { REQUIRE_PTR(dk); REQUIRE_PTR(dv); }
+    return (int)staged_bwd(p, desc->in_dtype, desc->out_dtype, q, k, v, d_o, D, lse, w, workspace, dq, dk, dv, dw,
+                           static_cast<hipStream_t>(stream));
+}
+
 size_t convattn_decode_partial_bytes(const convattn_desc *desc) {
     Problem p;
     if (validate(desc, CONVATTN_OP_DECODE, &p)) return 0;

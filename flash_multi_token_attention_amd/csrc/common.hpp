@@ -69,6 +69,16 @@ hipError_t generic_decode(const Problem &p, int in_dt, const void *q, const void
                           const float *w, float *o_part, float *m_part, float *l_part, hipStream_t s);
 inline int generic_q_tiles(const Problem &p) { return (p.Nq + kGenTR - 1) / kGenTR; }
 
+// ---- the same arithmetic with score-sized matrices in a workspace (staged_fp32.hip) ----
+bool staged_ok(const Problem &p);
+size_t staged_fwd_bytes(const Problem &p);
+size_t staged_bwd_bytes(const Problem &p);
+hipError_t staged_fwd(const Problem &p, int in_dt, int out_dt, const void *q, const void *k, const void *v, const float *w, void *ws,
+                      void *o, float *m, float *l, hipStream_t s);
+hipError_t staged_bwd(const Problem &p, int in_dt, int out_dt, const void *q, const void *k, const void *v, const void *d_o,
+                      const float *D, const float *lse, const float *w, void *ws, void *dq, void *dk, void *dv, float *dw,
+                      hipStream_t s);
+
 // ---- shape-independent helpers (reduce_kernels.hip) ----
 hipError_t bwd_preprocess(const Problem &p, int in_dt, int out_dt, const void *o, const void *d_o,
                           const float *m, const float *l, float *D, float *lse, hipStream_t s);

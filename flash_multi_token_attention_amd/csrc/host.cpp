@@ -28,7 +28,8 @@ using torch::autograd::variable_list;
 // ---- the C ABI, from the library Python has loaded ----
 #define API_LIST(F)                                                                                                   \
     F(convattn_strerror) F(convattn_fwd) F(convattn_bwd_preprocess) F(convattn_bwd_fused_workspace_bytes)              \
-    F(convattn_bwd_fused) F(convattn_decode_strided) F(convattn_decode_kv) F(convattn_decode_combine)                 \
+    F(convattn_bwd_fused) F(convattn_staged_workspace_bytes) F(convattn_staged_fwd) F(convattn_staged_bwd)               \
+    F(convattn_decode_strided) F(convattn_decode_kv) F(convattn_decode_combine)                 \
     F(convattn_headmix_validate) F(convattn_headmix_fwd_workspace_bytes) F(convattn_headmix_fwd_ws)                   \
     F(convattn_headmix_bwd_fused_workspace_bytes) F(convattn_headmix_bwd_fused)
 struct Api {
@@ -83,6 +84,7 @@ bool plain(const Tensor &t) {
                                                      c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize}));
 }
 int dt_of(const Tensor &t) { return t.scalar_type() == at::kBFloat16 ? CONVATTN_BF16 : CONVATTN_F32; }
+int64_t padded(int64_t n) { return (n + 3) & ~int64_t(3); }   // floats up to the next 16-byte boundary
 bool aligned(const Tensor &t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 
 bool same_rows(const Tensor &Q, const Tensor &K, const Tensor &V) {
@@ -117,7 +119,7 @@ py::object *window_slow_backward = nullptr, *mix_slow_backward = nullptr;
 // ------------------------------------------------------------------ window attention
 struct WindowBackward : torch::autograd::Node {
     SavedVariable q, k, v, w, o;
-    Tensor stats;        // M then L, fp32 [2][B][H][Nq]
+    Tensor stats;        // M then (from the next 16-byte boundary) L, fp32 [B][H][Nq]
     double scale = 1;
     int64_t pad_q = 0, pad_k = 0;
     bool causal = false;
@@ -144,20 +146,22 @@ struct WindowBackward : torch::autograd::Node {
             const Tensor Wf = window(W, Q.size(1), pad_q, pad_k, Q);
             convattn_desc d = window_desc(Q, K.size(2), Wf, scale, causal, dt_of(Q));
             const size_t rows = (size_t)Q.size(0) * Q.size(1) * Q.size(2), stat = (rows * 4 + 255) / 256 * 256;
-            const size_t bytes = api.convattn_bwd_fused_workspace_bytes(&d);
             // (D and LSE ahead of the workspace, which counts for the cap alone as in the Python op)
-            Tensor ws = bytes <= workspace_cap() && bytes ? workspace(bytes + 2 * stat, Q) : Tensor();
+            auto reserve = [&](size_t bytes) { return bytes && bytes <= workspace_cap() ? workspace(bytes + 2 * stat, Q) : Tensor(); };
+            Tensor ws = reserve(api.convattn_staged_workspace_bytes(&d, CONVATTN_OP_BWD));
+            const bool staged = ws.defined();
+            if (!staged) ws = reserve(api.convattn_bwd_fused_workspace_bytes(&d));
             if (ws.defined()) {
                 char *base = static_cast<char *>(ws.data_ptr());
                 float *D = reinterpret_cast<float *>(base), *lse = reinterpret_cast<float *>(base + stat);
-                const float *M = stats.const_data_ptr<float>(), *L = M + rows;
+                const float *M = stats.const_data_ptr<float>(), *L = M + padded(rows);
                 void *s = stream_of(Q);
                 Tensor dQ = empty(Q.sizes(), Q.scalar_type(), Q), dK = empty(K.sizes(), Q.scalar_type(), Q),
                        dV = empty(V.sizes(), Q.scalar_type(), Q), dW = empty(W.sizes(), at::kFloat, Q);
                 convattn_desc pre = d;
                 pre.Nk = pre.Nq; pre.c_q = pre.c_k = 1; pre.scale = 1; pre.causal = 0;
                 check(api.convattn_bwd_preprocess(&pre, O.data_ptr(), dO.data_ptr(), M, L, D, lse, s), "conv_attn.bwd_preprocess");
-                check(api.convattn_bwd_fused(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), dO.data_ptr(), D, lse,
+                check((staged ? api.convattn_staged_bwd : api.convattn_bwd_fused)(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), dO.data_ptr(), D, lse,
                                              Wf.const_data_ptr<float>(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
                                              dW.mutable_data_ptr<float>(), base + 2 * stat, s),
                       "conv_attn.backward");
@@ -168,7 +172,7 @@ struct WindowBackward : torch::autograd::Node {
         }
         const int64_t rows = Q.size(0) * Q.size(1) * Q.size(2);
         const Tensor M = stats.narrow(0, 0, rows).view({Q.size(0), Q.size(1), Q.size(2)}),
-                     L = stats.narrow(0, rows, rows).view({Q.size(0), Q.size(1), Q.size(2)});
+                     L = stats.narrow(0, padded(rows), rows).view({Q.size(0), Q.size(1), Q.size(2)});
         py::gil_scoped_acquire gil;
         auto r = (*window_slow_backward)(Q, K, V, W.detach(), M, L, O.detach(), dO, scale, pad_q, pad_k, causal,
                                          (bool)task_should_compute_output(0), (bool)task_should_compute_output(1),
@@ -203,10 +207,13 @@ std::optional<Tensor> window_attention(const Tensor &Q, const Tensor &K, const T
         if (!V.is_contiguous()) Vc = V.contiguous();
         convattn_desc d = window_desc(Qc, K.size(2), Wf, scale, causal, dt_of(Q));
         O = empty(Q.sizes(), Q.scalar_type(), Q);
-        stats = empty({2 * rows}, at::kFloat, Q);
+        stats = empty({2 * padded(rows)}, at::kFloat, Q);
         float *M = stats.mutable_data_ptr<float>();
-        check(api.convattn_fwd(&d, Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), Wf.const_data_ptr<float>(), O.data_ptr(), M,
-                               M + rows, stream_of(Q)),
+        const Tensor ws = workspace(api.convattn_staged_workspace_bytes(&d, CONVATTN_OP_FWD), Q);
+        const float *w = Wf.const_data_ptr<float>();
+        check(ws.defined() ? api.convattn_staged_fwd(&d, Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), w, ws.data_ptr(), O.data_ptr(), M,
+                                                     M + padded(rows), stream_of(Q))
+                           : api.convattn_fwd(&d, Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), w, O.data_ptr(), M, M + padded(rows), stream_of(Q)),
               "conv_attn.forward");
     }
     if (node) {

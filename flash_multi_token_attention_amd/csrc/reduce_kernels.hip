@@ -53,9 +53,10 @@ __global__ __launch_bounds__(256) void preprocess_kernel(size_t rows, int d, con
 // dW[h][tap] = sum over (batch, tile) of the partials, in a fixed order: a workgroup takes 64 taps
 // of one head (lane = tap, so a partial is read with contiguous loads); wave w adds the partials
 // w, w+4, ... in four independent chains, and the four waves' sums are added in wave order.
-__global__ __launch_bounds__(256) void dw_reduce_kernel(int B, int H, int n_tiles, int ntap,
-                                                        const float *__restrict__ part, float *__restrict__ dW) {
-    __shared__ float red[4][64];
+__global__ __launch_bounds__(1024) void dw_reduce_kernel(int B, int H, int n_tiles, int ntap,
+                                                         const float *__restrict__ part, float *__restrict__ dW) {
+    constexpr int NW = 16;
+    __shared__ float red[NW][64];
     const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int tap = blockIdx.y * 64 + lane;
     const int n = B * n_tiles;
@@ -66,16 +67,20 @@ __global__ __launch_bounds__(256) void dw_reduce_kernel(int B, int H, int n_tile
             return part[(((size_t)b * H + h) * n_tiles + t) * ntap + tap];
         };
         int q = wave;
-        for (; q + 12 < n; q += 16) {
+        for (; q + 3 * NW < n; q += 4 * NW) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] += at(q + 4 * c);
+            for (int c = 0; c < 4; ++c) s[c] += at(q + NW * c);
         }
-        for (int c = 0; q < n; q += 4, ++c) s[c] += at(q);
+        for (int c = 0; q < n; q += NW, ++c) s[c] += at(q);
     }
     red[wave][lane] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
-    if (wave == 0 && tap < ntap)
-        dW[(size_t)h * ntap + tap] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    if (wave == 0 && tap < ntap) {
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) v += red[w][lane];
+        dW[(size_t)h * ntap + tap] = v;
+    }
 }
 
 // Merge of a few decode splits: one workgroup per (batch, head), one thread per output column walks the splits.
@@ -170,7 +175,7 @@ hipError_t bwd_preprocess(const Problem &p, int in_dt, int out_dt, const void *o
 }
 
 hipError_t dw_reduce(const Problem &p, int n_tiles, const float *dw_part, float *dw, hipStream_t s) {
-    dw_reduce_kernel<<<dim3(p.H, (p.c_q * p.c_k + 63) / 64), 256, 0, s>>>(p.B, p.H, n_tiles, p.c_q * p.c_k, dw_part, dw);
+    dw_reduce_kernel<<<dim3(p.H, (p.c_q * p.c_k + 63) / 64), 1024, 0, s>>>(p.B, p.H, n_tiles, p.c_q * p.c_k, dw_part, dw);
     return hipGetLastError();
 }
 

@@ -198,6 +198,19 @@ int convattn_bwd_fused_dq(const convattn_desc *desc, const void *q, const void *
                           void *dq, void *workspace, void *stream);
 int convattn_bwd_fused_dw(const convattn_desc *desc, const void *workspace, float *dw, void *stream);
 
+/*
+ * Forward and whole backward of the fp32-arithmetic path with score-sized fp32 matrices in the caller's workspace: each
+ * (row, key) pair is convolved once instead of once per pass and tile (what convattn_fwd and convattn_bwd_fused compute
+ * for these descriptors, several times faster).  convattn_staged_workspace_bytes: 4 bytes per pair forward, 12 backward,
+ * 0 for a descriptor the matrix-core bf16 kernels run (or a bad one); the buffer is not initialised by the caller.  dq and
+ * dw, or dk and dv, may be null together.
+ */
+size_t convattn_staged_workspace_bytes(const convattn_desc *desc, int op);
+int convattn_staged_fwd(const convattn_desc *desc, const void *q, const void *k, const void *v, const float *w, void *workspace,
+                        void *o, float *m, float *l, void *stream);
+int convattn_staged_bwd(const convattn_desc *desc, const void *q, const void *k, const void *v, const void *d_o, const float *D,
+                        const float *lse, const float *w, void *dq, void *dk, void *dv, float *dw, void *workspace, void *stream);
+
 /* Bytes of o_part (fp32 [B,H,n_splits,d]); m_part and l_part are fp32 [B,H,n_splits]. */
 size_t convattn_decode_partial_bytes(const convattn_desc *desc);
 
