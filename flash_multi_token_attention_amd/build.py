@@ -44,6 +44,7 @@ UNITS = [
     ("bwd_chain3_mfma.hip", "bwd_chain3_mfma_qw", ["-DCONVATTN_CHAIN_UNIT=2"]),
     ("bwd_dq_rows.hip", "bwd_dq_rows", []),
     ("decode_stream.hip", "decode_stream", []),
+    ("decode_shared.hip", "decode_shared", []),
     ("headmix_attn.hip", "headmix_attn", []),
     ("headmix_probs.hip", "headmix_probs", []),
     ("headmix_scores.hip", "headmix_scores", []),

@@ -319,12 +319,21 @@ def backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
     return dQ, dK, dV, dW
 
 
-def default_k_splits(B: int, H: int, Nk: int) -> int:
-    """Enough (batch, head, split) workgroups to fill 256 CUs eight times over: where the read
-    stream of this machine peaks (a pure non-temporal read stream: 6.6 TB/s with 1024 workgroups
-    of 256 threads, 7.2 with 2048, 6.4 with 4096)."""
-    want = max(1, (8 * 256 + B * H - 1) // (B * H))
-    return max(1, min(want, Nk // 256 if Nk >= 256 else 1, 1024))
+def default_k_splits(B: int, H: int, Nk: int, ragged: bool = False) -> int:
+    """Split count by the model the measurements follow: a workgroup (4 waves of 64 keys per iteration) costs its iterations
+    plus about one for set-up and wind-down, and the (batch, head, split) workgroups run in rounds of one per CU.
+    The best of 1 to 4 rounds (B1 H8 N65536 d128: 32 splits 48.5 us, 64: 54, 256: 82; B8 H32 N8192 with 11 x 11
+    windows: 1 split 161 us, 8: 198; B32 H32 N8192: 1 split 616 us, 2: 630); more rounds than that where the sequences
+    have lengths of their own, since only the longest costs a whole round (B16 H8 of lengths 2048 to 8192)."""
+    most = min(Nk // 256, 1024)
+    best, splits = None, 1
+    for rounds in (1, 2, 3, 4):
+        n = min(rounds * 256 // (B * H), most)
+        if n >= 1:
+            cost = (0.7 * rounds + 0.3 if ragged else rounds) * (-(-Nk // (256 * n)) + 1)
+            if best is None or cost < best:
+                best, splits = cost, n
+    return splits
 
 
 def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.float32,
@@ -378,12 +387,21 @@ def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.
     return O, M, L, (O_part, M_part, L_part)
 
 
-def _kv_splits(B: int, H: int, H_kv: int, Nk: int, c_q: int) -> int:
-    """Default split count with shared KV heads: a workgroup takes 4 or 2 query heads of one KV head when the window has at
-    most 8 query taps."""
+def _kv_splits(B: int, H: int, H_kv: int, Nk: int, d: int, c_q: int, ragged: bool) -> int:
+    """Default split count with shared KV heads.  With d = 64 or 128 a workgroup takes 4 or 2 query heads of one KV head and
+    an even share of all keys of the batch, in tiles of 64 (512 workgroups, at least 4 tiles each): room for the parts a
+    longest entry is cut into, and for twice as many where the other entries may be shorter (the shares are smaller then).
+    With d = 32 a workgroup takes them when the window has at most 8 query taps, and a fixed split of the keys."""
     group = H // max(1, H_kv or H)
-    heads_per_wg = 1 if c_q > 8 else 4 if group % 4 == 0 else 2 if group % 2 == 0 else 1
-    return default_k_splits(B, H // heads_per_wg, Nk)
+    heads_per_wg = 4 if group % 4 == 0 else 2 if group % 2 == 0 else 1
+    if d == 32 or heads_per_wg == 1:
+        return default_k_splits(B, H // (1 if c_q > 8 else heads_per_wg), Nk, ragged)
+    tiles = -(-Nk // 64)
+    share = max(4, -(-B * (H // heads_per_wg) * tiles // 512))
+    if tiles <= 4:
+        return 1
+    parts = -(-tiles // share)
+    return min((2 if ragged and B > 1 else 1) * parts + 1, 1024, Nk)
 
 
 def _decode_kv_native(Q, K, V, block_table, seq_lens, Nk, conv_kernel, k_splits, scale, causal, out_dtype, what):
@@ -392,7 +410,8 @@ def _decode_kv_native(Q, K, V, block_table, seq_lens, Nk, conv_kernel, k_splits,
             and K.shape[1] > 0 and Q.shape[1] % K.shape[1] == 0):
         return None
     r = _lib.host().decode_kv(Q, K, V, block_table, seq_lens, Nk, conv_kernel,
-                              k_splits or _kv_splits(Q.shape[0], Q.shape[1], K.shape[1], Nk, conv_kernel.shape[1]),
+                              k_splits or _kv_splits(Q.shape[0], Q.shape[1], K.shape[1], Nk, Q.shape[3], conv_kernel.shape[1],
+                                                      seq_lens is not None),
                               scale, bool(causal), out_dtype, what)
     return r if r is None else (r[0], r[1], r[2], r[3:])
 
@@ -402,7 +421,7 @@ def _decode_kv(Q, K, V, layout: "_lib.KvLayout", Nk: int, conv_kernel, k_splits,
     c_q, c_k = conv_kernel.shape[1], conv_kernel.shape[2]
     W = _weights(conv_kernel, H, c_q - 1, (c_k - 1) // 2, Q.device)
     if not k_splits:
-        k_splits = _kv_splits(B, H, layout.H_kv, Nk, c_q)
+        k_splits = _kv_splits(B, H, layout.H_kv, Nk, d, c_q, bool(layout.seq_lens))
     if out_dtype not in _DT:
         raise RuntimeError("out_dtype must be bfloat16 or float32")
     desc = _lib.Desc(B, H, r, Nk, d, c_q, c_k, float(scale), int(bool(causal)), _DT[Q.dtype], _DT[out_dtype],

@@ -25,10 +25,11 @@
 // pages named by a block table (PAGED instance: the page numbers of the 80 rows around a 64-key
 // iteration are fetched by scalar loads one iteration ahead and handed to the lanes through LDS,
 // so the lookups do not sit in the vector-load queue between the K / V loads), and every batch
-// entry may have its own number of keys.  With shared KV heads a workgroup takes HG = 2 or 4 query
-// heads of one KV head (windows of up to 8 query taps): two heads' tap rows fill one 16-row MFMA
-// (rows 0..7 and 8..15), so the K / V stream of the KV head is read once for all of them, and only
-// the window, the softmax and P.V are repeated per head.
+// entry may have its own number of keys.  Shared KV heads with d = 64 or 128 have a kernel of their own
+// (decode_shared.hip); with d = 32 a workgroup takes HG = 2 or 4 query heads of one KV head (windows
+// of up to 8 query taps): two heads' tap rows fill one 16-row MFMA (rows 0..7 and 8..15), so the
+// K / V stream of the KV head is read once for all of them, and only the window, the softmax and P.V
+// are repeated per head.
 #include "mfma_common.hpp"
 
 namespace convattn {
@@ -349,16 +350,12 @@ bool decode_stream_ok(const Problem &p, int in_dt, unsigned flags) {
            p.pk <= 8 && p.c_q <= 16;
 }
 
-// Query heads a workgroup takes together: 4 or 2 heads of one KV head when the window's query taps
-// fit half an MFMA (8 rows), else 1.
-int decode_heads_per_wg(const Problem &p, int group) {
-    if (p.c_q > 8) return 1;
-    return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-}
-
 hipError_t decode_stream_kv(const Problem &p, const KvArgs &kv, const void *q, const void *k, const void *v,
                             const float *w, float *o_part, float *m_part, float *l_part, hipStream_t s) {
-    const int hg = decode_heads_per_wg(p, kv.group);
+    // Heads that share KV heads go to decode_shared.hip where its V fragments fit the row width (d = 64, 128); with
+    // d = 32 a workgroup here takes 4 or 2 heads of a KV head when the query taps fit half an MFMA (8 rows).
+    if (p.d != 32 && kv.group % 2 == 0) return decode_shared(p, kv, q, k, v, w, o_part, m_part, l_part, s);
+    const int hg = p.d != 32 || p.c_q > 8 ? 1 : kv.group % 4 == 0 ? 4 : kv.group % 2 == 0 ? 2 : 1;
     dim3 grid(p.n_splits, p.H / hg, p.B);
 #define CONVATTN_DECODE_LAUNCH(DD, PG, HH)                                                                   \
     decode_stream_kernel<DD, PG, HH><<<grid, NW * 64, 0, s>>>(p, kv, (const bf16_t *)q, (const bf16_t *)k,     \
@@ -370,14 +367,14 @@ hipError_t decode_stream_kv(const Problem &p, const KvArgs &kv, const void *q, c
         else CONVATTN_DECODE_LAUNCH(DD, PG, 1);                                                               \
     } while (0)
     if (p.d == 128) {
-        if (kv.table) CONVATTN_DECODE_PICK_HG(128, true);
-        else CONVATTN_DECODE_PICK_HG(128, false);
+        if (kv.table) CONVATTN_DECODE_LAUNCH(128, true, 1);
+        else CONVATTN_DECODE_LAUNCH(128, false, 1);
     } else if (p.d == 32) {
         if (kv.table) CONVATTN_DECODE_PICK_HG(32, true);
         else CONVATTN_DECODE_PICK_HG(32, false);
     } else {
-        if (kv.table) CONVATTN_DECODE_PICK_HG(64, true);
-        else CONVATTN_DECODE_PICK_HG(64, false);
+        if (kv.table) CONVATTN_DECODE_LAUNCH(64, true, 1);
+        else CONVATTN_DECODE_LAUNCH(64, false, 1);
     }
 #undef CONVATTN_DECODE_PICK_HG
 #undef CONVATTN_DECODE_LAUNCH
