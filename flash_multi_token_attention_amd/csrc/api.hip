@@ -549,7 +549,7 @@ static HeadmixFusedWs headmix_fused_ws(const convattn_headmix_desc *d) {
     HeadmixFusedWs w;
     w.lse_off = stat;
     w.part_off = 2 * stat;
-    w.kv_off = w.part_off + align256((size_t)d->B * headmix_score_wgs(d->B, d->H, d->N, p.causal) * d->H * d->H * sizeof(float));
+    w.kv_off = w.part_off + align256((size_t)headmix_score_wgs(d->B, d->H, d->N, p.causal) * d->H * d->H * sizeof(float));
     w.ds_off = w.kv_off + 2 * align256(headmix_frag_bytes(p));
     w.p_off = w.ds_off + ds;
     w.total = w.p_off + ds;

@@ -51,39 +51,76 @@ template <int H_, int WAVES_, int R_> struct Tile {
     }
 };
 
-// Key steps per workgroup and the workgroups of a batch entry (chunks of key steps, row tiles within).
-struct Plan { int steps_per_wg, n_wg, n_chunks; };
-template <typename T> Plan make_plan(int B, int N, int causal, int wgs_per_cu, int least, int most) {
-    constexpr int unit = 32 / T::KT;   // whole blocks of 32 keys
-    const int n_rt32 = (N + 31) / 32, n_tiles = n_rt32 * (32 / T::R), all = n_rt32 * unit;
-    const long long steps = causal ? (long long)n_tiles * (all + unit) / 2 : (long long)n_tiles * all;
-    long long per = steps * B / (256 * wgs_per_cu);
-    per = per < least ? least : per > most ? most : per;
+// The work of a launch: the key steps of all row tiles of all batch entries laid end to end, cut into even shares, one
+// per workgroup; a share's part of a row tile is a segment.  One round of workgroups, all done at the same time:
+// chunks of keys per row tile left the CUs with up to 335 of 258 steps at B4 H16 N4096 (55 of 33 at B2 H32 N2048), the
+// causal tiles being of all lengths and a launch five rounds.  Row tiles lie in pairs last, first, last but
+// one, second, ..: the pairs are equally long under the causal mask, so that where a share is about a pair (or a
+// simple fraction of one) neighbours walk the same keys at the same time.
+struct Plan {
+    int n_tiles, unit, split_shift;   // row tiles of a batch entry; key steps per 32 keys; log2 of the row tiles per 32 rows
+    int pair_len, entry_len;          // steps of a pair of row tiles, of a batch entry
+    int share, n_wg, max_segments;    // steps per workgroup, workgroups, segments of a row tile at most
+    int causal, n_rt32, B;
+
+    __host__ __device__ int len(int rt) const { return (causal ? (rt >> split_shift) + 1 : n_rt32) * unit; }
+    // position of row tile rt of batch entry b
+    __host__ __device__ int start(int b, int rt) const {
+        const int p = n_tiles - 1 - rt, first = p <= rt ? p * pair_len : rt * pair_len + len(p);
+        return b * entry_len + first;
+    }
+};
+template <typename T> Plan make_plan(int B, int N, int causal) {
     Plan p;
-    p.steps_per_wg = (int)((per + unit - 1) / unit) * unit;
-    p.n_chunks = (all + p.steps_per_wg - 1) / p.steps_per_wg;
-    p.n_wg = 0;
-    for (int c = 0; c < p.n_chunks; ++c) p.n_wg += n_tiles - (causal ? (c * p.steps_per_wg * T::KT / 32) * (32 / T::R) : 0);
+    p.n_rt32 = (N + 31) / 32;
+    p.causal = causal;
+    p.B = B;
+    p.unit = 32 / T::KT;
+    p.split_shift = T::R == 16;
+    p.n_tiles = p.n_rt32 << p.split_shift;
+    p.pair_len = p.len(0) + p.len(p.n_tiles - 1);
+    p.entry_len = p.n_tiles / 2 * p.pair_len + (p.n_tiles & 1 ? p.len(p.n_tiles / 2) : 0);
+    const long long total = (long long)B * p.entry_len;
+    p.share = (int)((total + 255) / 256);
+    p.n_wg = (int)((total + p.share - 1) / p.share);
+    p.max_segments = (p.len(p.n_tiles - 1) + p.share - 1) / p.share + 1;
     return p;
 }
-// Workgroup `id` of the n_wg of a batch entry -> row tile, chunk and its key steps.  Tiles of one chunk are
-// neighbours, and neighbours run on the same XCD (workgroup ids go round robin over the eight), so that the rows
-// of K and V of a chunk come from one L2.
-template <typename T>
-__device__ __forceinline__ bool find_unit(int causal, int n_rt32, const Plan &pl, int &id, int &rt, int &chunk, int &s0, int &s_end) {
-    const int n_tiles = n_rt32 * (32 / T::R), per = (pl.n_wg + 7) / 8;
-    id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || id >= pl.n_wg) return false;
-    int i = id;
-    for (chunk = 0;; ++chunk) {
-        s0 = chunk * pl.steps_per_wg;
-        const int first = causal ? (s0 * T::KT / 32) * (32 / T::R) : 0;   // first row tile that sees the chunk
-        if (i < n_tiles - first) break;
-        i -= n_tiles - first;
+// Neighbouring shares run on the same XCD (workgroup ids go round robin over the eight): the rows of K and V that
+// they walk come from one L2.
+__device__ __forceinline__ int share_of_workgroup(const Plan &pl) {
+    const int per = (pl.n_wg + 7) / 8, w = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    return (int)(blockIdx.x >> 3) < per && w < pl.n_wg ? w : -1;
+}
+inline int plan_grid(const Plan &pl) { return (pl.n_wg + 7) / 8 * 8; }
+// A segment: steps s0 .. s_end-1 of row tile rt of batch entry b.  A workgroup takes them in the order step(0),
+// step(1), ..: rotated, so that at a time t all workgroups are at key steps of the residue t modulo the share, i.e. at few
+// different keys (from s0 on, segments beginning anywhere, the workgroups of an XCD found 10 % of the rows of K
+// and V in its L2; rotated 65 to 85 %).
+struct Segment {
+    int b, rt, s0, s_end, rot;
+    __device__ __forceinline__ int len() const { return s_end - s0; }
+    __device__ __forceinline__ int step(int i) const {
+        const int s = s0 + rot + i;
+        return s >= s_end ? s - (s_end - s0) : s;
     }
-    rt = n_tiles - 1 - i;
-    s_end = min(s0 + pl.steps_per_wg, causal ? (rt * T::R / 32 + 1) * (32 / T::KT) : n_rt32 * (32 / T::KT));
-    return true;
+};
+// the one at position x of share `id`
+__device__ __forceinline__ Segment find_segment(const Plan &pl, int id, int x) {
+    const int begin = id * pl.share;
+    const int end = (int)min((long long)begin + pl.share, (long long)pl.entry_len * pl.B);
+    Segment sg;
+    sg.b = __builtin_amdgcn_readfirstlane(x / pl.entry_len);
+    const int r = x - sg.b * pl.entry_len, p = __builtin_amdgcn_readfirstlane(r / pl.pair_len);
+    sg.s0 = r - p * pl.pair_len;
+    sg.rt = pl.n_tiles - 1 - p;
+    const int first = pl.len(sg.rt);
+    if (sg.s0 >= first) { sg.s0 -= first; sg.rt = p; }
+    sg.s_end = min(pl.len(sg.rt), sg.s0 + end - x);
+    int rot = (x - begin - sg.s0) % pl.share;
+    rot = __builtin_amdgcn_readfirstlane(rot < 0 ? rot + pl.share : rot);
+    sg.rot = rot < sg.len() ? rot : 0;
+    return sg;
 }
 
 // Row fragments (lane 16g + n: tile row 16 rb + n, columns 32 ks + 8g ..) of rows i0 .. i0+R-1 of a head: whole rows

@@ -7,7 +7,7 @@
 // product), un-normalised, and headmix_pv_kernel multiplies them with V and divides by the row sums.
 //
 // Probabilities are exp2(z - ref) with one whole-number reference per (row, head): the largest score of the row's
-// first tile of keys, rounded up.  Every chunk of a row's keys derives the same reference from that tile, so that chunks
+// first tile of keys, rounded up.  Every segment of a row's keys derives the same reference from that tile, so that segments
 // need no merging, and a row has no running maximum: bf16 and fp32 keep their relative precision over
 // 2^+-126, and only a score more than kSlack above the reference moves it (the workgroup then rescales what it has
 // written so far; exact, the factor being a power of two).
@@ -26,7 +26,7 @@ constexpr float kSlack = 60.f;   // log2 units: sums of 2^60 terms times V stay 
 template <int H, int D> struct ProbTile : Tile<H, H == 16 ? 16 : 8, H == 16 ? 32 : 16> {
     using B = Tile<H, H == 16 ? 16 : 8, H == 16 ? 32 : 16>;
     static constexpr int ROOM = B::R * (D * 2 + 16);        // a head's rows while they are turned
-    static constexpr int w_off = 2 * B::arr, used = (w_off + H * B::WST) * 4, lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
+    static constexpr int w_off = 2 * B::arr * 4 > B::WAVES * ROOM ? 2 * B::arr : B::WAVES * ROOM / 4, lds = (w_off + H * B::WST) * 4;
 };
 
 struct ProbArgs {
@@ -36,7 +36,7 @@ struct ProbArgs {
     const bf16_t *Q, *KF;    // KF: fragment order
     const float *W;
     bf16_t *P;               // blocks
-    float *stats;            // [B][chunk][reference, largest score, sum, sum of the rounded][H][N]
+    float *stats;            // [B][segment][reference, largest score, sum, sum of the rounded][H][N]
 };
 
 template <int H, int D>
@@ -46,11 +46,18 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
                   KS = D / 32, NCH = HPW * KB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     float *lds = reinterpret_cast<float *>(smem);
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
-    const int b = blockIdx.y;
-    int id, rt, chunk, s0, s_end;
-    if (!find_unit<T>(a.causal, a.n_rt32, a.plan, id, rt, chunk, s0, s_end)) return;
-    const int i0 = rt * R, N = a.N, h0 = wave * HPW;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane_id = threadIdx.x & 63;
+    const int id = share_of_workgroup(a.plan), N = a.N, h0 = wave * HPW;
+    if (id < 0) return;
+    for (int i = threadIdx.x; i < H * H; i += T::WAVES * 64) lds[T::w_off + (i / H) * T::WST + i % H] = a.W[i] * (a.scale * kLog2e);
+    for (int x_pos = id * a.plan.share, x_end = (int)min((long long)x_pos + a.plan.share, (long long)a.B * a.plan.entry_len); x_pos < x_end;) {
+    const Segment sg = find_segment(a.plan, id, x_pos);
+    const int b = sg.b, rt = sg.rt, n_steps = sg.len();
+    x_pos += n_steps;
+    const int segment = __builtin_amdgcn_readfirstlane(id - a.plan.start(b, rt) / a.plan.share);
+    int lane = lane_id;
+    asm volatile("" : "+v"(lane));   // (no registers for what could be kept from segment to segment)
+    const int g = lane >> 4, n = lane & 15, i0 = rt * R;
 
     bf16x8 qf[HPW][RB][KS];
     {
@@ -59,7 +66,6 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
             turn_rows<T, D>(qf[t], a.Q + ((size_t)b * H + h0 + t) * N * D, i0, N, smem + wave * T::ROOM);
         lds_barrier();
     }
-    for (int i = tid; i < H * H; i += T::WAVES * 64) lds[T::w_off + (i / H) * T::WST + i % H] = a.W[i] * (a.scale * kLog2e);
     const float *wf_l = lds + T::w_off + n * T::WST + 4 * g;
 
     // ---- score phase: chunks of one head and 16 keys, K rows two chunks ahead ----
@@ -92,17 +98,18 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     // ---- mixing phase: lane (g, n) = heads 16x + 4g .. +3, tile row lr, keys 4q4 .. 4q4+3 ----
     const int lr = wave * RW + (n & (RW - 1)), q4 = n / RW, row = T::row(i0, lr), brow = row & 31;
     const int pos = lr * KT + 4 * T::slot(lr, q4);
-    f32x4 ref[HB], top[HB], l_sum[HB], l_hat[HB];
+    f32x4 nref[HB], top[HB], l_sum[HB], l_hat[HB];   // negative reference; largest score above the reference
 #pragma unroll
     for (int x = 0; x < HB; ++x) {
-        l_sum[x] = l_hat[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        nref[x] = l_sum[x] = l_hat[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
         top[x] = (f32x4){kNegInf, kNegInf, kNegInf, kNegInf};
     }
-    auto mix = [&](f32x4 (&z)[HB][4], const float *S, int step) {
+    // (z starts at from[]: the negative references of the lane's row)
+    auto mix = [&](f32x4 (&z)[HB][4], const f32x4 (&from)[HB], const float *S, int step) {
 #pragma unroll
         for (int x = 0; x < HB; ++x)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) z[x][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 4; ++t) z[x][t] = from[x];
 #pragma unroll
         for (int y = 0; y < HB; ++y) {
             f32x4 wf[HB];
@@ -143,9 +150,10 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     const int out = (((brow & 1) * 2 + ((4 * q4) >> 4)) * 16 + (brow >> 1)) * 16 + ((4 * q4) & 15) + 4 * g * kBlock;
     static_assert(KT == 32, "a step is a column of blocks");
 
-    auto probs = [&](const float *S, int step) {
+    auto probs = [&](const float *S, int u) {
+        const int step = sg.step(u);
         f32x4 z[HB][4];
-        mix(z, S, step);
+        mix(z, nref, S, step);
         bool over = false;
 #pragma unroll
         for (int x = 0; x < HB; ++x)
@@ -153,7 +161,7 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
             for (int r = 0; r < 4; ++r) {
                 const float m = fmaxf(fmaxf(z[x][0][r], z[x][1][r]), fmaxf(z[x][2][r], z[x][3][r]));
                 top[x][r] = fmaxf(top[x][r], m);
-                over |= m > ref[x][r] + kSlack;
+                over |= m > kSlack;
             }
         if (__any(over)) {
             // rare: move the references of the wave's rows; this wave wrote all of their probabilities itself, lane by lane
@@ -161,13 +169,15 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
             for (int x = 0; x < HB; ++x)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float m_new = fmaxf(ref[x][r], ceilf(row_max(top[x][r])));
-                    const float f = fast_exp2(ref[x][r] - m_new);
+                    const float up = fmaxf(0.f, ceilf(row_max(top[x][r]))), f = fast_exp2(-up);
                     l_sum[x][r] *= f;
                     l_hat[x][r] *= f;
-                    ref[x][r] = m_new;
-                    for (int e = s0; e < step; ++e) {
-                        bf16x4 *pp = reinterpret_cast<bf16x4 *>(block_of(e) + out + (16 * x + r) * kBlock);
+                    nref[x][r] -= up;
+                    top[x][r] -= up;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) z[x][t][r] -= up;
+                    for (int e = 0; e < u; ++e) {
+                        bf16x4 *pp = reinterpret_cast<bf16x4 *>(block_of(sg.step(e)) + out + (16 * x + r) * kBlock);
                         bf16x4 pb = *pp;
 #pragma unroll
                         for (int t = 0; t < 4; ++t) pb[t] = (bf16_t)((float)pb[t] * f);
@@ -183,7 +193,7 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
                 bf16x4 pb;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const float p = fast_exp2(z[x][t][r] - ref[x][r]);
+                    const float p = fast_exp2(z[x][t][r]);
                     l_sum[x][r] += p;
                     pb[t] = (bf16_t)p;
                     l_hat[x][r] += (float)pb[t];
@@ -196,32 +206,33 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     float *buf0 = lds, *buf1 = lds + T::arr;
     load_chunk(0, 0);
     load_chunk(0, 1);
-    scores(buf1, 0, s0);
-    scores(buf0, s0, min(s0 + 1, s_end - 1));
+    const auto later = [&](int i) { return sg.step(min(i, n_steps - 1)); };
+    scores(buf1, 0, sg.step(0));
+    scores(buf0, sg.step(0), later(1));
     lds_barrier();
     {
         f32x4 z[HB][4];
-        mix(z, buf1, 0);
+        mix(z, nref, buf1, 0);
 #pragma unroll
         for (int x = 0; x < HB; ++x)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                ref[x][r] = ceilf(row_max(fmaxf(fmaxf(z[x][0][r], z[x][1][r]), fmaxf(z[x][2][r], z[x][3][r]))));
+                nref[x][r] = -ceilf(row_max(fmaxf(fmaxf(z[x][0][r], z[x][1][r]), fmaxf(z[x][2][r], z[x][3][r]))));
     }
     lds_barrier();
-    for (int u = s0; u < s_end; ++u) {
-        float *cur = (u - s0) & 1 ? buf1 : buf0, *nxt = (u - s0) & 1 ? buf0 : buf1;
+    for (int u = 0; u < n_steps; ++u) {
+        float *cur = u & 1 ? buf1 : buf0, *nxt = u & 1 ? buf0 : buf1;
         // (half of the waves take the scores of the next step first, half the mix of this one: one half's LDS and vector work
         // runs under the other's products)
-        const bool first = wave < T::WAVES / 2, more = u + 1 < s_end;
-        const int ahead = min(u + 2, s_end - 1);
-        if (more && first) scores(nxt, u + 1, ahead);
+        const bool first = wave < T::WAVES / 2, more = u + 1 < n_steps;
+        const int next = later(u + 1), ahead = later(u + 2);
+        if (more && first) scores(nxt, next, ahead);
         probs(cur, u);
-        if (more && !first) scores(nxt, u + 1, ahead);
+        if (more && !first) scores(nxt, next, ahead);
         lds_barrier();
     }
 
-    float *st = a.stats + ((size_t)b * a.plan.n_chunks + chunk) * 4 * H * N;
+    float *st = a.stats + ((size_t)b * a.plan.max_segments + segment) * 4 * H * N;
 #pragma unroll
     for (int x = 0; x < HB; ++x)
 #pragma unroll
@@ -230,15 +241,16 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
             l += row16_rot<8>(l); lh += row16_rot<8>(lh);
             l += row16_rot<4>(l); lh += row16_rot<4>(lh);
             if constexpr (RW == 2) { l += row16_rot<2>(l); lh += row16_rot<2>(lh); }
-            const float m = row_max(top[x][r]);
+            const float m = row_max(top[x][r]) - nref[x][r];
             const size_t o = (size_t)(16 * x + 4 * g + r) * N + row, hn = (size_t)H * N;
             if (q4 == 0 && row < N) {
-                st[o] = ref[x][r];
+                st[o] = -nref[x][r];
                 st[hn + o] = m;
                 st[2 * hn + o] = l;
                 st[3 * hn + o] = lh;
             }
         }
+    }   // segments
 }
 
 // O = P V / (sum of P): the product kernel of dQ = dS K (bwd_dq_rows.hip) with the row sums, L and M at the end.
@@ -247,7 +259,7 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
 constexpr int PV_WAVES = 4, PV_ROWS = 128, PV_KEYS = 64;
 
 template <int D, typename TO>
-__global__ __launch_bounds__(PV_WAVES * 64) void headmix_pv_kernel(ProbArgs a, int H, int tile_keys, int tile_rows, const bf16_t *__restrict__ V,
+__global__ __launch_bounds__(PV_WAVES * 64) void headmix_pv_kernel(ProbArgs a, int H, const bf16_t *__restrict__ V,
                                                                    TO *__restrict__ O, float *__restrict__ L, float *__restrict__ M) {
     constexpr int RST = D * 2 + 16, DB = D / 16, CPR = D / 8, LD = PV_KEYS * CPR / (PV_WAVES * 64);
     __shared__ __attribute__((aligned(16))) unsigned char smem[2 * PV_KEYS * RST];
@@ -259,16 +271,17 @@ __global__ __launch_bounds__(PV_WAVES * 64) void headmix_pv_kernel(ProbArgs a, i
     const bf16_t *Vb = V + bh * N * D;
     const bf16_t *ws = a.P + ((size_t)b * chain_ds_block_off(causal, n_rt, a.n_kt) * H + h) * kBlock;
 
-    // ---- the rows' statistics over the chunks of their keys: lane n of block ob = row 2n + ob ----
-    const int chunk_keys = a.plan.steps_per_wg * tile_keys;
-    const int n_ch = causal ? min(min(rt, n_rt - 1) * 32 / chunk_keys + 1, a.plan.n_chunks) : a.plan.n_chunks;
+    // ---- the rows' statistics over the segments of their keys: lane n of block ob = row 2n + ob ----
+    const int tile = (min(rt, n_rt - 1) << a.plan.split_shift) + (a.plan.split_shift ? n >> 3 : 0);   // the rows' tile
+    const int t_start = a.plan.start(b, tile), t_first = t_start / a.plan.share;
+    const int n_ch = (t_start + a.plan.len(tile) - 1) / a.plan.share - t_first + 1;
     float ref[2], inv[2];
     bool moved = false;
 #pragma unroll
     for (int ob = 0; ob < 2; ++ob) {
         const int row = min(rw + 2 * n + ob, N - 1);
         const size_t hn = (size_t)H * N;
-        const float *st = a.stats + (size_t)b * a.plan.n_chunks * 4 * hn + (size_t)h * N + row;
+        const float *st = a.stats + (size_t)b * a.plan.max_segments * 4 * hn + (size_t)h * N + row;
         float r = st[0], m = st[hn], l = st[2 * hn], lh = st[3 * hn];
         for (int c = 1; c < n_ch; ++c) {
             const float *s = st + (size_t)c * 4 * hn;
@@ -329,8 +342,9 @@ __global__ __launch_bounds__(PV_WAVES * 64) void headmix_pv_kernel(ProbArgs a, i
             const bool ok = row_ok && kt < n_rt && (!causal || kt <= rt);
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) pf[kp][ob] = __builtin_bit_cast(bf16x8, zero_unless(ok, pr[kp][ob]));
-            if (moved && ok) {   // rare: a chunk of some row has a reference of its own
-                const float *st = a.stats + ((size_t)b * a.plan.n_chunks + min(kt * 32 / chunk_keys, n_ch - 1)) * 4 * H * N + (size_t)h * N;
+            if (moved && ok) {   // rare: a segment of some row has a reference of its own
+                const int seg = (t_start + kt * a.plan.unit) / a.plan.share - t_first;
+                const float *st = a.stats + ((size_t)b * a.plan.max_segments + seg) * 4 * H * N + (size_t)h * N;
 #pragma unroll
                 for (int ob = 0; ob < 2; ++ob) {
                     const float f = fast_exp2(st[min(rw + 2 * n + ob, N - 1)] - ref[ob]);
@@ -380,12 +394,8 @@ __global__ __launch_bounds__(PV_WAVES * 64) void headmix_pv_kernel(ProbArgs a, i
     }
 }
 
-// Four workgroups per CU level out the tail of the launch; a chunk repeats the first tile of its rows for the reference:
-// at least eight steps where there are enough workgroups without more.
 Plan prob_plan(const Problem &p) {
-    const long long all = (long long)((p.Nq + 31) / 32) * ((p.Nq + 31) / 32) * p.B / (p.causal ? 2 : 1) / 256;
-    const int least = all >= 16 ? 8 : all >= 4 ? 4 : 2;
-    return p.H == 16 ? make_plan<ProbTile<16, 32>>(p.B, p.Nq, p.causal, 4, least, 64) : make_plan<ProbTile<32, 32>>(p.B, p.Nq, p.causal, 4, least, 64);
+    return p.H == 16 ? make_plan<ProbTile<16, 32>>(p.B, p.Nq, p.causal) : make_plan<ProbTile<32, 32>>(p.B, p.Nq, p.causal);
 }
 
 template <int H, int D, typename TO>
@@ -395,15 +405,15 @@ hipError_t launch(const Problem &p, const ProbArgs &a, const void *k, const void
     launch_frag_order<D>(p.B * H, a.N, k, nullptr, a.KF, nullptr, s);
     hipError_t e = set_max_lds_once<headmix_probs_kernel<H, D>>(T::lds);
     if (e != hipSuccess) return e;
-    headmix_probs_kernel<H, D><<<dim3((a.plan.n_wg + 7) / 8 * 8, p.B), T::WAVES * 64, T::lds, s>>>(a);
-    headmix_pv_kernel<D, TO><<<dim3(H, p.B, (a.N + PV_ROWS - 1) / PV_ROWS), PV_WAVES * 64, 0, s>>>(a, H, T::KT, T::R, (const bf16_t *)v, (TO *)o, l, m);
+    headmix_probs_kernel<H, D><<<plan_grid(a.plan), T::WAVES * 64, T::lds, s>>>(a);
+    headmix_pv_kernel<D, TO><<<dim3(H, p.B, (a.N + PV_ROWS - 1) / PV_ROWS), PV_WAVES * 64, 0, s>>>(a, H, (const bf16_t *)v, (TO *)o, l, m);
     return hipGetLastError();
 }
 
 }  // namespace
 
-// K in fragment order, statistics of the chunks, blocks
-static size_t prob_stats_bytes(const Problem &p) { return ((size_t)p.B * prob_plan(p).n_chunks * 4 * p.H * p.Nq * sizeof(float) + 255) / 256 * 256; }
+// K in fragment order, statistics of the segments, blocks
+static size_t prob_stats_bytes(const Problem &p) { return ((size_t)p.B * prob_plan(p).max_segments * 4 * p.H * p.Nq * sizeof(float) + 255) / 256 * 256; }
 size_t headmix_fwd_workspace(const Problem &p) { return headmix_frag_bytes(p) + prob_stats_bytes(p) + chain_ds_bytes(p); }
 
 hipError_t headmix_fwd_blocks(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const float *w,

@@ -30,7 +30,7 @@ template <int H, int D> struct ScoreTile : Tile<H, 8, H == 16 ? 32 : 16> {
     static constexpr int w_off = NBUF * H * HS, wt_off = w_off + H * B::WST, st_off = wt_off + H * B::WST,
                          used = (st_off + (STATS_LDS ? 2 * B::R * B::WST : 0)) * 4, lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
     // chunks (one head, 16 keys) of K or V rows in registers, and how many of them stay in flight during the mixing phase
-    static constexpr int RING = H == 16 ? 4 : 2, AHEAD = H == 16 ? (D == 128 ? 2 : 4) : D == 128 ? 0 : 2;
+    static constexpr int RING = H == 16 || D < 128 ? 4 : 2, AHEAD = D == 128 ? (H == 16 ? 2 : 0) : 4;
     // (B4 H16 N4096 d128: 2 / 3 / 4 chunks in flight 1.27 / 1.33 / 1.32 ms; without the two orders of scores and mix 1.34)
     static_assert(SPW * B::KB % RING == 0, "a chunk's registers are the same in every step");
 };
@@ -42,7 +42,7 @@ struct ScoreArgs {
     const bf16_t *Q, *KF, *VF, *dO;   // KF, VF: fragment order
     const float *W, *lse, *Dl;
     bf16_t *P, *dS;      // blocks
-    float *dw_part;      // [B][n_wg][H][H], or null
+    float *dw_part;      // [n_wg][H][H], or null
 };
 
 template <int H, int D>
@@ -52,15 +52,33 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                   HB = T::HB, KS = D / 32, NCH = SPW * KB;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     float *lds = reinterpret_cast<float *>(smem);
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
-              n = lane & 15;
-    const int b = blockIdx.y;
-    int id, rt, chunk, s0, s_end;
-    if (!find_unit<T>(a.causal, a.n_rt32, a.plan, id, rt, chunk, s0, s_end)) return;
-    const int i0 = rt * R, N = a.N;
-    const size_t bo = (size_t)b * H * N * D;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane_id = threadIdx.x & 63;
+    const int id = share_of_workgroup(a.plan), N = a.N;
+    if (id < 0) return;
     // score phase: the first half of the waves takes S = Q K^T, the second half dP = dO V^T, SPW heads each
     const int mat = wave / (T::WAVES / 2), h0 = (wave - mat * (T::WAVES / 2)) * SPW;
+
+    // w of the mix and its transpose, with the scales of the two products, in LDS (read as four k steps at a time:
+    // k slot g of step s is head 4g + s)
+    for (int i = threadIdx.x; i < H * H; i += T::WAVES * 64) {
+        const float w = a.W[i];
+        lds[T::w_off + (i / H) * T::WST + i % H] = w * (a.scale * kLog2e);
+        lds[T::wt_off + (i % H) * T::WST + i / H] = w * a.scale;
+    }
+    f32x4 acc_w[HB][HB];
+#pragma unroll
+    for (int x = 0; x < HB; ++x)
+#pragma unroll
+        for (int y = 0; y < HB; ++y) acc_w[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    for (int x_pos = id * a.plan.share, x_end = (int)min((long long)x_pos + a.plan.share, (long long)a.B * a.plan.entry_len); x_pos < x_end;) {
+    const Segment sg = find_segment(a.plan, id, x_pos);
+    const int b = sg.b, rt = sg.rt, n_steps = sg.len();
+    x_pos += n_steps;
+    int lane = lane_id;
+    asm volatile("" : "+v"(lane));   // (no registers for what could be kept from segment to segment)
+    const int tid = wave * 64 + lane, g = lane >> 4, n = lane & 15, i0 = rt * R;
+    const size_t bo = (size_t)b * H * N * D;
 
     // ---- resident: Q or dO fragments of this wave's heads ----
     bf16x8 qf[SPW][RB][KS];
@@ -78,7 +96,7 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         for (int i = tid; i < R * H; i += T::WAVES * 64) {
             const int hh = i / R, lr2 = i % R, rr = T::row(i0, lr2);
             const size_t o = ((size_t)b * H + hh) * N + min(rr, N - 1);
-            st_l[lr2 * T::WST + hh] = rr < N ? a.lse[o] * kLog2e : 1e30f;
+            st_l[lr2 * T::WST + hh] = rr < N ? a.lse[o] * -kLog2e : -1e30f;
             st_l[(R + lr2) * T::WST + hh] = a.Dl[o];
         }
     } else {
@@ -87,24 +105,11 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const size_t o = ((size_t)b * H + 16 * hb + 4 * g + r) * N + min(row, N - 1);
-                lse_r[hb][r] = row < N ? a.lse[o] * kLog2e : 1e30f;
+                lse_r[hb][r] = row < N ? a.lse[o] * -kLog2e : -1e30f;
                 dl_r[hb][r] = a.Dl[o];
             }
     }
-    // w of the mix and its transpose, with the scales of the two products, in LDS (read as four k steps at a time:
-    // k slot g of step s is head 4g + s)
-    for (int i = tid; i < H * H; i += T::WAVES * 64) {
-        const float w = a.W[i];
-        lds[T::w_off + (i / H) * T::WST + i % H] = w * (a.scale * kLog2e);
-        lds[T::wt_off + (i % H) * T::WST + i / H] = w * a.scale;
-    }
     const float *wf_l = lds + T::w_off + n * T::WST + 4 * g, *wb_l = lds + T::wt_off + n * T::WST + 4 * g;
-    f32x4 acc_w[HB][HB];
-#pragma unroll
-    for (int x = 0; x < HB; ++x)
-#pragma unroll
-        for (int y = 0; y < HB; ++y) acc_w[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
     // ---- score phase, in chunks of one head and 16 keys whose rows are loaded two chunks ahead ----
     bf16x8 kf[T::RING][KS];
     const int n_t16 = a.n_rt32 * 2;
@@ -134,11 +139,14 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
     auto mix = [&](float *S, int step) {
         float *dP = S + DP;
         const int j0 = step * KT;
-        f32x4 z[HB][4];
+        f32x4 z[HB][4];   // starting at -LSE
 #pragma unroll
-        for (int x = 0; x < HB; ++x)
+        for (int x = 0; x < HB; ++x) {
+            f32x4 nlse = lse_r[x];
+            if constexpr (T::STATS_LDS) nlse = *reinterpret_cast<const f32x4 *>(st_l + lr * T::WST + 16 * x + 4 * g);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) z[x][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 4; ++t) z[x][t] = nlse;
+        }
 #pragma unroll
         for (int y = 0; y < HB; ++y) {
             f32x4 wf[HB];
@@ -173,11 +181,8 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         bf16_t *p_out = a.P + first + half, *ds_out = a.dS + first + half;
 #pragma unroll
         for (int x = 0; x < HB; ++x) {
-            f32x4 lse2 = lse_r[x], dl = dl_r[x];
-            if constexpr (T::STATS_LDS) {
-                lse2 = *reinterpret_cast<const f32x4 *>(st_l + lr * T::WST + 16 * x + 4 * g);
-                dl = *reinterpret_cast<const f32x4 *>(st_l + (R + lr) * T::WST + 16 * x + 4 * g);
-            }
+            f32x4 dl = dl_r[x];
+            if constexpr (T::STATS_LDS) dl = *reinterpret_cast<const f32x4 *>(st_l + (R + lr) * T::WST + 16 * x + 4 * g);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float *dz = dP + (16 * x + 4 * g + r) * HS + pos;
@@ -185,7 +190,7 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                 bf16x4 pb;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const float p = fast_exp2(z[x][t][r] - lse2[r]);
+                    const float p = fast_exp2(z[x][t][r]);
                     pb[t] = (bf16_t)p;
                     d[t] = p * (d[t] - dl[r]);
                     z[x][t][r] = d[t];
@@ -249,33 +254,35 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         }
     };
 #pragma unroll
-    for (int c = 0; c < T::AHEAD; ++c) load_chunk(s0, c);
+    for (int c = 0; c < T::AHEAD; ++c) load_chunk(sg.step(0), c);
+    const auto later = [&](int i) { return sg.step(min(i, n_steps - 1)); };
     if constexpr (T::NBUF == 2) {
         // One barrier per step.  Of the two waves of a SIMD one takes the scores of the next step first, the other the mix of
         // this one, so that one's LDS and vector work runs under the other's products.
-        scores(lds, s0, min(s0 + 1, s_end - 1));
+        scores(lds, sg.step(0), later(1));
         lds_barrier();
-        for (int u = s0; u < s_end; ++u) {
-            float *cur = lds + ((u - s0) & 1) * H * HS, *nxt = lds + ((u - s0 + 1) & 1) * H * HS;
-            const bool first = wave < T::WAVES / 2, more = u + 1 < s_end;
-            const int ahead = min(u + 2, s_end - 1);
-            if (more && first) scores(nxt, u + 1, ahead);
-            mix(cur, u);
-            if (more && !first) scores(nxt, u + 1, ahead);
+        for (int u = 0; u < n_steps; ++u) {
+            float *cur = lds + (u & 1) * H * HS, *nxt = lds + ((u + 1) & 1) * H * HS;
+            const bool first = wave < T::WAVES / 2, more = u + 1 < n_steps;
+            const int next = later(u + 1), ahead = later(u + 2);
+            if (more && first) scores(nxt, next, ahead);
+            mix(cur, sg.step(u));
+            if (more && !first) scores(nxt, next, ahead);
             lds_barrier();
         }
     } else {
-        for (int u = s0; u < s_end; ++u) {
-            scores(lds, u, min(u + 1, s_end - 1));
+        for (int u = 0; u < n_steps; ++u) {
+            scores(lds, sg.step(u), later(u + 1));
             lds_barrier();
-            mix(lds, u);
+            mix(lds, sg.step(u));
             lds_barrier();
         }
     }
+    }   // segments
 
     // ---- the workgroup's dw partial: the waves' accumulators added in wave order ----
     if (a.dw_part) {
-        lds_barrier();
+        const int g = lane_id >> 4, n = lane_id & 15;
 #pragma unroll
         for (int x = 0; x < HB; ++x)
 #pragma unroll
@@ -283,8 +290,8 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
 #pragma unroll
                 for (int r = 0; r < 4; ++r) lds[(wave * H + 16 * x + 4 * g + r) * H + 16 * y + n] = acc_w[x][y][r];
         lds_barrier();
-        float *part = a.dw_part + ((size_t)b * a.plan.n_wg + id) * H * H;
-        for (int i = tid; i < H * H; i += T::WAVES * 64) {
+        float *part = a.dw_part + (size_t)id * H * H;
+        for (int i = threadIdx.x; i < H * H; i += T::WAVES * 64) {
             float s = 0.f;
 #pragma unroll
             for (int w = 0; w < T::WAVES; ++w) s += lds[w * H * H + i];
@@ -441,22 +448,19 @@ __global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, i
     }
 }
 
-// Four workgroups per CU level out the tail of the launch; fewer than eight steps do not pay for a workgroup's
-// resident fragments while there are CUs for longer ones, more than 64 gain nothing.
 Plan score_plan(int B, int H, int N, int causal) {
-    const long long all = (long long)((N + 31) / 32) * ((N + 31) / 32) * B / (causal ? 2 : 1);
-    const int least = all >= 2048 ? 8 : 2;
-    return H == 16 ? make_plan<ScoreTile<16, 32>>(B, N, causal, 4, least, 64) : make_plan<ScoreTile<32, 32>>(B, N, causal, 4, least, 64);
+    return H == 16 ? make_plan<ScoreTile<16, 32>>(B, N, causal) : make_plan<ScoreTile<32, 32>>(B, N, causal);
 }
 
 template <int H, int D>
 hipError_t launch_scores(const ScoreArgs &a, const void *k, const void *v, hipStream_t s) {
     launch_frag_order<D>(a.B * H, a.N, k, v, a.KF, a.VF, s);
     constexpr int lds = ScoreTile<H, D>::lds;
+    static_assert(ScoreTile<H, D>::WAVES * ScoreTile<H, D>::ROOM <= ScoreTile<H, D>::w_off * 4, "w stays where the rows are turned");
     static_assert(lds <= 160 * 1024 && ScoreTile<H, D>::WAVES * H * H * 4 <= lds, "LDS budget");
     hipError_t e = set_max_lds_once<headmix_scores_kernel<H, D>>(lds);
     if (e != hipSuccess) return e;
-    headmix_scores_kernel<H, D><<<dim3((a.plan.n_wg + 7) / 8 * 8, a.B), ScoreTile<H, D>::WAVES * 64, lds, s>>>(a);
+    headmix_scores_kernel<H, D><<<plan_grid(a.plan), ScoreTile<H, D>::WAVES * 64, lds, s>>>(a);
     return hipGetLastError();
 }
 
@@ -499,7 +503,7 @@ hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const
     if (dq) {
         e = mfma_dq_from_rows(p, grad_dt, k, dS, nullptr, dq, s, true);
         if (e != hipSuccess) return e;
-        headmix_dw_sum_kernel<<<p.H * p.H / 16, 256, 0, s>>>(p.B * plan.n_wg, p.H * p.H, dw_part, dw);
+        headmix_dw_sum_kernel<<<p.H * p.H / 16, 256, 0, s>>>(plan.n_wg, p.H * p.H, dw_part, dw);
         e = hipGetLastError();
     }
     return e;
