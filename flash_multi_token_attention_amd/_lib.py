@@ -67,6 +67,10 @@ _SIGNATURES = {
     "convattn_bwd_fused_dkdv": (C.c_int, [_D] + [_P] * 11),
     "convattn_bwd_fused_dq": (C.c_int, [_D] + [_P] * 10),
     "convattn_bwd_fused_dw": (C.c_int, [_D] + [_P] * 3),
+    "convattn_fwd_split_workspace_bytes": (C.c_size_t, [_D]),
+    "convattn_fwd_split": (C.c_int, [_D] + [_P] * 9),
+    "convattn_bwd_split_workspace_bytes": (C.c_size_t, [_D]),
+    "convattn_bwd_split": (C.c_int, [_D] + [_P] * 13),
     "convattn_staged_workspace_bytes": (C.c_size_t, [_D, C.c_int]),
     "convattn_staged_fwd": (C.c_int, [_D] + [_P] * 9),
     "convattn_staged_bwd": (C.c_int, [_D] + [_P] * 13),

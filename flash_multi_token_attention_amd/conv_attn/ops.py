@@ -119,10 +119,9 @@ def kernel_path(Q, K, conv_kernel, causal=True, op="fwd", exact=False) -> str:
     return "mfma" if code == 1 else "fp32"
 
 
-def _staged_workspace(desc, op: int, device):
-    """Workspace of the fp32-arithmetic path's staged kernels; None when the call does not run them (bf16 matrix-core path, a
-    workspace above the cap or one that cannot be allocated: the kernels without score-sized scratch run then)."""
-    nbytes = _lib.load().convattn_staged_workspace_bytes(C.byref(desc), op)
+def _workspace(nbytes: int, device):
+    """Workspace of a form of an op that has one; None when the op does not run in that form (0 bytes), above the cap, or when
+    the allocation fails: the form that needs less runs then."""
     if nbytes == 0 or nbytes > max_workspace_bytes():
         return None
     try:
@@ -133,7 +132,7 @@ def _staged_workspace(desc, op: int, device):
 
 def _staged_backward(desc, Q, K, V, dO, D, L, W, out_dtype, want_q: bool, want_kv: bool, what: str):
     """(dQ, dK, dV, dW), None for those not wanted, from the staged kernels; None when they do not run."""
-    ws = _staged_workspace(desc, _lib.OP_BWD, Q.device)
+    ws = _workspace(_lib.load().convattn_staged_workspace_bytes(C.byref(desc), _lib.OP_BWD), Q.device)
     if ws is None:
         return None
     dQ = torch.empty(Q.shape, dtype=out_dtype, device=Q.device) if want_q else None
@@ -157,9 +156,11 @@ def forward(Q, K, V, conv_kernel, scale, pad_q, pad_k, causal, out_dtype=torch.f
     M = torch.empty((B, H, Nq), dtype=torch.float32, device=Q.device)
     L = torch.empty((B, H, Nq), dtype=torch.float32, device=Q.device)
     lib = _lib.load()
-    ws = _staged_workspace(desc, _lib.OP_FWD, Q.device)
+    ws, run = _workspace(lib.convattn_staged_workspace_bytes(C.byref(desc), _lib.OP_FWD), Q.device), lib.convattn_staged_fwd
+    if ws is None:   # (few heads or rows: the form whose workgroups share the keys of a tile of rows)
+        ws, run = _workspace(lib.convattn_fwd_split_workspace_bytes(C.byref(desc)), Q.device), lib.convattn_fwd_split
     if ws is not None:
-        rc = lib.convattn_staged_fwd(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), _ptr(ws), _ptr(O), _ptr(M), _ptr(L),
+        rc = run(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), _ptr(ws), _ptr(O), _ptr(M), _ptr(L),
                                      _stream(Q))
     else:
         rc = lib.convattn_fwd(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), _ptr(O), _ptr(M), _ptr(L), _stream(Q))
@@ -298,12 +299,10 @@ def backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
                     dQ[sl], dK[sl], dV[sl] = gq, gk, gv
                     dW[sl[1]] += gw
             return dQ, dK, dV, dW
-    ws = None
-    if nbytes <= cap:
-        try:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=Q.device)
-        except torch.OutOfMemoryError:
-            ws = None
+    # (few heads or rows: the form whose workgroups share the rows of a block of keys, where its workspace fits too)
+    ws, run = _workspace(lib.convattn_bwd_split_workspace_bytes(C.byref(desc)), Q.device), lib.convattn_bwd_split
+    if ws is None:
+        ws, run = _workspace(nbytes, Q.device), lib.convattn_bwd_fused
     if ws is None:
         dQ, dW = dq_backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal, out_dtype, exact,
                              low_memory=True)
@@ -313,8 +312,8 @@ def backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
     dK = torch.empty(K.shape, dtype=out_dtype, device=Q.device)
     dV = torch.empty(V.shape, dtype=out_dtype, device=Q.device)
     dW = torch.empty(W.shape, dtype=torch.float32, device=Q.device)
-    rc = lib.convattn_bwd_fused(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(dO), _ptr(D), _ptr(L),
-                                _ptr(W), _ptr(dQ), _ptr(dK), _ptr(dV), _ptr(dW), _ptr(ws), _stream(Q))
+    rc = run(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(dO), _ptr(D), _ptr(L), _ptr(W), _ptr(dQ), _ptr(dK), _ptr(dV),
+             _ptr(dW), _ptr(ws), _stream(Q))
     _lib.check(rc, "conv_attn.backward")
     return dQ, dK, dV, dW
 

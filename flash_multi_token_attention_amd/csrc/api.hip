@@ -147,6 +147,23 @@ int convattn_fwd(const convattn_desc *desc, const void *q, const void *k, const 
     return (int)generic_fwd(p, desc->in_dtype, desc->out_dtype, q, k, v, w, o, m, l, s);
 }
 
+size_t convattn_fwd_split_workspace_bytes(const convattn_desc *desc) {
+    Problem p;
+    if (validate(desc, CONVATTN_OP_FWD, &p) || pick_path(desc, p, CONVATTN_OP_FWD) != 1) return 0;
+    return mfma_fwd_split_bytes(p);
+}
+
+int convattn_fwd_split(const convattn_desc *desc, const void *q, const void *k, const void *v, const float *w, void *workspace,
+                       void *o, float *m, float *l, void *stream) {
+    Problem p;
+    int rc = validate(desc, CONVATTN_OP_FWD, &p);
+    if (rc) return rc;
+    if (convattn_fwd_split_workspace_bytes(desc) == 0) return CONVATTN_ERR_SHAPE;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(w); REQUIRE_PTR(workspace);
+    REQUIRE_PTR(o); REQUIRE_PTR(m); REQUIRE_PTR(l);
+    return (int)mfma_fwd(p, desc->out_dtype, q, k, v, w, o, m, l, static_cast<hipStream_t>(stream), static_cast<float *>(workspace));
+}
+
 int convattn_bwd_preprocess(const convattn_desc *desc, const void *o, const void *d_o,
                             const float *m, const float *l, float *D, float *lse, void *stream) {
     Problem p;
@@ -264,6 +281,52 @@ int convattn_bwd_fused_dkdv(const convattn_desc *desc, const void *q, const void
     hipError_t e = mfma_dc_scale(p, d_o, v, scale, s);
     if (e != hipSuccess) return (int)e;
     return (int)mfma_bwd_chain(p, desc->out_dtype, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s);
+}
+
+// The one-pass backward with the row tiles of a key block shared by several workgroups: the workspace of the fused one, more
+// dW partials, then the partial dK / dV.
+struct SplitWs {
+    size_t part_off, scale_off, kv_off, total;
+    int share, n_wg;
+};
+static SplitWs split_ws(const Problem &p) {
+    SplitWs w{};
+    w.share = chain_share(p);
+    if (!w.share) return w;
+    w.n_wg = chain_wgs(p, w.share);
+    w.part_off = align256(chain_ds_bytes(p));
+    w.scale_off = w.part_off + align256((size_t)p.B * p.H * w.n_wg * p.c_q * p.c_k * sizeof(float));
+    w.kv_off = w.scale_off + align256(chain_scale_bytes(p));
+    w.total = w.kv_off + align256(chain_part_bytes(p, w.share));
+    return w;
+}
+
+size_t convattn_bwd_split_workspace_bytes(const convattn_desc *desc) {
+    Problem p;
+    if (validate(desc, CONVATTN_OP_BWD, &p) || pick_path(desc, p, CONVATTN_OP_BWD) != 1) return 0;
+    return split_ws(p).total;
+}
+
+int convattn_bwd_split(const convattn_desc *desc, const void *q, const void *k, const void *v, const void *d_o,
+                       const float *D, const float *lse, const float *w, void *dq, void *dk, void *dv, float *dw,
+                       void *workspace, void *stream) {
+    Problem p;
+    int rc = validate(desc, CONVATTN_OP_BWD, &p);
+    if (rc) return rc;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(d_o); REQUIRE_PTR(D); REQUIRE_PTR(lse); REQUIRE_PTR(w);
+    REQUIRE_PTR(dq); REQUIRE_PTR(dk); REQUIRE_PTR(dv); REQUIRE_PTR(dw); REQUIRE_PTR(workspace);
+    const SplitWs lay = pick_path(desc, p, CONVATTN_OP_BWD) == 1 ? split_ws(p) : SplitWs{};
+    if (!lay.total) return CONVATTN_ERR_SHAPE;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    unsigned char *ws = static_cast<unsigned char *>(workspace);
+    float *part = reinterpret_cast<float *>(ws + lay.part_off), *scale = reinterpret_cast<float *>(ws + lay.scale_off);
+    float *kv = reinterpret_cast<float *>(ws + lay.kv_off);
+    hipError_t e = mfma_dc_scale(p, d_o, v, scale, s);
+    if (e == hipSuccess) e = mfma_bwd_chain(p, desc->out_dtype, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s, lay.share, kv);
+    if (e == hipSuccess) e = chain_reduce(p, desc->out_dtype, lay.share, kv, dk, dv, s);
+    if (e == hipSuccess) e = mfma_dq_from_rows(p, desc->out_dtype, k, ws, scale, dq, s);
+    if (e == hipSuccess) e = dw_reduce(p, lay.n_wg, part, dw, s);
+    return (int)e;
 }
 
 int convattn_bwd_fused_dq(const convattn_desc *desc, const void *q, const void *k, const void *v,

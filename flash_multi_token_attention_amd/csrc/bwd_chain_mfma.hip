@@ -95,7 +95,8 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
 
     // x = head, y = batch, z = key tile: the first key tiles see the most rows and go first
     const int h = blockIdx.x, b = blockIdx.y;
-    const int k0 = blockIdx.z * BKW, c0 = k0 + pr * WK;
+    const ChainSpan span = chain_span(p, blockIdx.z, args.share);
+    const int k0 = span.kb * BKW, c0 = k0 + pr * WK;
     const int pk = p.pk, cq = p.c_q, ck = p.c_k;
     const bool causal = p.causal != 0;
     const size_t bh = (size_t)b * p.H + h;
@@ -116,8 +117,13 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
     }
 
     // Causal: rows before the first key this workgroup touches (k0 - 8) see none of its keys.
-    const int r_begin = causal ? (max(0, k0 - 8) / BR) * BR : 0;
-    const int n_tiles = (p.Nq - r_begin + BR - 1) / BR;
+    const int t_begin = span.len * span.part / span.parts, t_end = span.len * (span.part + 1) / span.parts;
+    const int r_begin = (span.first_rt + t_begin) * BR, n_tiles = t_end - t_begin;
+    // The window of the last tile's rows reaches into the tile after it, whose dC is computed here too where it is
+    // another workgroup's: n_scored tiles have scores and dC, n_tiles of them everything else.
+    const int n_scored = n_tiles + (t_end < span.len ? 1 : 0);
+    // this workgroup's partial dK / dV, or null: it writes the results itself
+    float *kv_part = span.parts > 1 ? args.kv_part + (bh * gridDim.z + blockIdx.z) * (2 * BKW * D) : nullptr;
     // masks are needed next to the diagonal, at both ends of the key axis and past the last row
     const bool always_edge = c0 < 8 || c0 + 40 > p.Nk;
     auto is_edge = [&](int r0) { return always_edge || (causal && r0 < c0 + 64) || r0 + BR > p.Nq; };
@@ -315,9 +321,9 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
             tiles_landed(false);
             __syncthreads();
             // (the LSE / D loads before the tile loads: the wait above is for the youngest loads of the wave)
-            if (it + 1 < n_tiles) stage_stats(it + 1);
+            if (it + 1 < n_scored) stage_stats(it + 1);
             load_stats(r0 + 2 * BR);
-            if (it + 1 < n_tiles) fetch_tile(it + 1);
+            if (it + 1 < n_scored) fetch_tile(it + 1);
             // dC of a tile that has none (entirely above the diagonal, or the one after the last):
             // zeros, so that the consumers read every tile alike
             auto zero_dc = [&] {
@@ -330,8 +336,8 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
                     for (int ob = 0; ob < 2; ++ob)
                         *reinterpret_cast<u32x2 *>(Cs + ob * CST + cb * 32) = (u32x2){0u, 0u};
             };
-            if (it == n_tiles) zero_dc();
-            if (it >= n_tiles) continue;
+            if (it == n_scored) zero_dc();
+            if (it >= n_scored) continue;
 
             auto ptile = [&](auto edge_tag, auto full_tag) {
                 constexpr bool EDGE = decltype(edge_tag)::value;
@@ -508,7 +514,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
         for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
             for (int f = 0; f < 2; ++f) prev_dc[cb][f][0] = prev_dc[cb][f][1] = 0u;
-        const int n_kt = gridDim.z * NP, kt = blockIdx.z * NP + pr;
+        const int n_kt = (p.Nk + 8 + BKW - 1) / BKW * NP, kt = span.kb * NP + pr;
         // (causal: the pair's first block is row tile kt - 1)
         bf16_t *ds_pair = dS_ws + (bh * (size_t)chain_ds_block_off(causal, n_rt, n_kt) + (size_t)chain_ds_block_off(causal, n_rt, kt) -
                                    chain_ds_first_rt(causal, kt)) * (WK * BR);
@@ -518,9 +524,9 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
             ds_stored = false;
             __syncthreads();
             // (the LSE / D loads before the tile loads: the counted wait above relies on that order)
-            if (it + 1 < n_tiles) stage_stats(it + 1);
+            if (it + 1 < n_scored) stage_stats(it + 1);
             load_stats(r_begin + (it + 2) * BR);
-            if (it + 1 < n_tiles) fetch_tile(it + 1);
+            if (it + 1 < n_scored) fetch_tile(it + 1);
             const int u = it - 1, v = it - 2;
             const int r0u = r_begin + u * BR, r0v = r_begin + v * BR;
             const bool u_in = it >= 1 && u < n_tiles;
@@ -764,6 +770,12 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 const int col = db * 16 + 4 * g;
+                if (WANT_KV && kv_part) {
+                    float *dst = kv_part + (pr * WK + m * 16 + n) * D + col;
+                    *reinterpret_cast<f32x4 *>(dst) = acc_k[m][db] * inv;
+                    *reinterpret_cast<f32x4 *>(dst + BKW * D) = acc_v[m][db] * inv;
+                    continue;
+                }
                 if (WANT_KV && key_k < p.Nk) {
                     TO *dst = dK + (bh * p.Nk + key_k) * D + col;
                     if constexpr (sizeof(TO) == 2) {
@@ -858,15 +870,15 @@ __global__ void dc_scale_finish_kernel(int n_bh, int d, const float *__restrict_
 template <int D, int CQT, typename TO, int WANT>
 hipError_t launch_chain(const Problem &p, const void *q, const void *k, const void *v, const void *d_o,
                         const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk,
-                        void *dv, void *ds_ws, float *dw_part, hipStream_t s) {
+                        void *dv, void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
     auto kern = bwd_chain_kernel<D, CQT, TO, WANT>;
     constexpr int lds = ChainLds<D, CQT>::total;
     static_assert(lds <= 160 * 1024, "LDS budget");
     hipError_t e = set_max_lds_once<bwd_chain_kernel<D, CQT, TO, WANT>>(lds);
     if (e != hipSuccess) return e;
-    dim3 grid(p.H, p.B, mfma_kv_tiles(p));
+    dim3 grid(p.H, p.B, chain_wgs(p, share));
     ChainArgs args{p, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)d_o, Dl, lse, w,
-                   dc_scale, dk, dv, (bf16_t *)ds_ws, dw_part, chain_row_tiles(p)};
+                   dc_scale, dk, dv, (bf16_t *)ds_ws, dw_part, chain_row_tiles(p), share, kv_part};
     kern<<<grid, NT, lds, s>>>(args);
     return hipGetLastError();
 }
@@ -874,26 +886,26 @@ hipError_t launch_chain(const Problem &p, const void *q, const void *k, const vo
 template <int D, typename TO, int WANT>
 hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v, const void *d_o,
                    const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv,
-                   void *ds_ws, float *dw_part, hipStream_t s) {
+                   void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
     // (windows of up to 6 query taps run the three-role kernel of bwd_chain3_mfma.hip)
-    if (p.c_q <= 8) return launch_chain<D, 8, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-    return launch_chain<D, 12, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+    if (p.c_q <= 8) return launch_chain<D, 8, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    return launch_chain<D, 12, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 
 template <int WANT>
 hipError_t pick_shape(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const void *d_o,
                       const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv,
-                      void *ds_ws, float *dw_part, hipStream_t s) {
+                      void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
     if (p.d == 128) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-        return pick_cq<128, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+        return pick_cq<128, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     }
     if (p.d == 32) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-        return pick_cq<32, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+        return pick_cq<32, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     }
-    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-    return pick_cq<64, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    return pick_cq<64, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 
 }  // namespace
@@ -926,8 +938,8 @@ hipError_t mfma_dc_scale(const Problem &p, const void *d_o, const void *v, float
 #endif
 hipError_t CHAIN_ENTRY(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
                        const void *d_o, const float *Dl, const float *lse, const float *w,
-                       const float *dc_scale, void *dk, void *dv, void *ds_ws, float *dw_part, hipStream_t s) {
-    return pick_shape<CONVATTN_CHAIN_UNIT>(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+                       const float *dc_scale, void *dk, void *dv, void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
+    return pick_shape<CONVATTN_CHAIN_UNIT>(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 
 }  // namespace convattn

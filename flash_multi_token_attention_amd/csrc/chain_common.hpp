@@ -176,7 +176,8 @@ struct ChainArgs {
     void *dK, *dV;
     bf16_t *dS_ws;
     float *dW_part;
-    int n_rt;
+    int n_rt, share;    // share, kv_part: see ChainSpan
+    float *kv_part;
 };
 
 // The kernel argument segment lives in the constant address space; host passes of the compiler

@@ -70,9 +70,26 @@ template <int D> struct FwdLds {
     static constexpr int total = n_buf * buf_bytes;
 };
 
-template <int D, int CQT, typename TO>
+// A query tile's key steps cut into parts of at most `share` steps, one workgroup each (0: one workgroup per tile); a part
+// leaves its O (not normalised), row sums, exponent bases and maxima in `part`, [batch, head][workgroup][BQ][D + 4] fp32, for
+// fwd_merge_kernel.
+struct FwdSplit { int share; float *part; };
+template <int BQ>
+__host__ __device__ inline int fwd_steps(const Problem &p, int qt) {
+    const int k_end = p.causal ? (p.Nk < (qt + 1) * BQ ? p.Nk : (qt + 1) * BQ) : p.Nk;
+    return (k_end + 16 + BK - 1) / BK;
+}
+__host__ __device__ inline int fwd_parts(int steps, int share) { return share > 0 && steps > share ? (steps + share - 1) / share : 1; }
+template <int BQ> inline int fwd_wgs(const Problem &p, int share) {
+    int n = 0;
+    for (int qt = 0; qt < (p.Nq + BQ - 1) / BQ; ++qt) n += fwd_parts(fwd_steps<BQ>(p, qt), share);
+    return n;
+}
+
+// (SPLIT: an instance of its own, the other one is a percent slower with the parts' bounds at run time)
+template <int D, int CQT, typename TO, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
-    Problem p, const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
+    Problem p, FwdSplit split, const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
     const bf16_t *__restrict__ V, const float *__restrict__ W, TO *__restrict__ O,
     float *__restrict__ M, float *__restrict__ L) {
     using Lds = FwdLds<D>;
@@ -89,7 +106,10 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     // x = head, y = batch, z = query tile: the dispatcher hands out every (batch, head) of the
     // longest (causal) tiles first, so the tail of the launch is made of short tiles
     const int h = blockIdx.x, b = blockIdx.y;
-    const int qt = gridDim.z - 1 - blockIdx.z;
+    int qt = gridDim.z - 1 - blockIdx.z, part_no = 0;
+    if constexpr (SPLIT)
+        for (qt = (p.Nq + BQ - 1) / BQ - 1, part_no = blockIdx.z; part_no >= fwd_parts(fwd_steps<BQ>(p, qt), split.share); --qt)
+            part_no -= fwd_parts(fwd_steps<BQ>(p, qt), split.share);
     const int i0 = qt * BQ, i0w = i0 + wave * WR;
     const int base = i0w - (CQT - 1);  // first score row of the wave
     const int pk = p.pk, cq = p.c_q;
@@ -398,10 +418,38 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         }
     };
 
-    const int k_end = causal ? min(p.Nk, i0 + BQ) : p.Nk;
-    const int n_steps = (k_end + 16 + BK - 1) / BK;
-    fetch_step(0);
-    if constexpr (Lds::n_buf == 3) fetch_step(1);
+    const int all_steps = fwd_steps<BQ>(p, qt), parts = SPLIT ? fwd_parts(all_steps, split.share) : 1;
+    const int u_lo = SPLIT ? all_steps * part_no / parts : 0, n_steps = SPLIT ? all_steps * (part_no + 1) / parts : all_steps;   // this workgroup's steps
+    // (a part that does not begin with the first step takes the scores of the step before it along the way: the window
+    // needs the last block of them)
+    const int u_first = SPLIT ? max(u_lo - 1, 0) : 0;
+    fetch_step(u_first);
+    if constexpr (Lds::n_buf == 3) fetch_step(u_first + 1);
+    if constexpr (SPLIT) {
+        const int to_first = (u_first % Lds::n_buf) * Lds::buf_bytes;
+        ka += to_first;
+        va[0] += to_first;
+        va[1] += to_first;
+    }
+    auto carry_only = [&](int u) {
+        const int jk = 32 * u + 8;   // keys of the step's second block
+        f32x4 acc[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+                acc[f] = mfma_bf16(*(lds_bf16x8_ptr)(size_t)(ka + 1024 + ks * 2048), qf[f][ks], acc[f]);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            const int qpos = base + 2 * n + f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (causal && jk + 4 * g + r > qpos) acc[f][r] = 0.f;
+            const u32x2 two = pack_scores_f16(acc[f]);
+            carry[f][0] = two[0];
+            carry[f][1] = two[1];
+        }
+    };
     // Along the keys a wave's steps are: step 0 (keys before the first one to mask), steps whose
     // keys all lie at or before its first score row (no masks), steps on the diagonal or at the
     // end of the keys (masks), and steps entirely after its rows (it only takes part in the
@@ -415,8 +463,9 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
             if constexpr (Lds::n_buf == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * N_LD) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();  // step u-1 is done everywhere: its buffer is free, and step u's is written
-            fetch_step(u + Lds::n_buf - 1);
-            if constexpr (KIND != 2) step(u, std::integral_constant<bool, KIND == 1>{});
+            if (!SPLIT || u + Lds::n_buf - 1 < n_steps) fetch_step(u + Lds::n_buf - 1);
+            if constexpr (KIND == 3) carry_only(u);
+            else if constexpr (KIND != 2) step(u, std::integral_constant<bool, KIND == 1>{});
             const int to_other = (u % Lds::n_buf == Lds::n_buf - 1) ? -(Lds::n_buf - 1) * Lds::buf_bytes : Lds::buf_bytes;
             ka += to_other;
             va[0] += to_other;
@@ -427,10 +476,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     const int u_tail = p.Nk < 24 ? 1 : (p.Nk - 24) / 32 + 1;    // first u >= 1 with 32u + 24 > Nk
     const int u1 = min(causal ? min(u_diag, u_tail) : u_tail, n_steps);
     const int u2 = max(u1, causal ? min((i0w + WR + 15) / 32 + 1, n_steps) : n_steps);  // 32u - 16 > i0w + WR - 1
-    run(0, 1, std::integral_constant<int, 1>{});
-    run(1, u1, std::integral_constant<int, 0>{});
-    run(u1, u2, std::integral_constant<int, 1>{});
-    run(u2, n_steps, std::integral_constant<int, 2>{});
+    if constexpr (SPLIT) run(u_first, u_lo, std::integral_constant<int, 3>{});
+    run(u_lo, 1, std::integral_constant<int, 1>{});
+    run(max(1, u_lo), u1, std::integral_constant<int, 0>{});
+    run(max(u1, u_lo), u2, std::integral_constant<int, 1>{});
+    run(max(u2, u_lo), n_steps, std::integral_constant<int, 2>{});
     // ---- epilogue: finish the row sums and maxima, normalise, store O, M, L ----
 #pragma unroll
     for (int ob = 0; ob < 2; ++ob) {
@@ -441,6 +491,15 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         mt = fmaxf(mt, __shfl_xor(mt, 16, kWave));
         mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));
         const int qpos = base + 2 * n + ob;
+        if (SPLIT && parts > 1) {
+            if (qpos >= i0w && qpos < p.Nq) {
+                float *dst = split.part + ((bh * gridDim.z + blockIdx.z) * BQ + qpos - i0) * (D + 4);
+#pragma unroll
+                for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4 *>(dst + db * 16 + 4 * g) = acc_o[ob][db];
+                if (g == 0) *reinterpret_cast<f32x4 *>(dst + D) = (f32x4){l, m_ref[ob], mt, 0.f};
+            }
+            continue;
+        }
         if (qpos >= i0w && qpos < p.Nq) {
             const float inv = 1.f / l;
             TO *orow = O + (bh * p.Nq + qpos) * D;
@@ -465,46 +524,130 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     }
 }
 
+// O, M and L of the rows of a split query tile from its parts: 4 columns of a row per thread.
+// x = 256 threads of the tile, y = tile from the last on, z = (batch, head).
+template <int D, int BQ, typename TO>
+__global__ __launch_bounds__(256) void fwd_merge_kernel(Problem p, FwdSplit split, int n_wg, TO *__restrict__ O, float *__restrict__ M,
+                                                        float *__restrict__ L) {
+    int z = 0, qt = (p.Nq + BQ - 1) / BQ - 1;
+    for (int i = 0; i < (int)blockIdx.y; ++i, --qt) z += fwd_parts(fwd_steps<BQ>(p, qt), split.share);
+    const int parts = fwd_parts(fwd_steps<BQ>(p, qt), split.share);
+    const int e = blockIdx.x * 256 + threadIdx.x, r = e / (D / 4), col = (e % (D / 4)) * 4, row = qt * BQ + r;
+    if (r >= BQ || row >= p.Nq) return;
+    const float *src = split.part + (((size_t)blockIdx.z * n_wg + z) * BQ + r) * (D + 4);
+    const size_t step = (size_t)BQ * (D + 4);
+    float ref = kNegInf, m = kNegInf, l = 0.f;
+    for (int i = 0; i < parts; ++i) {
+        const f32x4 st = *reinterpret_cast<const f32x4 *>(src + i * step + D);
+        ref = fmaxf(ref, st[1]);
+        m = fmaxf(m, st[2]);
+    }
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < parts; ++i) {   // (a part none of whose keys the row sees has base -inf: factor 0)
+        const f32x4 st = *reinterpret_cast<const f32x4 *>(src + i * step + D);
+        const float f = fast_exp2(st[1] - ref);
+        l = fmaf(st[0], f, l);
+        o += *reinterpret_cast<const f32x4 *>(src + i * step + col) * f;
+    }
+    o *= 1.f / l;
+    const size_t at = (size_t)blockIdx.z * p.Nq + row;
+    if constexpr (sizeof(TO) == 2) {
+        const bf16x4 ov = {(bf16_t)o[0], (bf16_t)o[1], (bf16_t)o[2], (bf16_t)o[3]};
+        *reinterpret_cast<bf16x4 *>(O + at * D + col) = ov;
+    } else {
+        *reinterpret_cast<f32x4 *>(O + at * D + col) = o;
+    }
+    if (col == 0) {
+        M[at] = m * (1.f / kLog2e);
+        L[at] = l * fast_exp2(ref - m);
+    }
+}
+
+// Steps per workgroup, or 0: one workgroup per query tile.  In units of a key step of a workgroup that has a CU to itself:
+// a workgroup costs its steps and about 4 (5 where it is a part); with two per CU each runs at 0.6 of that; the merge
+// kernel about 8.  Few (batch, head) pairs or rows leave the launch as long as its longest tile
+// (B1 H8 N2048 d64 7x7: 49 -> 30 + 7 us, B1 H8 N1000 d128 6x11: 30 -> 16 + 6).  From 8192 rows on nothing is split, whatever the number of heads is.
+template <int BQ> int fwd_share(const Problem &p) {
+    const int n_qt = (p.Nq + BQ - 1) / BQ, most = fwd_steps<BQ>(p, n_qt - 1);
+    if (most < 32 || p.Nq >= 8192 || p.Nk >= 8192 || p.B * (long long)p.H > 64) return 0;
+    float none = 0.f, best = 0.f;
+    int share = 0;
+    for (int cut = 1; cut <= 6; ++cut) {
+        const int sh = cut == 1 ? 0 : (most + cut - 1) / cut;
+        if (cut > 1 && sh < 6) break;
+        float total = 0.f, longest = 0.f;
+        int jobs = 0;
+        for (int qt = 0; qt < n_qt; ++qt) {
+            const int st = fwd_steps<BQ>(p, qt), parts = fwd_parts(st, sh);
+            const float one = (float)((st + parts - 1) / parts) + (parts > 1 ? 5.f : 4.f);
+            longest = one > longest ? one : longest;
+            total += one * parts;
+            jobs += parts;
+        }
+        const float n = (float)p.B * p.H, even = total * n / (256.f * 1.22f) + 0.35f * longest;
+        const float alone = jobs * n <= 256.f ? longest : jobs * n >= 512.f ? 1.64f * longest : (1.f + 0.64f * (jobs * n - 256.f) / 256.f) * longest;
+        const float t = jobs * n <= 256.f || alone > even ? alone : even;
+        if (cut == 1) none = best = t;
+        else if (1.1f * t + 8.f < none && t < best) { best = t; share = sh; }
+    }
+    return share;
+}
+
 template <int D, int CQT, typename TO>
-hipError_t launch_fwd(const Problem &p, const void *q, const void *k, const void *v, const float *w,
+hipError_t launch_fwd(const Problem &p, float *part, const void *q, const void *k, const void *v, const float *w,
                       void *o, float *m, float *l, hipStream_t s) {
-    auto kern = fwd_reg_mfma_kernel<D, CQT, TO>;
-    constexpr int lds = FwdLds<D>::total;
+    constexpr int lds = FwdLds<D>::total, BQ = NW * wave_rows(CQT);
     if (lds > 64 * 1024) {
-        hipError_t e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO>>(lds);
+        hipError_t e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, false>>(lds);
+        if (e == hipSuccess) e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, true>>(lds);
         if (e != hipSuccess) return e;
     }
-    constexpr int BQ = NW * wave_rows(CQT);
-    dim3 grid(p.H, p.B, (p.Nq + BQ - 1) / BQ);
-    kern<<<grid, NW * 64, lds, s>>>(p, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, w,
-                                    (TO *)o, m, l);
+    const FwdSplit split{part ? fwd_share<BQ>(p) : 0, part};
+    const int n_wg = fwd_wgs<BQ>(p, split.share);
+    auto kern = split.share ? fwd_reg_mfma_kernel<D, CQT, TO, true> : fwd_reg_mfma_kernel<D, CQT, TO, false>;
+    kern<<<dim3(p.H, p.B, n_wg), NW * 64, lds, s>>>(p, split, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, w, (TO *)o, m, l);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !split.share) return e;
+    int tiles = 0;   // (the split tiles are the last ones)
+    const int n_qt = (p.Nq + BQ - 1) / BQ;
+    while (tiles < n_qt && fwd_parts(fwd_steps<BQ>(p, n_qt - 1 - tiles), split.share) > 1) ++tiles;
+    fwd_merge_kernel<D, BQ, TO><<<dim3((BQ * D / 4 + 255) / 256, tiles, p.B * p.H), 256, 0, s>>>(p, split, n_wg, (TO *)o, m, l);
     return hipGetLastError();
 }
 
 template <int D, typename TO>
-hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v, const float *w,
+hipError_t pick_cq(const Problem &p, float *part, const void *q, const void *k, const void *v, const float *w,
                    void *o, float *m, float *l, hipStream_t s) {
-    if (p.c_q <= 3) return launch_fwd<D, 3, TO>(p, q, k, v, w, o, m, l, s);
-    if (p.c_q <= 6) return launch_fwd<D, 6, TO>(p, q, k, v, w, o, m, l, s);
-    if (p.c_q <= 8) return launch_fwd<D, 8, TO>(p, q, k, v, w, o, m, l, s);
-    return launch_fwd<D, 11, TO>(p, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 3) return launch_fwd<D, 3, TO>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 6) return launch_fwd<D, 6, TO>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 8) return launch_fwd<D, 8, TO>(p, part, q, k, v, w, o, m, l, s);
+    return launch_fwd<D, 11, TO>(p, part, q, k, v, w, o, m, l, s);
+}
+
+template <int CQT> size_t split_bytes(const Problem &p) {
+    constexpr int BQ = NW * wave_rows(CQT);
+    const int share = fwd_share<BQ>(p);
+    return share ? (size_t)p.B * p.H * fwd_wgs<BQ>(p, share) * BQ * (p.d + 4) * sizeof(float) : 0;
 }
 
 }  // namespace
 
+size_t mfma_fwd_split_bytes(const Problem &p) {
+    return p.c_q <= 3 ? split_bytes<3>(p) : p.c_q <= 6 ? split_bytes<6>(p) : p.c_q <= 8 ? split_bytes<8>(p) : split_bytes<11>(p);
+}
 
 hipError_t mfma_fwd(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
-                    const float *w, void *o, float *m, float *l, hipStream_t s) {
+                    const float *w, void *o, float *m, float *l, hipStream_t s, float *part) {
     if (p.d == 128) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t>(p, q, k, v, w, o, m, l, s);
-        return pick_cq<128, float>(p, q, k, v, w, o, m, l, s);
+        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t>(p, part, q, k, v, w, o, m, l, s);
+        return pick_cq<128, float>(p, part, q, k, v, w, o, m, l, s);
     }
     if (p.d == 32) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t>(p, q, k, v, w, o, m, l, s);
-        return pick_cq<32, float>(p, q, k, v, w, o, m, l, s);
+        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t>(p, part, q, k, v, w, o, m, l, s);
+        return pick_cq<32, float>(p, part, q, k, v, w, o, m, l, s);
     }
-    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t>(p, q, k, v, w, o, m, l, s);
-    return pick_cq<64, float>(p, q, k, v, w, o, m, l, s);
+    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t>(p, part, q, k, v, w, o, m, l, s);
+    return pick_cq<64, float>(p, part, q, k, v, w, o, m, l, s);
 }
 
 }  // namespace convattn

@@ -27,8 +27,8 @@ using torch::autograd::variable_list;
 
 // ---- the C ABI, from the library Python has loaded ----
 #define API_LIST(F)                                                                                                   \
-    F(convattn_strerror) F(convattn_fwd) F(convattn_bwd_preprocess) F(convattn_bwd_fused_workspace_bytes)              \
-    F(convattn_bwd_fused) F(convattn_staged_workspace_bytes) F(convattn_staged_fwd) F(convattn_staged_bwd)               \
+    F(convattn_strerror) F(convattn_fwd) F(convattn_fwd_split_workspace_bytes) F(convattn_fwd_split) F(convattn_bwd_preprocess) F(convattn_bwd_fused_workspace_bytes)              \
+    F(convattn_bwd_fused) F(convattn_bwd_split_workspace_bytes) F(convattn_bwd_split) F(convattn_staged_workspace_bytes) F(convattn_staged_fwd) F(convattn_staged_bwd)               \
     F(convattn_decode_strided) F(convattn_decode_kv) F(convattn_decode_combine)                 \
     F(convattn_headmix_validate) F(convattn_headmix_fwd_workspace_bytes) F(convattn_headmix_fwd_ws)                   \
     F(convattn_headmix_bwd_fused_workspace_bytes) F(convattn_headmix_bwd_fused)
@@ -149,8 +149,15 @@ struct WindowBackward : torch::autograd::Node {
             // (D and LSE ahead of the workspace, which counts for the cap alone as in the Python op)
             auto reserve = [&](size_t bytes) { return bytes && bytes <= workspace_cap() ? workspace(bytes + 2 * stat, Q) : Tensor(); };
             Tensor ws = reserve(api.convattn_staged_workspace_bytes(&d, CONVATTN_OP_BWD));
-            const bool staged = ws.defined();
-            if (!staged) ws = reserve(api.convattn_bwd_fused_workspace_bytes(&d));
+            auto backward = api.convattn_staged_bwd;
+            if (!ws.defined()) {
+                ws = reserve(api.convattn_bwd_split_workspace_bytes(&d));
+                backward = api.convattn_bwd_split;
+            }
+            if (!ws.defined()) {
+                ws = reserve(api.convattn_bwd_fused_workspace_bytes(&d));
+                backward = api.convattn_bwd_fused;
+            }
             if (ws.defined()) {
                 char *base = static_cast<char *>(ws.data_ptr());
                 float *D = reinterpret_cast<float *>(base), *lse = reinterpret_cast<float *>(base + stat);
@@ -161,9 +168,8 @@ struct WindowBackward : torch::autograd::Node {
                 convattn_desc pre = d;
                 pre.Nk = pre.Nq; pre.c_q = pre.c_k = 1; pre.scale = 1; pre.causal = 0;
                 check(api.convattn_bwd_preprocess(&pre, O.data_ptr(), dO.data_ptr(), M, L, D, lse, s), "conv_attn.bwd_preprocess");
-                check((staged ? api.convattn_staged_bwd : api.convattn_bwd_fused)(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), dO.data_ptr(), D, lse,
-                                             Wf.const_data_ptr<float>(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(),
-                                             dW.mutable_data_ptr<float>(), base + 2 * stat, s),
+                check(backward(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), dO.data_ptr(), D, lse, Wf.const_data_ptr<float>(),
+                               dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), dW.mutable_data_ptr<float>(), base + 2 * stat, s),
                       "conv_attn.backward");
                 out[0] = dQ; out[1] = dK; out[2] = dV;
                 out[3] = W.scalar_type() == at::kFloat ? dW : dW.to(W.scalar_type());
@@ -209,10 +215,15 @@ std::optional<Tensor> window_attention(const Tensor &Q, const Tensor &K, const T
         O = empty(Q.sizes(), Q.scalar_type(), Q);
         stats = empty({2 * padded(rows)}, at::kFloat, Q);
         float *M = stats.mutable_data_ptr<float>();
-        const Tensor ws = workspace(api.convattn_staged_workspace_bytes(&d, CONVATTN_OP_FWD), Q);
+        Tensor ws = workspace(api.convattn_staged_workspace_bytes(&d, CONVATTN_OP_FWD), Q);
+        auto forward = api.convattn_staged_fwd;
+        if (!ws.defined()) {
+            ws = workspace(api.convattn_fwd_split_workspace_bytes(&d), Q);
+            forward = api.convattn_fwd_split;
+        }
         const float *w = Wf.const_data_ptr<float>();
-        check(ws.defined() ? api.convattn_staged_fwd(&d, Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), w, ws.data_ptr(), O.data_ptr(), M,
-                                                     M + padded(rows), stream_of(Q))
+        check(ws.defined() ? forward(&d, Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), w, ws.data_ptr(), O.data_ptr(), M, M + padded(rows),
+                                     stream_of(Q))
                            : api.convattn_fwd(&d, Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), w, O.data_ptr(), M, M + padded(rows), stream_of(Q)),
               "conv_attn.forward");
     }

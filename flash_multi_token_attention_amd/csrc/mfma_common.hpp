@@ -233,7 +233,9 @@ inline hipError_t set_max_lds_once(int bytes) {
 
 // ---- bf16 MFMA kernels ----
 hipError_t mfma_fwd(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
-                    const float *w, void *o, float *m, float *l, hipStream_t s);
+                    const float *w, void *o, float *m, float *l, hipStream_t s, float *part = nullptr);
+// room for the parts of the query tiles whose keys several workgroups share (`part` above), 0 where none do
+size_t mfma_fwd_split_bytes(const Problem &p);
 
 constexpr int kMfmaDqRows = 128;   // query rows per dQ/dW workgroup (= one dW partial)
 inline int mfma_dq_tiles(const Problem &p) { return (p.Nq + kMfmaDqRows - 1) / kMfmaDqRows; }
@@ -249,6 +251,42 @@ inline int mfma_kv_tiles(const Problem &p) { return (p.Nk + 8 + kKvKeysPerWg - 1
 // [key tile of 32][row tile of 32][32 rows][32 keys], which mfma_dq_from_rows multiplies with K.
 // dc_scale holds {s, log2 s} per (batch, head): the power of two dC is carried at (mfma_dc_scale).
 constexpr int kChainKeys = 32, kChainRows = 32;
+// A workgroup walks the row tiles (of 32) that see its keys: under the causal mask those from key block kb's own rows on.
+// share > 0: a key block's tiles are cut into parts of at most `share` tiles, one workgroup each (partial dK / dV in
+// fp32, added by chain_reduce).  Few (batch, head) pairs or rows leave the launch with less than a round of
+// workgroups, as long as its longest one (chain_share has the rule).
+struct ChainSpan { int kb, first_rt, len, part, parts; };
+__host__ __device__ inline int chain_first_tile(const Problem &p, int kb) {
+    return p.causal && kb > 0 ? (kb * kKvKeysPerWg - 8) / kChainRows : 0;
+}
+__host__ __device__ inline int chain_len(const Problem &p, int kb) { return (p.Nq + kChainRows - 1) / kChainRows - chain_first_tile(p, kb); }
+__host__ __device__ inline int chain_parts(const Problem &p, int kb, int share) {
+    const int len = chain_len(p, kb);
+    return share > 0 && len > share ? (len + share - 1) / share : 1;
+}
+// workgroup z of a (batch, head)
+__host__ __device__ inline ChainSpan chain_span(const Problem &p, int z, int share) {
+    ChainSpan s;
+    s.kb = z;
+    s.part = 0;
+    if (share > 0)
+        for (s.kb = 0, s.part = z; s.part >= chain_parts(p, s.kb, share); ++s.kb) s.part -= chain_parts(p, s.kb, share);
+    s.first_rt = chain_first_tile(p, s.kb);
+    s.len = chain_len(p, s.kb);
+    s.parts = chain_parts(p, s.kb, share);
+    return s;
+}
+inline int chain_wgs(const Problem &p, int share) {
+    int n = 0;
+    for (int kb = 0; kb < mfma_kv_tiles(p); ++kb) n += chain_parts(p, kb, share);
+    return n;
+}
+// bytes of the partial dK and dV: [batch, head][workgroup][dK, dV][128 keys][d] fp32
+inline size_t chain_part_bytes(const Problem &p, int share) {
+    return share > 0 ? (size_t)p.B * p.H * chain_wgs(p, share) * 2 * kKvKeysPerWg * p.d * sizeof(float) : 0;
+}
+int chain_share(const Problem &p);
+hipError_t chain_reduce(const Problem &p, int out_dt, int share, const float *part, void *dk, void *dv, hipStream_t s);
 inline int chain_key_tiles(const Problem &p) { return mfma_kv_tiles(p) * (kKvKeysPerWg / kChainKeys); }
 __host__ __device__ inline int chain_row_tiles(const Problem &p) { return (p.Nq + kChainRows - 1) / kChainRows; }
 // The dS blocks of one (batch, head) are kept as [key tile][row tile]; under the causal mask key tile kt has
@@ -272,7 +310,7 @@ hipError_t mfma_dc_scale(const Problem &p, const void *d_o, const void *v, float
 #define CHAIN_DECL(name)                                                                                   \
     hipError_t name(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const void *d_o, \
                     const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv, \
-                    void *ds_ws, float *dw_part, hipStream_t s)
+                    void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s)
 CHAIN_DECL(mfma_bwd_chain_kv);
 CHAIN_DECL(mfma_bwd_chain_qw);
 CHAIN_DECL(mfma_bwd_chain_all);
@@ -284,15 +322,15 @@ CHAIN_DECL(mfma_bwd_chain3_all);
 inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const void *q, const void *k, const void *v,
                                  const void *d_o, const float *Dl, const float *lse, const float *w,
                                  const float *dc_scale, void *dk, void *dv, void *ds_ws, float *dw_part,
-                                 hipStream_t s) {
+                                 hipStream_t s, int share = 0, float *kv_part = nullptr) {
     if (p.c_q <= 6) {
-        if (want == 1) return mfma_bwd_chain3_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-        if (want == 2) return mfma_bwd_chain3_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-        return mfma_bwd_chain3_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+        if (want == 1) return mfma_bwd_chain3_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+        if (want == 2) return mfma_bwd_chain3_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+        return mfma_bwd_chain3_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     }
-    if (want == 1) return mfma_bwd_chain_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-    if (want == 2) return mfma_bwd_chain_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
-    return mfma_bwd_chain_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, s);
+    if (want == 1) return mfma_bwd_chain_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    if (want == 2) return mfma_bwd_chain_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    return mfma_bwd_chain_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 // heads_inner: the blocks lie [batch][block][head] (all heads of a block side by side) instead of [batch, head][block]
 hipError_t mfma_dq_from_rows(const Problem &p, int out_dt, const void *k, const void *ds_ws,

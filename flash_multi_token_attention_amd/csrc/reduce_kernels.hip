@@ -1,7 +1,7 @@
 // Small bandwidth-bound helpers around the conv-attention kernels:
 // backward preparation (D, LSE), the ordered dW reduction and the decode
 // split merge.
-#include "common.hpp"
+#include "mfma_common.hpp"
 
 namespace convattn {
 namespace {
@@ -80,6 +80,33 @@ __global__ __launch_bounds__(1024) void dw_reduce_kernel(int B, int H, int n_til
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += red[w][lane];
         dW[(size_t)h * ntap + tap] = v;
+    }
+}
+
+// dK and dV of the key blocks whose row tiles several workgroups share: the partials added in the order of the rows.
+// x = 16-byte groups of a key block's dK, then dV, y = key block, z = (batch, head).
+template <typename TO>
+__global__ __launch_bounds__(256) void chain_reduce_kernel(Problem p, int share, int n_wg, const float *__restrict__ part,
+                                                           TO *__restrict__ dK, TO *__restrict__ dV) {
+    const int kb = blockIdx.y, parts = chain_parts(p, kb, share);
+    if (parts == 1) return;
+    int z = 0;
+    for (int i = 0; i < kb; ++i) z += chain_parts(p, i, share);
+    const int e = (blockIdx.x * 256 + threadIdx.x) * 4, per = kKvKeysPerWg * p.d;   // (2 per is a multiple of 1024)
+    const int is_v = e >= per, local = e - is_v * per, key = kb * kKvKeysPerWg + local / p.d - (is_v ? 8 : 0);
+    if (key < 0 || key >= p.Nk) return;
+    const float *src = part + ((size_t)blockIdx.z * n_wg + z) * 2 * per + e;
+    float4 sum = *reinterpret_cast<const float4 *>(src);
+    for (int i = 1; i < parts; ++i) {
+        const float4 v = *reinterpret_cast<const float4 *>(src + (size_t)i * 2 * per);
+        sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+    }
+    TO *dst = (is_v ? dV : dK) + ((size_t)blockIdx.z * p.Nk + key) * p.d + local % p.d;
+    if constexpr (sizeof(TO) == 2) {
+        bf16x4 o = {(bf16_t)sum.x, (bf16_t)sum.y, (bf16_t)sum.z, (bf16_t)sum.w};
+        *reinterpret_cast<bf16x4 *>(dst) = o;
+    } else {
+        *reinterpret_cast<float4 *>(dst) = sum;
     }
 }
 
@@ -176,6 +203,49 @@ hipError_t bwd_preprocess(const Problem &p, int in_dt, int out_dt, const void *o
 
 hipError_t dw_reduce(const Problem &p, int n_tiles, const float *dw_part, float *dw, hipStream_t s) {
     dw_reduce_kernel<<<dim3(p.H, (p.c_q * p.c_k + 63) / 64), 1024, 0, s>>>(p.B, p.H, n_tiles, p.c_q * p.c_k, dw_part, dw);
+    return hipGetLastError();
+}
+
+// Row tiles per workgroup of the split backward, or 0: one workgroup per key block.  In units of a row tile a workgroup
+// costs its tiles, about 4.5 for set-up and wind-down and one more where its range ends inside the key block; the launch
+// the longest workgroup or the CUs' even part of everything plus a third of the longest; the reduction kernel 6 to 8.
+// (B2 H8 N1531 d64 11x11: 167 -> 109 us, B1 H8 N2048 d64 7x7: 169 -> 72, B1 H8 N1000 d128 6x11: 78 -> 32.)
+// Sequences of less than 20 row tiles gain less than the reduction and its launch cost.  From 8192 rows on nothing is split, whatever
+// the number of heads is: a head's results do not depend on how many others there are.
+int chain_share(const Problem &p) {
+    const int n_rt = chain_row_tiles(p), n_kb = mfma_kv_tiles(p);
+    if (n_rt < 20 || p.Nq >= 8192 || p.B * (long long)p.H > 64) return 0;
+    float none = 0.f, best = 0.f;
+    int share = 0;
+    for (int cut = 1; cut <= 8; cut += cut < 4 ? 1 : 2) {
+        const int s = cut == 1 ? 0 : (n_rt + cut - 1) / cut;
+        if (cut > 1 && s < 6) break;
+        float total = 0.f, longest = 0.f;
+        int jobs = 0;
+        for (int kb = 0; kb < n_kb; ++kb) {
+            const int len = chain_len(p, kb) > 0 ? chain_len(p, kb) : 0, parts = chain_parts(p, kb, s);
+            const float one = (float)((len + parts - 1) / parts) + 4.5f + (parts > 1 ? 1.f : 0.f);
+            longest = one > longest ? one : longest;
+            total += one * parts;
+            jobs += parts;
+        }
+        const float n = (float)p.B * p.H, even = total * n / 256.f + longest / 3.f;
+        const float t = jobs * n <= 256.f || longest > even ? longest : even;
+        if (cut == 1) none = best = t;
+        else if (1.05f * t + 7.f < none && t < best) { best = t; share = s; }
+    }
+    return share;
+}
+
+hipError_t chain_reduce(const Problem &p, int out_dt, int share, const float *part, void *dk, void *dv, hipStream_t s) {
+    int split = 0;   // (the parts of a key block do not grow from block to block)
+    while (split < mfma_kv_tiles(p) && chain_parts(p, split, share) > 1) ++split;
+    const dim3 grid(2 * kKvKeysPerWg * p.d / 1024, split, p.B * p.H);
+    const int n_wg = chain_wgs(p, share);
+    if (out_dt == CONVATTN_BF16)
+        chain_reduce_kernel<bf16_t><<<grid, 256, 0, s>>>(p, share, n_wg, part, (bf16_t *)dk, (bf16_t *)dv);
+    else
+        chain_reduce_kernel<float><<<grid, 256, 0, s>>>(p, share, n_wg, part, (float *)dk, (float *)dv);
     return hipGetLastError();
 }
 

@@ -199,6 +199,24 @@ int convattn_bwd_fused_dq(const convattn_desc *desc, const void *q, const void *
 int convattn_bwd_fused_dw(const convattn_desc *desc, const void *workspace, float *dw, void *stream);
 
 /*
+ * What convattn_fwd computes for a bf16 problem with few (batch, head) pairs or rows: the keys of a tile of query rows are
+ * shared by several workgroups, their parts merged in a fixed order.  convattn_fwd_split_workspace_bytes is 0 for a
+ * descriptor that gains nothing from that (then convattn_fwd is the call).
+ */
+size_t convattn_fwd_split_workspace_bytes(const convattn_desc *desc);
+int convattn_fwd_split(const convattn_desc *desc, const void *q, const void *k, const void *v, const float *w, void *workspace,
+                       void *o, float *m, float *l, void *stream);
+
+/*
+ * What convattn_bwd_fused computes for a bf16 problem with few (batch, head) pairs or rows: the query rows of a block of 128
+ * keys are shared by several workgroups and their dK / dV added in a fixed order.  convattn_bwd_split_workspace_bytes is 0
+ * for a descriptor that gains nothing from that (then convattn_bwd_fused is the call).
+ */
+size_t convattn_bwd_split_workspace_bytes(const convattn_desc *desc);
+int convattn_bwd_split(const convattn_desc *desc, const void *q, const void *k, const void *v, const void *d_o, const float *D,
+                       const float *lse, const float *w, void *dq, void *dk, void *dv, float *dw, void *workspace, void *stream);
+
+/*
  * Forward and whole backward of the fp32-arithmetic path with score-sized fp32 matrices in the caller's workspace: each
  * (row, key) pair is convolved once instead of once per pass and tile (what convattn_fwd and convattn_bwd_fused compute
  * for these descriptors, several times faster).  convattn_staged_workspace_bytes: 4 bytes per pair forward, 12 backward,
