@@ -14,7 +14,7 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("B,H,N,d,c_q,c_k,causal", [
-    (1, 2, 577, 64, 3, 3, True), (1, 3, 641, 128, 6, 11, True), (2, 8, 1531, 64, 11, 11, True), (1, 8, 1000, 128, 8, 15, True),
+    (1, 2, 641, 64, 3, 3, True), (1, 3, 705, 128, 6, 11, True), (2, 8, 1531, 64, 11, 11, True), (1, 8, 1000, 128, 8, 15, True),
     (1, 4, 700, 32, 6, 5, False), (1, 2, 2049, 128, 9, 11, False), (1, 8, 1157, 32, 11, 7, True), (1, 1, 4000, 64, 6, 11, True),
 ])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
@@ -39,7 +39,7 @@ def test_split_equals_unsplit(B, H, N, d, c_q, c_k, causal, out_dtype, monkeypat
 
 
 @pytest.mark.parametrize("B,H,N,d,c_q,c_k,causal", [
-    (1, 2, 900, 64, 3, 3, True), (2, 8, 1531, 64, 11, 11, True), (1, 8, 1000, 128, 8, 15, True), (1, 4, 1217, 32, 6, 17, False),
+    (1, 2, 1100, 64, 3, 3, True), (2, 8, 1531, 64, 11, 11, True), (1, 8, 1000, 128, 8, 15, True), (1, 4, 1217, 32, 6, 17, False),
     (1, 2, 2049, 128, 9, 11, False), (1, 8, 1157, 32, 11, 7, True), (1, 1, 4000, 64, 6, 11, True), (1, 3, 1600, 128, 6, 11, True),
 ])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
