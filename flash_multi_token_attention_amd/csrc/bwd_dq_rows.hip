@@ -28,7 +28,10 @@ template <int D> struct RowsLds {
     static constexpr int total = 2 * k_bytes;
 };
 
-template <int D, typename TO>
+// KEYS: the four waves of a workgroup share 32 rows, wave w takes the key steps w, w + 4, .. through LDS room of its own, and
+// their sums are added at the end: for launches that would leave CUs idle or end with a few long workgroups.
+// (B1 H8 N2048 d64 27.8 -> 14.8 us, B2 H8 N1531 22.6 -> 15.3, B1 H8 N1000 d128 19.2 -> 11.6.)
+template <int D, typename TO, bool KEYS>
 __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_t *__restrict__ K,
                                                           const bf16_t *__restrict__ dS_ws,
                                                           const float *__restrict__ dc_scale, int n_kt,
@@ -37,7 +40,7 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
     constexpr int RST = Lds::RST;
     constexpr int DB = D / 16, CPR = D / 8;
     constexpr int K_CH = BKS * CPR;                 // 16-byte chunks of a K step
-    constexpr int K_LD = K_CH / (NW * 64);          // 4 (D = 128) or 2 (D = 64)
+    constexpr int K_LD = K_CH / (KEYS ? 64 : NW * 64);   // per lane
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
     const int tid = threadIdx.x;
@@ -45,7 +48,8 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
     const int g = lane >> 4, n = lane & 15;
     const int h = blockIdx.x, b = blockIdx.y;
     const int qt = gridDim.z - 1 - blockIdx.z;  // longest (causal) row tiles first
-    const int i0 = qt * BQ, rw = i0 + wave * 32, rt = rw / kChainRows;
+    const int i0 = qt * (KEYS ? kChainRows : BQ), rw = KEYS ? i0 : i0 + wave * 32, rt = rw / kChainRows;
+    const int s0 = KEYS ? wave : 0, ds = KEYS ? NW : 1;   // this wave's first step and stride
     const bool causal = p.causal != 0;
     const size_t bh = (size_t)b * p.H + h;
     const bf16_t *Kb = K + bh * p.Nk * D;
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
 #pragma unroll
         for (int db = 0; db < DB; ++db) acc[ob][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-    const int k_end = causal ? min(p.Nk, i0 + BQ) : p.Nk;
+    const int k_end = causal ? min(p.Nk, i0 + (KEYS ? kChainRows : BQ)) : p.Nk;
     const int n_steps = (k_end + BKS - 1) / BKS;
     const bool row_ok = rt < n_rt;
 
@@ -69,7 +73,7 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
     auto load_k = [&](int s) {
 #pragma unroll
         for (int i = 0; i < K_LD; ++i) {
-            const int c = tid + i * NW * 64, row = c / CPR, cc = c % CPR;
+            const int c = KEYS ? lane + i * 64 : tid + i * NW * 64, row = c / CPR, cc = c % CPR;
             kr[i] = load_row16_clamped<D>(Kb, s * BKS + row, p.Nk, cc * 8);
         }
     };
@@ -92,10 +96,10 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
     };
 
     auto run_step = [&](int s, u32x4 (&sr)[2][2]) {
-        unsigned char *Ks = smem + (s & 1) * Lds::k_bytes;
+        unsigned char *Ks = smem + (KEYS ? wave : s & 1) * Lds::k_bytes;
 #pragma unroll
         for (int i = 0; i < K_LD; ++i) {
-            const int c = tid + i * NW * 64, row = c / CPR, cc = c % CPR;
+            const int c = KEYS ? lane + i * 64 : tid + i * NW * 64, row = c / CPR, cc = c % CPR;
             *reinterpret_cast<u32x4 *>(Ks + row * RST + cc * 16) = zero_unless(s * BKS + row < p.Nk, kr[i]);
         }
         bf16x8 sf[2][2];
@@ -107,9 +111,14 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) sf[kp][ob] = __builtin_bit_cast(bf16x8, zero_unless(ok, sr[kp][ob]));
         }
-        __syncthreads();
-        load_k(s + 1);
-        load_ds(s + 2, sr);
+        if constexpr (KEYS) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
+        load_k(s + ds);
+        load_ds(s + 2 * ds, sr);
         if (causal && s * BKS > rw + 31) return;  // every key of the step is after the wave's rows
 
 #pragma unroll
@@ -125,12 +134,35 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
             }
         }
     };
-    load_k(0);
-    load_ds(0, sr_a);
-    load_ds(1, sr_b);
-    for (int s = 0; s < n_steps; s += 2) {
+    load_k(s0);
+    load_ds(s0, sr_a);
+    load_ds(s0 + ds, sr_b);
+    for (int s = s0; s < n_steps; s += 2 * ds) {
         run_step(s, sr_a);
-        if (s + 1 < n_steps) run_step(s + 1, sr_b);
+        if constexpr (KEYS) {   // (this wave's reads of its room before its next writes)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (s + ds < n_steps) run_step(s + ds, sr_b);
+        if constexpr (KEYS) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    if constexpr (KEYS) {
+        static_assert(2 * DB * 1024 <= Lds::k_bytes, "a wave's sums fit its room");
+        f32x4 *mine = reinterpret_cast<f32x4 *>(smem + wave * Lds::k_bytes);
+#pragma unroll
+        for (int e = 0; e < 2 * DB; ++e) mine[e * 64 + lane] = acc[e / DB][e % DB];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 2 * DB; ++e) {
+            if (e % NW != wave) continue;
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v += reinterpret_cast<const f32x4 *>(smem + w * Lds::k_bytes)[e * 64 + lane];
+            acc[e / DB][e % DB] = v;
+        }
     }
 
     // lane n of block ob = row 2 n + ob of the wave's 32; 4 consecutive head-dim columns per block
@@ -142,6 +174,7 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
             TO *orow = dQ + (bh * p.Nq + qpos) * D;
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
+                if (KEYS && (ob * DB + db) % NW != wave) continue;
                 const int col = db * 16 + 4 * g;
                 if constexpr (sizeof(TO) == 2) {
                     bf16x4 ov;
@@ -159,11 +192,21 @@ __global__ __launch_bounds__(NW * 64) void dq_rows_kernel(Problem p, const bf16_
 template <int D, typename TO>
 hipError_t launch(const Problem &p, const void *k, const void *ds_ws, const float *dc_scale, void *dq,
                   hipStream_t s, int heads_inner) {
-    auto kern = dq_rows_kernel<D, TO>;
-    constexpr int lds = RowsLds<D>::total;
-    dim3 grid(p.H, p.B, (p.Nq + BQ - 1) / BQ);
-    kern<<<grid, NW * 64, lds, s>>>(p, (const bf16_t *)k, (const bf16_t *)ds_ws, dc_scale, chain_key_tiles(p),
-                                    chain_row_tiles(p), heads_inner, (TO *)dq);
+    // With two workgroups per CU or fewer the launch is as long as its longest workgroup: the waves share the keys then.
+    // (Not from 8192 rows on: a head's results do not depend on how many others there are.)
+    const long long wgs = (long long)p.B * p.H * ((p.Nq + BQ - 1) / BQ);
+    if (wgs <= 512 && p.Nq < 8192) {
+        constexpr int lds = NW * RowsLds<D>::k_bytes;
+        if (lds > 64 * 1024) {
+            hipError_t e = set_max_lds_once<dq_rows_kernel<D, TO, true>>(lds);
+            if (e != hipSuccess) return e;
+        }
+        dq_rows_kernel<D, TO, true><<<dim3(p.H, p.B, chain_row_tiles(p)), NW * 64, lds, s>>>(
+            p, (const bf16_t *)k, (const bf16_t *)ds_ws, dc_scale, chain_key_tiles(p), chain_row_tiles(p), heads_inner, (TO *)dq);
+        return hipGetLastError();
+    }
+    dq_rows_kernel<D, TO, false><<<dim3(p.H, p.B, (p.Nq + BQ - 1) / BQ), NW * 64, RowsLds<D>::total, s>>>(
+        p, (const bf16_t *)k, (const bf16_t *)ds_ws, dc_scale, chain_key_tiles(p), chain_row_tiles(p), heads_inner, (TO *)dq);
     return hipGetLastError();
 }
 
