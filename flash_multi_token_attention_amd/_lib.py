@@ -71,6 +71,7 @@ _SIGNATURES = {
     "convattn_fwd_split": (C.c_int, [_D] + [_P] * 9),
     "convattn_bwd_split_workspace_bytes": (C.c_size_t, [_D]),
     "convattn_bwd_split": (C.c_int, [_D] + [_P] * 13),
+    "convattn_bwd_all": (C.c_int, [_D] + [_P] * 14 + [C.c_int] + [_P] * 2),
     "convattn_staged_workspace_bytes": (C.c_size_t, [_D, C.c_int]),
     "convattn_staged_fwd": (C.c_int, [_D] + [_P] * 9),
     "convattn_staged_bwd": (C.c_int, [_D] + [_P] * 13),

@@ -301,6 +301,20 @@ static SplitWs split_ws(const Problem &p) {
     return w;
 }
 
+// everything but the dC scale
+static hipError_t run_split(const Problem &p, int out_dt, const SplitWs &lay, const void *q, const void *k, const void *v,
+                            const void *d_o, const float *D, const float *lse, const float *w, void *dq, void *dk, void *dv,
+                            float *dw, void *workspace, hipStream_t s) {
+    unsigned char *ws = static_cast<unsigned char *>(workspace);
+    float *part = reinterpret_cast<float *>(ws + lay.part_off), *scale = reinterpret_cast<float *>(ws + lay.scale_off);
+    float *kv = reinterpret_cast<float *>(ws + lay.kv_off);
+    hipError_t e = mfma_bwd_chain(p, out_dt, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s, lay.share, kv);
+    if (e == hipSuccess) e = chain_reduce(p, out_dt, lay.share, kv, dk, dv, s);
+    if (e == hipSuccess) e = mfma_dq_from_rows(p, out_dt, k, ws, scale, dq, s);
+    if (e == hipSuccess) e = dw_reduce(p, lay.n_wg, part, dw, s);
+    return e;
+}
+
 size_t convattn_bwd_split_workspace_bytes(const convattn_desc *desc) {
     Problem p;
     if (validate(desc, CONVATTN_OP_BWD, &p) || pick_path(desc, p, CONVATTN_OP_BWD) != 1) return 0;
@@ -318,14 +332,33 @@ int convattn_bwd_split(const convattn_desc *desc, const void *q, const void *k, 
     const SplitWs lay = pick_path(desc, p, CONVATTN_OP_BWD) == 1 ? split_ws(p) : SplitWs{};
     if (!lay.total) return CONVATTN_ERR_SHAPE;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    float *scale = reinterpret_cast<float *>(static_cast<unsigned char *>(workspace) + lay.scale_off);
+    const hipError_t e = mfma_dc_scale(p, d_o, v, scale, s);
+    return e == hipSuccess ? (int)run_split(p, desc->out_dtype, lay, q, k, v, d_o, D, lse, w, dq, dk, dv, dw, workspace, s) : (int)e;
+}
+
+int convattn_bwd_all(const convattn_desc *desc, const void *q, const void *k, const void *v, const void *o, const void *d_o,
+                     const float *m, const float *l, const float *w, float *D, float *lse, void *dq, void *dk, void *dv,
+                     float *dw, int split, void *workspace, void *stream) {
+    Problem p;
+    int rc = validate(desc, CONVATTN_OP_BWD, &p);
+    if (rc) return rc;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(o); REQUIRE_PTR(d_o); REQUIRE_PTR(m); REQUIRE_PTR(l); REQUIRE_PTR(w);
+    REQUIRE_PTR(D); REQUIRE_PTR(lse); REQUIRE_PTR(dq); REQUIRE_PTR(dk); REQUIRE_PTR(dv); REQUIRE_PTR(dw); REQUIRE_PTR(workspace);
+    if (pick_path(desc, p, CONVATTN_OP_BWD) != 1) return CONVATTN_ERR_SHAPE;
+    const SplitWs cut = split ? split_ws(p) : SplitWs{};
+    if (split && !cut.total) return CONVATTN_ERR_SHAPE;
+    const FusedWs lay = fused_ws(p);
+    hipStream_t s = static_cast<hipStream_t>(stream);
     unsigned char *ws = static_cast<unsigned char *>(workspace);
-    float *part = reinterpret_cast<float *>(ws + lay.part_off), *scale = reinterpret_cast<float *>(ws + lay.scale_off);
-    float *kv = reinterpret_cast<float *>(ws + lay.kv_off);
-    hipError_t e = mfma_dc_scale(p, d_o, v, scale, s);
-    if (e == hipSuccess) e = mfma_bwd_chain(p, desc->out_dtype, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s, lay.share, kv);
-    if (e == hipSuccess) e = chain_reduce(p, desc->out_dtype, lay.share, kv, dk, dv, s);
+    float *scale = reinterpret_cast<float *>(ws + (split ? cut.scale_off : lay.scale_off));
+    hipError_t e = bwd_prepare(p, desc->out_dtype, o, d_o, v, m, l, D, lse, scale, s);
+    if (e != hipSuccess) return (int)e;
+    if (split) return (int)run_split(p, desc->out_dtype, cut, q, k, v, d_o, D, lse, w, dq, dk, dv, dw, workspace, s);
+    float *part = reinterpret_cast<float *>(ws + lay.part_off);
+    e = mfma_bwd_chain(p, desc->out_dtype, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s);
     if (e == hipSuccess) e = mfma_dq_from_rows(p, desc->out_dtype, k, ws, scale, dq, s);
-    if (e == hipSuccess) e = dw_reduce(p, lay.n_wg, part, dw, s);
+    if (e == hipSuccess) e = dw_reduce(p, mfma_kv_tiles(p), part, dw, s);
     return (int)e;
 }
 

@@ -821,7 +821,6 @@ __global__ __launch_bounds__(NT) void bwd_chain_kernel(ChainArgs args) {
 // amax|dO| and amax|V| of one (batch, head) -> {s, log2 s}, s the power of two that brings
 // sqrt(d) * amax|dO| * amax|V| (a few times a typical |dP|) to about 2^12.  Two steps: kScaleChunks
 // workgroups per (batch, head) leave their maxima in `part`, one thread per (batch, head) finishes.
-constexpr int kScaleChunks = 32;
 __global__ __launch_bounds__(256) void dc_scale_partial_kernel(int Nq, int Nk, int d, const bf16_t *__restrict__ dO,
                                                                const bf16_t *__restrict__ V, float *__restrict__ part) {
     const size_t bh = (size_t)blockIdx.z * gridDim.y + blockIdx.y;   // y = head, z = batch
@@ -858,11 +857,7 @@ __global__ void dc_scale_finish_kernel(int n_bh, int d, const float *__restrict_
         a = fmaxf(a, part[((size_t)bh * kScaleChunks + c) * 2]);
         v = fmaxf(v, part[((size_t)bh * kScaleChunks + c) * 2 + 1]);
     }
-    const float prod = sqrtf((float)d) * a * v;
-    float e = 0.f;
-    if (prod > 0.f && prod < 3e38f) e = fminf(fmaxf(floorf(12.f - log2f(prod)), -60.f), 60.f);
-    out[2 * bh] = exp2f(e);
-    out[2 * bh + 1] = e;
+    write_dc_scale(d, a, v, out + 2 * bh);
 }
 
 #endif
@@ -917,9 +912,11 @@ hipError_t mfma_dc_scale(const Problem &p, const void *d_o, const void *v, float
     float *part = dc_scale + (size_t)p.B * p.H * 2;
     dc_scale_partial_kernel<<<dim3(kScaleChunks, p.H, p.B), 256, 0, s>>>(p.Nq, p.Nk, p.d, (const bf16_t *)d_o,
                                                                           (const bf16_t *)v, part);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    dc_scale_finish_kernel<<<dim3((p.B * p.H + 255) / 256), 256, 0, s>>>(p.B * p.H, p.d, part, dc_scale);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? dc_scale_finish(p, dc_scale, s) : e;
+}
+hipError_t dc_scale_finish(const Problem &p, float *dc_scale, hipStream_t s) {
+    dc_scale_finish_kernel<<<dim3((p.B * p.H + 255) / 256), 256, 0, s>>>(p.B * p.H, p.d, dc_scale + (size_t)p.B * p.H * 2, dc_scale);
     return hipGetLastError();
 }
 #endif

@@ -28,7 +28,7 @@ using torch::autograd::variable_list;
 // ---- the C ABI, from the library Python has loaded ----
 #define API_LIST(F)                                                                                                   \
     F(convattn_strerror) F(convattn_fwd) F(convattn_fwd_split_workspace_bytes) F(convattn_fwd_split) F(convattn_bwd_preprocess) F(convattn_bwd_fused_workspace_bytes)              \
-    F(convattn_bwd_fused) F(convattn_bwd_split_workspace_bytes) F(convattn_bwd_split) F(convattn_staged_workspace_bytes) F(convattn_staged_fwd) F(convattn_staged_bwd)               \
+    F(convattn_bwd_fused) F(convattn_bwd_split_workspace_bytes) F(convattn_bwd_all) F(convattn_staged_workspace_bytes) F(convattn_staged_fwd) F(convattn_staged_bwd)               \
     F(convattn_decode_strided) F(convattn_decode_kv) F(convattn_decode_combine)                 \
     F(convattn_headmix_validate) F(convattn_headmix_fwd_workspace_bytes) F(convattn_headmix_fwd_ws)                   \
     F(convattn_headmix_bwd_fused_workspace_bytes) F(convattn_headmix_bwd_fused)
@@ -149,14 +149,12 @@ struct WindowBackward : torch::autograd::Node {
             // (D and LSE ahead of the workspace, which counts for the cap alone as in the Python op)
             auto reserve = [&](size_t bytes) { return bytes && bytes <= workspace_cap() ? workspace(bytes + 2 * stat, Q) : Tensor(); };
             Tensor ws = reserve(api.convattn_staged_workspace_bytes(&d, CONVATTN_OP_BWD));
-            auto backward = api.convattn_staged_bwd;
-            if (!ws.defined()) {
+            const bool staged = ws.defined();
+            int split = 0;
+            if (!staged) {
                 ws = reserve(api.convattn_bwd_split_workspace_bytes(&d));
-                backward = api.convattn_bwd_split;
-            }
-            if (!ws.defined()) {
-                ws = reserve(api.convattn_bwd_fused_workspace_bytes(&d));
-                backward = api.convattn_bwd_fused;
+                split = ws.defined();
+                if (!split) ws = reserve(api.convattn_bwd_fused_workspace_bytes(&d));
             }
             if (ws.defined()) {
                 char *base = static_cast<char *>(ws.data_ptr());
@@ -165,12 +163,20 @@ struct WindowBackward : torch::autograd::Node {
                 void *s = stream_of(Q);
                 Tensor dQ = empty(Q.sizes(), Q.scalar_type(), Q), dK = empty(K.sizes(), Q.scalar_type(), Q),
                        dV = empty(V.sizes(), Q.scalar_type(), Q), dW = empty(W.sizes(), at::kFloat, Q);
-                convattn_desc pre = d;
-                pre.Nk = pre.Nq; pre.c_q = pre.c_k = 1; pre.scale = 1; pre.causal = 0;
-                check(api.convattn_bwd_preprocess(&pre, O.data_ptr(), dO.data_ptr(), M, L, D, lse, s), "conv_attn.bwd_preprocess");
-                check(backward(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), dO.data_ptr(), D, lse, Wf.const_data_ptr<float>(),
-                               dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), dW.mutable_data_ptr<float>(), base + 2 * stat, s),
-                      "conv_attn.backward");
+                const float *w = Wf.const_data_ptr<float>();
+                if (staged) {
+                    convattn_desc pre = d;
+                    pre.Nk = pre.Nq; pre.c_q = pre.c_k = 1; pre.scale = 1; pre.causal = 0;
+                    check(api.convattn_bwd_preprocess(&pre, O.data_ptr(), dO.data_ptr(), M, L, D, lse, s), "conv_attn.bwd_preprocess");
+                    check(api.convattn_staged_bwd(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), dO.data_ptr(), D, lse, w, dQ.data_ptr(),
+                                                  dK.data_ptr(), dV.data_ptr(), dW.mutable_data_ptr<float>(), base + 2 * stat, s),
+                          "conv_attn.backward");
+                } else {
+                    check(api.convattn_bwd_all(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), dO.data_ptr(), M, L, w, D, lse,
+                                               dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), dW.mutable_data_ptr<float>(), split,
+                                               base + 2 * stat, s),
+                          "conv_attn.backward");
+                }
                 out[0] = dQ; out[1] = dK; out[2] = dV;
                 out[3] = W.scalar_type() == at::kFloat ? dW : dW.to(W.scalar_type());
                 return out;

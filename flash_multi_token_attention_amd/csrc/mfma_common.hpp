@@ -216,6 +216,18 @@ __device__ __forceinline__ float dc_scale_log2_from_d(const float *__restrict__ 
 }
 #endif
 
+#if defined(__HIPCC__)
+// {s, log2 s} of a (batch, head) from amax|dO| and amax|V|: s the power of two that brings sqrt(d) amax|dO| amax|V| (a few
+// times a typical |dP|) to about 2^12
+__device__ __forceinline__ void write_dc_scale(int d, float a, float v, float *out) {
+    const float prod = sqrtf((float)d) * a * v;
+    float e = 0.f;
+    if (prod > 0.f && prod < 3e38f) e = fminf(fmaxf(floorf(12.f - log2f(prod)), -60.f), 60.f);
+    out[0] = exp2f(e);
+    out[1] = e;
+}
+#endif
+
 // Raises a kernel's dynamic LDS limit once per device (the attribute is sticky; setting it on every
 // launch costs a driver call).  One instance, and one flag word, per kernel instantiation.
 template <auto Kern>
@@ -305,6 +317,11 @@ inline size_t chain_ds_bytes(const Problem &p) {
 // {s, log2 s} per (batch, head) followed by 32 x 2 partial maxima per (batch, head)
 inline size_t chain_scale_bytes(const Problem &p) { return (size_t)p.B * p.H * (2 + 64) * sizeof(float); }
 hipError_t mfma_dc_scale(const Problem &p, const void *d_o, const void *v, float *dc_scale, hipStream_t s);
+// its second step alone; D, LSE and the dC scale together (reduce_kernels.hip)
+constexpr int kScaleChunks = 32;
+hipError_t dc_scale_finish(const Problem &p, float *dc_scale, hipStream_t s);
+hipError_t bwd_prepare(const Problem &p, int out_dt, const void *o, const void *d_o, const void *v, const float *m, const float *l,
+                       float *D, float *lse, float *dc_scale, hipStream_t s);
 // want: bit 0 = dK and dV, bit 1 = dS blocks (for dQ) and the dW partial; dc_scale may be null when
 // bit 1 is clear (the kernel then takes the scale from D).
 #define CHAIN_DECL(name)                                                                                   \

@@ -50,6 +50,67 @@ __global__ __launch_bounds__(256) void preprocess_kernel(size_t rows, int d, con
     }
 }
 
+// D, LSE and the dC scale of the bf16 backward from one reading of O, dO and V: D / 8 lanes per row, x = rows of one of
+// `chunks` parts of a (batch, head).  One part: the workgroup has the maxima of all of them and writes the scale;
+// several: it leaves its maxima (the layout of dc_scale_partial_kernel) for dc_scale_finish.
+template <int D, typename TO>
+__global__ void bwd_prepare_kernel(int Nq, int Nk, const TO *__restrict__ O, const bf16_t *__restrict__ dO,
+                                   const bf16_t *__restrict__ V, const float *__restrict__ M, const float *__restrict__ L,
+                                   float *__restrict__ Dl, float *__restrict__ LSE, float *__restrict__ part,
+                                   float *__restrict__ scale) {
+    constexpr int LPR = D / 8;
+    __shared__ float red[2][16];
+    const size_t bh = (size_t)blockIdx.z * gridDim.y + blockIdx.y;   // y = head, z = batch
+    const int tid = threadIdx.x, sub = tid % LPR, step = blockDim.x / LPR;
+    float top[2] = {0.f, 0.f};
+    auto bounds = [&](int n, int &lo, int &hi) {
+        const int per = (n + gridDim.x - 1) / gridDim.x;
+        lo = blockIdx.x * per;
+        hi = min(n, lo + per);
+    };
+    int lo, hi;
+    bounds(Nq, lo, hi);
+    for (int r = lo + tid / LPR; r < hi; r += step) {
+        const size_t row = bh * Nq + r;
+        float o[8], g[8], s = 0.f;
+        load8(O + row * D + sub * 8, o);
+        load8(dO + row * D + sub * 8, g);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            s = fmaf(o[i], g[i], s);
+            top[0] = fmaxf(top[0], fabsf(g[i]));
+        }
+#pragma unroll
+        for (int m = LPR / 2; m >= 1; m >>= 1) s += __shfl_xor(s, m, LPR);
+        if (sub == 0) {
+            Dl[row] = s;
+            LSE[row] = M[row] + __logf(L[row]);
+        }
+    }
+    bounds(Nk, lo, hi);
+    for (int r = lo + tid / LPR; r < hi; r += step) {
+        float v[8];
+        load8(V + (bh * Nk + r) * D + sub * 8, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) top[1] = fmaxf(top[1], fabsf(v[i]));
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        top[x] = wave_max(top[x]);
+        if ((tid & 63) == 0) red[x][tid >> 6] = top[x];
+    }
+    __syncthreads();
+    if (tid < 2) {
+        float mx = 0.f;
+        for (int w = 0; w < (int)blockDim.x / 64; ++w) mx = fmaxf(mx, red[tid][w]);
+        red[tid][0] = mx;
+        if (gridDim.x > 1) part[(bh * gridDim.x + blockIdx.x) * 2 + tid] = mx;
+    }
+    if (gridDim.x > 1) return;
+    __syncthreads();
+    if (tid == 0) write_dc_scale(D, red[0][0], red[1][0], scale + 2 * bh);
+}
+
 // dW[h][tap] = sum over (batch, tile) of the partials, in a fixed order: a workgroup takes 64 taps
 // of one head (lane = tap, so a partial is read with contiguous loads); wave w adds the partials
 // w, w+4, ... in four independent chains, and the four waves' sums are added in wave order.
@@ -199,6 +260,26 @@ hipError_t bwd_preprocess(const Problem &p, int in_dt, int out_dt, const void *o
     else CALL(float, float);
 #undef CALL
     return hipGetLastError();
+}
+
+// part: dc_scale as mfma_dc_scale leaves it ({s, log2 s} per (batch, head), then the maxima of kScaleChunks parts)
+hipError_t bwd_prepare(const Problem &p, int out_dt, const void *o, const void *d_o, const void *v, const float *m, const float *l,
+                       float *D, float *lse, float *dc_scale, hipStream_t s) {
+    // (one workgroup reads 64 K elements of each tensor in about 4 us, as long as the second launch would take)
+    const bool one = (long long)(p.Nq > p.Nk ? p.Nq : p.Nk) * p.d <= 65536;
+    const dim3 grid(one ? 1 : kScaleChunks, p.H, p.B);
+    float *part = dc_scale + (size_t)p.B * p.H * 2;
+#define CALL(DD, TO)                                                                                                            \
+    bwd_prepare_kernel<DD, TO><<<grid, one ? 1024 : 256, 0, s>>>(p.Nq, p.Nk, (const TO *)o, (const bf16_t *)d_o, (const bf16_t *)v, m, \
+                                                                 l, D, lse, part, dc_scale)
+#define PICK(DD) (out_dt == CONVATTN_BF16 ? CALL(DD, bf16_t) : CALL(DD, float))
+    if (p.d == 32) PICK(32);
+    else if (p.d == 64) PICK(64);
+    else PICK(128);
+#undef PICK
+#undef CALL
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess || one ? e : dc_scale_finish(p, dc_scale, s);
 }
 
 hipError_t dw_reduce(const Problem &p, int n_tiles, const float *dw_part, float *dw, hipStream_t s) {

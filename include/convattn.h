@@ -217,6 +217,14 @@ int convattn_bwd_split(const convattn_desc *desc, const void *q, const void *k, 
                        const float *lse, const float *w, void *dq, void *dk, void *dv, float *dw, void *workspace, void *stream);
 
 /*
+ * convattn_bwd_preprocess and convattn_bwd_fused (split = 0) or convattn_bwd_split (split = 1) of a bf16 problem in one
+ * call, with the workspace of the latter: D, LSE (both written) and the dC scale come from one reading of O, dO and V.
+ */
+int convattn_bwd_all(const convattn_desc *desc, const void *q, const void *k, const void *v, const void *o, const void *d_o,
+                     const float *m, const float *l, const float *w, float *D, float *lse, void *dq, void *dk, void *dv,
+                     float *dw, int split, void *workspace, void *stream);
+
+/*
  * Forward and whole backward of the fp32-arithmetic path with score-sized fp32 matrices in the caller's workspace: each
  * (row, key) pair is convolved once instead of once per pass and tile (what convattn_fwd and convattn_bwd_fused compute
  * for these descriptors, several times faster).  convattn_staged_workspace_bytes: 4 bytes per pair forward, 12 backward,
