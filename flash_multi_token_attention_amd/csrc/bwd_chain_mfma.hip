@@ -95,7 +95,9 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
 
     // x = head, y = batch, z = key tile: the first key tiles see the most rows and go first
     const int h = blockIdx.x, b = blockIdx.y;
-    const ChainSpan span = chain_span(p, blockIdx.z, args.share);
+    // (SPLIT: instances of their own, the others are up to 2 % slower with the parts' bounds at run time)
+    constexpr bool SPLIT = (WANT & 4) != 0;
+    const ChainSpan span = SPLIT ? chain_span(p, blockIdx.z, args.share) : ChainSpan{(int)blockIdx.z, 0, 0, 0, 1};
     const int k0 = span.kb * BKW, c0 = k0 + pr * WK;
     const int pk = p.pk, cq = p.c_q, ck = p.c_k;
     const bool causal = p.causal != 0;
@@ -117,13 +119,14 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
     }
 
     // Causal: rows before the first key this workgroup touches (k0 - 8) see none of its keys.
-    const int t_begin = span.len * span.part / span.parts, t_end = span.len * (span.part + 1) / span.parts;
-    const int r_begin = (span.first_rt + t_begin) * BR, n_tiles = t_end - t_begin;
+    const int t_begin = SPLIT ? span.len * span.part / span.parts : 0, t_end = SPLIT ? span.len * (span.part + 1) / span.parts : 0;
+    const int r_begin = SPLIT ? (span.first_rt + t_begin) * BR : causal ? (max(0, k0 - 8) / BR) * BR : 0;
+    const int n_tiles = SPLIT ? t_end - t_begin : (p.Nq - r_begin + BR - 1) / BR;
     // The window of the last tile's rows reaches into the tile after it, whose dC is computed here too where it is
     // another workgroup's: n_scored tiles have scores and dC, n_tiles of them everything else.
-    const int n_scored = n_tiles + (t_end < span.len ? 1 : 0);
+    const int n_scored = n_tiles + (SPLIT && t_end < span.len ? 1 : 0);
     // this workgroup's partial dK / dV, or null: it writes the results itself
-    float *kv_part = span.parts > 1 ? args.kv_part + (bh * gridDim.z + blockIdx.z) * (2 * BKW * D) : nullptr;
+    float *kv_part = SPLIT && span.parts > 1 ? args.kv_part + (bh * gridDim.z + blockIdx.z) * (2 * BKW * D) : nullptr;
     // masks are needed next to the diagonal, at both ends of the key axis and past the last row
     const bool always_edge = c0 < 8 || c0 + 40 > p.Nk;
     auto is_edge = [&](int r0) { return always_edge || (causal && r0 < c0 + 64) || r0 + BR > p.Nq; };
@@ -514,7 +517,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
         for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
             for (int f = 0; f < 2; ++f) prev_dc[cb][f][0] = prev_dc[cb][f][1] = 0u;
-        const int n_kt = (p.Nk + 8 + BKW - 1) / BKW * NP, kt = span.kb * NP + pr;
+        const int n_kt = (SPLIT ? (p.Nk + 8 + BKW - 1) / BKW : (int)gridDim.z) * NP, kt = span.kb * NP + pr;
         // (causal: the pair's first block is row tile kt - 1)
         bf16_t *ds_pair = dS_ws + (bh * (size_t)chain_ds_block_off(causal, n_rt, n_kt) + (size_t)chain_ds_block_off(causal, n_rt, kt) -
                                    chain_ds_first_rt(causal, kt)) * (WK * BR);
@@ -770,7 +773,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 const int col = db * 16 + 4 * g;
-                if (WANT_KV && kv_part) {
+                if (SPLIT && WANT_KV && kv_part) {
                     float *dst = kv_part + (pr * WK + m * 16 + n) * D + col;
                     *reinterpret_cast<f32x4 *>(dst) = acc_k[m][db] * inv;
                     *reinterpret_cast<f32x4 *>(dst + BKW * D) = acc_v[m][db] * inv;
@@ -922,12 +925,14 @@ hipError_t dc_scale_finish(const Problem &p, float *dc_scale, hipStream_t s) {
 #endif
 
 // This file is compiled once per value of CONVATTN_CHAIN_UNIT (1 = dK and dV only, 2 = dS and dW
-// only, 3 = everything), so that the three sets of instances build in parallel.
+// only, 3 = everything, 7 = everything with split row ranges), so that the three sets of instances build in parallel.
 #ifndef CONVATTN_CHAIN_UNIT
 #define CONVATTN_CHAIN_UNIT 3
 #endif
 #if CONVATTN_CHAIN_UNIT == 1
 #define CHAIN_ENTRY mfma_bwd_chain_kv
+#elif CONVATTN_CHAIN_UNIT == 7
+#define CHAIN_ENTRY mfma_bwd_chain_split
 #elif CONVATTN_CHAIN_UNIT == 2
 #define CHAIN_ENTRY mfma_bwd_chain_qw
 #else

@@ -54,7 +54,7 @@ constexpr float kMaxSlack = 6.f;  // log2 units a score may exceed its row's exp
 constexpr int wave_rows(int cqt) { return 33 - cqt; }
 
 constexpr int kFwdPfv = 2;    // V^T fragments read ahead of their MFMAs in the P V phase
-constexpr int kFwdNbuf = 2;   // LDS buffers: the rows of step u+1 arrive during step u (3, two steps ahead, measured no faster)
+constexpr int kFwdNbuf = 2;   // LDS buffers: the rows of step u+1 arrive during step u (3 or 4, two or three steps ahead, measured no faster, with one workgroup per CU neither)
 template <int D> struct FwdLds {
     // K / V rows go from global memory straight into LDS (buffer loads with the LDS modifier: the
     // 64 lanes of a load fill 1 KB of consecutive LDS, which rules out padded rows).  A tile of 32
@@ -424,7 +424,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     // needs the last block of them)
     const int u_first = SPLIT ? max(u_lo - 1, 0) : 0;
     fetch_step(u_first);
-    if constexpr (Lds::n_buf == 3) fetch_step(u_first + 1);
+#pragma unroll
+    for (int x = 1; x < Lds::n_buf - 1; ++x) fetch_step(u_first + x);
     if constexpr (SPLIT) {
         const int to_first = (u_first % Lds::n_buf) * Lds::buf_bytes;
         ka += to_first;
@@ -460,10 +461,10 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         for (int u = ua; u < ub; ++u) {
             // this wave's rows of step u have landed (with three buffers those of step u + 1 may be on their way:
             // 2 * N_LD loads per step, and the loop body issues no other vector memory operation before this wait)
-            if constexpr (Lds::n_buf == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * N_LD) : "memory");
+            if constexpr (Lds::n_buf > 2) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((Lds::n_buf - 2) * 2 * N_LD) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();  // step u-1 is done everywhere: its buffer is free, and step u's is written
-            if (!SPLIT || u + Lds::n_buf - 1 < n_steps) fetch_step(u + Lds::n_buf - 1);
+            if (!SPLIT || Lds::n_buf > 2 || u + Lds::n_buf - 1 < n_steps) fetch_step(u + Lds::n_buf - 1);
             if constexpr (KIND == 3) carry_only(u);
             else if constexpr (KIND != 2) step(u, std::integral_constant<bool, KIND == 1>{});
             const int to_other = (u % Lds::n_buf == Lds::n_buf - 1) ? -(Lds::n_buf - 1) * Lds::buf_bytes : Lds::buf_bytes;

@@ -331,10 +331,12 @@ hipError_t bwd_prepare(const Problem &p, int out_dt, const void *o, const void *
 CHAIN_DECL(mfma_bwd_chain_kv);
 CHAIN_DECL(mfma_bwd_chain_qw);
 CHAIN_DECL(mfma_bwd_chain_all);
+CHAIN_DECL(mfma_bwd_chain_split);   // everything, with share > 0
 // the same with three waves per SIMD (bwd_chain3_mfma.hip): windows of up to 6 query taps
 CHAIN_DECL(mfma_bwd_chain3_kv);
 CHAIN_DECL(mfma_bwd_chain3_qw);
 CHAIN_DECL(mfma_bwd_chain3_all);
+CHAIN_DECL(mfma_bwd_chain3_split);
 #undef CHAIN_DECL
 inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const void *q, const void *k, const void *v,
                                  const void *d_o, const float *Dl, const float *lse, const float *w,
@@ -343,10 +345,12 @@ inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const v
     if (p.c_q <= 6) {
         if (want == 1) return mfma_bwd_chain3_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
         if (want == 2) return mfma_bwd_chain3_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+        if (share) return mfma_bwd_chain3_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
         return mfma_bwd_chain3_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     }
     if (want == 1) return mfma_bwd_chain_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     if (want == 2) return mfma_bwd_chain_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    if (share) return mfma_bwd_chain_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     return mfma_bwd_chain_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 // heads_inner: the blocks lie [batch][block][head] (all heads of a block side by side) instead of [batch, head][block]
