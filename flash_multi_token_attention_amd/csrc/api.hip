@@ -685,10 +685,8 @@ int convattn_headmix_bwd_fused(const convattn_headmix_desc *desc, int grad_dtype
     const HeadmixFusedWs ws = headmix_fused_ws(desc);
     unsigned char *base = static_cast<unsigned char *>(workspace);
     float *Dl = reinterpret_cast<float *>(base), *lse = reinterpret_cast<float *>(base + ws.lse_off);
-    rc = (int)bwd_preprocess(p, desc->in_dtype, desc->out_dtype, o, d_o, m, l, Dl, lse, s);
-    if (rc) return rc;
-    return (int)headmix_bwd_fused(p, grad_dtype, q, k, v, w, d_o, lse, Dl, base + ws.p_off, base + ws.ds_off, base + ws.kv_off,
-                                  reinterpret_cast<float *>(base + ws.part_off), dq, dk, dv, dw, s);
+    return (int)headmix_bwd_fused(p, grad_dtype, q, k, v, w, desc->out_dtype, o, d_o, m, l, lse, Dl, base + ws.p_off, base + ws.ds_off,
+                                  base + ws.kv_off, reinterpret_cast<float *>(base + ws.part_off), dq, dk, dv, dw, s);
 }
 
 }  // extern "C"

@@ -103,8 +103,8 @@ hipError_t headmix_fwd_blocks(const Problem &p, int out_dt, const void *q, const
 // one pass for all gradients (headmix_scores.hip); p: B, H, Nq = Nk = N, d, scale, causal.  dk / dv or dq / dw may be null.
 size_t headmix_frag_bytes(const Problem &p);              // kv_frag holds two of these
 int headmix_score_wgs(int B, int H, int N, int causal);   // dw partials
-hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,
-                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, void *kv_frag, float *dw_part,
-                             void *dq, void *dk, void *dv, float *dw, hipStream_t s);
+hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w, int o_dt,
+                             const void *o, const void *d_o, const float *m, const float *l, float *lse, float *Dl, void *P,
+                             void *dS, void *kv_frag, float *dw_part, void *dq, void *dk, void *dv, float *dw, hipStream_t s);
 
 }  // namespace convattn

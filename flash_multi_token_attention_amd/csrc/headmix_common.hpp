@@ -156,11 +156,9 @@ __device__ __forceinline__ void turn_rows(bf16x8 (&f)[T::RB][D / 32], const bf16
 // bound by them (3.3 M of its 4.1 M clocks per CU at B4 H16 N4096 d128).  One copy of K and V (0.04 ms there) is read
 // N / 32 times.  V may be null.
 template <int D>
-__global__ __launch_bounds__(256) void frag_order_kernel(int N, int n_t16, const bf16_t *__restrict__ K,
-                                                         const bf16_t *__restrict__ V, bf16_t *__restrict__ KF,
-                                                         bf16_t *__restrict__ VF, size_t n_frag) {
-    const size_t f = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // one 1 KB fragment per wave
-    if (f >= n_frag) return;
+__device__ __forceinline__ void frag_order(size_t f, int N, int n_t16, const bf16_t *__restrict__ K, const bf16_t *__restrict__ V,
+                                           bf16_t *__restrict__ KF, bf16_t *__restrict__ VF, size_t n_frag) {
+    if (f >= n_frag) return;   // (one 1 KB fragment per wave)
     constexpr int KS = D / 32;
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const size_t bh = f / ((size_t)n_t16 * KS);
@@ -168,13 +166,7 @@ __global__ __launch_bounds__(256) void frag_order_kernel(int N, int n_t16, const
     *reinterpret_cast<u32x4 *>(KF + f * 512 + lane * 8) = load_row16<D>(K + bh * N * D, row, N, col);
     if (V) *reinterpret_cast<u32x4 *>(VF + f * 512 + lane * 8) = load_row16<D>(V + bh * N * D, row, N, col);
 }
-template <int D>
-void launch_frag_order(int BH, int N, const void *k, const void *v, const bf16_t *kf, const bf16_t *vf, hipStream_t s) {
-    const int n_t16 = (N + 31) / 32 * 2;
-    const size_t n_frag = (size_t)BH * n_t16 * (D / 32);
-    frag_order_kernel<D><<<(unsigned)((n_frag + 3) / 4), 256, 0, s>>>(N, n_t16, (const bf16_t *)k, (const bf16_t *)v, const_cast<bf16_t *>(kf),
-                                                                     const_cast<bf16_t *>(vf), n_frag);
-}
+inline size_t frag_count(int BH, int N, int d) { return (size_t)BH * ((N + 31) / 32 * 2) * (d / 32); }
 
 }  // namespace headmix
 }  // namespace convattn

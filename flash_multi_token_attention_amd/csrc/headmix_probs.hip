@@ -398,11 +398,18 @@ Plan prob_plan(const Problem &p) {
     return p.H == 16 ? make_plan<ProbTile<16, 32>>(p.B, p.Nq, p.causal) : make_plan<ProbTile<32, 32>>(p.B, p.Nq, p.causal);
 }
 
+template <int D>
+__global__ __launch_bounds__(256) void frag_order_kernel(int N, int n_t16, const bf16_t *__restrict__ K, bf16_t *__restrict__ KF,
+                                                         size_t n_frag) {
+    frag_order<D>((size_t)blockIdx.x * 4 + (threadIdx.x >> 6), N, n_t16, K, nullptr, KF, nullptr, n_frag);
+}
+
 template <int H, int D, typename TO>
 hipError_t launch(const Problem &p, const ProbArgs &a, const void *k, const void *v, void *o, float *l, float *m, hipStream_t s) {
     using T = ProbTile<H, D>;
     static_assert(T::lds <= 160 * 1024, "LDS budget");
-    launch_frag_order<D>(p.B * H, a.N, k, nullptr, a.KF, nullptr, s);
+    const size_t n_frag = frag_count(p.B * H, a.N, D);
+    frag_order_kernel<D><<<(unsigned)((n_frag + 3) / 4), 256, 0, s>>>(a.N, a.n_rt32 * 2, (const bf16_t *)k, const_cast<bf16_t *>(a.KF), n_frag);
     hipError_t e = set_max_lds_once<headmix_probs_kernel<H, D>>(T::lds);
     if (e != hipSuccess) return e;
     headmix_probs_kernel<H, D><<<plan_grid(a.plan), T::WAVES * 64, T::lds, s>>>(a);

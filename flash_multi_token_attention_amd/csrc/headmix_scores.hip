@@ -11,7 +11,9 @@
 // blocks of 32 rows x 32 keys (the operand precision of the products that follow); dQ = dS K is
 // the product kernel of the window backward (bwd_dq_rows.hip, same block layout) and
 // headmix_dkdv_kernel takes dV = P^T dO and dK = dS^T Q from one walk over the blocks of 128 keys.
+#include "dq_rows.hpp"
 #include "headmix_common.hpp"
+#include "row_stats.hpp"
 
 namespace convattn {
 namespace {
@@ -302,10 +304,9 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
 
 // dw[h][h'] = sum of the partials in a fixed order: a workgroup takes 16 entries, 16 threads per entry each
 // add every 16th partial, the sixteen sums are added in order.
-__global__ __launch_bounds__(256) void headmix_dw_sum_kernel(int n_part, int hh, const float *__restrict__ part,
-                                                             float *__restrict__ dW) {
-    __shared__ float red[16][17];
-    const int e = threadIdx.x & 15, c = threadIdx.x >> 4, idx = blockIdx.x * 16 + e;
+__device__ __forceinline__ void dw_sum(int n_part, int hh, const float *__restrict__ part, float *__restrict__ dW, int block,
+                                       float (*red)[17]) {
+    const int e = threadIdx.x & 15, c = threadIdx.x >> 4, idx = block * 16 + e;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
     int q = c;
     for (; q + 48 < n_part; q += 64) {
@@ -321,8 +322,13 @@ __global__ __launch_bounds__(256) void headmix_dw_sum_kernel(int n_part, int hh,
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) s += red[i][threadIdx.x];
-        dW[blockIdx.x * 16 + threadIdx.x] = s;
+        dW[block * 16 + threadIdx.x] = s;
     }
+}
+__global__ __launch_bounds__(256) void headmix_dw_sum_kernel(int n_part, int hh, const float *__restrict__ part,
+                                                             float *__restrict__ dW) {
+    __shared__ float red[16][17];
+    dw_sum(n_part, hh, part, dW, blockIdx.x, red);
 }
 
 // ------------------------------------------------------------------ dV = P^T dO, dK = dS^T Q
@@ -340,25 +346,21 @@ template <int D> struct KvLds {
 };
 
 template <int D, typename TO>
-__global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, int H, int N, int causal, int n_rt, int n_kt,
-                                                                     const bf16_t *__restrict__ Q,
-                                                                     const bf16_t *__restrict__ dO,
-                                                                     const bf16_t *__restrict__ Pws,
-                                                                     const bf16_t *__restrict__ dSws,
-                                                                     TO *__restrict__ dK, TO *__restrict__ dV) {
+__device__ __forceinline__ void dkdv_tile(int B, int H, int N, int causal, int n_rt, int n_kt, const bf16_t *__restrict__ Q,
+                                          const bf16_t *__restrict__ dO, const bf16_t *__restrict__ Pws,
+                                          const bf16_t *__restrict__ dSws, TO *__restrict__ dK, TO *__restrict__ dV, int h, int b,
+                                          int z, unsigned char *smem) {
     using Lds = KvLds<D>;
     constexpr int DB = D / 16, CPR = D / 8, LD = 32 * CPR / (KV_WAVES * 64) > 0 ? 32 * CPR / (KV_WAVES * 64) : 1;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int kt = blockIdx.z * KV_WAVES + wave;          // this wave's block column
+    const int kt = z * KV_WAVES + wave;          // this wave's block column
     const size_t bh = (size_t)b * H + h;
     const bf16_t *Qb = Q + bh * N * D, *Ob = dO + bh * N * D;
     const size_t wso = (size_t)b * chain_ds_block_off(causal != 0, n_rt, n_kt) * H + h;   // blocks lie [batch][block][head]
     const int kt_c = min(kt, n_rt - 1);                   // (N keys and N rows: n_rt columns exist)
     const bool own = kt < n_rt;
     const size_t col = wso + (chain_ds_block_off(causal != 0, n_rt, kt_c) - chain_ds_first_rt(causal != 0, kt_c)) * H;
-    const int rt0 = causal ? blockIdx.z * KV_WAVES : 0;
+    const int rt0 = causal ? z * KV_WAVES : 0;
 
     f32x4 acc_v[2][DB], acc_k[2][DB];
 #pragma unroll
@@ -448,13 +450,71 @@ __global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, i
     }
 }
 
+template <int D, typename TO>
+__global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_dkdv_kernel(int B, int H, int N, int causal, int n_rt, int n_kt,
+                                                                     const bf16_t *__restrict__ Q,
+                                                                     const bf16_t *__restrict__ dO,
+                                                                     const bf16_t *__restrict__ Pws,
+                                                                     const bf16_t *__restrict__ dSws,
+                                                                     TO *__restrict__ dK, TO *__restrict__ dV) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    dkdv_tile<D, TO>(B, H, N, causal, n_rt, n_kt, Q, dO, Pws, dSws, dK, dV, blockIdx.x, blockIdx.y, blockIdx.z, smem);
+}
+
+// What follows the score kernel, in one launch: workgroups for dK and dV, then for dQ, then for dw.  Problems whose dQ tiles
+// share keys among the waves (small ones) are bound by launches: three of 3 us of host time and 2 us of GPU time become one.
+template <int D, typename TO>
+__global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_products_kernel(Problem p, int n_rt, int n_kt, const bf16_t *__restrict__ Q,
+                                                                            const bf16_t *__restrict__ K, const bf16_t *__restrict__ dO,
+                                                                            const bf16_t *__restrict__ Pws, const bf16_t *__restrict__ dSws,
+                                                                            int n_part, const float *__restrict__ dw_part,
+                                                                            TO *__restrict__ dQ, TO *__restrict__ dK,
+                                                                            TO *__restrict__ dV, float *__restrict__ dW) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int BH = p.B * p.H, kv = BH * ((p.Nk + 127) / 128), i = blockIdx.x;
+    if (i < kv) {
+        const int bh = i % BH;
+        dkdv_tile<D, TO>(p.B, p.H, p.Nk, p.causal, n_rt, n_kt, Q, dO, Pws, dSws, dK, dV, bh % p.H, bh / p.H, i / BH, smem);
+    } else if (i < kv + BH * n_rt) {
+        const int j = i - kv, bh = j % BH;
+        dq_rows::tile<D, TO, true>(p, K, dSws, nullptr, n_kt, n_rt, 1, dQ, bh % p.H, bh / p.H, n_rt - 1 - j / BH, smem);
+    } else {
+        dw_sum(n_part, p.H * p.H, dw_part, dW, i - kv - BH * n_rt, reinterpret_cast<float (*)[17]>(smem));
+    }
+}
+
 Plan score_plan(int B, int H, int N, int causal) {
     return H == 16 ? make_plan<ScoreTile<16, 32>>(B, N, causal) : make_plan<ScoreTile<32, 32>>(B, N, causal);
 }
 
+// What precedes the score kernel, in one launch: K and V in fragment order, then D and LSE of the rows.
+template <int D, typename TO>
+__global__ __launch_bounds__(256) void headmix_prepare_kernel(int N, int n_t16, size_t n_frag, size_t rows, const bf16_t *__restrict__ K,
+                                                              const bf16_t *__restrict__ V, const TO *__restrict__ O,
+                                                              const bf16_t *__restrict__ dO, const float *__restrict__ M,
+                                                              const float *__restrict__ L, bf16_t *__restrict__ KF,
+                                                              bf16_t *__restrict__ VF, float *__restrict__ Dl, float *__restrict__ LSE) {
+    const size_t first = (n_frag + 3) / 4;
+    if (blockIdx.x < first) frag_order<D>((size_t)blockIdx.x * 4 + (threadIdx.x >> 6), N, n_t16, K, V, KF, VF, n_frag);
+    else row_stats(blockIdx.x - first, rows, D, O, dO, M, L, Dl, LSE);
+}
+template <int D>
+hipError_t launch_prepare(const Problem &p, int o_dt, const void *k, const void *v, const void *o, const void *d_o, const float *m,
+                          const float *l, void *kf, void *vf, float *Dl, float *lse, hipStream_t s) {
+    const size_t n_frag = frag_count(p.B * p.H, p.Nk, D), rows = (size_t)p.B * p.H * p.Nq;
+    const unsigned grid = (unsigned)((n_frag + 3) / 4 + (rows + 15) / 16);
+    const int n_t16 = chain_row_tiles(p) * 2;
+#define CALL(TO)                                                                                                              \
+    headmix_prepare_kernel<D, TO><<<grid, 256, 0, s>>>(p.Nk, n_t16, n_frag, rows, (const bf16_t *)k, (const bf16_t *)v, (const TO *)o, \
+                                                       (const bf16_t *)d_o, m, l, (bf16_t *)kf, (bf16_t *)vf, Dl, lse)
+    if (o_dt == CONVATTN_BF16) CALL(bf16_t);
+    else CALL(float);
+#undef CALL
+    return hipGetLastError();
+}
+
 template <int H, int D>
-hipError_t launch_scores(const ScoreArgs &a, const void *k, const void *v, hipStream_t s) {
-    launch_frag_order<D>(a.B * H, a.N, k, v, a.KF, a.VF, s);
+hipError_t launch_scores(const ScoreArgs &a, hipStream_t s) {
     constexpr int lds = ScoreTile<H, D>::lds;
     static_assert(ScoreTile<H, D>::WAVES * ScoreTile<H, D>::ROOM <= ScoreTile<H, D>::w_off * 4, "w stays where the rows are turned");
     static_assert(lds <= 160 * 1024 && ScoreTile<H, D>::WAVES * H * H * 4 <= lds, "LDS budget");
@@ -475,6 +535,17 @@ hipError_t launch_dkdv(const Problem &p, const void *q, const void *d_o, const b
     return hipGetLastError();
 }
 
+template <int D, typename TO>
+hipError_t launch_products(const Problem &p, const ScoreArgs &a, const void *k, void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
+    constexpr int lds = KvLds<D>::total > dq_rows::lds_by_keys<D> ? KvLds<D>::total : dq_rows::lds_by_keys<D>;
+    hipError_t e = set_max_lds_once<headmix_products_kernel<D, TO>>(lds);
+    if (e != hipSuccess) return e;
+    const int n_rt = chain_row_tiles(p), grid = p.B * p.H * ((p.Nk + 127) / 128 + n_rt) + p.H * p.H / 16;
+    headmix_products_kernel<D, TO><<<grid, KV_WAVES * 64, lds, s>>>(p, n_rt, chain_key_tiles(p), a.Q, (const bf16_t *)k, a.dO, a.P, a.dS,
+                                                                   a.plan.n_wg, a.dw_part, (TO *)dq, (TO *)dk, (TO *)dv, dw);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 // K (or V) in fragment order
@@ -482,17 +553,28 @@ size_t headmix_frag_bytes(const Problem &p) { return (size_t)p.B * p.H * chain_r
 int headmix_score_wgs(int B, int H, int N, int causal) { return score_plan(B, H, N, causal).n_wg; }
 
 hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const void *k, const void *v, const float *w,
-                             const void *d_o, const float *lse, const float *Dl, void *P, void *dS, void *kv_frag, float *dw_part,
-                             void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
+                             int o_dt, const void *o, const void *d_o, const float *m, const float *l, float *lse, float *Dl, void *P,
+                             void *dS, void *kv_frag, float *dw_part, void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
     const Plan plan = score_plan(p.B, p.H, p.Nq, p.causal);
     const bool want_kv = dk != nullptr;
     const ScoreArgs a{p.B, p.Nq, p.causal, chain_row_tiles(p), chain_key_tiles(p), plan, p.scale,
                       (const bf16_t *)q, (const bf16_t *)kv_frag, (const bf16_t *)kv_frag + headmix_frag_bytes(p) / 2, (const bf16_t *)d_o, w, lse, Dl,
                       (bf16_t *)P, (bf16_t *)dS, dq ? dw_part : nullptr};
-    hipError_t e = hipErrorInvalidValue;
-    if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, k, v, s) : p.d == 64 ? launch_scores<16, 64>(a, k, v, s) : launch_scores<16, 128>(a, k, v, s);
-    if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, k, v, s) : p.d == 64 ? launch_scores<32, 64>(a, k, v, s) : launch_scores<32, 128>(a, k, v, s);
+    void *kf = kv_frag, *vf = static_cast<unsigned char *>(kv_frag) + headmix_frag_bytes(p);
+    hipError_t e = p.d == 32   ? launch_prepare<32>(p, o_dt, k, v, o, d_o, m, l, kf, vf, Dl, lse, s)
+                   : p.d == 64 ? launch_prepare<64>(p, o_dt, k, v, o, d_o, m, l, kf, vf, Dl, lse, s)
+                               : launch_prepare<128>(p, o_dt, k, v, o, d_o, m, l, kf, vf, Dl, lse, s);
     if (e != hipSuccess) return e;
+    e = hipErrorInvalidValue;
+    if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, s) : p.d == 64 ? launch_scores<16, 64>(a, s) : launch_scores<16, 128>(a, s);
+    if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, s) : p.d == 64 ? launch_scores<32, 64>(a, s) : launch_scores<32, 128>(a, s);
+    if (e != hipSuccess) return e;
+    if (want_kv && dq && dq_rows::by_keys(p)) {
+#define CALL(DD) (grad_dt == CONVATTN_BF16 ? launch_products<DD, bf16_t>(p, a, k, dq, dk, dv, dw, s) \
+                                           : launch_products<DD, float>(p, a, k, dq, dk, dv, dw, s))
+        return p.d == 32 ? CALL(32) : p.d == 64 ? CALL(64) : CALL(128);
+#undef CALL
+    }
     if (want_kv) {
 #define CALL(DD) (grad_dt == CONVATTN_BF16 ? launch_dkdv<DD, bf16_t>(p, q, d_o, a.P, a.dS, dk, dv, s) \
                                            : launch_dkdv<DD, float>(p, q, d_o, a.P, a.dS, dk, dv, s))
