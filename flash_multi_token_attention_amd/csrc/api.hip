@@ -309,9 +309,7 @@ static hipError_t run_split(const Problem &p, int out_dt, const SplitWs &lay, co
     float *part = reinterpret_cast<float *>(ws + lay.part_off), *scale = reinterpret_cast<float *>(ws + lay.scale_off);
     float *kv = reinterpret_cast<float *>(ws + lay.kv_off);
     hipError_t e = mfma_bwd_chain(p, out_dt, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s, lay.share, kv);
-    if (e == hipSuccess) e = chain_reduce(p, out_dt, lay.share, kv, dk, dv, s);
-    if (e == hipSuccess) e = mfma_dq_from_rows(p, out_dt, k, ws, scale, dq, s);
-    if (e == hipSuccess) e = dw_reduce(p, lay.n_wg, part, dw, s);
+    if (e == hipSuccess) e = mfma_bwd_products(p, out_dt, k, ws, scale, lay.n_wg, part, lay.share, kv, dq, dk, dv, dw, s);
     return e;
 }
 
@@ -357,8 +355,7 @@ int convattn_bwd_all(const convattn_desc *desc, const void *q, const void *k, co
     if (split) return (int)run_split(p, desc->out_dtype, cut, q, k, v, d_o, D, lse, w, dq, dk, dv, dw, workspace, s);
     float *part = reinterpret_cast<float *>(ws + lay.part_off);
     e = mfma_bwd_chain(p, desc->out_dtype, 3, q, k, v, d_o, D, lse, w, scale, dk, dv, ws, part, s);
-    if (e == hipSuccess) e = mfma_dq_from_rows(p, desc->out_dtype, k, ws, scale, dq, s);
-    if (e == hipSuccess) e = dw_reduce(p, mfma_kv_tiles(p), part, dw, s);
+    if (e == hipSuccess) e = mfma_bwd_products(p, desc->out_dtype, k, ws, scale, mfma_kv_tiles(p), part, 0, nullptr, dq, dk, dv, dw, s);
     return (int)e;
 }
 

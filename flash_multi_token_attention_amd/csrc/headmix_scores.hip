@@ -13,7 +13,7 @@
 // headmix_dkdv_kernel takes dV = P^T dO and dK = dS^T Q from one walk over the blocks of 128 keys.
 #include "dq_rows.hpp"
 #include "headmix_common.hpp"
-#include "row_stats.hpp"
+#include "reduce_common.hpp"
 
 namespace convattn {
 namespace {

@@ -297,6 +297,12 @@ inline int chain_wgs(const Problem &p, int share) {
 inline size_t chain_part_bytes(const Problem &p, int share) {
     return share > 0 ? (size_t)p.B * p.H * chain_wgs(p, share) * 2 * kKvKeysPerWg * p.d * sizeof(float) : 0;
 }
+// key blocks with several parts (they are the first ones: the parts do not grow from block to block)
+inline int chain_split_blocks(const Problem &p, int share) {
+    int n = 0;
+    while (n < mfma_kv_tiles(p) && chain_parts(p, n, share) > 1) ++n;
+    return n;
+}
 int chain_share(const Problem &p);
 hipError_t chain_reduce(const Problem &p, int out_dt, int share, const float *part, void *dk, void *dv, hipStream_t s);
 inline int chain_key_tiles(const Problem &p) { return mfma_kv_tiles(p) * (kKvKeysPerWg / kChainKeys); }
@@ -353,6 +359,11 @@ inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const v
     if (share) return mfma_bwd_chain_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
     return mfma_bwd_chain_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
+// What follows the key-stationary kernel: dQ, the sum of the n_wg dW partials per (batch, head) and, with share > 0, dK and dV from
+// their parts.  One launch where dQ's waves share keys (small problems), else one each.
+hipError_t mfma_bwd_products(const Problem &p, int out_dt, const void *k, const void *ds_ws, const float *dc_scale, int n_wg,
+                             const float *dw_part, int share, const float *kv_part, void *dq, void *dk, void *dv, float *dw,
+                             hipStream_t s);
 // heads_inner: the blocks lie [batch][block][head] (all heads of a block side by side) instead of [batch, head][block]
 hipError_t mfma_dq_from_rows(const Problem &p, int out_dt, const void *k, const void *ds_ws,
                              const float *dc_scale, void *dq, hipStream_t s, bool heads_inner = false);

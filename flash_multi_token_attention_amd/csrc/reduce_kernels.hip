@@ -1,7 +1,7 @@
 // Small bandwidth-bound helpers around the conv-attention kernels:
 // backward preparation (D, LSE), the ordered dW reduction and the decode
 // split merge.
-#include "row_stats.hpp"
+#include "reduce_common.hpp"
 
 namespace convattn {
 namespace {
@@ -76,64 +76,17 @@ __global__ void bwd_prepare_kernel(int Nq, int Nk, const TO *__restrict__ O, con
     if (tid == 0) write_dc_scale(D, red[0][0], red[1][0], scale + 2 * bh);
 }
 
-// dW[h][tap] = sum over (batch, tile) of the partials, in a fixed order: a workgroup takes 64 taps
-// of one head (lane = tap, so a partial is read with contiguous loads); wave w adds the partials
-// w, w+4, ... in four independent chains, and the four waves' sums are added in wave order.
 __global__ __launch_bounds__(1024) void dw_reduce_kernel(int B, int H, int n_tiles, int ntap,
                                                          const float *__restrict__ part, float *__restrict__ dW) {
-    constexpr int NW = 16;
-    __shared__ float red[NW][64];
-    const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int tap = blockIdx.y * 64 + lane;
-    const int n = B * n_tiles;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    if (tap < ntap) {
-        auto at = [&](int q) {
-            const int b = q / n_tiles, t = q - b * n_tiles;
-            return part[(((size_t)b * H + h) * n_tiles + t) * ntap + tap];
-        };
-        int q = wave;
-        for (; q + 3 * NW < n; q += 4 * NW) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] += at(q + NW * c);
-        }
-        for (int c = 0; q < n; q += NW, ++c) s[c] += at(q);
-    }
-    red[wave][lane] = (s[0] + s[1]) + (s[2] + s[3]);
-    __syncthreads();
-    if (wave == 0 && tap < ntap) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) v += red[w][lane];
-        dW[(size_t)h * ntap + tap] = v;
-    }
+    __shared__ float red[kDwChains][64];
+    dw_reduce_block<1024>(B, H, n_tiles, ntap, part, dW, blockIdx.x, blockIdx.y, red);
 }
 
-// dK and dV of the key blocks whose row tiles several workgroups share: the partials added in the order of the rows.
-// x = 16-byte groups of a key block's dK, then dV, y = key block, z = (batch, head).
+// x = 16-byte groups of a key block's dK, then dV, y = key block, z = (batch, head)
 template <typename TO>
 __global__ __launch_bounds__(256) void chain_reduce_kernel(Problem p, int share, int n_wg, const float *__restrict__ part,
                                                            TO *__restrict__ dK, TO *__restrict__ dV) {
-    const int kb = blockIdx.y, parts = chain_parts(p, kb, share);
-    if (parts == 1) return;
-    int z = 0;
-    for (int i = 0; i < kb; ++i) z += chain_parts(p, i, share);
-    const int e = (blockIdx.x * 256 + threadIdx.x) * 4, per = kKvKeysPerWg * p.d;   // (2 per is a multiple of 1024)
-    const int is_v = e >= per, local = e - is_v * per, key = kb * kKvKeysPerWg + local / p.d - (is_v ? 8 : 0);
-    if (key < 0 || key >= p.Nk) return;
-    const float *src = part + ((size_t)blockIdx.z * n_wg + z) * 2 * per + e;
-    float4 sum = *reinterpret_cast<const float4 *>(src);
-    for (int i = 1; i < parts; ++i) {
-        const float4 v = *reinterpret_cast<const float4 *>(src + (size_t)i * 2 * per);
-        sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
-    }
-    TO *dst = (is_v ? dV : dK) + ((size_t)blockIdx.z * p.Nk + key) * p.d + local % p.d;
-    if constexpr (sizeof(TO) == 2) {
-        bf16x4 o = {(bf16_t)sum.x, (bf16_t)sum.y, (bf16_t)sum.z, (bf16_t)sum.w};
-        *reinterpret_cast<bf16x4 *>(dst) = o;
-    } else {
-        *reinterpret_cast<float4 *>(dst) = sum;
-    }
+    chain_reduce_block(p, share, n_wg, part, dK, dV, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Merge of a few decode splits: one workgroup per (batch, head), one thread per output column walks the splits.
@@ -284,9 +237,7 @@ int chain_share(const Problem &p) {
 }
 
 hipError_t chain_reduce(const Problem &p, int out_dt, int share, const float *part, void *dk, void *dv, hipStream_t s) {
-    int split = 0;   // (the parts of a key block do not grow from block to block)
-    while (split < mfma_kv_tiles(p) && chain_parts(p, split, share) > 1) ++split;
-    const dim3 grid(2 * kKvKeysPerWg * p.d / 1024, split, p.B * p.H);
+    const dim3 grid(2 * kKvKeysPerWg * p.d / 1024, chain_split_blocks(p, share), p.B * p.H);
     const int n_wg = chain_wgs(p, share);
     if (out_dt == CONVATTN_BF16)
         chain_reduce_kernel<bf16_t><<<grid, 256, 0, s>>>(p, share, n_wg, part, (bf16_t *)dk, (bf16_t *)dv);
