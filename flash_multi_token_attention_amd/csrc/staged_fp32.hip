@@ -243,21 +243,25 @@ __device__ __forceinline__ void tile_dw_any(float *__restrict__ part, float *red
     }
 }
 
-// LDS of window_kernel: rows of Q and K (then of dO and V, then dP / dC), the score tile with its halo
+// LDS of window_kernel: rows of Q and K, then in their place dP / dC (backward), the sums of dW and the score tile with its halo.
+// (The score tile beside the rows, and rows of dO and V staged as well, took 60 KB at d = 64: two workgroups per CU, and one at
+// d = 128.  Now 39: B1 H8 N1024 d64 6x11 backward 73 -> 58 us, forward 42 -> 36.)
 struct WinLds {
-    int dst, sst, q_f, k_f, w_f, s_f, total_f;   // floats
+    int dst, sst, k_f, dp_f, w_f, s_f, total_f;   // floats
 };
-__host__ __device__ inline WinLds win_lds(const Problem &p) {
+__host__ __device__ inline WinLds win_lds(const Problem &p, bool bwd) {
     WinLds l;
     l.dst = ((p.d + 15) & ~15) + 4;
     // a patch reads whole 16-byte quantities: columns 60 .. 60 + c_k + 3 rounded up
     l.sst = TT - 4 + ((p.c_k + 3 + 3) & ~3);
-    l.q_f = (TT + p.pq) * l.dst;
-    l.k_f = (TT + 2 * p.pk) * l.dst;
-    const int op = l.q_f + l.k_f, need = TT * (TT + 4) + (p.c_k <= 15 ? 8 * p.c_q * p.c_k : 0);   // dP, sums of dW
-    l.w_f = op > need ? op : need;                // window
-    l.s_f = l.w_f + p.c_q * win_stride(p.c_k);    // score tile
-    l.total_f = l.s_f + (TT + p.pq) * l.sst;
+    l.w_f = 0;                                            // window
+    const int rows = p.c_q * win_stride(p.c_k);           // first float of the rows of Q
+    l.k_f = rows + (TT + p.pq) * l.dst;
+    l.s_f = rows;                                         // score tile
+    l.dp_f = l.s_f + (TT + p.pq) * l.sst;
+    const int one = l.k_f + (TT + 2 * p.pk) * l.dst;
+    const int two = l.dp_f + (bwd ? TT * (TT + 4) + (p.c_k <= 15 ? 8 * p.c_q * p.c_k : 0) : 0);
+    l.total_f = one > two ? one : two;
     return l;
 }
 
@@ -275,57 +279,83 @@ __global__ __launch_bounds__(NT, 2) void window_kernel(StArgs a, const TI *__res
     long long tile;
     find_tile(p, a.n_rt, a.n_ct, bh, rt, ct, tile);
     const int h = (int)(bh % p.H), r0 = rt * TT, c0 = ct * TT, d = p.d, pq = p.pq, pk = p.pk, Kd = round16(d);
-    const WinLds L = win_lds(p);
-    float *Qs = lds, *Ks = lds + L.q_f, *Ss = lds + L.s_f, *Ws = lds + L.w_f;
+    const WinLds L = win_lds(p, BWD);
+    float *Qs = lds + L.s_f, *Ks = lds + L.k_f, *Ss = lds + L.s_f, *Ws = lds + L.w_f, *dPs = lds + L.dp_f;   // dP: [64][68]
+    constexpr int PST = TT + 4;
     const int nr = TT + pq, nc = TT + 2 * pk;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
 
     stage_window<false>(Ws, W + (size_t)h * p.c_q * p.c_k, p.c_q, p.c_k);
     stage_rows(Qs, L.dst, Q + bh * p.Nq * d, r0 - pq, nr, p.Nq, d);
     stage_rows(Ks, L.dst, K + bh * p.Nk * d, c0 - pk, nc, p.Nk, d);
-    // (columns past the halo that a patch's last 16 bytes touch: multiplied by nothing, but not to be NaN patterns either)
-    for (int r = tid; r < nr; r += NT)
-        for (int c = nc; c < L.sst; ++c) Ss[r * L.sst + c] = 0.f;
     __syncthreads();
-    {
-        const int nrb = (nr + 15) / 16, ncb = (nc + 15) / 16, ncp = (ncb + 1) / 2;
-        for (int it = wave; it < nrb * ncp; it += NT / 64) {
+    // score blocks of 16 rows x 32 keys, held until the rows have been read by everyone
+    constexpr int HELD = 4;   // (at most 5 x 3 blocks for four waves)
+    const int nrb = (nr + 15) / 16, ncb = (nc + 15) / 16, ncp = (ncb + 1) / 2;
+    f32x4 sc[HELD][2];
+#pragma unroll
+    for (int x = 0; x < HELD; ++x) {
+        const int it = wave + x * (NT / 64);
+        if (it < nrb * ncp) {
             const int rb = it / ncp, cb = (it - rb * ncp) * 2;
-            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            sc[x][0] = sc[x][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
             const float *bp[2] = {Ks + min(cb * 16 + n, nc - 1) * L.dst + 4 * g, Ks + min(cb * 16 + 16 + n, nc - 1) * L.dst + 4 * g};
-            mma_nt<2>(acc, Qs + min(rb * 16 + n, nr - 1) * L.dst + 4 * g, bp, Kd);
+            mma_nt<2>(sc[x], Qs + min(rb * 16 + n, nr - 1) * L.dst + 4 * g, bp, Kd);
+        }
+    }
+    f32x4 dp_acc[4];
+    if constexpr (BWD) {
+        // dP = dO V^T, the operands as they lie in memory (sixteen consecutive k of sixteen rows per load)
+        const TI *gp = dO + (bh * p.Nq + min(r0 + wave * 16 + n, p.Nq - 1)) * d, *vp[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            dp_acc[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            vp[u] = V + (bh * p.Nk + min(c0 + u * 16 + n, p.Nk - 1)) * d;   // (pairs past the last row or key are dropped below)
+        }
+        f32x4 av, bv[4];
+        auto fetch = [&](int k) {
+            const bool in = k + 4 * g < d;
+            const int at = in ? k + 4 * g : 0;
+            av = load4(gp + at);
+            if (!in) av = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) bv[u] = load4(vp[u] + at);
+        };
+        fetch(0);
+        for (int k = 0; k < Kd; k += 16) {
+            const f32x4 a0 = av, b0[4] = {bv[0], bv[1], bv[2], bv[3]};
+            fetch(min(k + 16, Kd - 16));
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) dp_acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[s], b0[u][s], dp_acc[u], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < HELD; ++x) {
+        const int it = wave + x * (NT / 64);
+        if (it < nrb * ncp) {
+            const int rb = it / ncp, cb = (it - rb * ncp) * 2;
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int i = rb * 16 + 4 * g + r, j = (cb + u) * 16 + n;
-                    if (i < nr && j < nc) Ss[i * L.sst + j] = p.causal && c0 - pk + j > r0 - pq + i ? 0.f : acc[u][r] * p.scale;
+                    if (i < nr && j < nc) Ss[i * L.sst + j] = p.causal && c0 - pk + j > r0 - pq + i ? 0.f : sc[x][u][r] * p.scale;
                 }
         }
     }
-    __syncthreads();
-    float *dPs = lds;                       // [64][68]
-    constexpr int PST = TT + 4;
+    // (columns past the halo that a patch's last 16 bytes touch: multiplied by nothing, but not to be NaN patterns either)
+    for (int r = tid; r < nr; r += NT)
+        for (int c = nc; c < L.sst; ++c) Ss[r * L.sst + c] = 0.f;
     if constexpr (BWD) {
-        float *Gs = lds, *Vs = lds + TT * L.dst;
-        stage_rows(Gs, L.dst, dO + bh * p.Nq * d, r0, TT, p.Nq, d);
-        stage_rows(Vs, L.dst, V + bh * p.Nk * d, c0, TT, p.Nk, d);
-        __syncthreads();
-        f32x4 acc[4];
-        const float *bp[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            acc[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
-            bp[u] = Vs + (u * 16 + n) * L.dst + 4 * g;
-        }
-        mma_nt<4>(acc, Gs + (wave * 16 + n) * L.dst + 4 * g, bp, Kd);
-        __syncthreads();
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) dPs[(wave * 16 + 4 * g + r) * PST + u * 16 + n] = acc[u][r];
-        __syncthreads();
+            for (int r = 0; r < 4; ++r) dPs[(wave * 16 + 4 * g + r) * PST + u * 16 + n] = dp_acc[u][r];
     }
+    __syncthreads();
     // ---- window: a thread has rows 4 ty .., keys 4 tx .. ----
     const int tx = tid & 15, ty = tid >> 4, key0 = c0 + 4 * tx;
     float c[4][4];
@@ -380,7 +410,7 @@ __global__ __launch_bounds__(NT) void unwindow_kernel(StArgs a, const float *__r
     int rt, ct;
     long long tile;
     find_tile(p, a.n_rt, a.n_ct, bh, rt, ct, tile);
-    const int h = (int)(bh % p.H), r0 = rt * TT, c0 = ct * TT, sst = win_lds(p).sst, nr = TT + p.pq, tid = threadIdx.x;
+    const int h = (int)(bh % p.H), r0 = rt * TT, c0 = ct * TT, sst = win_lds(p, true).sst, nr = TT + p.pq, tid = threadIdx.x;
     float *Ws = lds + nr * sst;
     stage_window<true>(Ws, W + (size_t)h * p.c_q * p.c_k, p.c_q, p.c_k);
     {
@@ -592,7 +622,7 @@ hipError_t launch_window(const StArgs &a, const void *q, const void *k, const vo
                          const float *w, float *part, hipStream_t s) {
     hipError_t e = set_max_lds_once<window_kernel<BWD, TI>>((int)kLdsBytes);
     if (e != hipSuccess) return e;
-    window_kernel<BWD, TI><<<dim3((unsigned)((size_t)a.p.B * a.p.H * dw_tiles(a))), NT, win_lds(a.p).total_f * sizeof(float), s>>>(
+    window_kernel<BWD, TI><<<dim3((unsigned)((size_t)a.p.B * a.p.H * dw_tiles(a))), NT, win_lds(a.p, BWD).total_f * sizeof(float), s>>>(
         a, (const TI *)q, (const TI *)k, (const TI *)v, (const TI *)d_o, D, lse, w, part);
     return hipGetLastError();
 }
@@ -602,7 +632,7 @@ hipError_t launch_window(const StArgs &a, const void *q, const void *k, const vo
 // Windows and sizes the staged kernels take: everything validate() lets through that fits their LDS and grids.
 bool staged_ok(const Problem &p) {
     const StArgs a = make_args(p);
-    return (size_t)win_lds(p).total_f * sizeof(float) <= kLdsBytes && 2 * a.n_rt <= 65535 && 2 * a.n_ct <= 65535 &&
+    return (size_t)win_lds(p, true).total_f * sizeof(float) <= kLdsBytes && 2 * a.n_rt <= 65535 && 2 * a.n_ct <= 65535 &&
            (double)p.B * p.H * (double)dw_tiles(a) < 2147483647.0 && (!p.causal || p.Nq == p.Nk);
 }
 size_t staged_fwd_bytes(const Problem &p) {
@@ -652,7 +682,7 @@ static hipError_t run_bwd(StArgs a, const void *q, const void *k, const void *v,
     e = set_max_lds_once<unwindow_kernel>((int)kLdsBytes);
     if (e != hipSuccess) return e;
     const unsigned BH = (unsigned)(a.p.B * a.p.H);
-    unwindow_kernel<<<dim3((unsigned)(BH * dw_tiles(a))), NT, ((TT + a.p.pq) * win_lds(a.p).sst + a.p.c_q * win_stride(a.p.c_k)) * sizeof(float), s>>>(a, w);
+    unwindow_kernel<<<dim3((unsigned)(BH * dw_tiles(a))), NT, ((TT + a.p.pq) * win_lds(a.p, true).sst + a.p.c_q * win_stride(a.p.c_k)) * sizeof(float), s>>>(a, w);
     const dim3 grid(BH, ((a.p.Nq > a.p.Nk ? a.p.Nq : a.p.Nk) + PM - 1) / PM, (dq ? 1 : 0) + (dk ? 2 : 0));
     if (a.p.d <= 64) bwd_product_kernel<4, TI, TO><<<grid, PNT, 0, s>>>(a, (const TI *)q, (const TI *)k, (const TI *)d_o, (TO *)dq, (TO *)dk, (TO *)dv);
     else bwd_product_kernel<8, TI, TO><<<grid, PNT, 0, s>>>(a, (const TI *)q, (const TI *)k, (const TI *)d_o, (TO *)dq, (TO *)dk, (TO *)dv);
