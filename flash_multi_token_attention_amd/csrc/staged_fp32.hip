@@ -403,7 +403,7 @@ __global__ __launch_bounds__(NT, 2) void window_kernel(StArgs a, const TI *__res
 
 // dS[r][c] = sum_ab W[a][b] dC[r - a + pq][c - b + pk]: the window turned by 180 degrees over the rows from r on and the keys from
 // c - pk on
-__global__ __launch_bounds__(NT) void unwindow_kernel(StArgs a, const float *__restrict__ W) {
+__global__ __launch_bounds__(NT, 5) void unwindow_kernel(StArgs a, const float *__restrict__ W) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const Problem &p = a.p;
     size_t bh;
