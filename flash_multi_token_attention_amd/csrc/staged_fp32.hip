@@ -402,7 +402,9 @@ __global__ __launch_bounds__(NT, 2) void window_kernel(StArgs a, const TI *__res
 }
 
 // dS[r][c] = sum_ab W[a][b] dC[r - a + pq][c - b + pk]: the window turned by 180 degrees over the rows from r on and the keys from
-// c - pk on
+// c - pk on.  A workgroup waits for its tile's rows first and multiplies afterwards, so what covers the wait is the others on the
+// CU: held to five (96 registers, 19 of them spilled around the taps), B1 H8 N1024 d64's 1088 workgroups are all resident at once
+// (23 -> 19 us at four; B1 H2 N2002 d128 21 -> 17).
 __global__ __launch_bounds__(NT, 5) void unwindow_kernel(StArgs a, const float *__restrict__ W) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const Problem &p = a.p;
