@@ -1,4 +1,4 @@
-// Whole backward of conv-attention on bf16 MFMA (gfx950), windows of up to 6 query taps: the
+// Whole backward of conv-attention on bf16 MFMA (gfx950), windows of up to 6 query taps, at head dimensions 32 and 64 of up to 11: the
 // key-stationary kernel of bwd_chain_mfma.hip with three waves per SIMD instead of two.
 //
 // A workgroup of 12 waves owns 128 keys of one (batch, head) and walks down the query rows in tiles
@@ -67,7 +67,6 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
     const int n_rt = args.n_rt;
     using Lds = Chain3Lds<D, CQT>;
     constexpr int KS = D / 32, DB = D / 16;
-    static_assert(CQT <= 6 && (2 * CQT) % 6 == 0, "whole dW units per value wave and half");
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
     const int tid = threadIdx.x;
@@ -257,7 +256,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
 #pragma unroll
                     for (int f = 0; f < 2; ++f) acc[kb][f] = mfma_bf16(kf[kb][ks], qf[f], acc[kb][f]);
             }
-            const int rbase = (tp * BR) % S_RING;
+            const int rbase = (tp * BR) % Lds::ring_rows;
 #pragma unroll
             for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
@@ -278,7 +277,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                     if constexpr (KB0 == 0) {
                         if (WANT_QW && kb < 3) {
                             const int rr = rbase + 2 * n + f;
-                            *reinterpret_cast<u32x2 *>(s_ring + (rr >= S_RING ? rr - S_RING : rr) * SST + (kb * 16 + 4 * g) * 2) =
+                            *reinterpret_cast<u32x2 *>(s_ring + (rr >= Lds::ring_rows ? rr - Lds::ring_rows : rr) * SST + (kb * 16 + 4 * g) * 2) =
                                 (u32x2){pd[kb][f][0], pd[kb][f][1]};
                         }
                     }
@@ -540,14 +539,16 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
             store_dv();
         } else {
             // dW: a unit is the key blocks of two triples (pair group) times one tap slot; the waves 0 .. 2
-            // take 2 CQT / 3 consecutive units each, in two passes of NU units of one pair group.
-            constexpr int NU = CQT / 3, NPASS = 2, TH = NU * NPASS;
+            // take 2 DWT / 3 consecutive units each, in passes of NU units of one pair group (DWT: the tap slots and what fills
+            // them up to a multiple of three, which is multiplied and dropped; four units per pass spilled 25 registers).
+            constexpr int DWT = (CQT + 2) / 3 * 3, TH = 2 * DWT / 3, NU = TH > 6 ? 2 : TH / 2, NPASS = TH / NU;
+            static_assert(NU * NPASS == TH && DWT % NU == 0, "a pass stays in one pair group");
             int dw_pg[NPASS], dw_t[NPASS];
 #pragma unroll
             for (int ps = 0; ps < NPASS; ++ps) {
                 const int q = pr * TH + ps * NU;
-                dw_pg[ps] = q / CQT;
-                dw_t[ps] = q - dw_pg[ps] * CQT;
+                dw_pg[ps] = q / DWT;
+                dw_t[ps] = q - dw_pg[ps] * DWT;
             }
             f32x4 acc_w[TH][2];
 #pragma unroll
@@ -566,15 +567,15 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 if (WANT_QW && u_in) static_for<NPASS>([&](auto PS) {
                     constexpr int ps = decltype(PS)::value;
                     const int pg = dw_pg[ps], t_lo = dw_t[ps];
-                    const int wbase = ((u + 1) * BR - (CQT - 1) + S_RING) % S_RING;
+                    const int wbase = ((u + 1) * BR - (CQT - 1) + Lds::ring_rows) % Lds::ring_rows;
                     const unsigned int c_lane = opaque(tr_lane_off(CST, g, n));
                     const unsigned int ring0 = Lds::pair_off + 2 * pg * Lds::pair_bytes + 4 * (n & 3) * 2;
                     unsigned int a_lo[NU], a_hi[NU];
 #pragma unroll
                     for (int tt = 0; tt < NU; ++tt) {
                         const unsigned int ra = wbase + 4 * g + (n >> 2) + min(t_lo + tt, CQT - 1), rb = ra + 16;
-                        a_lo[tt] = opaque(ring0 + min(ra, ra - S_RING) * SST);
-                        a_hi[tt] = opaque(ring0 + min(rb, rb - S_RING) * SST);
+                        a_lo[tt] = opaque(ring0 + min(ra, ra - Lds::ring_rows) * SST);
+                        a_hi[tt] = opaque(ring0 + min(rb, rb - Lds::ring_rows) * SST);
                     }
                     const unsigned int off4 = pg == NP / 2 - 1 ? Lds::pair_bytes + 64 : 2 * Lds::pair_bytes;
                     unsigned int a4_lo[NU], a4_hi[NU];
@@ -852,8 +853,16 @@ template <int D, typename TO, int WANT>
 hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v, const void *d_o,
                    const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv,
                    void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
-    if (p.c_q <= 3) return launch_chain3<D, 3, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    return launch_chain3<D, 6, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+#define CALL(CQT) launch_chain3<D, CQT, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s)
+    if (p.c_q <= 3) return CALL(3);
+    // (7 and 8 slots apart: a padding tap for 7 costs 2.5 % in the two-role kernel)
+    if constexpr (D <= 64) {
+        if (p.c_q == 7) return CALL(7);
+        if (p.c_q == 8) return CALL(8);
+        if (p.c_q > 8) return CALL(11);
+    }
+    return CALL(6);
+#undef CALL
 }
 
 template <int WANT>

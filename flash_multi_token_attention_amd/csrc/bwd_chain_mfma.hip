@@ -1,5 +1,5 @@
-// Whole backward of conv-attention on bf16 MFMA (gfx950), windows of 7 to 11 query taps (instances of 8 and
-// 12 tap slots): the score chain stays in registers.  (Windows of up to 6 query taps run the three-role kernel of bwd_chain3_mfma.hip,
+// Whole backward of conv-attention on bf16 MFMA (gfx950), windows of 7 to 11 query taps at head dimension 128 (instances of 7, 8
+// and 11 tap slots): the score chain stays in registers.  (Other windows run the three-role kernel of bwd_chain3_mfma.hip,
 // which shares this file's building blocks through chain_common.hpp; the per-(batch, head) dC scale
 // kernels of both live here.)
 //
@@ -494,8 +494,8 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
         // dW: a unit is the key blocks of two pairs (pair group) times one tap slot; every wave takes one pair
         // group and half of the tap slots, in one pass (two for more than 8 tap slots: the operands of a
         // pass are in registers three key blocks deep).
-        static_assert(CQT % 2 == 0, "half of the tap slots per wave");
-        constexpr int NPASS = CQT > 8 ? 2 : 1, TH = CQT / 2, NU = TH / NPASS;   // units per pass
+        // (an odd number of slots: the second wave of a group multiplies its last one twice and drops the copy)
+        constexpr int NPASS = CQT > 8 ? 2 : 1, TH = (CQT + 1) / 2, NU = TH / NPASS;   // units per pass
         static_assert(NU * NPASS == TH, "whole units per pass");
         int dw_pg[NPASS], dw_t[NPASS];   // pair group and first tap slot
 #pragma unroll
@@ -885,25 +885,19 @@ template <int D, typename TO, int WANT>
 hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v, const void *d_o,
                    const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv,
                    void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
-    // (windows of up to 6 query taps run the three-role kernel of bwd_chain3_mfma.hip)
-    if (p.c_q <= 8) return launch_chain<D, 8, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    return launch_chain<D, 12, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    // (the others run the three-role kernel of bwd_chain3_mfma.hip; forward + backward of B4 H16 N2048 d128 7x7 in 8 slots 682 us,
+    // in 7 665)
+#define CALL(CQT) launch_chain<D, CQT, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s)
+    return p.c_q <= 7 ? CALL(7) : p.c_q == 8 ? CALL(8) : CALL(11);
+#undef CALL
 }
 
 template <int WANT>
 hipError_t pick_shape(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const void *d_o,
                       const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv,
                       void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
-    if (p.d == 128) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-        return pick_cq<128, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    }
-    if (p.d == 32) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-        return pick_cq<32, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    }
-    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    return pick_cq<64, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    return pick_cq<128, float, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 
 }  // namespace

@@ -37,7 +37,7 @@ template <int D, int CQT> struct ChainLds {
     static constexpr int stat_bytes = 2 * (2 * BR * 4);
     // bands, then flipped bands: one KB of ready-made fragments per tap slot, or (windows of more than 8
     // query taps, where those do not fit) one compact table per tap slot that the lanes read their fragments from
-    static constexpr bool compact_bands = CQT > 8;
+    static constexpr bool compact_bands = CQT > 8 && D > 64;
     static constexpr int band_slot = compact_bands ? kBandTab : 1024;
     static constexpr int band_off = stat_off + stat_bytes;
     static constexpr int band_bytes = 2 * CQT * band_slot;

@@ -338,7 +338,7 @@ CHAIN_DECL(mfma_bwd_chain_kv);
 CHAIN_DECL(mfma_bwd_chain_qw);
 CHAIN_DECL(mfma_bwd_chain_all);
 CHAIN_DECL(mfma_bwd_chain_split);   // everything, with share > 0
-// the same with three waves per SIMD (bwd_chain3_mfma.hip): windows of up to 6 query taps
+// the same with three waves per SIMD (bwd_chain3_mfma.hip)
 CHAIN_DECL(mfma_bwd_chain3_kv);
 CHAIN_DECL(mfma_bwd_chain3_qw);
 CHAIN_DECL(mfma_bwd_chain3_all);
@@ -348,7 +348,11 @@ inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const v
                                  const void *d_o, const float *Dl, const float *lse, const float *w,
                                  const float *dc_scale, void *dk, void *dv, void *ds_ws, float *dw_part,
                                  hipStream_t s, int share = 0, float *kv_part = nullptr) {
-    if (p.c_q <= 6) {
+    // Three waves of 168 registers per SIMD hold any window's roles up to d = 64 (the second kernel computes a third C block per 32
+    // keys, which a neighbour has anyway); beyond 6 query taps the dV and dW accumulators of d = 128 do not fit.  Forward + backward, us, two
+    // waves in 8 or 12 slots and three in 7 or 11: B4 H16 N4096 11x11 d64 2406 and 2216, d32 2225 and 2032, 7x7 d64 1898 and 1797,
+    // d32 1742 and 1581, B2 H8 N1531 d64 11x11 168 and 156.
+    if (p.c_q <= 6 || p.d <= 64) {
         if (want == 1) return mfma_bwd_chain3_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
         if (want == 2) return mfma_bwd_chain3_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
         if (share) return mfma_bwd_chain3_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
