@@ -79,6 +79,10 @@ _SIGNATURES = {
     "convattn_decode_partial_bytes": (C.c_size_t, [_D]),
     "convattn_decode": (C.c_int, [_D] + [_P] * 8),
     "convattn_decode_strided": (C.c_int, [_D] + [_P] * 4 + [C.c_longlong] * 2 + [_P] * 4),
+    "convattn_decode_splits": (C.c_int, [C.c_int] * 5),
+    "convattn_decode_step_splits": (C.c_int, [C.c_int] * 5),
+    "convattn_decode_whole_ok": (C.c_int, [_D]),
+    "convattn_decode_whole": (C.c_int, [_D] + [_P] * 4 + [C.c_longlong] * 2 + [_P] * 4),
     "convattn_decode_kv": (C.c_int, [_D] + [_P] * 3 + [C.POINTER(KvLayout)] + [_P] * 5),
     "convattn_decode_combine": (C.c_int, [_D] + [_P] * 7),
     "convattn_decode_noalloc_bytes": (C.c_size_t, [_D]),

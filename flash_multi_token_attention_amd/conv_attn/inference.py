@@ -21,4 +21,4 @@ def fwd_conv_attn_inference(Q, K, V, conv_kernel, k_splits, scale, pad_q, pad_k,
         raise ValueError(f"Q sequence length must be <= 16 for inference, got {Q.shape[2]}")
     if conv_kernel.dim() != 3 or pad_q != conv_kernel.shape[1] - 1 or pad_k != (conv_kernel.shape[2] - 1) // 2:
         ops._weights(conv_kernel, Q.shape[1], pad_q, pad_k, Q.device)  # raises, naming what is wrong
-    return ops.decode(Q, K, V, conv_kernel, k_splits, scale, causal)[:3]
+    return ops.decode_whole(Q, K, V, conv_kernel, k_splits, scale, causal)

@@ -370,26 +370,9 @@ def backward(Q, K, V, dO, D, L, conv_kernel, scale, pad_q, pad_k, causal,
 
 
 def default_k_splits(B: int, H: int, Nk: int, ragged: bool = False, d: int = 128) -> int:
-    """Split count by the model the measurements follow: a workgroup (4 waves of 64 keys per iteration) costs its iterations
-    plus about one for set-up and wind-down, and the (batch, head, split) workgroups run in rounds of one per CU, two with
-    d = 32, whose workgroups have half the bytes in flight.
-    The best of 1 to 4 rounds (B1 H8 N65536 d128: 32 splits 48.5 us, 64: 54, 256: 82; B8 H32 N8192 with 11 x 11
-    windows: 1 split 161 us, 8: 198; B32 H32 N8192: 1 split 616 us, 2: 630); up to 16 rounds where the sequences of a batch
-    have lengths of their own, since only the longest costs a whole round (B32 H8 N43236 d64 of a quarter to the whole of it: 4 splits
-    328 us, 16: 299).  Two splits at least from 512 heads on with d = 32 or 64: in a cache whose heads lie 1 MiB and a few KiB
-    apart the unsplit heads keep to the same channels (B32 H32 N8192 d64 in a cache of 8256 rows: 1 split 385 us, 2: 329; dense 2 %
-    more).  Over 1842 shapes, d 32 to 128, the choice is 2 % from the best count on average (d = 128 1 to 2 %, d = 32 2 to 4 %)."""
-    ragged = ragged and B > 1
-    slots = 512 if d == 32 else 256
-    most = min(Nk // 256, 1024)
-    best, splits = None, 1
-    for rounds in (1, 2, 3, 4, 6, 8, 12, 16) if ragged else (1, 2, 3, 4):
-        n = min(rounds * slots // (B * H), most)
-        if n >= 1:
-            cost = (rounds + (0.5 if ragged else 0.0)) * (-(-Nk // (256 * n)) + 1)
-            if best is None or cost < best:
-                best, splits = cost, n
-    return max(splits, 2) if d <= 64 and B * H >= 512 and Nk >= 2048 else splits
+    """The library's split count for a step of B x H (batch, head) pairs; ``ragged``: the entries of the batch have lengths of
+    their own (csrc/decode_stream.hip has the rule and its measurements)."""
+    return _lib.load().convattn_decode_splits(B, H, Nk, int(ragged), d)
 
 
 def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.float32,
@@ -403,8 +386,7 @@ def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.
     if (host is not None and workspace is None and not exact and all(isinstance(t, torch.Tensor) for t in (Q, K, V, conv_kernel))
             and K.dim() == 4):
         # the ordinary case in one native call; anything it does not take comes back as None and is checked below
-        r = host.decode_dense(Q, K, V, conv_kernel, k_splits or default_k_splits(Q.shape[0], Q.shape[1], K.shape[2], d=Q.shape[-1]),
-                              scale, bool(causal), out_dtype)
+        r = host.decode_dense(Q, K, V, conv_kernel, k_splits or 0, scale, bool(causal), out_dtype, True)
         if r is not None:
             return r[0], r[1], r[2], r[3:]
     _check_qkv(Q, K, V, kv_views=True)
@@ -443,6 +425,18 @@ def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.
                                      _ptr(M), _ptr(L), st)
     _lib.check(rc, "conv_attn.forward_inference (combine)")
     return O, M, L, (O_part, M_part, L_part)
+
+
+def decode_whole(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.float32):
+    """``decode`` without the partials -> (O, M, L).  Nobody sees the splits, so ``k_splits`` is their most: no more are made
+    than the library would choose (B32 H32 N1000 d128 in 32 splits 663 us, in its own count 43), and one launch does it
+    where it takes the step as a whole."""
+    host = _lib.host()
+    if host is not None and all(isinstance(t, torch.Tensor) for t in (Q, K, V, conv_kernel)) and K.dim() == 4:
+        r = host.decode_dense(Q, K, V, conv_kernel, k_splits or 0, scale, bool(causal), out_dtype, False)
+        if r is not None:
+            return r[:3]
+    return decode(Q, K, V, conv_kernel, k_splits, scale, causal, out_dtype)[:3]
 
 
 def _kv_splits(B: int, H: int, H_kv: int, Nk: int, d: int, c_q: int, ragged: bool) -> int:

@@ -449,23 +449,50 @@ int convattn_decode(const convattn_desc *desc, const void *q, const void *k, con
     return convattn_decode_strided(desc, q, k, v, w, hs * desc->H, hs, o_part, m_part, l_part, stream);
 }
 
+// rows of a head stay dense (d elements apart) and 16-byte aligned; heads and batches must not overlap
+static bool kv_strides(long long batch, long long head, Problem *p) {
+    p->kv_bstride = batch;
+    p->kv_hstride = head;
+    return head < (long long)p->Nk * p->d || head % 8 != 0 || batch % 8 != 0 || (p->B > 1 && batch < (long long)p->Nk * p->d);
+}
+
 int convattn_decode_strided(const convattn_desc *desc, const void *q, const void *k, const void *v,
                             const float *w, long long kv_batch_stride, long long kv_head_stride,
                             float *o_part, float *m_part, float *l_part, void *stream) {
     Problem p;
     int rc = validate(desc, CONVATTN_OP_DECODE, &p);
     if (rc) return rc;
-    // rows of a head stay dense (d elements apart) and 16-byte aligned; heads and batches must not overlap
-    if (kv_head_stride < (long long)p.Nk * p.d || kv_head_stride % 8 != 0 || kv_batch_stride % 8 != 0 ||
-        (p.B > 1 && kv_batch_stride < (long long)p.Nk * p.d))
-        return CONVATTN_ERR_SHAPE;
-    p.kv_bstride = kv_batch_stride; p.kv_hstride = kv_head_stride;
+    if (kv_strides(kv_batch_stride, kv_head_stride, &p)) return CONVATTN_ERR_SHAPE;
     REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(w);
     REQUIRE_PTR(o_part); REQUIRE_PTR(m_part); REQUIRE_PTR(l_part);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (pick_path(desc, p, CONVATTN_OP_DECODE) == 1)
         return (int)decode_stream(p, q, k, v, w, o_part, m_part, l_part, s);
     return (int)generic_decode(p, desc->in_dtype, q, k, v, w, o_part, m_part, l_part, s);
+}
+
+int convattn_decode_splits(int B, int H, int Nk, int ragged, int d) {
+    return B > 0 && H > 0 && Nk > 0 ? decode_splits((long long)B * H, Nk, ragged && B > 1, d) : 1;
+}
+
+int convattn_decode_step_splits(int B, int H, int Nk, int d, int asked) {
+    return B > 0 && H > 0 && Nk > 0 ? decode_step_splits((long long)B * H, Nk, d, asked) : 1;
+}
+
+int convattn_decode_whole_ok(const convattn_desc *desc) {
+    Problem p;
+    return validate(desc, CONVATTN_OP_DECODE, &p) == 0 && pick_path(desc, p, CONVATTN_OP_DECODE) == 1 && decode_whole_waves(p) > 0;
+}
+
+int convattn_decode_whole(const convattn_desc *desc, const void *q, const void *k, const void *v, const float *w,
+                          long long kv_batch_stride, long long kv_head_stride, void *o, float *m, float *l, void *stream) {
+    Problem p;
+    int rc = validate(desc, CONVATTN_OP_DECODE, &p);
+    if (rc) return rc;
+    if (kv_strides(kv_batch_stride, kv_head_stride, &p)) return CONVATTN_ERR_SHAPE;
+    REQUIRE_PTR(q); REQUIRE_PTR(k); REQUIRE_PTR(v); REQUIRE_PTR(w); REQUIRE_PTR(o); REQUIRE_PTR(m); REQUIRE_PTR(l);
+    if (pick_path(desc, p, CONVATTN_OP_DECODE) != 1 || !decode_whole_waves(p)) return CONVATTN_ERR_SPLITS;
+    return (int)decode_whole(p, desc->out_dtype, q, k, v, w, o, m, l, static_cast<hipStream_t>(stream));
 }
 
 int convattn_decode_kv(const convattn_desc *desc, const void *q, const void *k, const void *v,

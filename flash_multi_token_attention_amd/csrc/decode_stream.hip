@@ -17,8 +17,9 @@
 //     the key phases are summed across lanes once at the end;
 //   * K of the next iteration and V of this one are in flight while the scores,
 //     window and softmax of this iteration are computed.
-// The 4 waves merge their (m, l, o) in LDS and store one un-normalised partial
-// per split; convattn_decode_combine merges the splits.
+// The waves merge their (m, l, o) in LDS and store one un-normalised partial
+// per split; convattn_decode_combine merges the splits.  WHOLE instances have all keys of a (batch, head) in one workgroup
+// and store the result itself.
 //
 // Where the rows live is a parameter of the kernel (KvArgs): query heads may share KV heads
 // (head h reads KV head h / group), the rows of a (batch, KV head) may be contiguous or come in
@@ -38,7 +39,7 @@ namespace {
 // Non-temporal loads below: every K / V row is read exactly once, and keeping it out of the
 // caches' replacement order is worth 10 % of the stream's bandwidth here.
 
-constexpr int NW = 4;
+constexpr int kWaves = 4;          // waves per workgroup of a split
 constexpr int IT = 64;             // keys per wave iteration
 constexpr int SW = IT + 16;        // score strip width: 16 carried + 64 new
 constexpr int SROW = SW + 4;       // floats per strip row (84)
@@ -46,11 +47,11 @@ constexpr int SROW = SW + 4;       // floats per strip row (84)
 __device__ __forceinline__ float bf16_lo(unsigned int w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(unsigned int w) { return __uint_as_float(w & 0xffff0000u); }
 
-template <int D, bool PAGED, int HG>
+template <int D, bool PAGED, int HG, int NW, bool WHOLE>
 __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(
     Problem p, KvArgs kv, const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
-    const bf16_t *__restrict__ V, const float *__restrict__ W, float *__restrict__ O_part,
-    float *__restrict__ M_part, float *__restrict__ L_part) {
+    const bf16_t *__restrict__ V, const float *__restrict__ W, void *__restrict__ O_out,
+    float *__restrict__ M_out, float *__restrict__ L_out, int out_dt) {
     constexpr int KS = D / 32;
     constexpr int CPR = D / 8;       // 16-byte chunks per K/V row
     constexpr int RPI = 64 / CPR;    // V rows one load instruction of the wave covers
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(
     // Causal variant: tap row a sits at position Nk - c_q + a and sees no later key.
     const int row_pos = p.causal ? Nk - cq + row_tap : 0x7fffffff;
 
-    // Key range of this wave: the split's chunk cut into 4 runs of whole iterations.
+    // Key range of this wave: the split's chunk cut into a run of whole iterations per wave.
     // (PAGED: splits start at multiples of 64 keys, so that an iteration's rows are a fixed window)
     const int chunk = PAGED ? ((Nk + p.n_splits - 1) / p.n_splits + IT - 1) / IT * IT : (Nk + p.n_splits - 1) / p.n_splits;
     const int s_lo = sp * chunk, s_hi = min(Nk, s_lo + chunk);
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(
         }
     }
 
-    // merge the 4 waves: o = sum o_w e^{m_w - m}, l = sum l_w e^{m_w - m}
+    // merge the waves: o = sum o_w e^{m_w - m}, l = sum l_w e^{m_w - m}
 #pragma unroll
     for (int hh = 0; hh < HG; ++hh) {
         if (lane < CPR) {
@@ -325,20 +326,23 @@ __global__ __launch_bounds__(NW * 64) void decode_stream_kernel(
 #pragma unroll
         for (int w = 0; w < NW; ++w) m = fmaxf(m, s_ml[w][hh][0]);
         const size_t slot = (bh + hh) * p.n_splits + sp;
+        float l = 0.f;
+        if (WHOLE || tid == 0) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w)
+                if (s_ml[w][hh][0] != kNegInf) l = fmaf(s_ml[w][hh][1], __expf(s_ml[w][hh][0] - m), l);
+        }
         if (tid < D) {
             float o = 0.f;
 #pragma unroll
             for (int w = 0; w < NW; ++w)
                 if (s_ml[w][hh][0] != kNegInf) o = fmaf(s_o[w][hh][tid], __expf(s_ml[w][hh][0] - m), o);
-            O_part[slot * D + tid] = o;
+            if (WHOLE && out_dt == CONVATTN_BF16) static_cast<bf16_t *>(O_out)[slot * D + tid] = (bf16_t)(o / l);
+            else static_cast<float *>(O_out)[slot * D + tid] = WHOLE ? o / l : o;
         }
         if (tid == 0) {
-            float l = 0.f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w)
-                if (s_ml[w][hh][0] != kNegInf) l = fmaf(s_ml[w][hh][1], __expf(s_ml[w][hh][0] - m), l);
-            M_part[slot] = m;
-            L_part[slot] = l;
+            M_out[slot] = m;
+            L_out[slot] = l;
         }
     }
 }
@@ -358,8 +362,8 @@ hipError_t decode_stream_kv(const Problem &p, const KvArgs &kv, const void *q, c
     const int hg = p.d != 32 || p.c_q > 8 ? 1 : kv.group % 4 == 0 ? 4 : kv.group % 2 == 0 ? 2 : 1;
     dim3 grid(p.n_splits, p.H / hg, p.B);
 #define CONVATTN_DECODE_LAUNCH(DD, PG, HH)                                                                   \
-    decode_stream_kernel<DD, PG, HH><<<grid, NW * 64, 0, s>>>(p, kv, (const bf16_t *)q, (const bf16_t *)k,     \
-                                                             (const bf16_t *)v, w, o_part, m_part, l_part)
+    decode_stream_kernel<DD, PG, HH, kWaves, false><<<grid, kWaves * 64, 0, s>>>(                              \
+        p, kv, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, w, o_part, m_part, l_part, CONVATTN_F32)
 #define CONVATTN_DECODE_PICK_HG(DD, PG)                                                                      \
     do {                                                                                                     \
         if (hg == 4) CONVATTN_DECODE_LAUNCH(DD, PG, 4);                                                       \
@@ -386,6 +390,74 @@ hipError_t decode_stream(const Problem &p, const void *q, const void *k, const v
     KvArgs kv = {};
     kv.group = 1;
     return decode_stream_kv(p, kv, q, k, v, w, o_part, m_part, l_part, s);
+}
+
+// Split count of a decode step, by the model the measurements follow: a workgroup (4 waves of 64 keys per iteration) costs its
+// iterations plus about one for set-up and wind-down, and the (batch, head, split) workgroups run in rounds of one per CU, two with
+// d = 32, whose workgroups have half the bytes in flight.
+// The best of 1 to 4 rounds (B1 H8 N65536 d128: 32 splits 48.5 us, 64: 54, 256: 82; B8 H32 N8192 with 11 x 11
+// windows: 1 split 161 us, 8: 198; B32 H32 N8192: 1 split 616 us, 2: 630); up to 16 rounds where the sequences of a batch
+// have lengths of their own, since only the longest costs a whole round (B32 H8 N43236 d64 of a quarter to the whole of it: 4 splits
+// 328 us, 16: 299).  Two splits at least from 512 heads on with d = 32 or 64: in a cache whose heads lie 1 MiB and a few KiB
+// apart the unsplit heads keep to the same channels (B32 H32 N8192 d64 in a cache of 8256 rows: 1 split 385 us, 2: 329; dense 2 %
+// more).  Over 1842 shapes, d 32 to 128, the choice is 2 % from the best count on average (d = 128 1 to 2 %, d = 32 2 to 4 %).
+static int slots_of(int d) { return d == 32 ? 512 : 256; }
+int decode_splits(long long heads, int Nk, bool ragged, int d) {
+    const int slots = slots_of(d), most = Nk / 256 < 1024 ? Nk / 256 : 1024;
+    static constexpr int kRounds[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    int splits = 1;
+    float best = 0.f;
+    for (int i = 0; i < (ragged ? 8 : 4); ++i) {
+        const long long fit = kRounds[i] * (long long)slots / heads;
+        const int n = (int)(fit < most ? fit : most);
+        if (n < 1) continue;
+        const float cost = (kRounds[i] + (ragged ? 0.5f : 0.f)) * (float)((Nk + 256LL * n - 1) / (256LL * n) + 1);
+        if (best == 0.f || cost < best) { best = cost; splits = n; }
+    }
+    return d <= 64 && heads >= 512 && Nk >= 2048 && splits < 2 ? 2 : splits;
+}
+
+// The split count of a step whose partials nobody sees, `asked` at most (0: no limit).  While the workgroups fit one round,
+// 128 keys each, two waves at work, are faster than 256: the four waves of a workgroup wait for each other's LDS reads (us, by the rule
+// above and now: B1 H8 d128 N1000 12.8 and 10.5, N2048 14.3 and 10.7, B4 H8 d64 N1000 12.0 and 9.3).  Up to 64, beyond which the merge
+// costs more than it gains.
+int decode_step_splits(long long heads, int Nk, int d, int asked) {
+    int n = decode_splits(heads, Nk, false, d);
+    const long long room = slots_of(d) / heads;
+    if (n <= room) {
+        const long long one = room < (Nk + 127) / 128 ? room : (Nk + 127) / 128;
+        if (one > n) n = one < 64 ? (int)one : n > 64 ? n : 64;
+    }
+    return asked > 0 && asked < n ? asked : n;
+}
+
+// Waves of the workgroup that takes all keys of a (batch, head), or 0: splits and a merge.  Without splits the merge is only a launch
+// of its own (B32 H32 N8192 d128 614 -> 611 us, B1 H8 N500 d64 10.9 -> 7.3).  With splits one workgroup has to be as fast as they
+// are in parallel: where eight waves have one iteration each (B2 H2 N512 d64 10.0 -> 7.8 us; at two, B1 H8 N1000 d128,
+// 12.8 -> 16.4; sixteen waves of one iteration, d64, 9.8: the window's LDS reads of the waves of a CU pass one after the other).
+constexpr int kWholeWaves = 8;
+int decode_whole_waves(const Problem &p) { return p.n_splits == 1 ? kWaves : p.Nk <= kWholeWaves * IT ? kWholeWaves : 0; }
+
+hipError_t decode_whole(Problem p, int out_dt, const void *q, const void *k, const void *v, const float *w, void *o, float *m, float *l,
+                        hipStream_t s) {
+    const bool many = decode_whole_waves(p) > kWaves;
+    p.n_splits = 1;
+    KvArgs kv = {};
+    kv.group = 1;
+#define CALL(DD, NW)                                                                                                       \
+    decode_stream_kernel<DD, false, 1, NW, true><<<dim3(1, p.H, p.B), NW * 64, 0, s>>>(p, kv, (const bf16_t *)q, (const bf16_t *)k, \
+                                                                                     (const bf16_t *)v, w, o, m, l, out_dt)
+    if (many) {
+        if (p.d == 128) CALL(128, kWholeWaves);
+        else if (p.d == 64) CALL(64, kWholeWaves);
+        else CALL(32, kWholeWaves);
+    } else {
+        if (p.d == 128) CALL(128, kWaves);
+        else if (p.d == 64) CALL(64, kWaves);
+        else CALL(32, kWaves);
+    }
+#undef CALL
+    return hipGetLastError();
 }
 
 }  // namespace convattn

@@ -31,7 +31,7 @@ using torch::autograd::variable_list;
 #define API_LIST(F)                                                                                                   \
     F(convattn_strerror) F(convattn_kernel_path) F(convattn_fwd) F(convattn_fwd_split_workspace_bytes) F(convattn_fwd_split) F(convattn_bwd_preprocess) F(convattn_bwd_fused_workspace_bytes)              \
     F(convattn_bwd_fused) F(convattn_bwd_split_workspace_bytes) F(convattn_bwd_all) F(convattn_staged_workspace_bytes) F(convattn_staged_fwd) F(convattn_staged_bwd)               \
-    F(convattn_decode_strided) F(convattn_decode_kv) F(convattn_decode_combine)                 \
+    F(convattn_decode_strided) F(convattn_decode_splits) F(convattn_decode_step_splits) F(convattn_decode_whole_ok) F(convattn_decode_whole) F(convattn_decode_kv) F(convattn_decode_combine)                 \
     F(convattn_headmix_validate) F(convattn_headmix_fwd_workspace_bytes) F(convattn_headmix_fwd_ws)                   \
     F(convattn_headmix_bwd_fused_workspace_bytes) F(convattn_headmix_bwd_fused_dq_dw_workspace_bytes) F(convattn_headmix_bwd_fused)
 struct Api {
@@ -406,17 +406,41 @@ std::optional<at::ScalarType> out_type(const py::object &dtype) {
     return t;
 }
 
-// k_splits > 0
+// k_splits > 0, or 0: the library's choice.  Without `partials` k_splits is a most, and they may be missing from the result.
 std::optional<Decoded> decode_dense(const Tensor &Q, const Tensor &K, const Tensor &V, const Tensor &W, int64_t k_splits, double scale,
-                                    bool causal, const py::object &out_dtype) {
+                                    bool causal, const py::object &out_dtype, bool partials) {
     const auto out = out_type(out_dtype);
     if (!out || watched() || !same_rows(Q, K, V) || K.size(1) != Q.size(1) || !Q.is_contiguous() || !cache_rows(K) || K.strides() != V.strides() ||
-        Q.size(2) > 16 || k_splits < 1 || k_splits > 1024 || W.dim() != 3)
+        Q.size(2) > 16 || k_splits < 0 || k_splits > 1024 || k_splits > K.size(2) || W.dim() != 3)
         return std::nullopt;
     const Tensor Wf = window(W, Q.size(1), W.size(1) - 1, (W.size(2) - 1) / 2, Q);
     if (!Wf.defined()) return std::nullopt;
     convattn_desc d = window_desc(Q, K.size(2), Wf, scale, causal, *out == at::kFloat ? CONVATTN_F32 : CONVATTN_BF16);
-    d.n_splits = (int)k_splits;
+    d.n_splits = k_splits > 0 ? (int)k_splits : 1;
+    if (!partials && api.convattn_kernel_path(&d, CONVATTN_OP_DECODE) == 1) {
+        d.n_splits = api.convattn_decode_step_splits(d.B, d.H, d.Nk, d.d, (int)k_splits);
+        const bool whole = api.convattn_decode_whole_ok(&d) != 0;
+        const char *what = "conv_attn.forward_inference";
+        py::gil_scoped_release no_gil;
+        c10::DeviceGuard dev(Q.device());
+        at::AutoDispatchBelowADInplaceOrView guard;
+        Tensor O = empty({d.B, d.H, 1, d.d}, *out, Q), M = empty({d.B, d.H, 1}, at::kFloat, Q), L = empty({d.B, d.H, 1}, at::kFloat, Q);
+        const int64_t slots = (int64_t)d.B * d.H * d.n_splits;
+        const Tensor part = whole ? Tensor() : empty({slots * d.d + 2 * padded(slots)}, at::kFloat, Q);
+        const void *q = Q.data_ptr(), *k = K.data_ptr(), *v = V.data_ptr();
+        const float *w = Wf.const_data_ptr<float>();
+        float *m = M.mutable_data_ptr<float>(), *l = L.mutable_data_ptr<float>();
+        void *s = stream_of(Q);
+        if (whole) {
+            check(api.convattn_decode_whole(&d, q, k, v, w, batch_stride(K), head_stride(K), O.data_ptr(), m, l, s), what);
+        } else {
+            float *op = part.mutable_data_ptr<float>(), *mp = op + slots * d.d, *lp = mp + padded(slots);
+            check(api.convattn_decode_strided(&d, q, k, v, w, batch_stride(K), head_stride(K), op, mp, lp, s), what);
+            check(api.convattn_decode_combine(&d, op, mp, lp, O.data_ptr(), m, l, s), what);
+        }
+        return Decoded{O, M, L, Tensor(), Tensor(), Tensor()};
+    }
+    if (k_splits == 0) d.n_splits = api.convattn_decode_splits(d.B, d.H, d.Nk, 0, d.d);
     return run_decode(d, Q, *out, "conv_attn.forward_inference", [&](float *o, float *m, float *l, void *s) {
         return api.convattn_decode_strided(&d, Q.data_ptr(), K.data_ptr(), V.data_ptr(), Wf.const_data_ptr<float>(), batch_stride(K),
                                            head_stride(K), o, m, l, s);

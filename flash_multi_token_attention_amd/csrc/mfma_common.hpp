@@ -390,5 +390,12 @@ hipError_t decode_stream_kv(const Problem &p, const KvArgs &kv, const void *q, c
                             const float *w, float *o_part, float *m_part, float *l_part, hipStream_t s);
 hipError_t decode_stream(const Problem &p, const void *q, const void *k, const void *v, const float *w,
                          float *o_part, float *m_part, float *l_part, hipStream_t s);
+// a step's split count (ragged: the entries of the batch have lengths of their own)
+int decode_splits(long long heads, int Nk, bool ragged, int d);
+int decode_step_splits(long long heads, int Nk, int d, int asked);
+// The whole step in one launch, where decode_whole_waves is not 0
+int decode_whole_waves(const Problem &p);
+hipError_t decode_whole(Problem p, int out_dt, const void *q, const void *k, const void *v, const float *w, void *o, float *m, float *l,
+                        hipStream_t s);
 
 }  // namespace convattn

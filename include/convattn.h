@@ -264,6 +264,20 @@ int convattn_decode_strided(const convattn_desc *desc, const void *q, const void
                             const float *w, long long kv_batch_stride, long long kv_head_stride,
                             float *o_part, float *m_part, float *l_part, void *stream);
 
+/* The split count to be preferred for a step of B x H (batch, head) pairs; ragged: entries of the batch have fewer than Nk keys. */
+int convattn_decode_splits(int B, int H, int Nk, int ragged, int d);
+/* The same for a step whose partials nobody reads, and at most `asked` where that is > 0. */
+int convattn_decode_step_splits(int B, int H, int Nk, int d, int asked);
+
+/*
+ * A whole decode step in one launch, without partials: O [B,H,1,d] (out_dtype), M, L [B,H,1] fp32.  Taken (convattn_decode_whole_ok
+ * != 0) for one split, and for caches short enough for one workgroup per (batch, head), whatever n_splits is;
+ * CONVATTN_ERR_SPLITS otherwise.  Strides as in convattn_decode_strided.
+ */
+int convattn_decode_whole_ok(const convattn_desc *desc);
+int convattn_decode_whole(const convattn_desc *desc, const void *q, const void *k, const void *v, const float *w,
+                          long long kv_batch_stride, long long kv_head_stride, void *o, float *m, float *l, void *stream);
+
 /*
  * Where K and V of a decode step live, beyond the dense and strided [B,H,Nk,d] forms above: shared
  * KV heads (grouped-query attention), a paged cache and per-sequence lengths.  The reference has

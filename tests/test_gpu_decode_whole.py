@@ -1,0 +1,54 @@
+"""Decode steps whose splits nobody sees: one workgroup per (batch, head) or fewer splits than asked for, against the CPU oracle and
+against the step that returns its partials."""
+import pytest
+import torch
+
+from flash_multi_token_attention_amd.conv_attn import fwd_conv_attn_inference, ops
+from oracle import conv_attn_oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _case(B, H, r, Nk, d, c_q, c_k, seed):
+    g = torch.Generator().manual_seed(seed)
+    Q, K, V = (torch.randn(B, H, n, d, generator=g).to(torch.bfloat16) for n in (r, Nk, Nk))
+    W = 0.05 * torch.randn(H, c_q, c_k, generator=g)
+    W[:, c_q - 1, (c_k - 1) // 2] += 1.0
+    return Q, K, V, W
+
+
+# around a wave's 64 keys, four and eight waves of them
+@pytest.mark.parametrize("Nk", [1, 63, 65, 257, 511, 512, 513, 1100])
+@pytest.mark.parametrize("d,c_q,c_k,r", [(32, 3, 3, 16), (64, 7, 7, 16), (128, 6, 11, 6), (64, 16, 17, 5)])
+@pytest.mark.parametrize("splits", [0, 1, 32])
+def test_result_without_partials(Nk, d, c_q, c_k, r, splits):
+    if splits > Nk:
+        splits = Nk
+    Q, K, V, W = _case(2, 3, r, Nk, d, c_q, c_k, seed=Nk + d)
+    ref = orc.decode(Q.float(), K.float(), V.float(), W, d ** -0.5)
+    q, k, v, w = (t.to(DEV) for t in (Q, K, V, W))
+    got = fwd_conv_attn_inference(q, k, v, w, splits, d ** -0.5, c_q - 1, (c_k - 1) // 2, False)
+    want = ops.decode(q, k, v, w, splits, d ** -0.5)[:3]
+    for a, b, o in zip(got, want, ref):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        # sums of at most 1100 fp32 terms in another order; the oracle's own products are rounded once more
+        assert float((a - b).abs().max()) <= 1e-5 * max(1.0, float(b.abs().max()))
+        assert float((a.cpu() - o).abs().max()) <= 2e-2 * max(1.0, float(o.abs().max()))
+    bf = ops.decode_whole(q, k, v, w, splits, d ** -0.5, out_dtype=torch.bfloat16)
+    assert bf[0].dtype == torch.bfloat16 and torch.equal(bf[0], got[0].to(torch.bfloat16))
+
+
+def test_views_causal_and_refused_counts():
+    Q, K, V, W = _case(2, 2, 6, 300, 64, 6, 11, seed=1)
+    q, w = Q.to(DEV), W.to(DEV)
+    room = torch.empty(2, 2, 2, 512, 64, dtype=torch.bfloat16, device=DEV)
+    room[0, :, :, :300], room[1, :, :, :300] = K.to(DEV), V.to(DEV)
+    k, v = room[0, :, :, :300], room[1, :, :, :300]
+    for causal in (False, True):
+        got = fwd_conv_attn_inference(q, k, v, w, 4, 0.125, 5, 5, causal)
+        want = ops.decode(q, k, v, w, 4, 0.125, causal)[:3]
+        assert all(float((a - b).abs().max()) <= 1e-5 * max(1.0, float(b.abs().max())) for a, b in zip(got, want))
+    for bad in (-1, 301, 1025):
+        with pytest.raises(RuntimeError, match="k_splits"):
+            fwd_conv_attn_inference(q, k, v, w, bad, 0.125, 5, 5, False)
