@@ -630,6 +630,8 @@ hipError_t pick_cq(const Problem &p, float *part, const void *q, const void *k, 
                    void *o, float *m, float *l, hipStream_t s) {
     if (p.c_q <= 3) return launch_fwd<D, 3, TO>(p, part, q, k, v, w, o, m, l, s);
     if (p.c_q <= 6) return launch_fwd<D, 6, TO>(p, part, q, k, v, w, o, m, l, s);
+    // (7 taps in 8 slots: B2 H12 N4691 d128 7x7 281 us, in 7 266)
+    if (p.c_q <= 7) return launch_fwd<D, 7, TO>(p, part, q, k, v, w, o, m, l, s);
     if (p.c_q <= 8) return launch_fwd<D, 8, TO>(p, part, q, k, v, w, o, m, l, s);
     return launch_fwd<D, 11, TO>(p, part, q, k, v, w, o, m, l, s);
 }
@@ -643,7 +645,11 @@ template <int CQT> size_t split_bytes(const Problem &p) {
 }  // namespace
 
 size_t mfma_fwd_split_bytes(const Problem &p) {
-    return p.c_q <= 3 ? split_bytes<3>(p) : p.c_q <= 6 ? split_bytes<6>(p) : p.c_q <= 8 ? split_bytes<8>(p) : split_bytes<11>(p);
+    return p.c_q <= 3   ? split_bytes<3>(p)
+           : p.c_q <= 6 ? split_bytes<6>(p)
+           : p.c_q <= 7 ? split_bytes<7>(p)
+           : p.c_q <= 8 ? split_bytes<8>(p)
+                        : split_bytes<11>(p);
 }
 
 hipError_t mfma_fwd(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
