@@ -97,16 +97,22 @@ inline int plan_grid(const Plan &pl) { return (pl.n_wg + 7) / 8 * 8; }
 // step(1), ..: rotated, so that at a time t all workgroups are at key steps of the residue t modulo the share, i.e. at few
 // different keys (from s0 on, segments beginning anywhere, the workgroups of an XCD found 10 % of the rows of K
 // and V in its L2; rotated, 78 and 66 % of all accesses of the forward and the backward hit, B4 H16 N4096 d128).
+// `down` (long shares of the backward, score_plan): a segment that ends with its share, and does not begin with it, is
+// walked from its last step down.  The shares end at the same time, so at a time t those on the short tiles of an entry
+// are all at the step that many from the start, whatever their lengths; rotated, neighbours are two steps apart, and the
+// blocks that are written meanwhile (1 MB per step on an XCD) push the rows out of the L2.
 struct Segment {
     int b, rt, s0, s_end, rot;
+    bool down;
     __device__ __forceinline__ int len() const { return s_end - s0; }
     __device__ __forceinline__ int step(int i) const {
+        if (down) return s_end - 1 - i;
         const int s = s0 + rot + i;
         return s >= s_end ? s - (s_end - s0) : s;
     }
 };
 // the one at position x of share `id`
-__device__ __forceinline__ Segment find_segment(const Plan &pl, int id, int x) {
+__device__ __forceinline__ Segment find_segment(const Plan &pl, int id, int x, bool down) {
     const int begin = id * pl.share;
     const int end = (int)min((long long)begin + pl.share, (long long)pl.entry_len * pl.B);
     Segment sg;
@@ -120,6 +126,7 @@ __device__ __forceinline__ Segment find_segment(const Plan &pl, int id, int x) {
     int rot = (x - begin - sg.s0) % pl.share;
     rot = __builtin_amdgcn_readfirstlane(rot < 0 ? rot + pl.share : rot);
     sg.rot = rot < sg.len() ? rot : 0;
+    sg.down = down && __builtin_amdgcn_readfirstlane(x > begin && x + sg.len() == begin + pl.share) != 0;
     return sg;
 }
 

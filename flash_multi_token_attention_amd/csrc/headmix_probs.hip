@@ -56,7 +56,7 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     if (id < 0) return;
     for (int i = threadIdx.x; i < H * H; i += T::WAVES * 64) lds[T::w_off + (i / H) * T::WST + i % H] = a.W[i] * (a.scale * kLog2e);
     for (int x_pos = id * a.plan.share, x_end = (int)min((long long)x_pos + a.plan.share, (long long)a.B * a.plan.entry_len); x_pos < x_end;) {
-    const Segment sg = find_segment(a.plan, id, x_pos);
+    const Segment sg = find_segment(a.plan, id, x_pos, false);
     const int b = sg.b, rt = sg.rt, n_steps = sg.len();
     x_pos += n_steps;
     const int segment = __builtin_amdgcn_readfirstlane(id - a.plan.start(b, rt) / a.plan.share);

@@ -34,6 +34,12 @@ template <int H, int D> struct ScoreTile : Tile<H, 8, H == 16 ? 32 : 16> {
     // chunks (one head, 16 keys) of K or V rows in registers, and how many of them stay in flight during the mixing phase
     static constexpr int RING = H == 16 || D < 128 ? 4 : 2, AHEAD = D == 128 ? (H == 16 ? 2 : 0) : 4;
     // (B4 H16 N4096 d128: 2 / 3 / 4 chunks in flight 1.27 / 1.33 / 1.32 ms; without the two orders of scores and mix 1.34)
+    // Key steps ahead of its use that a step's K and V are asked for, a dword of each 128-byte line, so that the fragment loads
+    // find them in the L2: the workgroups of an XCD walk the same keys in step, so all of them wait for each of its misses
+    // (a fragment load comes two chunks ahead, and the memory takes a whole step under the stores of the blocks).  The
+    // workgroups of an XCD take the heads in turn; a value is dropped two steps later, when it has arrived.
+    // B4 H16 N4096 d128, us: none 1231, 3 steps 1100, 6 steps 1095.
+    static constexpr int ASK = 6;
     static_assert(SPW * B::KB % RING == 0, "a chunk's registers are the same in every step");
 };
 
@@ -47,7 +53,8 @@ struct ScoreArgs {
     float *dw_part;      // [n_wg][H][H], or null
 };
 
-template <int H, int D>
+// AHEAD: K and V are asked for ahead of their use, and short tiles walked down (score_ahead)
+template <int H, int D, bool AHEAD>
 __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_kernel(ScoreArgs a) {
     using T = ScoreTile<H, D>;
     constexpr int RB = T::RB, R = T::R, KT = T::KT, KB = T::KB, NQ = T::NQ, RW = T::RW, HS = T::HS, DP = T::DP, SPW = T::SPW,
@@ -74,7 +81,7 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         for (int y = 0; y < HB; ++y) acc_w[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
     for (int x_pos = id * a.plan.share, x_end = (int)min((long long)x_pos + a.plan.share, (long long)a.B * a.plan.entry_len); x_pos < x_end;) {
-    const Segment sg = find_segment(a.plan, id, x_pos);
+    const Segment sg = find_segment(a.plan, id, x_pos, AHEAD);
     const int b = sg.b, rt = sg.rt, n_steps = sg.len();
     x_pos += n_steps;
     int lane = lane_id;
@@ -263,7 +270,17 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         // this one, so that one's LDS and vector work runs under the other's products.
         scores(lds, sg.step(0), later(1));
         lds_barrier();
+        unsigned asked[2] = {0, 0};
         for (int u = 0; u < n_steps; ++u) {
+            if constexpr (AHEAD) {
+                if (wave == 0) {
+                    static_assert(H == 16 && KB * KS * 8 == 32, "a line of a head's K or V per lane");
+                    const size_t tile = ((size_t)b * H + (blockIdx.x >> 3) % H) * n_t16 + later(u + T::ASK);
+                    asm volatile("" ::"v"(asked[0]));
+                    asked[0] = asked[1];
+                    asked[1] = *reinterpret_cast<const unsigned *>((lane < 32 ? a.KF : a.VF) + tile * KS * 512 + lane % 32 * 64);
+                }
+            }
             float *cur = lds + (u & 1) * H * HS, *nxt = lds + ((u + 1) & 1) * H * HS;
             const bool first = wave < T::WAVES / 2, more = u + 1 < n_steps;
             const int next = later(u + 1), ahead = later(u + 2);
@@ -486,6 +503,11 @@ __global__ __launch_bounds__(KV_WAVES * 64, 2) void headmix_products_kernel(Prob
 Plan score_plan(int B, int H, int N, int causal) {
     return H == 16 ? make_plan<ScoreTile<16, 32>>(B, N, causal) : make_plan<ScoreTile<32, 32>>(B, N, causal);
 }
+// Asking ahead pays where a workgroup has many steps: us without and with it, B4 N4096 (258 steps) 1231 / 1098, B4 N3700 (210)
+// 995 / 974, B8 N2048 (130) 634 / 596; B3 N3000 (105) 472 / 482, B1 N2500 non-causal (49) 217 / 215, B2 N3000 (70) 305 / 312;
+// non-causal B2 N3900 (233) 1077 / 1055, B1 N4096 (128) 518 / 534.  d = 64, whose loads have more chunks in flight, and 32 heads,
+// whose steps take longer, gain nothing.
+bool score_ahead(const Problem &p, const Plan &plan) { return p.H == 16 && p.d == 128 && plan.share > 128; }
 
 // What precedes the score kernel, in one launch: K and V in fragment order, then D and LSE of the rows.
 template <int D, typename TO>
@@ -513,14 +535,14 @@ hipError_t launch_prepare(const Problem &p, int o_dt, const void *k, const void 
     return hipGetLastError();
 }
 
-template <int H, int D>
+template <int H, int D, bool AHEAD = false>
 hipError_t launch_scores(const ScoreArgs &a, hipStream_t s) {
     constexpr int lds = ScoreTile<H, D>::lds;
     static_assert(ScoreTile<H, D>::WAVES * ScoreTile<H, D>::ROOM <= ScoreTile<H, D>::w_off * 4, "w stays where the rows are turned");
     static_assert(lds <= 160 * 1024 && ScoreTile<H, D>::WAVES * H * H * 4 <= lds, "LDS budget");
-    hipError_t e = set_max_lds_once<headmix_scores_kernel<H, D>>(lds);
+    hipError_t e = set_max_lds_once<headmix_scores_kernel<H, D, AHEAD>>(lds);
     if (e != hipSuccess) return e;
-    headmix_scores_kernel<H, D><<<plan_grid(a.plan), ScoreTile<H, D>::WAVES * 64, lds, s>>>(a);
+    headmix_scores_kernel<H, D, AHEAD><<<plan_grid(a.plan), ScoreTile<H, D>::WAVES * 64, lds, s>>>(a);
     return hipGetLastError();
 }
 
@@ -566,7 +588,11 @@ hipError_t headmix_bwd_fused(const Problem &p, int grad_dt, const void *q, const
                                : launch_prepare<128>(p, o_dt, k, v, o, d_o, m, l, kf, vf, Dl, lse, s);
     if (e != hipSuccess) return e;
     e = hipErrorInvalidValue;
-    if (p.H == 16) e = p.d == 32 ? launch_scores<16, 32>(a, s) : p.d == 64 ? launch_scores<16, 64>(a, s) : launch_scores<16, 128>(a, s);
+    if (p.H == 16)
+        e = p.d == 32              ? launch_scores<16, 32>(a, s)
+            : p.d == 64            ? launch_scores<16, 64>(a, s)
+            : score_ahead(p, plan) ? launch_scores<16, 128, true>(a, s)
+                                   : launch_scores<16, 128>(a, s);
     if (p.H == 32) e = p.d == 32 ? launch_scores<32, 32>(a, s) : p.d == 64 ? launch_scores<32, 64>(a, s) : launch_scores<32, 128>(a, s);
     if (e != hipSuccess) return e;
     if (want_kv && dq && dq_rows::by_keys(p, true)) {
