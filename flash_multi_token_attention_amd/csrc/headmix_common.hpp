@@ -3,7 +3,7 @@
 //
 // A workgroup owns R query rows of all heads of a batch entry and walks KT keys per step, alternating between
 // "a wave takes heads" (products of rows, bf16 MFMA) and "a wave takes rows" (the head mix as a product over the head
-// index on the fp32 MFMA); the two meet in LDS arrays [head][tile row][key].  What the tiles leave
+// index with fp32's precision); the two meet in LDS arrays [head][tile row][key].  What the tiles leave
 // (probabilities, dS) goes to global memory as bf16 blocks of 32 rows x 32 keys in the layout of the
 // product kernels, [row parity][key half][row pair][16 keys], the blocks of all heads side by side:
 // [batch][block][head].
@@ -30,6 +30,89 @@ template <typename V> __device__ __forceinline__ const V *at(const bf16_t *base,
 }
 template <typename V> __device__ __forceinline__ V *at(bf16_t *base, unsigned off) {
     return reinterpret_cast<V *>(reinterpret_cast<char *>(base) + off);
+}
+
+// The mix of 32 heads on the bf16 MFMA: every operand is the sum of three bf16 numbers, x = hi + mid + lo exactly (8 significant
+// bits each, rounded to nearest), and six of the nine products are taken; each of the others is below 2^-26 |a b|.  96 clocks for a
+// contraction over 32 heads where the fp32 MFMA takes 256; that was 60 % of the time of headmix_scores_kernel<32, 64>, whose vector ALUs
+// were 7 % busy.  B2 H32 N2048 d64, us: scores 346 -> 305, probabilities 170 -> 152; B2 H32 N1500 d32 182 -> 157 and 89 -> 82; d128 252 -> 248
+// and 119 -> 110.  log L of the forward against 64 bits: 1.59e-8 -> 1.57e-8 of its norm (N500 d64), 1.53 -> 1.48e-8 (N700 d128), its
+// gradients as before.  With 16 heads three of five clocks stay and the matrix pipe does not bind.  dw (a sum over pairs, whose operands
+// would both have to be split) stays on the fp32 MFMA: 305 us, on this one 311.
+// Infinities and NaN leave a NaN in a rest, so in every head's sum: such a step is repeated on the fp32 MFMA (has_nan).
+struct Split { bf16x8 hi, mid, lo; };
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, (bf16x2){(__bf16)a, (__bf16)b});
+}
+__device__ __forceinline__ Split split8(const float (&v)[8]) {
+#pragma clang fp contract(off)   // (a product whose rest is taken would be computed again, its factors kept)
+    u32x4 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = v[2 * i], b = v[2 * i + 1];
+        h[i] = bf16_pair(a, b);
+        a -= __uint_as_float(h[i] << 16);
+        b -= __uint_as_float(h[i] & 0xffff0000u);
+        m[i] = bf16_pair(a, b);
+        a -= __uint_as_float(m[i] << 16);
+        b -= __uint_as_float(m[i] & 0xffff0000u);
+        l[i] = bf16_pair(a, b);
+    }
+    return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+// The split of a 32 x 32 matrix in LDS as A operands [hi, mid, lo][16 rows][lane][8]: lane (g, n) row n, k slot 4y + s of its eight = column
+// 16y + 4g + s, the heads of the fp32 path's accumulators
+constexpr int kSplitBytes = 3 * 2 * 64 * 16;
+__device__ __forceinline__ void put_split(void *dst, int row, int col, float v) {
+    unsigned short *p = static_cast<unsigned short *>(dst) + ((row >> 4) * 64 + ((col >> 2) & 3) * 16 + (row & 15)) * 8 + (col >> 4) * 4 + (col & 3);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+        const unsigned u = bf16_pair(v, 0.f) & 0xffffu;
+        p[part * 1024] = (unsigned short)u;
+        v -= __uint_as_float(u << 16);
+    }
+}
+template <int HB> __device__ __forceinline__ bool has_nan(const f32x4 (&z)[HB][4]) {
+    bool nan = false;
+#pragma unroll
+    for (int x = 0; x < HB; ++x)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) nan |= __builtin_isunordered(z[x][t][0], z[x][t][1]) | __builtin_isunordered(z[x][t][2], z[x][t][3]);
+    return __any(nan);
+}
+// c[x][u] += A_x B_u for both 16 rows x of the matrix at `a`, the small products first.  (A part of the matrix is read when its
+// products are due: registers are short.)
+template <int U>
+__device__ __forceinline__ void mfma_split(f32x4 *const (&c)[2], const void *a, int lane, const Split (&b)[U]) {
+    const bf16x8 *p = static_cast<const bf16x8 *>(a) + lane;
+#pragma unroll
+    for (int part = 2; part >= 0; --part) {
+        asm volatile("" ::: "memory");
+        const bf16x8 w[2] = {p[part * 128], p[part * 128 + 64]};
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (part == 0) c[x][u] = mfma_bf16(w[x], b[u].lo, c[x][u]);
+                if (part <= 1) c[x][u] = mfma_bf16(w[x], b[u].mid, c[x][u]);
+                c[x][u] = mfma_bf16(w[x], b[u].hi, c[x][u]);
+            }
+    }
+}
+
+// z[x][t] += (the 32 x 32 matrix in `w`) S for the keys t of the lane's tile row, the heads in the order of put_split
+template <typename T>
+__device__ __forceinline__ void mix_split(f32x4 (&z)[T::HB][4], const float *S, int pos, int g, const void *w, int lane) {
+#pragma unroll
+    for (int t = 0; t < 4; t += 2) {   // (two keys at a time; four: 314 us where this is 305, one: 319, the matrix is read more often)
+        float2 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const float2 *>(S + (16 * (i >> 2) + 4 * g + (i & 3)) * T::HS + pos + t);
+        const Split sp[2] = {split8({v[0].x, v[1].x, v[2].x, v[3].x, v[4].x, v[5].x, v[6].x, v[7].x}),
+                             split8({v[0].y, v[1].y, v[2].y, v[3].y, v[4].y, v[5].y, v[6].y, v[7].y})};
+        mfma_split<2>({&z[0][t], &z[T::HB - 1][t]}, w, lane, sp);
+    }
 }
 
 constexpr int kBlock = kChainRows * kChainKeys;   // elements of a block

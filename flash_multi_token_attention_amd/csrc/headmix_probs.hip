@@ -30,7 +30,8 @@ constexpr float kFloor = -126.f;    // blocks whose scores are all below this, r
 template <int H, int D> struct ProbTile : Tile<H, H == 16 ? 16 : 8, H == 16 ? 32 : 16> {
     using B = Tile<H, H == 16 ? 16 : 8, H == 16 ? 32 : 16>;
     static constexpr int ROOM = B::R * (D * 2 + 16);        // a head's rows while they are turned
-    static constexpr int w_off = 2 * B::arr * 4 > B::WAVES * ROOM ? 2 * B::arr : B::WAVES * ROOM / 4, lds = (w_off + H * B::WST) * 4;
+    static constexpr int w_off = 2 * B::arr * 4 > B::WAVES * ROOM ? 2 * B::arr : B::WAVES * ROOM / 4, sp_off = w_off + H * B::WST,
+                         lds = sp_off * 4 + (H == 32 ? kSplitBytes : 0);   // (H = 32: the split of w behind it)
 };
 
 struct ProbArgs {
@@ -54,7 +55,11 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane_id = threadIdx.x & 63;
     const int id = share_of_workgroup(a.plan), N = a.N, h0 = wave * HPW;
     if (id < 0) return;
-    for (int i = threadIdx.x; i < H * H; i += T::WAVES * 64) lds[T::w_off + (i / H) * T::WST + i % H] = a.W[i] * (a.scale * kLog2e);
+    for (int i = threadIdx.x; i < H * H; i += T::WAVES * 64) {
+        const float w = a.W[i] * (a.scale * kLog2e);
+        lds[T::w_off + (i / H) * T::WST + i % H] = w;
+        if constexpr (H == 32) put_split(lds + T::sp_off, i / H, i % H, w);
+    }
     for (int x_pos = id * a.plan.share, x_end = (int)min((long long)x_pos + a.plan.share, (long long)a.B * a.plan.entry_len); x_pos < x_end;) {
     const Segment sg = find_segment(a.plan, id, x_pos, false);
     const int b = sg.b, rt = sg.rt, n_steps = sg.len();
@@ -111,23 +116,37 @@ __global__ __launch_bounds__((ProbTile<H, D>::WAVES * 64)) void headmix_probs_ke
     }
     // (z starts at from[]: the negative references of the lane's row)
     auto mix = [&](f32x4 (&z)[HB][4], const f32x4 (&from)[HB], const float *S, int step) {
+        auto start = [&] {
 #pragma unroll
-        for (int x = 0; x < HB; ++x)
+            for (int x = 0; x < HB; ++x)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) z[x][t] = from[x];
+                for (int t = 0; t < 4; ++t) z[x][t] = from[x];
+        };
+        auto mix_fp32 = [&] {
 #pragma unroll
-        for (int y = 0; y < HB; ++y) {
-            f32x4 wf[HB];
+            for (int y = 0; y < HB; ++y) {
+                f32x4 wf[HB];
 #pragma unroll
-            for (int x = 0; x < HB; ++x) wf[x] = *reinterpret_cast<const f32x4 *>(wf_l + 16 * x * T::WST + 16 * y);
+                for (int x = 0; x < HB; ++x) wf[x] = *reinterpret_cast<const f32x4 *>(wf_l + 16 * x * T::WST + 16 * y);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(S + (16 * y + 4 * g + s) * HS + pos);
+                for (int s = 0; s < 4; ++s) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(S + (16 * y + 4 * g + s) * HS + pos);
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
+                    for (int t = 0; t < 4; ++t)
 #pragma unroll
-                    for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
+                        for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
+                }
             }
+        };
+        start();
+        if constexpr (H == 32) {
+            mix_split<T>(z, S, pos, g, lds + T::sp_off, lane);
+            if (has_nan(z)) {
+                start();
+                mix_fp32();
+            }
+        } else {
+            mix_fp32();
         }
         // masks only where a key of the tile is past the tile's first row or past the last key
         if ((a.causal && step * KT + KT - 1 > i0) || step * KT + KT > N) {

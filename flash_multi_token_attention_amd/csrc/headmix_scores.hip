@@ -30,7 +30,8 @@ template <int H, int D> struct ScoreTile : Tile<H, 8, H == 16 ? 32 : 16> {
     static constexpr int DP = B::R * B::KT, HS = 2 * DP + 4, NBUF = H == 16 ? 2 : 1;
     static constexpr bool STATS_LDS = D >= 64;               // LSE and D of the tile rows: registers are short
     static constexpr int w_off = NBUF * H * HS, wt_off = w_off + H * B::WST, st_off = wt_off + H * B::WST,
-                         used = (st_off + (STATS_LDS ? 2 * B::R * B::WST : 0)) * 4, lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
+                         sp_off = st_off + (STATS_LDS ? 2 * B::R * B::WST : 0),   // H = 32: the split of w and its transpose
+                         used = sp_off * 4 + (H == 32 ? 2 * kSplitBytes : 0), lds = used > B::WAVES * ROOM ? used : B::WAVES * ROOM;
     // chunks (one head, 16 keys) of K or V rows in registers, and how many of them stay in flight during the mixing phase
     static constexpr int RING = H == 16 || D < 128 ? 4 : 2, AHEAD = D == 128 ? (H == 16 ? 2 : 0) : 4;
     // (B4 H16 N4096 d128: 2 / 3 / 4 chunks in flight 1.27 / 1.33 / 1.32 ms; without the two orders of scores and mix 1.34)
@@ -73,6 +74,10 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         const float w = a.W[i];
         lds[T::w_off + (i / H) * T::WST + i % H] = w * (a.scale * kLog2e);
         lds[T::wt_off + (i % H) * T::WST + i / H] = w * a.scale;
+        if constexpr (H == 32) {
+            put_split(lds + T::sp_off, i / H, i % H, w * (a.scale * kLog2e));
+            put_split(smem + T::sp_off * 4 + kSplitBytes, i % H, i / H, w * a.scale);
+        }
     }
     f32x4 acc_w[HB][HB];
 #pragma unroll
@@ -149,26 +154,40 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
         float *dP = S + DP;
         const int j0 = step * KT;
         f32x4 z[HB][4];   // starting at -LSE
+        auto start = [&] {
 #pragma unroll
-        for (int x = 0; x < HB; ++x) {
-            f32x4 nlse = lse_r[x];
-            if constexpr (T::STATS_LDS) nlse = *reinterpret_cast<const f32x4 *>(st_l + lr * T::WST + 16 * x + 4 * g);
+            for (int x = 0; x < HB; ++x) {
+                f32x4 nlse = lse_r[x];
+                if constexpr (T::STATS_LDS) nlse = *reinterpret_cast<const f32x4 *>(st_l + lr * T::WST + 16 * x + 4 * g);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) z[x][t] = nlse;
-        }
-#pragma unroll
-        for (int y = 0; y < HB; ++y) {
-            f32x4 wf[HB];
-#pragma unroll
-            for (int x = 0; x < HB; ++x) wf[x] = *reinterpret_cast<const f32x4 *>(wf_l + 16 * x * T::WST + 16 * y);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(S + (16 * y + 4 * g + s) * HS + pos);
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
+                for (int t = 0; t < 4; ++t) z[x][t] = nlse;
             }
+        };
+        auto mix_fp32 = [&] {
+#pragma unroll
+            for (int y = 0; y < HB; ++y) {
+                f32x4 wf[HB];
+#pragma unroll
+                for (int x = 0; x < HB; ++x) wf[x] = *reinterpret_cast<const f32x4 *>(wf_l + 16 * x * T::WST + 16 * y);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(S + (16 * y + 4 * g + s) * HS + pos);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int x = 0; x < HB; ++x) z[x][t] = mfma4(wf[x][s], v[t], z[x][t]);
+                }
+            }
+        };
+        start();
+        if constexpr (H == 32) {
+            mix_split<T>(z, S, pos, g, lds + T::sp_off, lane);
+            if (has_nan(z)) {
+                start();
+                mix_fp32();
+            }
+        } else {
+            mix_fp32();
         }
         // masks only where a key of the tile is past the tile's first row or past the last key
         if ((a.causal && j0 + KT - 1 > i0) || j0 + KT > N) {
@@ -208,27 +227,54 @@ __global__ __launch_bounds__((ScoreTile<H, D>::WAVES * 64)) void headmix_scores_
                 __builtin_nontemporal_store(__builtin_bit_cast(u32x2, pb), at<u32x2>(p_out, out + (16 * x + r) * SC_BLK * 2));
             }
         }
+        f32x4 ds[HB][4];
+        auto dmix_fp32 = [&] {
 #pragma unroll
-        for (int x = 0; x < HB; ++x) {
-            f32x4 ds[4];
+            for (int x = 0; x < HB; ++x) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) ds[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < 4; ++t) ds[x][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int y = 0; y < HB; ++y) {
-                const f32x4 wb = *reinterpret_cast<const f32x4 *>(wb_l + 16 * x * T::WST + 16 * y);
+                for (int y = 0; y < HB; ++y) {
+                    const f32x4 wb = *reinterpret_cast<const f32x4 *>(wb_l + 16 * x * T::WST + 16 * y);
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
+                    for (int s = 0; s < 4; ++s)
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) ds[t] = mfma4(wb[s], z[y][t][s], ds[t]);
+                        for (int t = 0; t < 4; ++t) ds[x][t] = mfma4(wb[s], z[y][t][s], ds[x][t]);
+                }
             }
+        };
+        if constexpr (H == 32) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {   // (a key at a time: two took up to 16 registers that are not there)
+                const f32x4 z0 = z[0][t], z1 = z[HB - 1][t];
+                const Split sp[1] = {split8({z0[0], z0[1], z0[2], z0[3], z1[0], z1[1], z1[2], z1[3]})};
+                ds[0][t] = ds[HB - 1][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                mfma_split<1>({&ds[0][t], &ds[HB - 1][t]}, smem + T::sp_off * 4 + kSplitBytes, lane, sp);
+            }
+            if (has_nan(ds)) {
+                asm volatile("" ::: "memory");   // (dZ from where it was put: kept in registers it would be in everyone's way)
+#pragma unroll
+                for (int x = 0; x < HB; ++x)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const f32x4 dz = *reinterpret_cast<const f32x4 *>(dP + (16 * x + 4 * g + r) * HS + pos);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) z[x][t][r] = dz[t];
+                    }
+                dmix_fp32();
+            }
+        } else {
+            dmix_fp32();
+        }
+#pragma unroll
+        for (int x = 0; x < HB; ++x)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 bf16x4 db;
 #pragma unroll
-                for (int t = 0; t < 4; ++t) db[t] = (bf16_t)ds[t][r];
+                for (int t = 0; t < 4; ++t) db[t] = (bf16_t)ds[x][t][r];
                 __builtin_nontemporal_store(__builtin_bit_cast(u32x2, db), at<u32x2>(ds_out, out + (16 * x + r) * SC_BLK * 2));
             }
-        }
         // dw += dZ S^T over the wave's own 64 pairs: lane n = head of either operand
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
