@@ -13,12 +13,14 @@
 // All operands, scores and sums are fp32, dW is summed in a fixed order, nothing is added with atomics.  The matrices take
 // 4 bytes per pair (forward one, backward three of them; the whole square under the causal mask too).  Above the caller's
 // workspace limit the Python ops run them by groups of heads; the other kernels run where one head does not fit.
-#include "mfma_common.hpp"
+#include "reduce_common.hpp"
 
 namespace convattn {
 namespace {
 
 constexpr int NT = 256, TT = 64;                 // threads; rows and keys of a tile
+constexpr int KC = 64;                           // columns of Q and K that a tile stages at a time: four workgroups per CU at d = 128 too
+                                                 // (whole rows, two: B1 H8 N1024 d128 6x11 backward 99 -> 83 us, forward 60 -> 49)
 
 struct StArgs {
     Problem p;
@@ -33,12 +35,12 @@ __device__ __forceinline__ f32x4 load4(const bf16_t *p) {
     const bf16x4 v = *reinterpret_cast<const bf16x4 *>(p);
     return (f32x4){(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
 }
-__device__ __forceinline__ int round16(int d) { return (d + 15) & ~15; }
+__host__ __device__ inline int round16(int d) { return (d + 15) & ~15; }
 
-// dst[r][0 .. round16(d)) = row row0 + r of src for r < rows; zeros outside [0, N) and past d
+// dst[r][0 .. width) = columns col0 .. of row row0 + r of src for r < rows; zeros outside [0, N) and past d
 template <typename TI>
-__device__ __forceinline__ void stage_rows(float *dst, int st, const TI *__restrict__ src, int row0, int rows, int N, int d) {
-    const int q = round16(d) / 4;
+__device__ __forceinline__ void stage_rows(float *dst, int st, const TI *__restrict__ src, int row0, int rows, int N, int d, int col0, int width) {
+    const int q = width / 4;
     constexpr int U = 8;   // loads in flight per thread
     if (NT % q == 0) {
         const int c = (threadIdx.x % q) * 4, step = NT / q;
@@ -48,7 +50,7 @@ __device__ __forceinline__ void stage_rows(float *dst, int st, const TI *__restr
             for (int u = 0; u < U; ++u) {
                 const int g = row0 + r + u * step;
                 v[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                if (r + u * step < rows && g >= 0 && g < N && c < d) v[u] = load4(src + (size_t)g * d + c);
+                if (r + u * step < rows && g >= 0 && g < N && col0 + c < d) v[u] = load4(src + (size_t)g * d + col0 + c);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -59,7 +61,7 @@ __device__ __forceinline__ void stage_rows(float *dst, int st, const TI *__restr
     for (int i = threadIdx.x; i < rows * q; i += NT) {
         const int r = i / q, c = (i - r * q) * 4, g = row0 + r;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (g >= 0 && g < N && c < d) v = load4(src + (size_t)g * d + c);
+        if (g >= 0 && g < N && col0 + c < d) v = load4(src + (size_t)g * d + col0 + c);
         *reinterpret_cast<f32x4 *>(dst + r * st + c) = v;
     }
 }
@@ -255,7 +257,7 @@ __device__ __forceinline__ void tile_dw_any(float *__restrict__ part, float *red
     }
 }
 
-// LDS of window_kernel: rows of Q and K, then in their place dP / dC (backward), the sums of dW and the score tile with its halo.
+// LDS of window_kernel: KC columns of the rows of Q and K, then in their place dP / dC (backward), the sums of dW and the score tile with its halo.
 // (The score tile beside the rows, and rows of dO and V staged as well, took 60 KB at d = 64: two workgroups per CU, and one at
 // d = 128.  Now 39: B1 H8 N1024 d64 6x11 backward 73 -> 58 us, forward 42 -> 36.)
 struct WinLds {
@@ -263,7 +265,7 @@ struct WinLds {
 };
 __host__ __device__ inline WinLds win_lds(const Problem &p, bool bwd) {
     WinLds l;
-    l.dst = ((p.d + 15) & ~15) + 4;
+    l.dst = (round16(p.d) < KC ? round16(p.d) : KC) + 4;
     // a patch reads whole 16-byte quantities: columns 60 .. 60 + c_k + 3 rounded up
     l.sst = TT - 4 + ((p.c_k + 3 + 3) & ~3);
     l.w_f = 0;                                            // window
@@ -300,21 +302,26 @@ __global__ __launch_bounds__(NT, 4) void window_kernel(StArgs a, const TI *__res
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
 
     stage_window<false>(Ws, W + (size_t)h * p.c_q * p.c_k, p.c_q, p.c_k);
-    stage_rows(Qs, L.dst, Q + bh * p.Nq * d, r0 - pq, nr, p.Nq, d);
-    stage_rows(Ks, L.dst, K + bh * p.Nk * d, c0 - pk, nc, p.Nk, d);
-    __syncthreads();
     // score blocks of 16 rows x 32 keys, held until the rows have been read by everyone
     constexpr int HELD = 4;   // (at most 5 x 3 blocks for four waves)
     const int nrb = (nr + 15) / 16, ncb = (nc + 15) / 16, ncp = (ncb + 1) / 2;
     f32x4 sc[HELD][2];
 #pragma unroll
-    for (int x = 0; x < HELD; ++x) {
-        const int it = wave + x * (NT / 64);
-        if (it < nrb * ncp) {
-            const int rb = it / ncp, cb = (it - rb * ncp) * 2;
-            sc[x][0] = sc[x][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-            const float *bp[2] = {Ks + min(cb * 16 + n, nc - 1) * L.dst + 4 * g, Ks + min(cb * 16 + 16 + n, nc - 1) * L.dst + 4 * g};
-            mma_nt<2>(sc[x], Qs + min(rb * 16 + n, nr - 1) * L.dst + 4 * g, bp, Kd);
+    for (int x = 0; x < HELD; ++x) sc[x][0] = sc[x][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < Kd; k0 += KC) {
+        const int width = min(KC, Kd - k0);
+        if (k0) __syncthreads();
+        stage_rows(Qs, L.dst, Q + bh * p.Nq * d, r0 - pq, nr, p.Nq, d, k0, width);
+        stage_rows(Ks, L.dst, K + bh * p.Nk * d, c0 - pk, nc, p.Nk, d, k0, width);
+        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < HELD; ++x) {
+            const int it = wave + x * (NT / 64);
+            if (it < nrb * ncp) {
+                const int rb = it / ncp, cb = (it - rb * ncp) * 2;
+                const float *bp[2] = {Ks + min(cb * 16 + n, nc - 1) * L.dst + 4 * g, Ks + min(cb * 16 + 16 + n, nc - 1) * L.dst + 4 * g};
+                mma_nt<2>(sc[x], Qs + min(rb * 16 + n, nr - 1) * L.dst + 4 * g, bp, width);
+            }
         }
     }
     f32x4 dp_acc[4];
@@ -467,17 +474,19 @@ __global__ __launch_bounds__(NT, 5) void unwindow_kernel(StArgs a, const float *
     }
 }
 
-// Products with a score-sized matrix X [rows][keys]: 32 rows (or keys) x d per workgroup of 8 waves, 128 of the contraction per
+// Products with a score-sized matrix X [rows][keys]: 32 rows (or keys) x d per workgroup of 8 waves, 64 of the contraction per
 // step:
 //   KIND 0: O = exp(C - M) V / L (also M, L)      1: dQ = scale dS K       (X as it lies)
 //   KIND 2: dV = P^T dO                           3: dK = scale dS^T Q     (X turned)
 // A wave has 16 rows of the result, all of d and one quarter of each step, the quarters are added at the end: a short sequence
 // has few row tiles, and the longest walk is the launch (B1 H8 N1024 d64 forward: 64 rows and steps of 32 37 us, 32 rows and
 // steps of 64 22 us).  The next step's operands are loaded into registers under this one's products.
-constexpr int PM = 32, PKS = 128, PNT = 512;
+// Steps of 64 instead of 128 leave room for more workgroups per CU (d = 64 three -> four, d = 128 one -> two): backward B1 H8 N2048 d64 98 -> 86 us,
+// B1 H8 N1024 d128 64 -> 48 (both with the order of bwd_product_kernel), forward of the latter 32 -> 30.
+constexpr int PM = 32, PKS = 64, PNT = 512;
 template <int DBLK> struct ProdLds {
-    static constexpr int BST = DBLK * 16 + 4, AST = PKS + 4, TST = PM + 4;
-    static constexpr int a_f = PM * AST > PKS * TST ? PM * AST : PKS * TST, total_f = a_f + PKS * BST;
+    static constexpr int BST = DBLK * 16 + 4, AST = PKS + 4, TST = PM + 4, hand_f = 3 * 2 * DBLK * 64 * 4;
+    static constexpr int a_f = PM * AST > PKS * TST ? PM * AST : PKS * TST, total_f = a_f + (PKS * BST > hand_f ? PKS * BST : hand_f);
 };
 template <int KIND, int DBLK, typename TI, typename TO>
 __device__ __forceinline__ void product(const StArgs &a, float *lds, size_t bh, int mt, const float *__restrict__ X, const TI *__restrict__ Y,
@@ -495,8 +504,8 @@ __device__ __forceinline__ void product(const StArgs &a, float *lds, size_t bh, 
     const TI *Yb = Y + bh * NK * d;
     float *As = lds, *Bs = lds + T::a_f;
 
-    // staging: A as it lies: row tid / 16, columns 8 (tid % 16) ..; turned: rows tid / 8 and + 64, columns 4 (tid % 8) ..
-    const int ar = TURN ? tid >> 3 : tid >> 4, ac = TURN ? 4 * (tid & 7) : 8 * (tid & 15);
+    // staging: A as it lies: row tid / 16, columns 4 (tid % 16) ..; turned: row tid / 8, columns 4 (tid % 8) ..
+    const int ar = TURN ? tid >> 3 : tid >> 4, ac = TURN ? 4 * (tid & 7) : 4 * (tid & 15);
     constexpr int BQ = PKS * DBLK * 4 / PNT;          // 16-byte quantities of Y per thread
     float mrow = 0.f, lsum = 0.f;
     if constexpr (KIND == 0) {
@@ -506,20 +515,17 @@ __device__ __forceinline__ void product(const StArgs &a, float *lds, size_t bh, 
 #pragma unroll
         for (int s = 8; s > 0; s >>= 1) mrow = fmaxf(mrow, __shfl_xor(mrow, s, 16));
     }
-    f32x4 xa[2], yb[BQ];
+    f32x4 xa, yb[BQ];
     auto load = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            if constexpr (TURN) {
-                const int row = k0 + ar + 64 * i;
-                xa[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                if (row < p.Nq) xa[i] = *reinterpret_cast<const f32x4 *>(Xb + (size_t)row * a.ld + m0 + ac);
-            } else {
-                // (a step may end past the row's last written tile, or past the matrix: -inf and 0 there)
-                const int key = k0 + ac + 4 * i;
-                xa[i] = KIND == 0 ? (f32x4){kNegInf, kNegInf, kNegInf, kNegInf} : (f32x4){0.f, 0.f, 0.f, 0.f};
-                if (key < x_end) xa[i] = *reinterpret_cast<const f32x4 *>(Xb + (size_t)min(m0 + ar, p.Nq - 1) * a.ld + key);
-            }
+        if constexpr (TURN) {
+            const int row = k0 + ar;
+            xa = (f32x4){0.f, 0.f, 0.f, 0.f};
+            if (row < p.Nq) xa = *reinterpret_cast<const f32x4 *>(Xb + (size_t)row * a.ld + m0 + ac);
+        } else {
+            // (a step may end past the row's last written tile, or past the matrix: -inf and 0 there)
+            const int key = k0 + ac;
+            xa = KIND == 0 ? (f32x4){kNegInf, kNegInf, kNegInf, kNegInf} : (f32x4){0.f, 0.f, 0.f, 0.f};
+            if (key < x_end) xa = *reinterpret_cast<const f32x4 *>(Xb + (size_t)min(m0 + ar, p.Nq - 1) * a.ld + key);
         }
 #pragma unroll
         for (int i = 0; i < BQ; ++i) {
@@ -535,16 +541,12 @@ __device__ __forceinline__ void product(const StArgs &a, float *lds, size_t bh, 
     for (int k0 = k_begin; k0 < k_end; k0 += PKS) {
         if constexpr (KIND == 0) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    xa[i][e] = __expf(xa[i][e] - mrow);
-                    lsum += xa[i][e];
-                }
+            for (int e = 0; e < 4; ++e) {
+                xa[e] = __expf(xa[e] - mrow);
+                lsum += xa[e];
+            }
         }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            *reinterpret_cast<f32x4 *>(As + (TURN ? (ar + 64 * i) * T::TST + ac : ar * T::AST + ac + 4 * i)) = xa[i];
+        *reinterpret_cast<f32x4 *>(As + ar * (TURN ? T::TST : T::AST) + ac) = xa;
 #pragma unroll
         for (int i = 0; i < BQ; ++i) {
             const int q = tid + i * PNT, r = q / (DBLK * 4), c = (q - r * (DBLK * 4)) * 4;
@@ -607,18 +609,30 @@ __global__ __launch_bounds__(PNT) void fwd_product_kernel(StArgs a, const TI *__
     __shared__ __attribute__((aligned(16))) float lds[ProdLds<DBLK>::total_f];
     product<0, DBLK, TI, TO>(a, lds, blockIdx.x, gridDim.y - 1 - blockIdx.y, a.c, V, O, M, L);   // longest (causal) tiles first
 }
+// y = the products that are wanted, z = row or key tiles: the workgroups of all products come in the order of their length under
+// the causal mask, the longest first (one product after the other B1 H8 N1024 d64 took 37 us, in this order 27).  The z behind the tiles
+// sum dW's partials (x = head): a launch of their own took 5 us of the 162 of that shape's training step.  At d = 128 held to two workgroups
+// per CU (126 registers instead of 138; 2 and 1 per CU: B1 H8 N2048 161 and 182 us, N1024 48 and 52, B1 H2 N2000, of 378 workgroups, 65 and 54).
 template <int DBLK, typename TI, typename TO>
-__global__ __launch_bounds__(PNT) void bwd_product_kernel(StArgs a, const TI *__restrict__ Q, const TI *__restrict__ K, const TI *__restrict__ dO,
-                                                         TO *__restrict__ dQ, TO *__restrict__ dK, TO *__restrict__ dV) {
+__global__ __launch_bounds__(PNT, 4) void bwd_product_kernel(StArgs a, const TI *__restrict__ Q, const TI *__restrict__ K, const TI *__restrict__ dO,
+                                                         TO *__restrict__ dQ, TO *__restrict__ dK, TO *__restrict__ dV, int n_tiles,
+                                                         const float *__restrict__ dw_part, float *__restrict__ dW) {
     __shared__ __attribute__((aligned(16))) float lds[ProdLds<DBLK>::total_f];
-    const int t = blockIdx.y, which = blockIdx.z + (dQ ? 0 : 1);
-    if (which == 0) {
-        const int rows = (a.p.Nq + PM - 1) / PM;
+    static_assert(ProdLds<DBLK>::total_f >= kDwChains * 64, "room for the dW chains");
+    const int t = blockIdx.z, which = blockIdx.y + (dQ ? 0 : 1), rows = (a.p.Nq + PM - 1) / PM, keys = (a.p.Nk + PM - 1) / PM;
+    if (t >= max(rows, keys)) {
+        const int ntap = a.p.c_q * a.p.c_k;
+        if (blockIdx.y != 0 || (int)blockIdx.x >= a.p.H) return;
+        for (int ty = t - max(rows, keys); ty * 64 < ntap; ty += gridDim.z - max(rows, keys)) {
+            dw_reduce_block<PNT>(a.p.B, a.p.H, n_tiles, ntap, dw_part, dW, blockIdx.x, ty, reinterpret_cast<float (*)[64]>(lds));
+            __syncthreads();
+        }
+    } else if (which == 0) {
         if (t < rows) product<1, DBLK, TI, TO>(a, lds, blockIdx.x, rows - 1 - t, a.ds, K, dQ, nullptr, nullptr);
     } else if (which == 1) {
-        if (t * PM < a.p.Nk) product<2, DBLK, TI, TO>(a, lds, blockIdx.x, t, a.pm, dO, dV, nullptr, nullptr);
+        if (t < keys) product<2, DBLK, TI, TO>(a, lds, blockIdx.x, t, a.pm, dO, dV, nullptr, nullptr);
     } else {
-        if (t * PM < a.p.Nk) product<3, DBLK, TI, TO>(a, lds, blockIdx.x, t, a.ds, Q, dK, nullptr, nullptr);
+        if (t < keys) product<3, DBLK, TI, TO>(a, lds, blockIdx.x, t, a.ds, Q, dK, nullptr, nullptr);
     }
 }
 
@@ -699,13 +713,17 @@ static hipError_t run_bwd(StArgs a, const void *q, const void *k, const void *v,
     e = set_max_lds_once<unwindow_kernel>((int)kLdsBytes);
     if (e != hipSuccess) return e;
     const unsigned BH = (unsigned)(a.p.B * a.p.H);
-    unwindow_kernel<<<dim3((unsigned)(BH * dw_tiles(a))), NT, ((TT + a.p.pq) * win_lds(a.p, true).sst + a.p.c_q * win_stride(a.p.c_k)) * sizeof(float), s>>>(a, w);
-    const dim3 grid(BH, ((a.p.Nq > a.p.Nk ? a.p.Nq : a.p.Nk) + PM - 1) / PM, (dq ? 1 : 0) + (dk ? 2 : 0));
-    if (a.p.d <= 64) bwd_product_kernel<4, TI, TO><<<grid, PNT, 0, s>>>(a, (const TI *)q, (const TI *)k, (const TI *)d_o, (TO *)dq, (TO *)dk, (TO *)dv);
-    else bwd_product_kernel<8, TI, TO><<<grid, PNT, 0, s>>>(a, (const TI *)q, (const TI *)k, (const TI *)d_o, (TO *)dq, (TO *)dk, (TO *)dv);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return dw ? dw_reduce(a.p, (int)dw_tiles(a), part, dw, s) : hipSuccess;
+    const int n_tiles = (int)dw_tiles(a);
+    unwindow_kernel<<<dim3(BH * n_tiles), NT, ((TT + a.p.pq) * win_lds(a.p, true).sst + a.p.c_q * win_stride(a.p.c_k)) * sizeof(float), s>>>(a, w);
+    const int tiles = ((a.p.Nq > a.p.Nk ? a.p.Nq : a.p.Nk) + PM - 1) / PM, tap_blocks = (a.p.c_q * a.p.c_k + 63) / 64;
+    const int sums = !dw ? 0 : tap_blocks < 65535 - tiles ? tap_blocks : 65535 - tiles;   // (tiles <= 65534, staged_ok)
+    const dim3 grid(BH, (dq ? 1 : 0) + (dk ? 2 : 0), tiles + sums);
+#define CALL(DB) \
+    bwd_product_kernel<DB, TI, TO><<<grid, PNT, 0, s>>>(a, (const TI *)q, (const TI *)k, (const TI *)d_o, (TO *)dq, (TO *)dk, (TO *)dv, n_tiles, part, dw)
+    if (a.p.d <= 64) CALL(4);
+    else CALL(8);
+#undef CALL
+    return hipGetLastError();
 }
 hipError_t staged_bwd(const Problem &p, int in_dt, int out_dt, const void *q, const void *k, const void *v, const void *d_o, const float *D,
                       const float *lse, const float *w, void *ws, void *dq, void *dk, void *dv, float *dw, hipStream_t s) {
