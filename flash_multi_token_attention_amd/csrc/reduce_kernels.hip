@@ -246,12 +246,13 @@ class Schedule {
 }  // namespace
 
 // Row tiles per workgroup of the split backward, or 0: one workgroup per key block.  The launch is laid out on 256 CUs for each
-// cut; in units of a row tile a workgroup costs its tiles, 8 for set-up and wind-down and 2 more where its range ends inside the
-// key block (the kernels of 7 to 11 query taps, whose tiles take longer, 4 and 1), the reduction 3 (2).  Against the unsplit
-// launch and every cut for 1 to 64 heads of 640 to 8000 rows (1205 shapes of 3x3 to 11x11 taps, d 32 to 128): 0.2 % over the best on
-// average, 1.5 % over the unsplit one at most.  (B2 H8 N1531 d64 11x11: 167 -> 109 us, B1 H8 N2048 d64 7x7:
-// 169 -> 72, B1 H8 N1000 d128 6x11: 78 -> 32; with more than two rounds of workgroups a split loses: B1 H8 N8000 d128 6x11 774 us
-// unsplit, 933 in parts, B1 H12 N5000 491 and 594.)
+// cut of the longest key block, from 1 1/4 to 8 parts; in units of a row tile a workgroup costs its tiles, 10 for set-up and wind-down and
+// 1 more where its range ends inside the key block (windows of 7 to 11 query taps, whose tiles take longer: 4 and 1 up to d = 64, 6 and
+// 2 at 128); what the reduction takes is in the margin over the unsplit launch.  Against every cut for 2 to 64 heads of 640 to
+// 8000 rows (482 shapes of 3x3 to 11x11 taps, d 32 to 128, a quarter of the last 221 not causal): 0.3 to 0.8 % over the best on
+// average (with cuts into 2, 3, 4, 6 and 8 parts only 1.9 to 2.5 %).  (B2 H8 N1531 d64 11x11, us, whole backward without D: unsplit 163,
+// into 3 parts 125, 1 1/2 parts 117; B1 H8 N2048 d64 7x7 164, 108 and, into 3 parts, 92; with more than two rounds of workgroups a split loses:
+// B1 H8 N8000 d128 6x11 774 us unsplit, 933 in parts, B1 H12 N5000 491 and 594.)
 // The limits: 12 to 19 row tiles would gain too (B1 H8 N512 d64 6x11 the whole backward 47 -> 31 us), which such calls, bound by
 // the host (75 us for a step), show in a captured graph only.  Beyond 64 heads no cut gains (5 to 45 % slower at 80 to
 // 256 heads of 640 to 4096 rows).  From 8192 rows on nothing is split, whatever the number of heads is, so that a head's results
@@ -261,21 +262,28 @@ int chain_share(const Problem &p) {
     const int n_rt = chain_row_tiles(p), n_kb = mfma_kv_tiles(p);
     const long long heads = (long long)p.B * p.H;
     if (n_rt < 20 || p.Nq >= 8192 || heads > 64 || heads * n_kb > 1024) return 0;
-    const bool wide = p.c_q > 6;
-    const float fixed = wide ? 4.f : 8.f, cut_end = wide ? 1.f : 2.f, margin = wide ? 1.f : 1.02f, reduction = wide ? 2.f : 3.f;
-    float none = 0.f, best = 0.f;
+    const bool wide = p.c_q > 6, small = p.d <= 64;
+    const float fixed = !wide ? 10.f : small ? 4.f : 6.f, cut_end = wide && !small ? 2.f : 1.f, margin = wide ? 1.04f : 1.06f;
+    const int n = (int)heads;
+    float best = 0.f, none = 0.f;
     int share = 0;
-    for (int cut = 1; cut <= 8; cut += cut < 4 ? 1 : 2) {
-        const int s = cut == 1 ? 0 : (n_rt + cut - 1) / cut;
-        if (cut > 1 && s < 6) break;
-        Schedule launch;
-        for (int kb = 0; kb < n_kb; ++kb) {
-            const int len = chain_len(p, kb) > 0 ? chain_len(p, kb) : 0, parts = chain_parts(p, kb, s);
-            launch.add((float)len / parts + fixed + (parts > 1 ? cut_end : 0.f), (int)heads * parts);
+    for (const int quarters : {4, 5, 6, 7, 8, 10, 12, 14, 16, 18, 20, 24, 28, 32}) {   // parts of the longest key block, in quarters
+        const int s = quarters == 4 ? 0 : (4 * n_rt + quarters - 1) / quarters;
+        if (quarters > 4 && s < 6) break;
+        auto cost = [&](int kb, int parts) {
+            const int len = chain_len(p, kb) > 0 ? chain_len(p, kb) : 0;
+            return (float)len / parts + fixed + (parts > 1 ? cut_end : 0.f);
+        };
+        if (quarters > 4) {   // (no better than even shares, and than its longest workgroup)
+            float sum = 0.f;
+            for (int kb = 0; kb < n_kb; ++kb) sum += cost(kb, chain_parts(p, kb, s)) * chain_parts(p, kb, s);
+            if (sum * n / 256.f >= best) continue;
         }
+        Schedule launch;
+        for (int kb = 0; kb < n_kb; ++kb) launch.add(cost(kb, chain_parts(p, kb, s)), n * chain_parts(p, kb, s));
         const float t = launch.end();
-        if (cut == 1) none = best = t;
-        else if (margin * t + reduction < none && t < best) { best = t; share = s; }
+        if (quarters == 4) none = best = t;
+        else if (margin * t < none && t < best) { best = t; share = s; }
     }
     return share;
 }
