@@ -73,7 +73,7 @@ template <int D> struct FwdLds {
 // A query tile's key steps cut into parts of at most `share` steps, one workgroup each (0: one workgroup per tile); a part
 // leaves its O (not normalised), row sums, exponent bases and maxima in `part`, [batch, head][workgroup][BQ][D + 4] fp32, for
 // fwd_merge_kernel.
-struct FwdSplit { int share; float *part; };
+struct FwdSplit { int share; float *part; int first_long; };
 template <int BQ>
 __host__ __device__ inline int fwd_steps(const Problem &p, int qt) {
     const int k_end = p.causal ? (p.Nk < (qt + 1) * BQ ? p.Nk : (qt + 1) * BQ) : p.Nk;
@@ -87,12 +87,15 @@ template <int BQ> inline int fwd_wgs(const Problem &p, int share) {
 }
 
 // (SPLIT: an instance of its own, the other one is a percent slower with the parts' bounds at run time)
-template <int D, int CQT, typename TO, bool SPLIT>
+// LONG: the tiles from split.first_long on run at a higher wave priority (long_tiles_first)
+enum { PLAIN, SPLIT_KEYS, LONG };
+template <int D, int CQT, typename TO, int FORM>
 __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     Problem p, FwdSplit split, const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
     const bf16_t *__restrict__ V, const float *__restrict__ W, TO *__restrict__ O,
     float *__restrict__ M, float *__restrict__ L) {
     using Lds = FwdLds<D>;
+    constexpr bool SPLIT = FORM == SPLIT_KEYS;
     constexpr int KST = Lds::KST;
     constexpr int KS = D / 32;   // MFMA k-steps over the head dimension
     constexpr int DB = D / 16;   // 16-wide blocks of the head dimension
@@ -111,6 +114,8 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         for (qt = (p.Nq + BQ - 1) / BQ - 1, part_no = blockIdx.z; part_no >= fwd_parts(fwd_steps<BQ>(p, qt), split.share); --qt)
             part_no -= fwd_parts(fwd_steps<BQ>(p, qt), split.share);
     const int i0 = qt * BQ, i0w = i0 + wave * WR;
+    const bool is_long = FORM == LONG && qt >= split.first_long;
+    if (is_long) __builtin_amdgcn_s_setprio(3);
     const int base = i0w - (CQT - 1);  // first score row of the wave
     const int pk = p.pk, cq = p.c_q;
     const bool causal = p.causal != 0;
@@ -331,7 +336,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         // The two waves of a SIMD are at different places of their steps: the one in an MFMA
         // phase (P V, S^T, the convolution) gets the issue slot first, the one in the softmax
         // arithmetic fills the gaps (measured: 1.5 % over equal priorities; the reverse is slower).
-        __builtin_amdgcn_s_setprio(0);
+        if (!is_long) __builtin_amdgcn_s_setprio(0);
         // ---- post-mask and softmax numerators (log2 domain).  The exponent base m_ref of a row
         //      only follows the row's maximum when some score exceeds it by more than kMaxSlack
         //      (then every lane group of the wave exchanges its maxima and rescales); otherwise no
@@ -397,7 +402,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         // ---- O^T += V^T P^T: V^T fragments through the LDS transpose read, P^T straight from
         //      the softmax registers (k slot 8g+e <-> key 4g+e of output block 0 for e < 4, of
         //      output block 1 for e >= 4) ----
-        __builtin_amdgcn_s_setprio(1);
+        if (!is_long) __builtin_amdgcn_s_setprio(1);
         bf16x8 pf[2];
 #pragma unroll
         for (int ob = 0; ob < 2; ++ob)
@@ -603,18 +608,32 @@ template <int BQ> int fwd_share(const Problem &p) {
     return share;
 }
 
+// Causal launches of 1.4 to 2 rounds of workgroups end with their longest tiles: a CU has three workgroups, a slot's tiles are shorter
+// together than the longest one alone (65 and 55 steps at B4 H16 N2048 d64 6x11), and that one runs at a third of the CU until the others
+// leave.  There the longer half of the tiles gets the issue slots first, us without and with it at B4 H16 N2048: d64 6x11 102.3 / 94.3, 3x3
+// 80.9 / 74.8, d32 6x11 82.8 / 78.7; 1.96 rounds (B1 H32 N5000 d64 6x11) 256 / 245.  Outside the two waves of a SIMD had better
+// take turns by phase: 1.2 rounds (B2 H12 N4096) 137 / 144, 1.3 (N5000 3x3) 133 / 140, 2.3 (N8000) 443 / 452, 3.2 (B4 H16 N4096) 320 / 342.  The
+// instances that have three workgroups per CU; the others (two, or four) gain nothing.
+constexpr bool has_long(int d, int cqt) { return (d == 64 && cqt <= 6) || (d == 32 && cqt == 6); }
+template <int BQ> bool long_tiles_first(const Problem &p) {
+    const long long wgs = (long long)p.B * p.H * ((p.Nq + BQ - 1) / BQ), round = 3 * 256;
+    return p.causal && 5 * wgs > 7 * round && wgs <= 2 * round;
+}
+
 template <int D, int CQT, typename TO>
 hipError_t launch_fwd(const Problem &p, float *part, const void *q, const void *k, const void *v, const float *w,
                       void *o, float *m, float *l, hipStream_t s) {
     constexpr int lds = FwdLds<D>::total, BQ = NW * wave_rows(CQT);
     if (lds > 64 * 1024) {
-        hipError_t e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, false>>(lds);
-        if (e == hipSuccess) e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, true>>(lds);
+        hipError_t e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, PLAIN>>(lds);
+        if (e == hipSuccess) e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS>>(lds);
         if (e != hipSuccess) return e;
     }
-    const FwdSplit split{part ? fwd_share<BQ>(p) : 0, part};
+    const FwdSplit split{part ? fwd_share<BQ>(p) : 0, part, (p.Nq + BQ - 1) / BQ / 2};
     const int n_wg = fwd_wgs<BQ>(p, split.share);
-    auto kern = split.share ? fwd_reg_mfma_kernel<D, CQT, TO, true> : fwd_reg_mfma_kernel<D, CQT, TO, false>;
+    auto kern = split.share ? fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS> : fwd_reg_mfma_kernel<D, CQT, TO, PLAIN>;
+    if constexpr (has_long(D, CQT))
+        if (!split.share && long_tiles_first<BQ>(p)) kern = fwd_reg_mfma_kernel<D, CQT, TO, LONG>;
     kern<<<dim3(p.H, p.B, n_wg), NW * 64, lds, s>>>(p, split, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, w, (TO *)o, m, l);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !split.share) return e;
