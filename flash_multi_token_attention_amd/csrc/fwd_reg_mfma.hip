@@ -73,7 +73,7 @@ template <int D> struct FwdLds {
 // A query tile's key steps cut into parts of at most `share` steps, one workgroup each (0: one workgroup per tile); a part
 // leaves its O (not normalised), row sums, exponent bases and maxima in `part`, [batch, head][workgroup][BQ][D + 4] fp32, for
 // fwd_merge_kernel.
-struct FwdSplit { int share; float *part; int first_long; };
+struct FwdSplit { int share, first_long; float *part; };
 template <int BQ>
 __host__ __device__ inline int fwd_steps(const Problem &p, int qt) {
     const int k_end = p.causal ? (p.Nk < (qt + 1) * BQ ? p.Nk : (qt + 1) * BQ) : p.Nk;
@@ -629,7 +629,7 @@ hipError_t launch_fwd(const Problem &p, float *part, const void *q, const void *
         if (e == hipSuccess) e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS>>(lds);
         if (e != hipSuccess) return e;
     }
-    const FwdSplit split{part ? fwd_share<BQ>(p) : 0, part, (p.Nq + BQ - 1) / BQ / 2};
+    const FwdSplit split{part ? fwd_share<BQ>(p) : 0, (p.Nq + BQ - 1) / BQ / 2, part};
     const int n_wg = fwd_wgs<BQ>(p, split.share);
     auto kern = split.share ? fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS> : fwd_reg_mfma_kernel<D, CQT, TO, PLAIN>;
     if constexpr (has_long(D, CQT))
