@@ -613,7 +613,8 @@ template <int BQ> int fwd_share(const Problem &p) {
 // leave.  There the longer half of the tiles gets the issue slots first, us without and with it at B4 H16 N2048: d64 6x11 102.3 / 94.3, 3x3
 // 80.9 / 74.8, d32 6x11 82.8 / 78.7; 1.96 rounds (B1 H32 N5000 d64 6x11) 256 / 245.  Outside the two waves of a SIMD had better
 // take turns by phase: 1.2 rounds (B2 H12 N4096) 137 / 144, 1.3 (N5000 3x3) 133 / 140, 2.3 (N8000) 443 / 452, 3.2 (B4 H16 N4096) 320 / 342.  The
-// instances that have three workgroups per CU; the others (two, or four) gain nothing.
+// instances that have three workgroups per CU; with two it costs up to 10 % in this band (B1 H32 N2500 d64 7x7 82 / 90, d128 6x11 101 / 110), with
+// four 1 to 3 %.
 constexpr bool has_long(int d, int cqt) { return (d == 64 && cqt <= 6) || (d == 32 && cqt == 6); }
 template <int BQ> bool long_tiles_first(const Problem &p) {
     const long long wgs = (long long)p.B * p.H * ((p.Nq + BQ - 1) / BQ), round = 3 * 256;
