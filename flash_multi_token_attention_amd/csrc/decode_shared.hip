@@ -17,9 +17,13 @@
 //   * a lane's V rows are consecutive keys of one page: one page lookup;
 //   * the workgroups of one round (two per CU) share all keys of the batch evenly, whatever the lengths of its entries
 //     are: a workgroup's set-up and wind-down cost as much as three iterations, and with n_splits equal
-//     parts per entry the round waited for the longest entry's.
+//     parts per entry the round waited for the longest entry's.  A workgroup that meets the start of a stream does set-up and
+//     wind-down twice, so the start counts as four tiles: without it the round waited for those workgroups
+//     (B8 H32 H_kv8 N4348 d128 3x3 39.6 -> 33.2 us, B16 H32 H_kv8 N2254 d64 11x11 38.8 -> 34.9, B4 H32 H_kv8 N20000 d128
+//     6x11 57.5 -> 52.5; 0 to 22 % over 100 shapes, 3 % on average with those of few keys, which go another way; 5 and 6 tiles
+//     give the same within 0.2 %, 3 and 8 half a per cent less).
 // B32 H32 H_kv8 N8192 d128 6x11, pages of 64, lengths from a quarter to all of N (684 MB of K / V): the whole call with the
-// merge 285 -> 140 us, this kernel about 135 of it.  No unit is full then (vector ALUs 22 %, LDS 19 %): each of the two waves per
+// merge 285 -> 138 us, this kernel about 133 of it.  No unit is full then (vector ALUs 22 %, LDS 19 %): each of the two waves per
 // SIMD is a chain of scores, window, softmax and P.V.  H32 H_kv8 N8192 d128 11x11, B16, pages of 256: kernel 258 -> 86 us.
 #include "mfma_common.hpp"
 
@@ -30,6 +34,7 @@ constexpr int NW = 4;
 constexpr int IT = 64;             // keys per wave iteration
 constexpr int SROW = IT + 16 + 4;  // floats per strip row: 16 carried + 64 new, padded
 constexpr int PROW = IT + 8;       // bf16 per row of probability parts
+constexpr int kHead = 4;           // tiles that the start of a stream counts for in the even share
 
 template <int ROR>
 __device__ __forceinline__ float row_rot(float v) {
@@ -135,8 +140,10 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_shared_kernel(
     // cut at the streams' ends; its part of a stream is partial w - (workgroup of the stream's first tile) of the n_splits.
     // parts > 0 instead: every stream has its own workgroup (1) or `parts` of them with one tile per wave.
     const int w = blockIdx.x, groups = p.H / HG;
-    int b, grp, Nk, t0, t1, nt, share = 1;
-    unsigned int pos = 0, end = 0, start = 0;   // tiles; start: the stream's first
+    // A workgroup that meets a stream's start goes through set-up and wind-down once more, so a stream counts as
+    // `head` tiles and then its own (a part of head tiles only is an empty one).
+    int b, grp, Nk, t0, t1, nt, share = 1, head = kHead;
+    unsigned int pos = 0, end = 0, start = 0;   // tiles with the heads; start: the stream's first
     if (parts) {
         const int s = w / parts;
         b = s / groups; grp = s % groups;
@@ -163,9 +170,21 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_shared_kernel(
             total = __builtin_amdgcn_readfirstlane(sum);
             longest = __builtin_amdgcn_readfirstlane(mx);
         }
-        total *= groups;
         // (a stream of n tiles meets at most ceil(n / share) + 1 workgroups; 4 tiles are one per wave)
-        share = max(max(NW, (int)((total + gridDim.x - 1) / gridDim.x)), (longest + p.n_splits - 2) / (p.n_splits - 1));
+        auto even_share = [&](unsigned int tiles, int most) {
+            return max(max(NW, (int)((tiles * groups + gridDim.x - 1) / gridDim.x)), (most + p.n_splits - 2) / (p.n_splits - 1));
+        };
+        share = even_share(total, longest);
+        // Streams of one length that the bare share divides: no workgroup meets two of them, and heads would only
+        // unsettle that (B32 H16 H_kv8 N718 d128, two workgroups per stream: 25.8 us, with heads 28.5).
+        if (total == (unsigned int)p.B * longest && longest % share == 0) {
+            head = 0;
+        } else {
+            longest += head;
+            total += (unsigned int)p.B * head;
+            share = even_share(total, longest);
+        }
+        total *= groups;
         const unsigned long long first = (unsigned long long)w * share;
         if (first >= total) return;
         pos = (unsigned int)first;
@@ -173,7 +192,7 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_shared_kernel(
         b = 0;
         if (kv.seq_lens) {
             for (;; b += 64) {   // (pos < total: some entry contains it)
-                const int mine = b + lane_id < p.B ? tiles_of(min(kv.seq_lens[b + lane_id], p.Nk)) : 0;
+                const int mine = b + lane_id < p.B ? tiles_of(min(kv.seq_lens[b + lane_id], p.Nk)) + head : 0;
                 int incl = mine;
 #pragma unroll
                 for (int o = 1; o < 64; o <<= 1) {
@@ -195,10 +214,10 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_shared_kernel(
         }
         Nk = keys_of(b);
         nt = tiles_of(Nk);
-        grp = (pos - start) / nt;
-        start += (unsigned int)grp * nt;
-        t0 = pos - start;
-        t1 = min(nt, t0 + (int)(end - pos));
+        grp = (pos - start) / (nt + head);
+        start += (unsigned int)grp * (nt + head);
+        t0 = max((int)(pos - start) - head, 0);
+        t1 = min(nt, max((int)(end - start) - head, 0));
     }
 
     for (;;) {   // parts of streams
@@ -487,15 +506,14 @@ __global__ __launch_bounds__(NW * 64, 2) void decode_shared_kernel(
         if (next >= (long long)p.B * groups) break;
         b = (int)(next / groups); grp = (int)(next % groups);
     } else {
-        pos += t1 - t0;
-        if (pos >= end) break;
-        start += nt;
+        start += nt + head;
+        if (start >= end) break;
         if (++grp == groups) { grp = 0; ++b; }
     }
     Nk = keys_of(b);
     nt = tiles_of(Nk);
     t0 = 0;
-    t1 = parts ? nt : min(nt, (int)(end - pos));
+    t1 = parts ? nt : min(nt, max((int)(end - start) - head, 0));
     }
 }
 
@@ -511,7 +529,7 @@ hipError_t launch(const Problem &p, const KvArgs &kv, const bf16_t *q, const bf1
     // (B1 H32 H_kv8 N700 d128: 28 against 17 us).
     const int most = 256 * (2 * L::bytes(p.c_q) <= (int)kLdsBytes ? 2 : 1), each = (p.Nk + NW * IT - 1) / (NW * IT);
     const long long streams = (long long)p.B * (p.H / HG), tiles = streams * ((p.Nk + IT - 1) / IT);
-    const int parts = p.n_splits == 1 || tiles > 0x7fffffffLL ? 1 : each <= p.n_splits && streams * each <= most ? each : 0;
+    const int parts = p.n_splits == 1 || tiles + kHead * streams > 0x7fffffffLL ? 1 : each <= p.n_splits && streams * each <= most ? each : 0;
     const long long wgs = parts > 1 ? streams * parts : parts ? streams : (tiles + NW - 1) / NW;
     decode_shared_kernel<D, PAGED, HG, WIDE><<<(int)(wgs < most ? wgs : most), NW * 64, L::bytes(p.c_q), s>>>(
         p, kv, parts, q, k, v, w, o_part, m_part, l_part);
