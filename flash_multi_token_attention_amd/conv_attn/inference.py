@@ -13,6 +13,8 @@ def fwd_conv_attn_inference(Q, K, V, conv_kernel, k_splits, scale, pad_q, pad_k,
     kernel_size_q-1 rows back; missing rows count as zero rows, which is what
     the reference's front padding to 16 rows amounts to), K, V [B,H,Nk,d].
     Returns O [B,H,1,d], M [B,H,1], L [B,H,1] in fp32, always normalised.
+    ``k_splits`` > 0 cuts the keys into that many parts (bf16: of 128 keys at least), whatever else is in
+    the batch; None/0 takes the count that is fastest for the whole batch.
     ``causal=False`` is the reference behaviour (its kernel ignores the flag);
     ``causal=True`` applies the training masks to the resident rows so that the
     result equals the last row of the causal training forward.

@@ -389,54 +389,69 @@ def decode(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.
         r = host.decode_dense(Q, K, V, conv_kernel, k_splits or 0, scale, bool(causal), out_dtype, True)
         if r is not None:
             return r[0], r[1], r[2], r[3:]
+    return _decode_dense(Q, K, V, conv_kernel, k_splits, scale, causal, out_dtype, exact, workspace, True)
+
+
+def decode_whole(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.float32):
+    """``decode`` without the partials -> (O, M, L).  Nobody sees the splits, so ``k_splits`` is their most (bf16): none has fewer than
+    128 keys, and one launch does the step where the library takes it as a whole.  How the keys of a head are cut follows from an
+    explicit count and their number alone, so its result has the same bits whatever else is in the batch; None/0 picks a count by
+    the shape, as in ``decode``."""
+    host = _lib.host()
+    if host is not None and all(isinstance(t, torch.Tensor) for t in (Q, K, V, conv_kernel)) and K.dim() == 4:
+        r = host.decode_dense(Q, K, V, conv_kernel, k_splits or 0, scale, bool(causal), out_dtype, False)
+        if r is not None:
+            return r[:3]
+    return _decode_dense(Q, K, V, conv_kernel, k_splits, scale, causal, out_dtype, False, None, False)[:3]
+
+
+def _decode_dense(Q, K, V, conv_kernel, k_splits, scale, causal, out_dtype, exact, workspace, partials):
+    """What the native call does, with all checks (csrc/host.cpp, decode_dense)."""
     _check_qkv(Q, K, V, kv_views=True)
     if K.stride() != V.stride():
         raise RuntimeError("K and V must have the same strides")
     B, H, r, d = Q.shape
+    Nk = K.shape[2]
     c_q, c_k = conv_kernel.shape[1], conv_kernel.shape[2]
     W = _weights(conv_kernel, H, c_q - 1, (c_k - 1) // 2, Q.device)
-    if not k_splits:
-        k_splits = default_k_splits(B, H, K.shape[2], d=d)
-    desc = _desc(Q, K, W, scale, causal, out_dtype, n_splits=k_splits, exact=exact)
+    desc = _desc(Q, K, W, scale, causal, out_dtype, n_splits=k_splits or 1, exact=exact)
     lib = _lib.load()
     if r > 16:
         raise ValueError(f"Q sequence length must be <= 16 for inference, got {r}")
-    if not 1 <= k_splits <= 1024:
+    if k_splits and not 1 <= k_splits <= min(Nk, 1024):
         # (every other argument is checked by the launch itself; a split count out of range would size the
         # partial buffers first)
+        desc.n_splits = 0   # (refused, also where the value itself does not fit the field)
         _lib.check(lib.convattn_validate(C.byref(desc), _lib.OP_DECODE), "conv_attn.forward_inference")
+    whole = False
+    if not partials and lib.convattn_kernel_path(C.byref(desc), _lib.OP_DECODE) == 1:
+        desc.n_splits = lib.convattn_decode_step_splits(B, H, Nk, d, k_splits or 0)
+        whole = lib.convattn_decode_whole_ok(C.byref(desc)) != 0
+    elif not k_splits:
+        desc.n_splits = default_k_splits(B, H, Nk, d=d)
+    k_splits = desc.n_splits
+    O = torch.empty((B, H, 1, d), dtype=out_dtype, device=Q.device)
+    M = torch.empty((B, H, 1), dtype=torch.float32, device=Q.device)
+    L = torch.empty((B, H, 1), dtype=torch.float32, device=Q.device)
+    st = _stream(Q)
+    kv = [C.c_longlong(n) for n in ((H * Nk * d, Nk * d) if K.is_contiguous() else (K.stride(0), K.stride(1)))]
+    if whole:
+        rc = lib.convattn_decode_whole(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), *kv, _ptr(O), _ptr(M), _ptr(L), st)
+        _lib.check(rc, "conv_attn.forward_inference")
+        return O, M, L, None
     if workspace is None:
         O_part = torch.empty((B, H, k_splits, d), dtype=torch.float32, device=Q.device)
         M_part = torch.empty((B, H, k_splits), dtype=torch.float32, device=Q.device)
         L_part = torch.empty((B, H, k_splits), dtype=torch.float32, device=Q.device)
     else:
         O_part, M_part, L_part = workspace
-    O = torch.empty((B, H, 1, d), dtype=out_dtype, device=Q.device)
-    M = torch.empty((B, H, 1), dtype=torch.float32, device=Q.device)
-    L = torch.empty((B, H, 1), dtype=torch.float32, device=Q.device)
-    st = _stream(Q)
-    Nk = K.shape[2]
-    kv_bs, kv_hs = (H * Nk * d, Nk * d) if K.is_contiguous() else (K.stride(0), K.stride(1))
-    rc = lib.convattn_decode_strided(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W),
-                                     C.c_longlong(kv_bs), C.c_longlong(kv_hs),
+    rc = lib.convattn_decode_strided(C.byref(desc), _ptr(Q), _ptr(K), _ptr(V), _ptr(W), *kv,
                                      _ptr(O_part), _ptr(M_part), _ptr(L_part), st)
     _lib.check(rc, "conv_attn.forward_inference")
     rc = lib.convattn_decode_combine(C.byref(desc), _ptr(O_part), _ptr(M_part), _ptr(L_part), _ptr(O),
                                      _ptr(M), _ptr(L), st)
     _lib.check(rc, "conv_attn.forward_inference (combine)")
     return O, M, L, (O_part, M_part, L_part)
-
-
-def decode_whole(Q, K, V, conv_kernel, k_splits, scale, causal=False, out_dtype=torch.float32):
-    """``decode`` without the partials -> (O, M, L).  Nobody sees the splits, so ``k_splits`` is their most: no more are made
-    than the library would choose (B32 H32 N1000 d128 in 32 splits 663 us, in its own count 43), and one launch does it
-    where it takes the step as a whole."""
-    host = _lib.host()
-    if host is not None and all(isinstance(t, torch.Tensor) for t in (Q, K, V, conv_kernel)) and K.dim() == 4:
-        r = host.decode_dense(Q, K, V, conv_kernel, k_splits or 0, scale, bool(causal), out_dtype, False)
-        if r is not None:
-            return r[:3]
-    return decode(Q, K, V, conv_kernel, k_splits, scale, causal, out_dtype)[:3]
 
 
 def _kv_splits(B: int, H: int, H_kv: int, Nk: int, d: int, c_q: int, ragged: bool) -> int:

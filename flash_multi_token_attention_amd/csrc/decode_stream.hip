@@ -417,18 +417,21 @@ int decode_splits(long long heads, int Nk, bool ragged, int d) {
     return d <= 64 && heads >= 512 && Nk >= 2048 && splits < 2 ? 2 : splits;
 }
 
-// The split count of a step whose partials nobody sees, `asked` at most (0: no limit).  While the workgroups fit one round,
-// 128 keys each, two waves at work, are faster than 256: the four waves of a workgroup wait for each other's LDS reads (us, by the rule
-// above and now: B1 H8 d128 N1000 12.8 and 10.5, N2048 14.3 and 10.7, B4 H8 d64 N1000 12.0 and 9.3).  Up to 64, beyond which the merge
-// costs more than it gains.
+// The split count of a step whose partials nobody sees.
+// `asked` for splits (> 0): that many, but none of fewer than 128 keys.  Two waves at work are faster than one and a longer merge (B2 H2
+// N2048 d64 7x7 in 32 splits 9.9 us, in 16 9.3; N1024 in 32 9.9, in 8 8.7; B1 H8 N2048 d128 11.1, in 16 10.8; B32 H32 N1000 d128 662, in 8
+// 196).  The count follows from the keys and nothing else, so a head's result has the same bits in any batch.
+// 0: by the rule above, and while the workgroups fit one round, 128 keys each: two waves at work are faster than four, which
+// wait for each other's LDS reads (us, by the rule above and now: B1 H8 d128 N1000 12.8 and 10.5, N2048 14.3 and 10.7, B4 H8 d64 N1000 12.0
+// and 9.3).  Up to 64, beyond which the merge costs more than it gains.
 int decode_step_splits(long long heads, int Nk, int d, int asked) {
-    int n = decode_splits(heads, Nk, false, d);
+    const int pairs_at_work = (Nk + 127) / 128;
+    if (asked > 0) return asked < pairs_at_work ? asked : pairs_at_work;
+    const int n = decode_splits(heads, Nk, false, d);
     const long long room = slots_of(d) / heads;
-    if (n <= room) {
-        const long long one = room < (Nk + 127) / 128 ? room : (Nk + 127) / 128;
-        if (one > n) n = one < 64 ? (int)one : n > 64 ? n : 64;
-    }
-    return asked > 0 && asked < n ? asked : n;
+    if (n > room) return n;
+    const long long one = room < pairs_at_work ? room : pairs_at_work;
+    return one <= n ? n : one < 64 ? (int)one : n > 64 ? n : 64;
 }
 
 // Waves of the workgroup that takes all keys of a (batch, head), or 0: splits and a merge.  Without splits the merge is only a launch

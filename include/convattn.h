@@ -266,7 +266,8 @@ int convattn_decode_strided(const convattn_desc *desc, const void *q, const void
 
 /* The split count to be preferred for a step of B x H (batch, head) pairs; ragged: entries of the batch have fewer than Nk keys. */
 int convattn_decode_splits(int B, int H, int Nk, int ragged, int d);
-/* The same for a step whose partials nobody reads, and at most `asked` where that is > 0. */
+/* The same for a step whose partials nobody reads.  asked > 0: that many, but no split of fewer than 128 keys (the count follows from
+ * Nk and `asked` alone). */
 int convattn_decode_step_splits(int B, int H, int Nk, int d, int asked);
 
 /*

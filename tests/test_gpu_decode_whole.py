@@ -3,6 +3,7 @@ against the step that returns its partials."""
 import pytest
 import torch
 
+from flash_multi_token_attention_amd import _lib
 from flash_multi_token_attention_amd.conv_attn import fwd_conv_attn_inference, ops
 from oracle import conv_attn_oracle as orc
 
@@ -52,3 +53,33 @@ def test_views_causal_and_refused_counts():
     for bad in (-1, 301, 1025):
         with pytest.raises(RuntimeError, match="k_splits"):
             fwd_conv_attn_inference(q, k, v, w, bad, 0.125, 5, 5, False)
+
+
+@pytest.mark.parametrize("Nk,splits", [(1, 1), (100, 32), (300, 3), (512, 32), (513, 4), (2048, 32), (2048, 1), (5000, 7), (40000, 700)])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_an_explicit_count_gives_a_head_the_same_bits_in_any_batch(Nk, splits, d):
+    B, H = (4, 16) if Nk > 5000 else (24, 24)   # two workgroups fit a CU with d = 32: 576 heads are more than 512
+    g = torch.Generator(device=DEV).manual_seed(Nk)
+    splits = min(splits, Nk)
+    Q, K, V = (torch.randn(B, H, n, d, generator=g, device=DEV, dtype=torch.bfloat16) for n in (6, Nk, Nk))
+    W = 0.3 * torch.randn(H, 6, 11, generator=g, device=DEV)
+    many = fwd_conv_attn_inference(Q, K, V, W, splits, d ** -0.5, 5, 5, False)
+    for b, h in ((0, 1), (B - 1, 2)):
+        few = fwd_conv_attn_inference(*(t[b:b + 1, :h].contiguous() for t in (Q, K, V)), W[:h].contiguous(), splits, d ** -0.5, 5, 5, False)
+        assert all(torch.equal(a[b:b + 1, :h], c) for a, c in zip(many, few))
+
+
+@pytest.mark.parametrize("Nk", [63, 300, 513, 2048])
+@pytest.mark.parametrize("splits", [0, 1, 3, 32])
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float32, 64), (torch.bfloat16, 40)])
+def test_the_python_op_makes_the_same_step(Nk, splits, dtype, d, monkeypatch):
+    # (where the native call declines: no host library, a dispatch mode)
+    Q, K, V, W = (t.to(DEV) for t in _case(2, 3, 6, Nk, d, 6, 11, seed=Nk))
+    Q, K, V = (t.to(dtype) for t in (Q, K, V))
+    native = fwd_conv_attn_inference(Q, K, V, W, splits, d ** -0.5, 5, 5, False)
+    monkeypatch.setattr(_lib, "host", lambda: None)
+    plain = fwd_conv_attn_inference(Q, K, V, W, splits, d ** -0.5, 5, 5, False)
+    assert all(a.dtype == b.dtype and torch.equal(a, b) for a, b in zip(native, plain))
+    for bad in (-1, Nk + 1, 1025, 2 ** 32 + 1):
+        with pytest.raises(RuntimeError, match="k_splits"):
+            fwd_conv_attn_inference(Q, K, V, W, bad, d ** -0.5, 5, 5, False)

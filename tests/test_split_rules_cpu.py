@@ -53,3 +53,11 @@ def test_decode_split_counts(args, low, high):
     assert low <= ops.default_k_splits(B, H, Nk, ragged, d) <= high
     # one sequence has no others that could be shorter
     assert ops.default_k_splits(1, H, Nk, True, d) == ops.default_k_splits(1, H, Nk, False, d)
+
+
+@pytest.mark.parametrize("Nk", [1, 128, 129, 513, 2048, 40000])
+@pytest.mark.parametrize("asked", [1, 2, 16, 32, 700])
+def test_an_explicit_count_does_not_follow_the_batch(Nk, asked):
+    lib = _lib.load()
+    counts = {lib.convattn_decode_step_splits(B, H, Nk, d, asked) for B, H in ((1, 1), (2, 2), (8, 32), (64, 64)) for d in (32, 64, 128)}
+    assert counts == {min(asked, -(-Nk // 128))}
