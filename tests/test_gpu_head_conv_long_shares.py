@@ -9,8 +9,9 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# steps per workgroup = B * (steps of the row tiles of 32 by keys of 16) / 256; the line is at 128
-@pytest.mark.parametrize("B,N,causal", [(4, 2900, True), (4, 4096, True), (124, 497, True), (60, 515, False), (2, 3001, False)])
+# steps per workgroup = B * (steps of the row tiles of 32 by keys of 16) / 256; the line is at 128, without the mask at 192
+@pytest.mark.parametrize("B,N,causal", [(4, 2900, True), (4, 4096, True), (124, 497, True), (60, 515, False), (2, 3001, False),
+                                        (90, 515, False), (4, 2501, False)])
 def test_entries_of_long_shares(B, N, causal):
     from flash_multi_token_attention_amd.head_conv_attn import ops
     H, d, tiles = 16, 128, -(-N // 32)
