@@ -610,15 +610,19 @@ template <int BQ> int fwd_share(const Problem &p) {
 
 // Causal launches of 1.4 to 2 rounds of workgroups end with their longest tiles: a CU has three workgroups, a slot's tiles are shorter
 // together than the longest one alone (65 and 55 steps at B4 H16 N2048 d64 6x11), and that one runs at a third of the CU until the others
-// leave.  There the longer half of the tiles gets the issue slots first, us without and with it at B4 H16 N2048: d64 6x11 102.3 / 94.3, 3x3
-// 80.9 / 74.8, d32 6x11 82.8 / 78.7; 1.96 rounds (B1 H32 N5000 d64 6x11) 256 / 245.  Outside the two waves of a SIMD had better
-// take turns by phase: 1.2 rounds (B2 H12 N4096) 137 / 144, 1.3 (N5000 3x3) 133 / 140, 2.3 (N8000) 443 / 452, 3.2 (B4 H16 N4096) 320 / 342.  The
-// instances that have three workgroups per CU; with two it costs up to 10 % in this band (B1 H32 N2500 d64 7x7 82 / 90, d128 6x11 101 / 110), with
+// leave.  There the longer half of the tiles gets the issue slots first; us without and with it at B4 H16 N2048 (1.6 rounds): d64 6x11
+// 95 / 90, 3x3 82 / 78, d32 6x11 77 / 74.
+// Below 1.4 and beyond 2 rounds the two waves of a SIMD had better take turns by phase (d64): B2 H12 6x11 of 1.25 rounds 139 / 148, 1.31 149 / 159,
+// 1.38 168 / 171, 1.41 178 / 176, 1.5 207 / 195; N8000 (2.3) 443 / 452, B4 H16 N4096 (3.2) 320 / 342.
+// The fewer tiles a head has, the less there is to put in order, and the earlier that ends: with 47 tiles (B1 H32 N5000) 1.96 rounds 256 / 245, with
+// 24 (B4 H16 N2581) 2.0 rounds 137 / 144, 22 tiles 1.83 rounds 119 / 116; 16 tiles 2.0 rounds 98 / 98, 14 1.75 80 / 79; 12 2.0 75 / 76, 12 1.5
+// 63 / 61; 7 (B12 H16 N745) 1.75 48.4 / 49.0, 6 2.0 49.3 / 50.4, 6 1.5 40.2 / 39.6; 3 1.5 25.3 / 25.6.  144 launches of 64 to 384 heads.
+// The instances that have three workgroups per CU; with two it costs up to 10 % in this band (B1 H32 N2500 d64 7x7 82 / 90, d128 6x11 101 / 110), with
 // four 1 to 3 %.
 constexpr bool has_long(int d, int cqt) { return (d == 64 && cqt <= 6) || (d == 32 && cqt == 6); }
 template <int BQ> bool long_tiles_first(const Problem &p) {
-    const long long wgs = (long long)p.B * p.H * ((p.Nq + BQ - 1) / BQ), round = 3 * 256;
-    return p.causal && 5 * wgs > 7 * round && wgs <= 2 * round;
+    const long long tiles = (p.Nq + BQ - 1) / BQ, wgs = p.B * p.H * tiles, round = 3 * 256;
+    return p.causal && 5 * wgs > 7 * round && wgs <= 2 * round && 10 * wgs * tiles <= (21 * tiles - 30) * round;   // (up to 2.1 - 3 / tiles rounds)
 }
 
 template <int D, int CQT, typename TO>

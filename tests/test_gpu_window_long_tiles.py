@@ -7,8 +7,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# workgroups of the whole batch: 1.4 to 2 rounds of 768; of its parts less than one (and too few key steps to be split)
-@pytest.mark.parametrize("d,c_q,c_k,B,H,N", [(64, 6, 11, 8, 16, 900), (64, 3, 3, 8, 16, 970), (32, 6, 11, 16, 16, 500), (64, 4, 5, 24, 12, 433)])
+# workgroups of the whole batch: 1.4 to 2 rounds of 768 (at most 2.1 - 3 / tiles of a head, which leaves two of these to the plain
+# instance); of its parts less than one (and too few key steps to be split)
+@pytest.mark.parametrize("d,c_q,c_k,B,H,N", [(64, 6, 11, 8, 16, 900), (64, 3, 3, 8, 16, 970), (32, 6, 11, 16, 16, 500), (64, 4, 5, 24, 12, 433),
+                                             (32, 6, 11, 8, 16, 961), (64, 4, 5, 12, 11, 962), (32, 4, 3, 12, 16, 560)])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
 def test_same_bits(d, c_q, c_k, B, H, N, out):
     from flash_multi_token_attention_amd.conv_attn import ops
