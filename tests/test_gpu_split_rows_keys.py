@@ -16,6 +16,10 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("B,H,N,d,c_q,c_k,causal", [
     (1, 2, 641, 64, 3, 3, True), (1, 3, 705, 128, 6, 11, True), (2, 8, 1531, 64, 11, 11, True), (1, 8, 1000, 128, 8, 15, True),
     (1, 4, 700, 32, 6, 5, False), (1, 2, 2049, 128, 9, 11, False), (1, 8, 1157, 32, 11, 7, True), (1, 1, 4000, 64, 6, 11, True),
+    # an instance per tap slot count: 7 and 8 up to d = 64, 7 at 128; 9 and 10 taps in 11 slots
+    (2, 8, 1531, 64, 7, 7, True), (1, 8, 700, 64, 8, 15, True), (1, 2, 1000, 32, 7, 7, False), (1, 8, 1153, 32, 8, 9, True),
+    (1, 2, 1100, 64, 8, 7, False), (1, 4, 1300, 64, 9, 5, True), (1, 4, 1300, 32, 10, 3, True), (1, 8, 2048, 128, 7, 7, True),
+    (1, 4, 1001, 128, 7, 15, False),
 ])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_split_equals_unsplit(B, H, N, d, c_q, c_k, causal, out_dtype, monkeypatch):
@@ -41,6 +45,8 @@ def test_split_equals_unsplit(B, H, N, d, c_q, c_k, causal, out_dtype, monkeypat
 @pytest.mark.parametrize("B,H,N,d,c_q,c_k,causal", [
     (1, 2, 1100, 64, 3, 3, True), (2, 8, 1531, 64, 11, 11, True), (1, 8, 1000, 128, 8, 15, True), (1, 4, 1217, 32, 6, 17, False),
     (1, 2, 2049, 128, 9, 11, False), (1, 8, 1157, 32, 11, 7, True), (1, 1, 4000, 64, 6, 11, True), (1, 3, 1600, 128, 6, 11, True),
+    (1, 8, 1200, 64, 7, 7, True), (1, 4, 1217, 32, 7, 17, False), (1, 3, 1600, 128, 7, 7, True), (1, 6, 1203, 64, 8, 9, True),
+    (1, 4, 1001, 128, 7, 15, False),
 ])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_split_forward_equals_unsplit(B, H, N, d, c_q, c_k, causal, out_dtype, monkeypatch):
