@@ -43,7 +43,7 @@ def test_result_without_partials(Nk, d, c_q, c_k, r, splits):
 def test_views_causal_and_refused_counts():
     Q, K, V, W = _case(2, 2, 6, 300, 64, 6, 11, seed=1)
     q, w = Q.to(DEV), W.to(DEV)
-    room = torch.empty(2, 2, 2, 512, 64, dtype=torch.bfloat16, device=DEV)
+    room = torch.full((2, 2, 2, 512, 64), float("nan"), dtype=torch.bfloat16, device=DEV)   # (not to be read into the result)
     room[0, :, :, :300], room[1, :, :, :300] = K.to(DEV), V.to(DEV)
     k, v = room[0, :, :, :300], room[1, :, :, :300]
     for causal in (False, True):

@@ -243,12 +243,16 @@ def test_decode_bf16_stream(r, Nk, d, c_q, c_k, splits, causal):
     O_ref, M_ref, L_ref = orc.decode(Q.float(), K.float(), V.float(), W, scale_of(d), causal=causal)
     g = [t.to(DEV) for t in (Q, K, V, W)]
     assert ops.kernel_path(g[0], g[1], g[3], causal, op="decode") == "mfma"
-    O, M, L = fwd_conv_attn_inference(g[0], g[1], g[2], g[3], splits, scale_of(d), c_q - 1,
-                                      (c_k - 1) // 2, causal)
-    assert O.shape == (2, 3, 1, d)
-    assert max_abs(O, O_ref) <= TOL_BF16
-    assert max_abs(M, M_ref) <= 1e-3
-    assert rel_max(L, L_ref) <= 1e-3
+    whole = fwd_conv_attn_inference(g[0], g[1], g[2], g[3], splits, scale_of(d), c_q - 1,
+                                    (c_k - 1) // 2, causal)
+    # (the function above makes no split of fewer than 128 keys: the op with partials makes as many as asked for)
+    O, M, L, (O_part, M_part, L_part) = ops.decode(*g, splits, scale_of(d), causal)
+    assert O_part.shape == (2, 3, splits, d) and M_part.shape == L_part.shape == (2, 3, splits)
+    for O, M, L in (whole, (O, M, L)):
+        assert O.shape == (2, 3, 1, d)
+        assert max_abs(O, O_ref) <= TOL_BF16
+        assert max_abs(M, M_ref) <= 1e-3
+        assert rel_max(L, L_ref) <= 1e-3
 
 
 @pytest.mark.parametrize("dtype,d,n_max", [(torch.bfloat16, 128, 700), (torch.bfloat16, 64, 512), (torch.float32, 64, 333)])
@@ -270,6 +274,11 @@ def test_decode_reads_views_of_a_longer_cache_in_place(dtype, d, n_max):
             dense = fwd_conv_attn_inference(g[0], g[1], g[2], g[3], splits, scale_of(d), c_q - 1, (c_k - 1) // 2, causal)
             view = fwd_conv_attn_inference(g[0], Kv, Vv, g[3], splits, scale_of(d), c_q - 1, (c_k - 1) // 2, causal)
             for a, b in zip(dense, view):
+                assert torch.equal(a, b)
+            # (bf16 in one launch above: the split kernel with its partials too)
+            dense, view = (ops.decode(g[0], k, v, g[3], splits, scale_of(d), causal) for k, v in ((g[1], g[2]), (Kv, Vv)))
+            assert view[3][0].shape[2] == splits
+            for a, b in zip((*dense[:3], *dense[3]), (*view[:3], *view[3])):
                 assert torch.equal(a, b)
     # a sequence-major cache ([B,N,H,d] permuted) has no dense rows per head: rejected, as a
     # non-contiguous tensor is by the reference
