@@ -35,6 +35,48 @@ def test_precision_of_the_scores(N, d, causal, spread):
     assert float(err) <= 2.0 ** -22 * float(size.gather(-1, top).norm())
 
 
+@pytest.mark.parametrize("N,d,causal", [(33, 64, False), (250, 128, True), (321, 32, True)])
+def test_precision_of_the_transposed_mix(N, d, causal):
+    # Heads 2p and 2p + 1 have the same scores' weights, V and dO, so the same dZ; head 16 + p, whose own scores are 0 (Q = 0), takes their
+    # difference: dS = a dZ - a (1 + e) dZ with e about 2^-13.  What a product is short of comes out 2^13 times as large: fp32's 2^-24
+    # (of w scale, and of the sum) 2^-11 each, beside the 2^-9 that the bf16 of dS leaves, half of it in the norm; without the lowest
+    # parts 2^-18 of a product are missing, 2^-19 on average, a sixty-fourth of dS.
+    from flash_multi_token_attention_amd.head_conv_attn import ops
+    g = torch.Generator().manual_seed(N + d)
+    Q, K, V, dO = (torch.randn(2, H, N, d, generator=g).to(torch.bfloat16) for _ in range(4))
+    Q[:, 16:] = 0
+    V[:, 1::2], dO[:, 1::2] = V[:, ::2], dO[:, ::2]
+    W = torch.zeros(H, H)
+    W[::2, :16] = torch.randn(16, 16, generator=g) / 4
+    W[1::2] = W[::2]
+    p = torch.arange(16)
+    W[2 * p, 16 + p] = 1 + torch.rand(16, generator=g)
+    W[2 * p + 1, 16 + p] = -W[2 * p, 16 + p] * (1 + 2.0 ** -13 * (1 + torch.rand(16, generator=g)))
+    sc = 1.0 / math.sqrt(d)
+    q, k, v, do, w = (t.to(DEV) for t in (Q, K, V, dO, W))
+    O, L, M = ops.forward(q, k, v, w, scale=sc, causal=causal)
+    got = ops.backward(q, k, v, w, O, do, L, M, causal=causal, scale=sc)[0].double().cpu()[:, 16:]
+    want, short = transposed_mix_dq(Q, K, V, dO, O.cpu(), W, sc, causal)
+    assert float((got - want).norm()) <= 2.0 ** -8 * float(want.norm())
+    assert float((short - want).norm()) > 2.0 ** -8 * float(want.norm())   # (two parts of w would fail)
+
+
+def transposed_mix_dq(Q, K, V, dO, O, W, sc, causal):
+    """dQ of heads 16.. in 64 bits, D from the O that was stored; with W and with its two highest bf16 parts."""
+    Q, K, V, dO, O = (t.double() for t in (Q, K, V, dO, O))
+    B, _, N, _ = Q.shape
+    kt, vt = K.transpose(-1, -2).contiguous(), V.transpose(-1, -2).contiguous()
+    Z = torch.matmul(W.double(), torch.matmul(Q, kt).mul(sc).reshape(B, H, N * N)).reshape(B, H, N, N)
+    if causal:
+        Z = Z.masked_fill(torch.ones(N, N, dtype=torch.bool).triu(1), -math.inf)
+    dZ = torch.softmax(Z, -1) * (torch.matmul(dO, vt) - (dO * O).sum(-1, keepdim=True))
+    ws = W * sc
+    hi = ws.to(torch.bfloat16).float()
+    two = hi + (ws - hi).to(torch.bfloat16).float()
+    return [torch.matmul(torch.matmul(w.double().t()[16:], dZ.reshape(B, H, N * N)).reshape(B, 16, N, N), K[:, 16:])
+            for w in (W.double() * sc, two)]
+
+
 def inputs(N, d, positive):
     g = torch.Generator().manual_seed(N)
     Q, K, V, dO = (torch.randn(1, H, N, d, generator=g) for _ in range(4))
