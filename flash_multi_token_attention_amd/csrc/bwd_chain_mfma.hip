@@ -73,6 +73,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
     bf16_t *__restrict__ dS_ws = args.dS_ws;
     float *__restrict__ dW_part = args.dW_part;
     const int n_rt = args.n_rt;
+    static_assert(D == 128 && CQT > 6, "the three-role kernel serves the others");
     using Lds = ChainLds<D, CQT>;
     constexpr int KS = D / 32, DB = D / 16;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -153,7 +154,6 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
 #pragma unroll
         for (int j0 = 0; j0 < 2 * KBT; j0 += 2 * NP) {
             const int j = j0 + wave, m = j / KBT, kb = j - m * KBT;
-            if (j >= 2 * KBT) break;   // (head dimension 32: four units for eight waves)
             const int row = 2 * (ln >> 2) + (kb & 1), chunk = (kb >> 1) * 4 + ((ln & 3) ^ ((ln >> 4) & 3));
             const int voff = ((r_begin + t * BR + row) * D + chunk * 8) * 2;
             const unsigned int dst = lds0 + (m ? Lds::g_off + (t % 3) * Lds::tile_bytes : Lds::q_off + (t & 3) * Lds::tile_bytes) + kb * 1024;
@@ -173,7 +173,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
         if (younger) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NDB * 2) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
-    static_assert((2 * KBT) % (2 * NP) == 0 || 2 * KBT < 2 * NP, "whole units per wave");
+    static_assert((2 * KBT) % (2 * NP) == 0, "whole units per wave");
     // LSE and D of a tile: loaded by the first 32 lanes of the first producer wave one iteration before they
     // are written to LDS.
     constexpr bool STAT_ROLE = ROLE == 0;
@@ -500,7 +500,6 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
         int dw_pg[NPASS], dw_t[NPASS];   // pair group and first tap slot
 #pragma unroll
         for (int ps = 0; ps < NPASS; ++ps) { dw_pg[ps] = pr >> 1; dw_t[ps] = (pr & 1) * TH + ps * NU; }
-        constexpr bool dw_wave = true;
         f32x4 acc_k[NDB][DB], acc_v[2][DB];
 #pragma unroll
         for (int m = 0; m < 2; ++m)
@@ -563,7 +562,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
                     SCHED_MFMA_ID(2, 60 + db);
                 });
             }
-                        // packed dC^T of tile u, as the producer's lanes held it (zeros when the tile has none)
+            // packed dC^T of tile u, as the producer's lanes held it (zeros when the tile has none)
             unsigned int cur_dc[NCB][2][2];
             {
                 // read unconditionally: the producer writes zeros for a tile without dC; what the first
@@ -640,11 +639,11 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
             for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
                 for (int f = 0; f < 2; ++f) { prev_dc[cb][f][0] = cur_dc[cb][f][0]; prev_dc[cb][f][1] = cur_dc[cb][f][1]; }
-                        // ---- dW, key blocks jb = 0..3 of the pairs 2 pg and 2 pg + 1 (block jb = dC block jb & 1 of
+            // ---- dW, key blocks jb = 0..3 of the pairs 2 pg and 2 pg + 1 (block jb = dC block jb & 1 of
             // pair 2 pg + jb / 2, keys k0 + 64 pg - 8 + 16 jb ..), tap slots t_lo .. t_lo + TH - 1:
             // G_t[j][j'] += sum_rows dC[row][j] S[row + t - (CQT-1)][j'] with j' in the score block
             // 8 keys before the dC block (x = 0) and the one 8 keys after it (x = 1) ----
-            if (WANT_QW && u_in && dw_wave) static_for<NPASS>([&](auto PS) {
+            if (WANT_QW && u_in) static_for<NPASS>([&](auto PS) {
                 constexpr int ps = decltype(PS)::value;
                 const int pg = dw_pg[ps], t_lo = dw_t[ps];
                 // Ring rows of this lane's two transpose reads at the wave's first tap slot: tile row 0
@@ -717,7 +716,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
                     for (int tt = 0; tt < NU; ++tt) { b0[tt] = b1[tt]; b1[tt] = b2[tt]; }
                 });
             });
-                        if (WANT_KV && v_ok) {
+            if (WANT_KV && v_ok) {
                 const unsigned char *Qs = smem + opaque((unsigned int)(q_slot(v) - smem) + tr_frag_off());
                 const unsigned char *Dsl = smem + opaque((unsigned int)(ds_tile - smem) + tr_lane_off(PST, g, n));
                 asm volatile("" ::: "memory");
@@ -760,7 +759,7 @@ __device__ __forceinline__ void chain_role(const CHAIN_CONST_AS ChainArgs *args_
                 for (int x = 0; x < 2; ++x)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        if (WANT_QW && dw_wave && dw_t[ps] + tt < CQT)
+                        if (WANT_QW && dw_t[ps] + tt < CQT)
                             red[(((dw_pg[ps] * CQT + dw_t[ps] + tt) * 2 + x) * 16 + 4 * g + r) * 16 + n] = acc_w[ps * NU + tt][x][r];
         __syncthreads();  // the producers add the dW partial up while the consumers store dK and dV
 
@@ -893,7 +892,7 @@ hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v
 }
 
 template <int WANT>
-hipError_t pick_shape(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const void *d_o,
+hipError_t pick_out(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const void *d_o,
                       const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv,
                       void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
     if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
@@ -935,7 +934,7 @@ hipError_t dc_scale_finish(const Problem &p, float *dc_scale, hipStream_t s) {
 hipError_t CHAIN_ENTRY(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
                        const void *d_o, const float *Dl, const float *lse, const float *w,
                        const float *dc_scale, void *dk, void *dv, void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
-    return pick_shape<CONVATTN_CHAIN_UNIT>(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    return pick_out<CONVATTN_CHAIN_UNIT>(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 
 }  // namespace convattn
