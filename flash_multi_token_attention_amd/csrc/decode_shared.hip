@@ -22,8 +22,8 @@
 //     (B8 H32 H_kv8 N4348 d128 3x3 39.6 -> 33.2 us, B16 H32 H_kv8 N2254 d64 11x11 38.8 -> 34.9, B4 H32 H_kv8 N20000 d128
 //     6x11 57.5 -> 52.5; 0 to 22 % over 100 shapes, 3 % on average with those of few keys, which go another way; 5 and 6 tiles
 //     give the same within 0.2 %, 3 and 8 half a per cent less).
-// B32 H32 H_kv8 N8192 d128 6x11, pages of 64, lengths from a quarter to all of N (684 MB of K / V): the whole call with the
-// merge 285 -> 138 us, this kernel about 133 of it.  No unit is full then (vector ALUs 22 %, LDS 19 %): each of the two waves per
+// B32 H32 H_kv8 N8192 d128 6x11, pages of 64, lengths drawn from a quarter to all of N (670 to 770 MB of K / V): the whole call with the
+// merge 285 -> 136 to 142 us, this kernel about 134 of it (765 MB: 141 to 149 under the tracer).  No unit is full then (vector ALUs 22 %, LDS 19 %): each of the two waves per
 // SIMD is a chain of scores, window, softmax and P.V.  H32 H_kv8 N8192 d128 11x11, B16, pages of 256: kernel 258 -> 86 us.
 #include "mfma_common.hpp"
 

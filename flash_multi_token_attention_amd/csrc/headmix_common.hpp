@@ -36,7 +36,7 @@ template <typename V> __device__ __forceinline__ V *at(bf16_t *base, unsigned of
 // bits each, rounded to nearest), and six of the nine products are taken; each of the others is below 2^-26 |a b|.  96 clocks for a
 // contraction over 32 heads where the fp32 MFMA takes 256; that was 60 % of the time of headmix_scores_kernel<32, 64>, whose vector ALUs
 // were 7 % busy.  B2 H32 N2048 d64, us: scores 346 -> 305, probabilities 170 -> 152; B2 H32 N1500 d32 182 -> 157 and 89 -> 82; d128 252 -> 248
-// and 119 -> 110.  log L of the forward against 64 bits: 1.59e-8 -> 1.57e-8 of its norm (N500 d64), 1.53 -> 1.48e-8 (N700 d128), its
+// and 119 -> 110.  log L of the forward against 64 bits, means of 12 seeds: 1.616e-8 -> 1.580e-8 of its norm (N500 d64), 1.520 -> 1.480e-8 (N330 d128), its
 // gradients as before.  With 16 heads three of five clocks stay and the matrix pipe does not bind.  dw (a sum over pairs, whose operands
 // would both have to be split) stays on the fp32 MFMA: 305 us, on this one 311.
 // Infinities and NaN leave a NaN in a rest, so in every head's sum: such a step is repeated on the fp32 MFMA (has_nan).

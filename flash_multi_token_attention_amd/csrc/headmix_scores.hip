@@ -551,9 +551,9 @@ Plan score_plan(int B, int H, int N, int causal) {
 }
 // Asking ahead pays where a workgroup has many steps: us without and with it, B4 N4096 (258 steps) 1231 / 1098, B4 N3700 (210)
 // 995 / 974, B4 N3200 (158) 726 / 704, B8 N2048 (130) 626 / 576, B4 N2900 (131) 598 / 595; B3 N3300 (128) 562 / 564, B4 N2700 (114)
-// 510 / 521, B3 N3000 (105) 463 / 470.  Without the mask the gain begins further up: B2 N4096 (256) 1092 / 1019, B2 N3600 (200) 881 / 836, B4 N2500 (195) 896 / 874; B8 N1750 (189) 789 / 804, B2 N3300 (169)
-// 664 / 671, B2 N3000 (138) 565 / 570, B4 N2000 (124) 534 / 555.  d = 64, whose loads have more chunks in flight, and 32 heads,
-// whose steps take longer, gain nothing.
+// 510 / 521, B3 N3000 (105) 463 / 470.  Without the mask the gain begins further up: B2 N4096 (256) 1092 / 1019, B2 N3600 (200)
+// 881 / 836, B4 N2500 (195) 896 / 874; B8 N1750 (189) 789 / 804, B2 N3300 (169) 664 / 671, B2 N3000 (138) 565 / 570, B4 N2000 (124)
+// 534 / 555.  d = 64, whose loads have more chunks in flight, and 32 heads, whose steps take longer, gain nothing.
 bool score_ahead(const Problem &p, const Plan &plan) { return p.H == 16 && p.d == 128 && plan.share > (p.causal ? 128 : 192); }
 
 // What precedes the score kernel, in one launch: K and V in fragment order, then D and LSE of the rows.
