@@ -35,6 +35,7 @@ UNITS = [
     ("staged_fp32.hip", "staged_fp32", []),
     ("reduce_kernels.hip", "reduce_kernels", []),
     ("fwd_reg_mfma.hip", "fwd_reg_mfma", []),
+    ("fwd_reg_mfma.hip", "fwd_reg_mfma_wide", ["-DCONVATTN_FWD_WIDE"]),
     ("bwd_dq_mfma.hip", "bwd_dq_mfma", VGPR_FORM),
     ("bwd_chain_mfma.hip", "bwd_chain_mfma_all", ["-DCONVATTN_CHAIN_UNIT=3"]),
     ("bwd_chain_mfma.hip", "bwd_chain_mfma_kv", ["-DCONVATTN_CHAIN_UNIT=1"]),

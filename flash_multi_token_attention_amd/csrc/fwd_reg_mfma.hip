@@ -11,16 +11,21 @@
 //      one lane address per matrix serves every fragment; one barrier per step);
 //   2. S^T = K Q^T for two 16-key blocks; the accumulator layout (lane = query row, 4 keys per
 //      lane group) is, packed to fp16 after the causal pre-mask, already the B operand layout of
-//      the convolution MFMA: k slots 0..3 of a lane group come from one block, 4..7 from the next
-//      (the Toeplitz bands are built for that order), so a window of 32 input keys is two packed
-//      blocks and the output block sits 8 keys into it.  The last block of a step is carried to
-//      the next step; no score is computed twice along the keys;
-//   3. convolution: C^T += T_a^T S^T(rows shifted by the tap).  A shift by an even number of
-//      rows is a DPP row shift of the packed registers, by an odd number the other fragment
-//      shifted; rows shifted in from above the wave's first row are zeros and only reach halo rows;
+//      the convolution MFMA: a window of 32 input keys is two packed blocks side by side in a lane
+//      and the output block sits 8 keys into it.  The last block of a step stays for the next
+//      step; no score is computed twice along the keys;
+//   3. convolution: C^T += T_a^T S^T(rows shifted by the tap), two taps per sparse product (SparseTaps).
+//      A shift by an even number of rows is a DPP row shift of the packed registers, by an odd number
+//      the other fragment shifted; rows shifted in from above the wave's first row are zeros and only
+//      reach halo rows.  A block's shifted rows are made once and kept for both windows it is in.
+//      What bounds the kernel is the issue of vector instructions (63 % of the cycles at B4 H16 N4096 d64 6x11)
+//      beside the matrix pipe (52 %), at a clock of 1.8 GHz.  Dense products of one tap each, whose windows were
+//      shifted anew and whose bands every lane gathered from memory, against these, us: B4 H16 N4096 6x11 d128
+//      440 -> 392, N2048 d64 88 -> 75, B1 H32 N5399 d64 11x11 452 -> 360, B4 H16 N4096 d64 7x7 357 -> 299, B1 H32 N4096 d64
+//      3x3 119 -> 110, B2 H8 N526 d32 6x11 14.5 -> 11.9;
 //   4. post-mask (-inf) and softmax numerators against a per-row base that is only raised (with
 //      a rescale of O and the row sums) when a score exceeds it by more than 2^6: no cross-lane
-//      traffic otherwise.  The true row maximum is kept per lane for the M output;
+//      traffic otherwise.  The true row maximum is kept per lane, relative to the base, for the M output;
 //   5. O^T += V^T P^T: V^T fragments through the LDS transpose read, P^T straight from the
 //      softmax registers.
 #include "mfma_common.hpp"
@@ -86,11 +91,15 @@ template <int BQ> inline int fwd_wgs(const Problem &p, int share) {
     return n;
 }
 
+// Waves per SIMD that the registers have to leave room for: windows of up to 6 slots fit three (168 registers) up to d = 64.  Forced to
+// three, 7 and 8 slots spill 8 to 15 registers (B4 H16 N4096 d64 7x7 299 -> 350 us, 8x9 324 -> 354); four at d = 32 with 3 slots: 19.0 -> 19.4.
+constexpr int fwd_waves(int d, int cqt) { return d <= 64 && cqt <= 6 ? 3 : 2; }
 // (SPLIT: an instance of its own, the other one is a percent slower with the parts' bounds at run time)
 // LONG: the tiles from split.first_long on run at a higher wave priority (long_tiles_first)
 enum { PLAIN, SPLIT_KEYS, LONG };
-template <int D, int CQT, typename TO, int FORM>
-__global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
+// WIDE: windows of 17 key taps, whose band the sparse product cannot hold (each tap a dense product of its own)
+template <int D, int CQT, typename TO, int FORM, bool WIDE>
+__global__ __launch_bounds__(NW * 64, fwd_waves(D, CQT)) void fwd_reg_mfma_kernel(
     Problem p, FwdSplit split, const bf16_t *__restrict__ Q, const bf16_t *__restrict__ K,
     const bf16_t *__restrict__ V, const float *__restrict__ W, TO *__restrict__ O,
     float *__restrict__ M, float *__restrict__ L) {
@@ -124,33 +133,38 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     const bf16_t *Kb = K + bh * p.Nk * D;
     const bf16_t *Vb = V + bh * p.Nk * D;
 
-    // Toeplitz bands of this head, one fragment per tap slot, pre-multiplied by
-    // scale * log2(e): the convolved scores come out in log2 units.  k slot 8g+e of a window
-    // is key 4g+e of its first 16-key block for e < 4, key 4g+e-4 of its second for e >= 4.
-    f16x8 tf[CQT];
+    const int all_steps = fwd_steps<BQ>(p, qt), parts = SPLIT ? fwd_parts(all_steps, split.share) : 1;
+    const int u_lo = SPLIT ? all_steps * part_no / parts : 0, n_steps = SPLIT ? all_steps * (part_no + 1) / parts : all_steps;   // this workgroup's steps
+    // (a part that does not begin with the first step takes the scores of the step before it along the way: the window
+    // needs the last block of them)
+    const int u_first = SPLIT ? max(u_lo - 1, 0) : 0;
+
+    // Toeplitz bands of this head, pre-multiplied by scale * log2(e): the convolved scores come out in log2 units.  WIDE: k slot
+    // 8g+e of a window is key 4g+e of its first 16-key block for e < 4, key 4g+e-4 of its second for e >= 4.
+    // (11 slots at d = 128 have no registers for the dense operands of the single slots)
+    constexpr bool DENSE_SINGLE = CQT <= 7 || D <= 64;
+    using Taps = SparseTaps<CQT, DENSE_SINGLE>;
+    f16x8 tf[WIDE ? CQT : 1];
+    SparseBands<CQT, DENSE_SINGLE> bands;
+    int index[2] = {0, 0};   // of the windows that end with a step's first and second score block
     {
-        const float *w_head = W + (size_t)h * cq * p.c_k;
-        // (unconditional loads from clamped indices, all in flight together; the select happens on the values)
-        float wv[CQT][8];
+        // (the table lies in the K / V buffer that the first step does not use)
+        static_assert(band_table_bytes<CQT>() <= Lds::buf_bytes, "room for the table");
+        unsigned int *tab = reinterpret_cast<unsigned int *>(smem + ((u_first & 1) ^ 1) * Lds::buf_bytes);
+        band_table_build<CQT>(tab, W + (size_t)h * cq * p.c_k, cq, p.c_k, pk, false, p.scale * kLog2e, tid, NW * 64);
+        __syncthreads();
+        if constexpr (WIDE) {
 #pragma unroll
-        for (int t = 0; t < CQT; ++t) {
-            const int a = t - (CQT - cq);
+            for (int t = 0; t < CQT; ++t) {
+                u32x4 v;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int kappa = e < 4 ? 4 * g + e : 16 + 4 * g + e - 4;
-                const int bb = kappa - kKeyHalo - n + pk;
-                wv[t][e] = w_head[max(a, 0) * p.c_k + min(max(bb, 0), p.c_k - 1)];
+                for (int q = 0; q < 4; ++q) v[q] = tab[t * kBandRow + 4 * g + 2 * (q & 1) + (q >> 1) * 16 - n + 16];
+                tf[t] = __builtin_bit_cast(f16x8, v);
             }
-        }
-#pragma unroll
-        for (int t = 0; t < CQT; ++t) {
-            const int a = t - (CQT - cq);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int kappa = e < 4 ? 4 * g + e : 16 + 4 * g + e - 4;
-                const int bb = kappa - kKeyHalo - n + pk;
-                tf[t][e] = (_Float16)((a >= 0 && bb >= 0 && bb < p.c_k) ? wv[t][e] * (p.scale * kLog2e) : 0.f);
-            }
+        } else {
+            bands.read(tab, g, n);
+            index[0] = sparse_index(g, n, true);
+            index[1] = sparse_index(g, n, false);
         }
     }
 
@@ -170,7 +184,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
 #pragma unroll
         for (int db = 0; db < DB; ++db) acc_o[ob][db] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float m_ref[2] = {kNegInf, kNegInf};   // exponent base of the row, in log2 units (same in the row's 4 lanes)
-    float m_true[2] = {kNegInf, kNegInf};  // maximum of the scores this lane has seen
+    float m_rel[2] = {kNegInf, kNegInf};   // maximum of the scores this lane has seen, relative to m_ref (or 0)
     // The convolution accumulates on top of minus the exponent base (0 while the row has none),
     // so its result is already the exponent; slack[ob]: how far it may go above 0 before the base
     // is raised (-inf while the row has no base: any visible score sets one).
@@ -250,6 +264,25 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
     // packed fp16 scores of the last score block of the previous step:
     // carry[f][dword] = row base + 2n + f, keys 4g .. 4g+3 of the block
     unsigned int carry[2][2] = {{0u, 0u}, {0u, 0u}};
+    // The sparse products' operands, kept from step to step: a step's first score block has the even dwords of the tuples, its
+    // second one the odd ones, and each takes the place of the block two before it.  Every row offset of a block is made once
+    // (CQT - 1 DPP moves of two dwords) and serves the two windows the block is in.
+    u32x8 rows[WIDE ? 1 : Taps::tuples];
+    if constexpr (!WIDE)
+#pragma unroll
+        for (int j = 0; j < Taps::tuples; ++j) rows[j] = (u32x8)0u;
+    // dwords of tuple j from the packed scores pd[f][dword] of a block
+    auto put_rows = [&](auto J, auto BLK, const unsigned int (&pd)[2][2]) {
+        constexpr int j = decltype(J)::value, blk = decltype(BLK)::value;
+        static_for<2>([&](auto HALF) {
+            constexpr int half = decltype(HALF)::value, delta = Taps::delta(j, half), f = delta & 1, s = (f - delta) / 2;
+#pragma unroll
+            for (int dw = 0; dw < 2; ++dw) {
+                if constexpr (s == 0) rows[j][4 * half + 2 * dw + blk] = pd[f][dw];
+                else rows[j][4 * half + 2 * dw + blk] = dpp_zero<0x110 + s>(pd[f][dw]);
+            }
+        });
+    };
 
     // One step of the wave; EDGE = the step touches the diagonal or an end of the keys
     // (wave-uniform), only then are the masks evaluated.
@@ -278,7 +311,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
             if constexpr (blk == 0) {
                 load_kf(1);
                 SCHED_DS_READ(KS);
-                SCHED_MFMA(2 * CQT);
+                SCHED_MFMA(WIDE ? 2 * CQT : 2 * (Taps::products + Taps::ONE));
             }
             const int key0 = jk + blk * 16 + 4 * g;
 #pragma unroll
@@ -302,7 +335,30 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
             //      before, 4..7 from this one ----
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) c[ob][blk] = neg_base[ob];
-            static_for<CQT + 1>([&](auto DL) {
+            if constexpr (!WIDE) {
+                auto single = [&](auto OB) {   // (the first product of its parity)
+                    constexpr int ob = decltype(OB)::value, j = Taps::single_tuple(ob);
+                    const u32x4 bv = {rows[j][4 * ob], rows[j][4 * ob + 1], rows[j][4 * ob + 2], rows[j][4 * ob + 3]};
+                    c[ob][blk] = mfma_f16(bands.one[Taps::ONE ? blk : 0][ob], __builtin_bit_cast(f16x8, bv), c[ob][blk]);
+                };
+                if constexpr (Taps::ONE) {
+                    put_rows(std::integral_constant<int, Taps::tuples - 1>{}, BL, pd[blk]);
+                    single(std::integral_constant<int, 0>{});
+                }
+                static_for<Taps::tuples>([&](auto J) {
+                    constexpr int j = decltype(J)::value;
+                    if constexpr (!Taps::ONE || j < Taps::tuples - 1) put_rows(J, BL, pd[blk]);
+                    if constexpr (Taps::ONE && j == 0) single(std::integral_constant<int, 1>{});
+                    static_for<2>([&](auto OB) {
+                        constexpr int ob = decltype(OB)::value;
+                        static_for<Taps::products>([&](auto I) {
+                            constexpr int i = decltype(I)::value;
+                            if constexpr (Taps::tuple(i, ob) == j) c[ob][blk] = smfmac_f16(bands.band[ob][i], rows[j], c[ob][blk], index[blk]);
+                        });
+                    });
+                });
+            }
+            else static_for<CQT + 1>([&](auto DL) {
                 constexpr int delta = decltype(DL)::value - (CQT - 1);
                 constexpr int f = delta & 1, s = (f - delta) / 2;
                 u32x4 bv;
@@ -319,10 +375,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
                 if constexpr (t0 >= 1) c[1][blk] = mfma_f16(tf[t0 - 1], __builtin_bit_cast(f16x8, bv), c[1][blk]);
             });
         });
+        if constexpr (WIDE)
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+            for (int f = 0; f < 2; ++f)
 #pragma unroll
-            for (int dw = 0; dw < 2; ++dw) carry[f][dw] = pd[1][f][dw];
+                for (int dw = 0; dw < 2; ++dw) carry[f][dw] = pd[1][f][dw];
         // V^T fragments of the first kFwdPfv head-dim blocks: in flight during the softmax
         constexpr int PFV = kFwdPfv < DB ? kFwdPfv : DB;
         bf16x8 vf[PFV + 1];
@@ -341,7 +398,6 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         //      only follows the row's maximum when some score exceeds it by more than kMaxSlack
         //      (then every lane group of the wave exchanges its maxima and rescales); otherwise no
         //      lane talks to another.  The true maximum is tracked per lane for the M output. ----
-        float mloc[2];
 #pragma unroll
         for (int ob = 0; ob < 2; ++ob) {
             if constexpr (EDGE) {
@@ -354,19 +410,17 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
                         if (key < 0 || key >= p.Nk || (causal && key > qpos)) c[ob][kb][r] = kNegInf;
                     }
             }
-            float mx = kNegInf;
+            // (the maximum so far never lies above the slack, so the test below may include it)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, c[ob][kb][r]);
-            mloc[ob] = mx;                                           // relative to the base
-            m_true[ob] = fmaxf(m_true[ob], mx - neg_base[ob][0]);   // absolute
+                for (int r = 0; r < 4; ++r) m_rel[ob] = fmaxf(m_rel[ob], c[ob][kb][r]);
         }
-        if (__builtin_amdgcn_ballot_w64(mloc[0] > slack[0] || mloc[1] > slack[1]) != 0) {
+        if (__builtin_amdgcn_ballot_w64(m_rel[0] > slack[0] || m_rel[1] > slack[1]) != 0) {
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) {
                 const float old_use = -neg_base[ob][0];
-                float mx = mloc[ob] + old_use;
+                float mx = m_rel[ob] + old_use;
                 mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
                 mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
                 const float m_new = fmaxf(m_ref[ob], mx);
@@ -375,6 +429,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
                 const float alpha = fast_exp2(m_ref[ob] - new_use);
                 const float delta = new_use - old_use;
                 m_ref[ob] = m_new;
+                m_rel[ob] -= delta;
                 slack[ob] = (m_new == kNegInf) ? kNegInf : kMaxSlack;
                 neg_base[ob] = (f32x4){-new_use, -new_use, -new_use, -new_use};
                 l_run[ob] *= alpha;
@@ -423,11 +478,6 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         }
     };
 
-    const int all_steps = fwd_steps<BQ>(p, qt), parts = SPLIT ? fwd_parts(all_steps, split.share) : 1;
-    const int u_lo = SPLIT ? all_steps * part_no / parts : 0, n_steps = SPLIT ? all_steps * (part_no + 1) / parts : all_steps;   // this workgroup's steps
-    // (a part that does not begin with the first step takes the scores of the step before it along the way: the window
-    // needs the last block of them)
-    const int u_first = SPLIT ? max(u_lo - 1, 0) : 0;
     fetch_step(u_first);
     if constexpr (SPLIT) {
         const int to_first = (u_first & 1) * Lds::buf_bytes;
@@ -453,6 +503,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
             carry[f][0] = two[0];
             carry[f][1] = two[1];
         }
+        if constexpr (!WIDE) static_for<Taps::tuples>([&](auto J) { put_rows(J, std::integral_constant<int, 1>{}, carry); });
     };
     // Along the keys a wave's steps are: step 0 (keys before the first one to mask), steps whose
     // keys all lie at or before its first score row (no masks), steps on the diagonal or at the
@@ -488,7 +539,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_reg_mfma_kernel(
         float l = l_run[ob];
         l += __shfl_xor(l, 16, kWave);
         l += __shfl_xor(l, 32, kWave);
-        float mt = m_true[ob];
+        float mt = m_rel[ob] - neg_base[ob][0];
         mt = fmaxf(mt, __shfl_xor(mt, 16, kWave));
         mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));
         const int qpos = base + 2 * n + ob;
@@ -625,20 +676,20 @@ template <int BQ> bool long_tiles_first(const Problem &p) {
     return p.causal && 5 * wgs > 7 * round && wgs <= 2 * round && 10 * wgs * tiles <= (21 * tiles - 30) * round;   // (up to 2.1 - 3 / tiles rounds)
 }
 
-template <int D, int CQT, typename TO>
+template <int D, int CQT, typename TO, bool WIDE>
 hipError_t launch_fwd(const Problem &p, float *part, const void *q, const void *k, const void *v, const float *w,
                       void *o, float *m, float *l, hipStream_t s) {
     constexpr int lds = FwdLds<D>::total, BQ = NW * wave_rows(CQT);
     if (lds > 64 * 1024) {
-        hipError_t e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, PLAIN>>(lds);
-        if (e == hipSuccess) e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS>>(lds);
+        hipError_t e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, PLAIN, WIDE>>(lds);
+        if (e == hipSuccess) e = set_max_lds_once<fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS, WIDE>>(lds);
         if (e != hipSuccess) return e;
     }
     const FwdSplit split{part ? fwd_share<BQ>(p) : 0, (p.Nq + BQ - 1) / BQ / 2, part};
     const int n_wg = fwd_wgs<BQ>(p, split.share);
-    auto kern = split.share ? fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS> : fwd_reg_mfma_kernel<D, CQT, TO, PLAIN>;
+    auto kern = split.share ? fwd_reg_mfma_kernel<D, CQT, TO, SPLIT_KEYS, WIDE> : fwd_reg_mfma_kernel<D, CQT, TO, PLAIN, WIDE>;
     if constexpr (has_long(D, CQT))
-        if (!split.share && long_tiles_first<BQ>(p)) kern = fwd_reg_mfma_kernel<D, CQT, TO, LONG>;
+        if (!split.share && long_tiles_first<BQ>(p)) kern = fwd_reg_mfma_kernel<D, CQT, TO, LONG, WIDE>;
     kern<<<dim3(p.H, p.B, n_wg), NW * 64, lds, s>>>(p, split, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, w, (TO *)o, m, l);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !split.share) return e;
@@ -649,15 +700,15 @@ hipError_t launch_fwd(const Problem &p, float *part, const void *q, const void *
     return hipGetLastError();
 }
 
-template <int D, typename TO>
+template <int D, typename TO, bool WIDE>
 hipError_t pick_cq(const Problem &p, float *part, const void *q, const void *k, const void *v, const float *w,
                    void *o, float *m, float *l, hipStream_t s) {
-    if (p.c_q <= 3) return launch_fwd<D, 3, TO>(p, part, q, k, v, w, o, m, l, s);
-    if (p.c_q <= 6) return launch_fwd<D, 6, TO>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 3) return launch_fwd<D, 3, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 6) return launch_fwd<D, 6, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
     // (7 taps in 8 slots: B2 H12 N4691 d128 7x7 281 us, in 7 266)
-    if (p.c_q <= 7) return launch_fwd<D, 7, TO>(p, part, q, k, v, w, o, m, l, s);
-    if (p.c_q <= 8) return launch_fwd<D, 8, TO>(p, part, q, k, v, w, o, m, l, s);
-    return launch_fwd<D, 11, TO>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 7) return launch_fwd<D, 7, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_q <= 8) return launch_fwd<D, 8, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
+    return launch_fwd<D, 11, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
 }
 
 template <int CQT> size_t split_bytes(const Problem &p) {
@@ -666,8 +717,31 @@ template <int CQT> size_t split_bytes(const Problem &p) {
     return share ? (size_t)p.B * p.H * fwd_wgs<BQ>(p, share) * BQ * (p.d + 4) * sizeof(float) : 0;
 }
 
+template <bool WIDE>
+hipError_t pick_shape(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
+                      const float *w, void *o, float *m, float *l, hipStream_t s, float *part) {
+    if (p.d == 128) {
+        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t, WIDE>(p, part, q, k, v, w, o, m, l, s);
+        return pick_cq<128, float, WIDE>(p, part, q, k, v, w, o, m, l, s);
+    }
+    if (p.d == 32) {
+        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t, WIDE>(p, part, q, k, v, w, o, m, l, s);
+        return pick_cq<32, float, WIDE>(p, part, q, k, v, w, o, m, l, s);
+    }
+    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t, WIDE>(p, part, q, k, v, w, o, m, l, s);
+    return pick_cq<64, float, WIDE>(p, part, q, k, v, w, o, m, l, s);
+}
+
 }  // namespace
 
+// This file is compiled twice, the second time (CONVATTN_FWD_WIDE) for the windows of 17 key taps, so that the two sets of instances
+// build in parallel.
+#ifdef CONVATTN_FWD_WIDE
+hipError_t mfma_fwd_wide(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
+                         const float *w, void *o, float *m, float *l, hipStream_t s, float *part) {
+    return pick_shape<true>(p, out_dt, q, k, v, w, o, m, l, s, part);
+}
+#else
 size_t mfma_fwd_split_bytes(const Problem &p) {
     return p.c_q <= 3   ? split_bytes<3>(p)
            : p.c_q <= 6 ? split_bytes<6>(p)
@@ -678,16 +752,9 @@ size_t mfma_fwd_split_bytes(const Problem &p) {
 
 hipError_t mfma_fwd(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
                     const float *w, void *o, float *m, float *l, hipStream_t s, float *part) {
-    if (p.d == 128) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<128, bf16_t>(p, part, q, k, v, w, o, m, l, s);
-        return pick_cq<128, float>(p, part, q, k, v, w, o, m, l, s);
-    }
-    if (p.d == 32) {
-        if (out_dt == CONVATTN_BF16) return pick_cq<32, bf16_t>(p, part, q, k, v, w, o, m, l, s);
-        return pick_cq<32, float>(p, part, q, k, v, w, o, m, l, s);
-    }
-    if (out_dt == CONVATTN_BF16) return pick_cq<64, bf16_t>(p, part, q, k, v, w, o, m, l, s);
-    return pick_cq<64, float>(p, part, q, k, v, w, o, m, l, s);
+    if (p.c_k > kSparseMaxCk) return mfma_fwd_wide(p, out_dt, q, k, v, w, o, m, l, s, part);
+    return pick_shape<false>(p, out_dt, q, k, v, w, o, m, l, s, part);
 }
+#endif
 
 }  // namespace convattn

@@ -22,11 +22,14 @@ namespace convattn {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x8 __attribute__((ext_vector_type(8)));
 // Five consecutive dwords at a 4-byte boundary of LDS, as 32-bit reads (the compiler pairs them
 // into ds_read2_b32).  A 128-bit LDS read that is not 16-byte aligned is legal on gfx950 but slow:
 // measured with four waves reading, one costs about 66 clocks of the LDS pipe against about 12 for
@@ -48,6 +51,108 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 __device__ __forceinline__ f32x4 mfma_f16(f16x8 a, f16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
+
+// ---- The window of two query taps as one sparse matrix product ----
+// v_smfmac_f32_16x16x64_f16 takes the issue time of the dense 16x16x32 (16.5 clocks per SIMD measured for both, one to four waves)
+// and twice its k: of every four consecutive k of the B operand each row of A uses two, which two an index says.  A band of at
+// most 15 keys fits that: of the keys kappa and kappa + 16 of a 32-key window an output key sees one at most.  With a dword (two
+// keys) of the window's first 16-key block beside the same dword of its second, every group of four k is {kappa, kappa + 1,
+// kappa + 16, kappa + 17}, and a row takes the first two or the last two.  Output key n sees the window's keys n + 1 .. n + 15,
+// so it takes the first block's keys kappa, kappa + 1 where kappa + 1 > n and the second block's otherwise.
+//
+// B operand of lane (g, n): dwords 0..3 belong to the first tap, 4..7 to the second, each as {first block keys 4g, 4g+1; second
+// block the same; first block keys 4g+2, 4g+3; second block}.  The two blocks may also stand the other way round, with the other index:
+// a window that moves on by one block replaces the dwords of its older block only.
+// A operand of lane (g, n): row n, the first tap for g < 2 and the second for the rest; its element 2q + e, q = 0..3, is key
+// 4 (2 (g & 1) + q / 2) + 2 (q & 1) + e of the block the row takes; the index has 4 bits for each q.
+__device__ __forceinline__ f32x4 smfmac_f16(f16x8 a, u32x8 b, f32x4 c, int index) {
+    return __builtin_amdgcn_smfmac_f32_16x16x64_f16(a, __builtin_bit_cast(f16x16, b), c, index, 0, 0);
+}
+constexpr int kSparseMaxCk = 15;
+__device__ __forceinline__ int sparse_key(int g, int q) { return 4 * (2 * (g & 1) + (q >> 1)) + 2 * (q & 1); }
+// index of a lane where the window's first block has the even dwords (`swapped`: the odd ones)
+__device__ __forceinline__ int sparse_index(int g, int n, bool swapped) {
+    int v = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v |= (((sparse_key(g, q) + 1 > n) != swapped) ? 0x4 : 0xE) << (4 * q);
+    return v;
+}
+// Which taps share a product.  A window of CQT tap slots needs, for output rows of parity ob = 0 and 1, the score rows at
+// offsets delta = slot - (CQT - 1) + ob, CQT + 1 of them.  Operand tuple j holds the offsets delta(j, 0) and delta(j, 1).  For an odd
+// CQT the tuples hold all offsets in pairs, and one slot of each parity stays single: a dense product of four dwords of a tuple,
+// which also brings the chain's starting value with it (ONE), or half of a sparse one (16 registers less).  For an even CQT they hold
+// the offsets of parity 1, and parity 0 has, for its first and its last slot, a tuple of its own in the place of the last one.
+template <int CQT, bool DENSE_SINGLE> struct SparseTaps {
+    static constexpr bool odd = CQT % 2 != 0, ONE = odd && DENSE_SINGLE;
+    static constexpr int tuples = odd ? (CQT + 1) / 2 : CQT / 2 + 1;        // operand tuples
+    static constexpr int products = odd && !ONE ? (CQT + 1) / 2 : CQT / 2;  // sparse products per output parity
+    static constexpr int delta(int j, int half) {
+        return !odd && j == CQT / 2 ? (half ? 0 : -(CQT - 1)) : -(CQT - (odd ? 1 : 2)) + 2 * j + half;
+    }
+    // tuple of product i of parity ob
+    static constexpr int tuple(int i, int ob) { return odd ? (ONE ? i + ob : i) : !ob && i == CQT / 2 - 1 ? CQT / 2 : i; }
+    // tap slot of a half of tuple j for parity ob; the table's row CQT (zeros) where it has none
+    static constexpr int slot(int j, int half, int ob) {
+        const int t = delta(j, half) + CQT - 1 - ob;
+        return t < 0 || t >= CQT ? CQT : t;
+    }
+    // the single slot of a parity (ONE): half ob of this tuple
+    static constexpr int single_tuple(int ob) { return ob ? 0 : tuples - 1; }
+    static constexpr int single_slot(int ob) { return slot(single_tuple(ob), ob, ob); }
+};
+// The bands of a head as a table in LDS: dword x + 16 of tap slot t's 48 holds the weights of two neighbouring keys, T[x] and T[x + 1]
+// with T[x] = w[a][pk + x - 8] * mul (`flip`: pk - (x - 8); zero outside the window), x = the key's place in the window less the output
+// key's; slot t stands for tap a = t - (CQT - c_q), and one more slot of zeros follows.  A lane finds the pairs of its operands there with
+// 4-byte reads: one or two loads of W per thread instead of the 48 to 88 gathers of every lane.
+constexpr int kBandRow = 48;
+template <int CQT> constexpr int band_table_bytes() { return (CQT + 1) * kBandRow * 4; }
+template <int CQT>
+__device__ __forceinline__ void band_table_build(unsigned int *tab, const float *__restrict__ w_head, int c_q, int c_k, int pk, bool flip,
+                                                 float mul, int tid, int nthreads) {
+    for (int i = tid; i < (CQT + 1) * kBandRow; i += nthreads) {
+        const int t = i / kBandRow, a = t - (CQT - c_q), off = i - t * kBandRow - 16 - kKeyHalo;
+        float v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int b = flip ? pk - off - e : pk + off + e;
+            v[e] = w_head[min(max(a, 0), c_q - 1) * c_k + min(max(b, 0), c_k - 1)];
+            v[e] = t < CQT && a >= 0 && b >= 0 && b < c_k ? v[e] * mul : 0.f;
+        }
+        const f16x2 two = {(_Float16)v[0], (_Float16)v[1]};
+        tab[i] = __builtin_bit_cast(unsigned int, two);
+    }
+}
+// The A operands of both parities: band[ob][i] of product i, one[w][ob] of the single slot where the window's first block has the
+// odd (w = 0) or the even (w = 1) dwords.
+template <int CQT, bool DENSE_SINGLE> struct SparseBands {
+    using T = SparseTaps<CQT, DENSE_SINGLE>;
+    f16x8 band[2][T::products], one[T::ONE ? 2 : 1][2];
+    __device__ __forceinline__ void read(const unsigned int *tab, int g, int n) {
+#pragma unroll
+        for (int ob = 0; ob < 2; ++ob) {
+#pragma unroll
+            for (int i = 0; i < T::products; ++i) {
+                const int j = T::tuple(i, ob);
+                u32x4 v;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int kappa = sparse_key(g, q), x = kappa + (kappa + 1 > n ? 0 : 16) - n;
+                    v[q] = tab[(g < 2 ? T::slot(j, 0, ob) : T::slot(j, 1, ob)) * kBandRow + x + 16];
+                }
+                band[ob][i] = __builtin_bit_cast(f16x8, v);
+            }
+            if constexpr (T::ONE)
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    u32x4 v;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        v[q] = tab[T::single_slot(ob) * kBandRow + 4 * g + 2 * (q >> 1) + ((q & 1) == w ? 16 : 0) - n + 16];
+                    one[w][ob] = __builtin_bit_cast(f16x8, v);
+                }
+        }
+    }
+};
 
 // Scheduling hints: the sequence of these calls in program order is the order in which the
 // backend lays out groups of LDS reads and MFMAs.  Used as "reads of stage s+1, then MFMAs
@@ -246,6 +351,9 @@ inline hipError_t set_max_lds_once(int bytes) {
 // ---- bf16 MFMA kernels ----
 hipError_t mfma_fwd(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
                     const float *w, void *o, float *m, float *l, hipStream_t s, float *part = nullptr);
+// the same for windows of more than kSparseMaxCk key taps (mfma_fwd calls it)
+hipError_t mfma_fwd_wide(const Problem &p, int out_dt, const void *q, const void *k, const void *v,
+                         const float *w, void *o, float *m, float *l, hipStream_t s, float *part);
 // room for the parts of the query tiles whose keys several workgroups share (`part` above), 0 where none do
 size_t mfma_fwd_split_bytes(const Problem &p);
 
