@@ -17,6 +17,12 @@
 // One workgroup barrier per tile.  With 168 registers per wave every role keeps its operands and
 // accumulators in registers, and a SIMD always has two other waves to issue from while one waits
 // for LDS data, the matrix pipe or the barrier.
+// What bounds it: a score wave's chain per tile alone takes two thirds of the kernel's time (d = 64, 6 taps: 680 of 1020 us with the
+// other roles' work left out), the other roles as much without it, and together they share the LDS (two thirds busy), the matrix
+// pipe and the vector ALUs.  So both convolutions take two tap slots per sparse product (SparseTaps in mfma_common.hpp), the key
+// waves keep their bands in registers, and dW's operands of neighbouring taps share their transpose reads (43 per wave and tile for
+// 56 at 6 slots, 61 for 112 at 11).  Kernel alone, B4 H16 N4096 causal, before -> after, us, in turn on one card: d 128 6x11 1409 -> 1310,
+// d 64 6x11 1097 -> 1048, 11x11 1442 -> 1283, 3x3 833 -> 804.
 #include <type_traits>
 
 #include "chain_common.hpp"
@@ -42,8 +48,8 @@ constexpr int NT3 = 3 * NP * 64;  // 768 threads
 #endif
 // LDS: the layout of the two-role kernel, then the V fragments of the block after the workgroup's keys
 // (16 rows; the wave that computes that block has no registers to keep them in)
-template <int D, int CQT> struct Chain3Lds : ChainLds<D, CQT> {
-    static constexpr int e_off = ChainLds<D, CQT>::total;
+template <int D, int CQT> struct Chain3Lds : ChainLds<D, CQT, true> {
+    static constexpr int e_off = ChainLds<D, CQT, true>::total;
     static constexpr int e_bytes = 16 * D * 2;
     static constexpr int total3 = e_off + e_bytes;
 };
@@ -237,6 +243,8 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
             for (int ks = 0; ks < KS; ++ks)
                 q_above[f][ks] = __builtin_bit_cast(bf16x8, load_row16_nb<D>(Qb, r_begin - BR + 2 * n + f, p.Nq, ks * 32 + g * 8));
 
+        using Taps = ChainTaps<CQT>;
+        const int sp_index = sparse_index(g, n, false);
         unsigned int prev_pd[NKB][2][2];
         // S^T of the 32 rows r0 .. r0+31 (ring tile tp), pre-masked, packed and stored for dW
         auto s_phase = [&](int r0, int tp, unsigned int (&pd)[NKB][2][2], auto edge_tag, auto &&load_qf) {
@@ -319,44 +327,17 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
                 if constexpr (FULL) {
                     unsigned char *Cs = c_stage(it), *Ps = p_stage(it);
-                    // ---- convolution: C^T block cb from score blocks cb (k slots 0..3 of a lane
-                    // group) and cb+1 (4..7).  Operand of row offset delta = DL - (CQT-1): fragment
-                    // f = delta & 1 shifted s = (f - delta) / 2 lanes down; it serves output parity
-                    // 0 with tap slot DL and parity 1 with tap slot DL - 1. ----
+                    // ---- convolution: C^T block cb from score blocks cb and cb+1, two tap slots per sparse product.
+                    // Operand of row offset delta: fragment f = delta & 1 shifted s = (f - delta) / 2 lanes down.  Block 2
+                    // takes the place of block 0 in an operand tuple (the other index). ----
                     f32x4 c[NCBL][2];
 #pragma unroll
                     for (int cb = 0; cb < NCBL; ++cb) {
                         c[cb][0] = (f32x4){-l2.x, -l2.x, -l2.x, -l2.x};
                         c[cb][1] = (f32x4){-l2.y, -l2.y, -l2.y, -l2.y};
                     }
-                    f16x8 tf_prev = (f16x8)(_Float16)0.f;
-                    static_for<CQT + 1>([&](auto DL) {
-                        constexpr int t0 = decltype(DL)::value;
-                        constexpr int delta = t0 - (CQT - 1);
-                        constexpr int f = delta & 1, s = (f - delta) / 2;
-                        f16x8 tf_cur = tf_prev;
-                        if constexpr (t0 < CQT) tf_cur = *reinterpret_cast<const f16x8 *>(bands + t0 * 1024);
-                        unsigned int sh[NKB][2];
-#pragma unroll
-                        for (int kb = CB0 - KB0; kb < CB0 - KB0 + NCBL + 1; ++kb)
-#pragma unroll
-                            for (int dw = 0; dw < 2; ++dw) sh[kb][dw] = win_up<s>(prev_pd[kb][f][dw], pd[kb][f][dw]);
-#pragma unroll
-                        for (int cb = 0; cb < NCBL; ++cb) {
-                            constexpr int o = CB0 - KB0;
-                            const u32x4 bv = {sh[o + cb][0], sh[o + cb][1], sh[o + cb + 1][0], sh[o + cb + 1][1]};
-                            if constexpr (t0 < CQT) c[cb][0] = mfma_f16(tf_cur, __builtin_bit_cast(f16x8, bv), c[cb][0]);
-                            if constexpr (t0 >= 1) c[cb][1] = mfma_f16(tf_prev, __builtin_bit_cast(f16x8, bv), c[cb][1]);
-                        }
-                        tf_prev = tf_cur;
-                    });
-#pragma unroll
-                    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                        for (int f = 0; f < 2; ++f) { prev_pd[kb][f][0] = pd[kb][f][0]; prev_pd[kb][f][1] = pd[kb][f][1]; }
                     // ---- dP^T = V dO^T - D, after the convolution (the shifted score windows are no longer live) ----
-                    if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
-                    {
+                    auto dp_phase = [&] {
                         const float2 d2 = *reinterpret_cast<const float2 *>(stat_slot(it) + BR + 2 * n);
 #pragma unroll
                         for (int cb = 0; cb < NCBL; ++cb) {
@@ -377,7 +358,37 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                                 for (int f = 0; f < 2; ++f) dp[cb][f] = mfma_bf16(vk, gf[f], dp[cb][f]);
                             }
                         }
-                    }
+                    };
+                    static_for<Taps::tuples>([&](auto J) {
+                        constexpr int j = decltype(J)::value;
+                        u32x8 rows;
+                        auto put = [&](auto KB, auto POS) {   // score block KB to the even (POS 0) or the odd dwords
+                            static_for<2>([&](auto HALF) {
+                                constexpr int half = decltype(HALF)::value, delta = Taps::delta(j, half), f = delta & 1, s = (f - delta) / 2;
+#pragma unroll
+                                for (int dw = 0; dw < 2; ++dw)
+                                    rows[4 * half + 2 * dw + decltype(POS)::value] = win_up<s>(prev_pd[decltype(KB)::value][f][dw], pd[decltype(KB)::value][f][dw]);
+                            });
+                        };
+                        put(std::integral_constant<int, CB0 - KB0>{}, std::integral_constant<int, 0>{});
+                        put(std::integral_constant<int, CB0 - KB0 + 1>{}, std::integral_constant<int, 1>{});
+                        static_for<NCBL>([&](auto CB) {
+                            constexpr int cb = decltype(CB)::value;
+                            if constexpr (cb > 0) put(std::integral_constant<int, CB0 - KB0 + cb + 1>{}, std::integral_constant<int, (cb + 1) % 2>{});
+                            static_for<2 * Taps::products>([&](auto X) {
+                                constexpr int ob = decltype(X)::value / Taps::products, i = decltype(X)::value % Taps::products;
+                                if constexpr (Taps::tuple(i, ob) == j)
+                                    c[cb][ob] = smfmac_f16(*reinterpret_cast<const f16x8 *>(bands + decltype(X)::value * 1024), rows, c[cb][ob],
+                                                           cb ? sp_index ^ 0xAAAA : sp_index);
+                            });
+                        });
+                    });
+#pragma unroll
+                    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+                        for (int f = 0; f < 2; ++f) { prev_pd[kb][f][0] = pd[kb][f][0]; prev_pd[kb][f][1] = pd[kb][f][1]; }
+                    if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
+                    dp_phase();
                     // ---- P = exp2(C - LSE) (times the dC scale), dC = P dP ----
                     if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
                     static_for<NCBL>([&](auto CB) {
@@ -431,11 +442,10 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
     if constexpr (ROLE == 0) {
         // ================================ score waves ================================
         // bands (times scale * log2 e: the convolved scores come out in log2 units) in LDS, one KB
-        // per tap slot, the slots dealt out to the four waves; the first barrier of the tile loop
-        // publishes them
-        for (int t = pr; t < CQT; t += NP)
+        // per product, dealt out to the four waves; the first barrier of the tile loop publishes them
+        for (int t = pr; t < 2 * ChainTaps<CQT>::products; t += NP)
             *reinterpret_cast<f16x8 *>(smem + Lds::band_off + t * 1024 + lane * 16) =
-                band_frag<CQT>(t, W + (size_t)h * cq * ck, cq, ck, pk, g, n, false, p.scale * kLog2e);
+                sparse_band_frag<CQT>(t, W + (size_t)h * cq * ck, cq, ck, pk, g, n, false, p.scale * kLog2e);
         score_chain(I0{}, I3{}, I0{}, I2{}, [&](auto &&tile) {
             for (int it = 0; it <= n_tiles + 1; ++it) {
                 __syncthreads();
@@ -444,17 +454,13 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
         });
         __syncthreads();  // the value waves' barrier before they hand over their dW accumulators
         __syncthreads();  // ... and the one after it
-        // ---- dW partial of this workgroup: G[m][n] of half x belongs to key tap b = n - m + 16 x - 8 + pk;
-        // the sum runs over the pair groups, the halves and the diagonals' elements in a fixed order.
+        // ---- dW partial of this workgroup: G[m][n] of half x belongs to key tap b = n - m + 16 x - 8 + pk.
         // S was raw, so * scale; dC was scaled, so / dcs. ----
-        static_assert(2 * CQT * 2 * 1024 <= NP * ChainLds<D, CQT>::pair_bytes, "room for the dW accumulators");
-        // Four lanes per tap (pair group, half), each adds its diagonal's elements in index order; the
-        // four sums are added as (0 + 1) + (2 + 3).
+        // Two lanes per tap (half), each adds its diagonal's elements in index order.
         const int ntap = cq * ck;
-        for (int q = tid; WANT_QW && (q >> 2) < ntap; q += NP * 64) {
-            const int tap = q >> 2, a = tap / ck, bb = tap - a * ck, t = a + CQT - cq;
-            const int pgi = (q >> 1) & 1, x = q & 1;
-            const float *red = reinterpret_cast<const float *>(smem + Lds::pair_off) + ((pgi * CQT + t) * 2 + x) * 256;
+        for (int q = tid; WANT_QW && (q >> 1) < ntap; q += NP * 64) {
+            const int tap = q >> 1, a = tap / ck, bb = tap - a * ck, t = a + CQT - cq, x = q & 1;
+            const float *red = reinterpret_cast<const float *>(smem + Lds::pair_off) + (t * 2 + x) * 256;
             float sum = 0.f;
 #pragma unroll
             for (int m = 0; m < 16; ++m) {
@@ -463,8 +469,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 if (nn >= 0 && nn < 16) sum += val;
             }
             sum += __shfl_xor(sum, 1);
-            sum += __shfl_xor(sum, 2);
-            if ((q & 3) == 0) dW_part[(bh * gridDim.z + blockIdx.z) * ntap + tap] = sum * p.scale / dcs;
+            if ((q & 1) == 0) dW_part[(bh * gridDim.z + blockIdx.z) * ntap + tap] = sum * p.scale / dcs;
         }
     } else if constexpr (ROLE == 1) {
         // ================================ value waves ================================
@@ -538,21 +543,12 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
             __syncthreads();
             store_dv();
         } else {
-            // dW: a unit is the key blocks of two triples (pair group) times one tap slot; the waves 0 .. 2
-            // take 2 DWT / 3 consecutive units each, in passes of NU units of one pair group (DWT: the tap slots and what fills
-            // them up to a multiple of three, which is multiplied and dropped; four units per pass spilled 25 registers).
-            constexpr int DWT = (CQT + 2) / 3 * 3, TH = 2 * DWT / 3, NU = TH > 6 ? 2 : TH / 2, NPASS = TH / NU;
-            static_assert(NU * NPASS == TH && DWT % NU == 0, "a pass stays in one pair group");
-            int dw_pg[NPASS], dw_t[NPASS];
+            // dW: the waves 0 .. 2 take TW consecutive tap slots each, for all key blocks (slots from CQT on are multiplied and dropped)
+            constexpr int TW = (CQT + 2) / 3;
+            const int t_lo = pr * TW;
+            f32x4 acc_w[TW][2];
 #pragma unroll
-            for (int ps = 0; ps < NPASS; ++ps) {
-                const int q = pr * TH + ps * NU;
-                dw_pg[ps] = q / DWT;
-                dw_t[ps] = q - dw_pg[ps] * DWT;
-            }
-            f32x4 acc_w[TH][2];
-#pragma unroll
-            for (int t = 0; t < TH; ++t) acc_w[t][0] = acc_w[t][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < TW; ++t) acc_w[t][0] = acc_w[t][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
             for (int it = 0; it <= n_tiles + 1; ++it) {
                 tiles_landed(false);
                 __syncthreads();
@@ -560,99 +556,88 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 const int u = it - 1;
                 const bool u_in = it >= 1 && u < n_tiles;
                 if (WANT_KV && u_in && !is_skipped(r_begin + u * BR)) dv_phase(u, std::integral_constant<int, C3_PRIO_VALUE>{});
-                // ---- dW, key blocks jb = 0..3 of the triples 2 pg and 2 pg + 1 (block jb = dC block jb & 1 of
-                // triple 2 pg + jb / 2, keys k0 + 64 pg - 8 + 16 jb ..), tap slots t_lo .. t_lo + NU - 1:
+                // ---- dW, key blocks jb = 0..7 (block jb = dC block jb & 1 of triple jb / 2, keys k0 - 8 + 16 jb ..):
                 // G_t[j][j'] += sum_rows dC[row][j] S[row + t - (CQT-1)][j'] with j' in the score block
-                // 8 keys before the dC block (x = 0) and the one 8 keys after it (x = 1) ----
-                if (WANT_QW && u_in) static_for<NPASS>([&](auto PS) {
-                    constexpr int ps = decltype(PS)::value;
-                    const int pg = dw_pg[ps], t_lo = dw_t[ps];
+                // 8 keys before the dC block (x = 0) and the one 8 keys after it (x = 1).
+                // A transpose read takes four rows from wherever its lanes point: k slot 4 m + r of a lane group is row
+                // 8 g + 2 r + m, so that a read of the rows one further down is the second half of one tap's operand and the
+                // first of the next one's: TW + 1 reads for TW taps.  (Eight such rows of 112 bytes cover every bank once.) ----
+                if (WANT_QW && u_in) {
                     const int wbase = ((u + 1) * BR - (CQT - 1) + Lds::ring_rows) % Lds::ring_rows;
-                    const unsigned int c_lane = opaque(tr_lane_off(CST, g, n));
-                    const unsigned int ring0 = Lds::pair_off + 2 * pg * Lds::pair_bytes + 4 * (n & 3) * 2;
-                    unsigned int a_lo[NU], a_hi[NU];
+                    const unsigned int row = 8 * g + 2 * (n >> 2), col = 4 * (n & 3) * 2;
+                    const unsigned int c_lane = opaque(Lds::pair_off + Lds::s_bytes + (u & 1) * (BR * CST) + row * CST + col);
+                    unsigned int a_s[TW + 1];
 #pragma unroll
-                    for (int tt = 0; tt < NU; ++tt) {
-                        const unsigned int ra = wbase + 4 * g + (n >> 2) + min(t_lo + tt, CQT - 1), rb = ra + 16;
-                        a_lo[tt] = opaque(ring0 + min(ra, ra - Lds::ring_rows) * SST);
-                        a_hi[tt] = opaque(ring0 + min(rb, rb - Lds::ring_rows) * SST);
+                    for (int m = 0; m <= TW; ++m) {
+                        const unsigned int r = wbase + row + min(t_lo + m, CQT);
+                        a_s[m] = opaque(Lds::pair_off + col + min(r, r - Lds::ring_rows) * SST);
                     }
-                    const unsigned int off4 = pg == NP / 2 - 1 ? Lds::pair_bytes + 64 : 2 * Lds::pair_bytes;
-                    unsigned int a4_lo[NU], a4_hi[NU];
-#pragma unroll
-                    for (int tt = 0; tt < NU; ++tt) { a4_lo[tt] = a_lo[tt] + off4; a4_hi[tt] = a_hi[tt] + off4; }
-                    auto s_frag = [&](auto JBP, int tt) {
+                    auto s_pair = [&](auto JBP, int m) {
                         constexpr int jbp = decltype(JBP)::value;
-                        constexpr int off = (jbp >> 1) * Lds::pair_bytes + (jbp & 1) * 32;
-                        bf16x4 l4, h4;
-                        if constexpr (jbp < 4) {
-                            l4 = lds_tr64(smem + a_lo[tt] + off);
-                            h4 = lds_tr64(smem + a_hi[tt] + off);
-                        } else {
-                            l4 = lds_tr64(smem + a4_lo[tt]);
-                            h4 = lds_tr64(smem + a4_hi[tt]);
-                        }
-                        return __builtin_bit_cast(f16x8, __builtin_shufflevector(l4, h4, 0, 1, 2, 3, 4, 5, 6, 7));
+                        constexpr int off = jbp < 2 * NP ? (jbp >> 1) * Lds::pair_bytes + (jbp & 1) * 32 : (NP - 1) * Lds::pair_bytes + 64;
+                        return __builtin_bit_cast(u32x2, lds_tr64(smem + a_s[m] + off));
                     };
                     auto c_frag = [&](int jb) {
-                        const int dq = jb >> 1;
-                        return __builtin_bit_cast(
-                            f16x8, read_tr(smem + Lds::pair_off + 2 * pg * Lds::pair_bytes + Lds::s_bytes + (u & 1) * (BR * CST) +
-                                               c_lane + dq * Lds::pair_bytes, CST, (jb & 1) * 16));
+                        const unsigned char *ptr = smem + c_lane + (jb >> 1) * Lds::pair_bytes + (jb & 1) * 32;
+                        const u32x2 lo = __builtin_bit_cast(u32x2, lds_tr64(ptr)), hi = __builtin_bit_cast(u32x2, lds_tr64(ptr + CST));
+                        return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3));
                     };
-                    f16x8 af = c_frag(0), b0[NU], b1[NU];
+                    auto tap_frag = [&](const u32x2 (&b)[TW + 1], int t) {
+                        return __builtin_bit_cast(f16x8, __builtin_shufflevector(b[t], b[t + 1], 0, 1, 2, 3));
+                    };
+                    f16x8 af = c_frag(0);
+                    u32x2 b0[TW + 1], b1[TW + 1];
 #pragma unroll
-                    for (int tt = 0; tt < NU; ++tt) {
-                        b0[tt] = s_frag(std::integral_constant<int, 0>{}, tt);
-                        b1[tt] = s_frag(std::integral_constant<int, 1>{}, tt);
+                    for (int m = 0; m <= TW; ++m) {
+                        b0[m] = s_pair(std::integral_constant<int, 0>{}, m);
+                        b1[m] = s_pair(std::integral_constant<int, 1>{}, m);
                     }
-                    static_for<4>([&](auto JB) {
+                    static_for<2 * NP>([&](auto JB) {
                         constexpr int jb = decltype(JB)::value;
-                        f16x8 af_n = af, b2[NU];
+                        f16x8 af_n = af;
+                        u32x2 b2[TW + 1];
 #pragma unroll
-                        for (int tt = 0; tt < NU; ++tt) b2[tt] = b1[tt];
-                        if constexpr (jb < 3) {
+                        for (int m = 0; m <= TW; ++m) b2[m] = b1[m];
+                        if constexpr (jb < 2 * NP - 1) {
                             af_n = c_frag(jb + 1);
 #pragma unroll
-                            for (int tt = 0; tt < NU; ++tt) b2[tt] = s_frag(std::integral_constant<int, jb + 2>{}, tt);
-                            SCHED_DS_READ_ID(2 + 2 * NU, 40 + 4 * ps + jb);
+                            for (int m = 0; m <= TW; ++m) b2[m] = s_pair(std::integral_constant<int, jb + 2>{}, m);
+                            SCHED_DS_READ_ID(3 + TW, 40 + jb);
                         }
 #pragma unroll
-                        for (int tt = 0; tt < NU; ++tt) {
-                            acc_w[ps * NU + tt][0] = mfma_f16(af, b0[tt], acc_w[ps * NU + tt][0]);
-                            acc_w[ps * NU + tt][1] = mfma_f16(af, b1[tt], acc_w[ps * NU + tt][1]);
+                        for (int t = 0; t < TW; ++t) {
+                            acc_w[t][0] = mfma_f16(af, tap_frag(b0, t), acc_w[t][0]);
+                            acc_w[t][1] = mfma_f16(af, tap_frag(b1, t), acc_w[t][1]);
                         }
-                        SCHED_MFMA_ID(2 * NU, 40 + 4 * ps + jb);
+                        SCHED_MFMA_ID(2 * TW, 40 + jb);
                         af = af_n;
 #pragma unroll
-                        for (int tt = 0; tt < NU; ++tt) { b0[tt] = b1[tt]; b1[tt] = b2[tt]; }
+                        for (int m = 0; m <= TW; ++m) { b0[m] = b1[m]; b1[m] = b2[m]; }
                     });
-                });
+                }
             }
-            // ---- dW accumulators of this wave to LDS as [pair group][tap slot][x][m][n], once every
-            // wave is done with the tiles ----
+            // ---- dW accumulators of this wave to LDS as [tap slot][x][m][n], once every wave is done with the tiles ----
             __syncthreads();
             float *red = reinterpret_cast<float *>(smem + Lds::pair_off);
 #pragma unroll
-            for (int ps = 0; ps < NPASS; ++ps)
+            for (int t = 0; t < TW; ++t)
 #pragma unroll
-                for (int tt = 0; tt < NU; ++tt)
+                for (int x = 0; x < 2; ++x)
 #pragma unroll
-                    for (int x = 0; x < 2; ++x)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (WANT_QW && dw_t[ps] + tt < CQT)
-                                red[(((dw_pg[ps] * CQT + dw_t[ps] + tt) * 2 + x) * 16 + 4 * g + r) * 16 + n] = acc_w[ps * NU + tt][x][r];
+                    for (int r = 0; r < 4; ++r)
+                        if (WANT_QW && t_lo + t < CQT) red[(((t_lo + t) * 2 + x) * 16 + 4 * g + r) * 16 + n] = acc_w[t][x][r];
             __syncthreads();  // the score waves add the dW partial up while the others store dK and dV
             store_dv();
         }
     } else {
         // ================================ key waves ================================
         const float *w_head = W + (size_t)h * cq * ck;
-        // flipped bands (times the softmax scale) in LDS, one KB per tap slot, dealt out to the four waves
-        unsigned char *bands = smem + opaque((unsigned int)Lds::band_off + CQT * 1024 + lane * 16);
-        for (int t = pr; t < CQT; t += NP)
-            *reinterpret_cast<f16x8 *>(bands + t * 1024) = band_frag<CQT>(t, w_head, cq, ck, pk, g, n, true, p.scale);
+        // flipped bands (times the softmax scale)
+        using Taps = ChainTaps<CQT>;
+        const int sp_index = sparse_index(g, n, false);
+        f16x8 bands[2 * Taps::products];
+#pragma unroll
+        for (int t = 0; t < 2 * Taps::products; ++t) bands[t] = sparse_band_frag<CQT>(t, w_head, cq, ck, pk, g, n, true, p.scale);
         stage_stats(0);
         load_stats(r_begin + BR);
         f32x4 acc_k[NDB][DB];
@@ -704,30 +689,32 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 bf16_t *ds_blk = ds_pair + (size_t)(r0v / BR) * (WK * BR);
                 __builtin_amdgcn_s_setprio(C3_PRIO_KEY);
                 // ---- dS^T of tile v: rows below it come from tile v+1.  Operand of row offset
-                // e = parity + (CQT-1 - tap slot): fragment e & 1 shifted e >> 1 lanes up. ----
+                // e = parity + (CQT-1 - tap slot): fragment e & 1 shifted e >> 1 lanes up; two tap slots per product. ----
                 f32x4 ds[NDB][2];
 #pragma unroll
                 for (int sb = 0; sb < NDB; ++sb) ds[sb][0] = ds[sb][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                auto band_of = [&](int e) { return *reinterpret_cast<const f16x8 *>(bands + (CQT - 1 - e) * 1024); };
-                f16x8 tbq[4];   // bands of steps e-1 .. e+2
-                tbq[0] = band_of(0);
-                tbq[1] = band_of(CQT >= 2 ? 1 : 0);
-                tbq[2] = tbq[3] = tbq[0];
-                static_for<CQT + 1>([&](auto E) {
-                    constexpr int e = decltype(E)::value, f = e & 1, s = e >> 1;
-                    if constexpr (e + 2 <= CQT - 1) tbq[(e + 2) % 4] = band_of(e + 2);
-                    const f16x8 tb_cur = tbq[e % 4], tb_prev = tbq[(e + 3) % 4];
-                    unsigned int sh[NCB][2];
+                static_for<Taps::tuples>([&](auto J) {
+                    constexpr int j = decltype(J)::value;
+                    u32x8 rows;
+                    auto put = [&](auto CB, auto POS) {
+                        static_for<2>([&](auto HALF) {
+                            constexpr int half = decltype(HALF)::value, e = Taps::delta(j, half) + CQT - 1, f = e & 1, s = e >> 1;
 #pragma unroll
-                    for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-                        for (int dw = 0; dw < 2; ++dw) sh[cb][dw] = win_down<s>(prev_dc[cb][f][dw], cur_dc[cb][f][dw]);
-#pragma unroll
-                    for (int sb = 0; sb < NDB; ++sb) {
-                        const u32x4 bv = {sh[sb][0], sh[sb][1], sh[sb + 1][0], sh[sb + 1][1]};
-                        if constexpr (e <= CQT - 1) ds[sb][0] = mfma_f16(tb_cur, __builtin_bit_cast(f16x8, bv), ds[sb][0]);
-                        if constexpr (e >= 1) ds[sb][1] = mfma_f16(tb_prev, __builtin_bit_cast(f16x8, bv), ds[sb][1]);
-                    }
+                            for (int dw = 0; dw < 2; ++dw)
+                                rows[4 * half + 2 * dw + decltype(POS)::value] = win_down<s>(prev_dc[decltype(CB)::value][f][dw], cur_dc[decltype(CB)::value][f][dw]);
+                        });
+                    };
+                    put(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+                    put(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+                    static_for<NDB>([&](auto SB) {
+                        constexpr int sb = decltype(SB)::value;
+                        if constexpr (sb > 0) put(std::integral_constant<int, sb + 1>{}, std::integral_constant<int, (sb + 1) % 2>{});
+                        static_for<2 * Taps::products>([&](auto X) {
+                            constexpr int ob = decltype(X)::value / Taps::products, i = decltype(X)::value % Taps::products;
+                            if constexpr (Taps::tuple(i, ob) == j)
+                                ds[sb][ob] = smfmac_f16(bands[decltype(X)::value], rows, ds[sb][ob], sb ? sp_index ^ 0xAAAA : sp_index);
+                        });
+                    });
                 });
                 auto ds_out = [&](auto edge_tag) {
                     constexpr bool EDGE = decltype(edge_tag)::value;

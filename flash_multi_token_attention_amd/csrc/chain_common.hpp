@@ -22,7 +22,8 @@ constexpr int CST = 112;         // bytes per row of the dC tile (48 keys fp16 +
 constexpr int PST = 72;          // bytes per row of the P and dS tiles (32 keys bf16 + 8)
 static_assert(BKW == kKvKeysPerWg && WK == kChainKeys && BR == kChainRows, "dS workspace layout");
 
-template <int D, int CQT> struct ChainLds {
+// THREE: the layout of the three-role kernel, whose key waves keep their bands in registers
+template <int D, int CQT, bool THREE = false> struct ChainLds {
     // Q / dO tiles are filled by buffer loads with the LDS modifier (64 lanes = 1 KB of consecutive
     // LDS), which rules out padded rows.  A tile of 32 rows is kept as [k-step ks][row parity f]
     // [row pair n][64 bytes]: the 4 chunks of 16 bytes that row 2n + f holds of head-dim columns
@@ -36,11 +37,12 @@ template <int D, int CQT> struct ChainLds {
     static constexpr int stat_off = g_off + g_slots * tile_bytes;   // LSE and D of a tile: two slots
     static constexpr int stat_bytes = 2 * (2 * BR * 4);
     // bands, then flipped bands: one KB of ready-made fragments per tap slot, or (windows of more than 8
-    // query taps, where those do not fit) one compact table per tap slot that the lanes read their fragments from
-    static constexpr bool compact_bands = CQT > 8 && D > 64;
+    // query taps, where those do not fit) one compact table per tap slot that the lanes read their fragments from;
+    // THREE: one KB per sparse product of two slots and output parity, the direct ones only
+    static constexpr bool compact_bands = !THREE && CQT > 8 && D > 64;
     static constexpr int band_slot = compact_bands ? kBandTab : 1024;
     static constexpr int band_off = stat_off + stat_bytes;
-    static constexpr int band_bytes = 2 * CQT * band_slot;
+    static constexpr int band_bytes = THREE ? (CQT + 1) / 2 * 2048 : 2 * CQT * band_slot;
     static constexpr int pair_off = band_off + band_bytes;
     static constexpr int ring_rows = CQT > 9 ? S_RING + 4 : S_RING;   // >= 64 + CQT - 1
     static constexpr int s_bytes = ring_rows * SST;
@@ -49,7 +51,7 @@ template <int D, int CQT> struct ChainLds {
     static constexpr int ds_bytes = BR * PST;
     static constexpr int pair_bytes = s_bytes + c_bytes + p_bytes + ds_bytes;
     static constexpr int total = pair_off + NP * pair_bytes;
-    static_assert(2 * CQT * 2 * 1024 <= NP * pair_bytes, "room for the dW accumulators (they take the place of the pairs' tiles)");
+    static_assert((THREE ? 1 : 2) * CQT * 2 * 1024 <= NP * pair_bytes, "room for the dW accumulators (they take the place of the pairs' tiles)");
 };
 
 // A lane-dependent LDS offset the compiler may not fold or hoist: what is added to it afterwards
@@ -132,6 +134,37 @@ __device__ __forceinline__ f16x8 band_frag(int t, const float *__restrict__ w_he
         v[e] = row[min(max(bb, 0), c_k - 1)];
         if (a < 0 || bb < 0 || bb >= c_k) v[e] = 0.f;
     }
+    f16x8 f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = (_Float16)(v[e] * mul);
+    return f;
+}
+
+// The bands of the sparse products (two tap slots each, see SparseTaps) for the same operand order: fragment `idx` = product i of
+// output parity ob at idx = ob * products + i.  `flip`: the transposed convolution, whose rows are counted downwards (row offset
+// e = delta + CQT - 1, tap slot CQT - 1 - slot).
+template <int CQT> using ChainTaps = SparseTaps<CQT, false>;
+template <int CQT>
+__device__ __forceinline__ f16x8 sparse_band_frag(int idx, const float *__restrict__ w_head, int c_q, int c_k, int pk,
+                                                  int g, int n, bool flip, float mul) {
+    using T = ChainTaps<CQT>;
+    const int ob = idx >= T::products ? 1 : 0, i = idx - ob * T::products;
+    int t = T::slot(T::tuple(i, ob), g >> 1, ob);
+    const bool none = t == CQT;
+    if (flip) t = CQT - 1 - t;
+    const int a = t - (CQT - c_q);
+    // (unconditional loads from clamped indices: the eight of a fragment are in flight together)
+    const float *row = w_head + min(max(a, 0), c_q - 1) * c_k;
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int kappa = sparse_key(g, q), off = kappa + e + (kappa + 1 > n ? 0 : 16) - kKeyHalo - n;
+            const int bb = flip ? pk - off : pk + off;
+            v[2 * q + e] = row[min(max(bb, 0), c_k - 1)];
+            if (none || a < 0 || bb < 0 || bb >= c_k) v[2 * q + e] = 0.f;
+        }
     f16x8 f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) f[e] = (_Float16)(v[e] * mul);
