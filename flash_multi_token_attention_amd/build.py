@@ -23,12 +23,11 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 
 # MFMA results in ordinary VGPRs (the 512-register dQ kernel otherwise copies every transient
-# accumulator out of the accumulation file).  Not for the dK/dV kernel: with its two tile loops
-# this compiler's MFMA rewrite pass crashes on it under this option.
+# accumulator out of the accumulation file).
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 
-# (source, object name, extra flags).  The dK/dV kernel is compiled as two objects (narrow /
-# 11-tap windows) so that they build in parallel.
+# (source, object name, extra flags).  The forward and the key-stationary backward are compiled as several
+# objects so that they build in parallel.
 UNITS = [
     ("api.hip", "api", []),
     ("generic_kernels.hip", "generic_kernels", []),
@@ -37,10 +36,6 @@ UNITS = [
     ("fwd_reg_mfma.hip", "fwd_reg_mfma", []),
     ("fwd_reg_mfma.hip", "fwd_reg_mfma_wide", ["-DCONVATTN_FWD_WIDE"]),
     ("bwd_dq_mfma.hip", "bwd_dq_mfma", VGPR_FORM),
-    ("bwd_chain_mfma.hip", "bwd_chain_mfma_all", ["-DCONVATTN_CHAIN_UNIT=3"]),
-    ("bwd_chain_mfma.hip", "bwd_chain_mfma_kv", ["-DCONVATTN_CHAIN_UNIT=1"]),
-    ("bwd_chain_mfma.hip", "bwd_chain_mfma_qw", ["-DCONVATTN_CHAIN_UNIT=2"]),
-    ("bwd_chain_mfma.hip", "bwd_chain_mfma_split", ["-DCONVATTN_CHAIN_UNIT=7"]),
     ("bwd_chain3_mfma.hip", "bwd_chain3_mfma_all", ["-DCONVATTN_CHAIN_UNIT=3"]),
     ("bwd_chain3_mfma.hip", "bwd_chain3_mfma_split", ["-DCONVATTN_CHAIN_UNIT=7"]),
     ("bwd_chain3_mfma.hip", "bwd_chain3_mfma_kv", ["-DCONVATTN_CHAIN_UNIT=1"]),

@@ -1,5 +1,4 @@
-// Whole backward of conv-attention on bf16 MFMA (gfx950), windows of up to 6 query taps, at head dimensions 32 and 64 of up to 11: the
-// key-stationary kernel of bwd_chain_mfma.hip with three waves per SIMD instead of two.
+// Whole backward of conv-attention on bf16 MFMA (gfx950): key-stationary, three waves per SIMD.
 //
 // A workgroup of 12 waves owns 128 keys of one (batch, head) and walks down the query rows in tiles
 // of 32.  Triple p (waves p, p+4, p+8: one SIMD) owns keys c0 = k0 + 32p .. c0+31 for dK and dS,
@@ -22,7 +21,8 @@
 // pipe and the vector ALUs.  So both convolutions take two tap slots per sparse product (SparseTaps in mfma_common.hpp), the key
 // waves keep their bands in registers, and dW's operands of neighbouring taps share their transpose reads (43 per wave and tile for
 // 56 at 6 slots, 61 for 112 at 11).  Kernel alone, B4 H16 N4096 causal, before -> after, us, in turn on one card: d 128 6x11 1409 -> 1310,
-// d 64 6x11 1097 -> 1048, 11x11 1442 -> 1283, 3x3 833 -> 804.
+// d 64 6x11 1097 -> 1048, 11x11 1442 -> 1283, 3x3 833 -> 804; at d 128 with more than 6 taps, in the place of a kernel of two waves per
+// SIMD and 256 registers, 7x7 1510 -> 1424, 11x11 1960 -> 1565 (B1 H8 N1500 61 -> 49).
 #include <type_traits>
 
 #include "chain_common.hpp"
@@ -46,14 +46,6 @@ constexpr int NT3 = 3 * NP * 64;  // 768 threads
 #ifndef C3_PRIO_KEY
 #define C3_PRIO_KEY 0     // key waves
 #endif
-// LDS: the layout of the two-role kernel, then the V fragments of the block after the workgroup's keys
-// (16 rows; the wave that computes that block has no registers to keep them in)
-template <int D, int CQT> struct Chain3Lds : ChainLds<D, CQT, true> {
-    static constexpr int e_off = ChainLds<D, CQT, true>::total;
-    static constexpr int e_bytes = 16 * D * 2;
-    static constexpr int total3 = e_off + e_bytes;
-};
-
 // One role of the workgroup: ROLE 0 = score waves, 1 = value waves (dV, dW, the block after the
 // workgroup's keys), 2 = key waves (dS, dK).  WANT: bit 0 = dK and dV, bit 1 = dS (for dQ) and dW.
 template <int D, int CQT, typename TO, int ROLE, int WANT>
@@ -71,7 +63,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
     bf16_t *__restrict__ dS_ws = args.dS_ws;
     float *__restrict__ dW_part = args.dW_part;
     const int n_rt = args.n_rt;
-    using Lds = Chain3Lds<D, CQT>;
+    using Lds = ChainLds<D, CQT>;
     constexpr int KS = D / 32, DB = D / 16;
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
@@ -378,7 +370,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                             static_for<2 * Taps::products>([&](auto X) {
                                 constexpr int ob = decltype(X)::value / Taps::products, i = decltype(X)::value % Taps::products;
                                 if constexpr (Taps::tuple(i, ob) == j)
-                                    c[cb][ob] = smfmac_f16(*reinterpret_cast<const f16x8 *>(bands + decltype(X)::value * 1024), rows, c[cb][ob],
+                                    c[cb][ob] = smfmac_f16(*reinterpret_cast<const f16x8 *>(bands + Lds::Bands::row(i, ob) * Lds::Bands::row_bytes), rows, c[cb][ob],
                                                            cb ? sp_index ^ 0xAAAA : sp_index);
                             });
                         });
@@ -441,11 +433,9 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
 
     if constexpr (ROLE == 0) {
         // ================================ score waves ================================
-        // bands (times scale * log2 e: the convolved scores come out in log2 units) in LDS, one KB
-        // per product, dealt out to the four waves; the first barrier of the tile loop publishes them
-        for (int t = pr; t < 2 * ChainTaps<CQT>::products; t += NP)
-            *reinterpret_cast<f16x8 *>(smem + Lds::band_off + t * 1024 + lane * 16) =
-                sparse_band_frag<CQT>(t, W + (size_t)h * cq * ck, cq, ck, pk, g, n, false, p.scale * kLog2e);
+        // bands (times scale * log2 e: the convolved scores come out in log2 units) in LDS;
+        // the first barrier of the tile loop publishes them
+        Lds::Bands::build(smem + Lds::band_off, 0, W + (size_t)h * cq * ck, cq, ck, pk, false, p.scale * kLog2e, pr, NP, g, n);
         score_chain(I0{}, I3{}, I0{}, I2{}, [&](auto &&tile) {
             for (int it = 0; it <= n_tiles + 1; ++it) {
                 __syncthreads();
@@ -632,12 +622,18 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
     } else {
         // ================================ key waves ================================
         const float *w_head = W + (size_t)h * cq * ck;
-        // flipped bands (times the softmax scale)
+        // bands of the transposed convolution (times the softmax scale): the first products' in registers, the others' in LDS
         using Taps = ChainTaps<CQT>;
         const int sp_index = sparse_index(g, n, false);
-        f16x8 bands[2 * Taps::products];
+        constexpr int KR = Lds::key_regs;
+        f16x8 band_regs[KR > 0 ? KR : 1][2];
 #pragma unroll
-        for (int t = 0; t < 2 * Taps::products; ++t) bands[t] = sparse_band_frag<CQT>(t, w_head, cq, ck, pk, g, n, true, p.scale);
+        for (int i = 0; i < KR; ++i)
+#pragma unroll
+            for (int ob = 0; ob < 2; ++ob) band_regs[i][ob] = Lds::Bands::frag(Lds::Bands::row(i, ob) + (g >> 1), w_head, cq, ck, pk, g, n, true, p.scale);
+        const unsigned char *bands = smem + opaque((unsigned int)Lds::key_band_off + lane * 16);
+        if constexpr (KR < Taps::products)
+            Lds::Bands::build(smem + Lds::key_band_off, Lds::key_row, w_head, cq, ck, pk, true, p.scale, pr, NP, g, n);
         stage_stats(0);
         load_stats(r_begin + BR);
         f32x4 acc_k[NDB][DB];
@@ -711,8 +707,12 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                         if constexpr (sb > 0) put(std::integral_constant<int, sb + 1>{}, std::integral_constant<int, (sb + 1) % 2>{});
                         static_for<2 * Taps::products>([&](auto X) {
                             constexpr int ob = decltype(X)::value / Taps::products, i = decltype(X)::value % Taps::products;
-                            if constexpr (Taps::tuple(i, ob) == j)
-                                ds[sb][ob] = smfmac_f16(bands[decltype(X)::value], rows, ds[sb][ob], sb ? sp_index ^ 0xAAAA : sp_index);
+                            if constexpr (Taps::tuple(i, ob) == j) {
+                                f16x8 band;
+                                if constexpr (i < KR) band = band_regs[i][ob];
+                                else band = *reinterpret_cast<const f16x8 *>(bands + (Lds::Bands::row(i, ob) - Lds::key_row) * Lds::Bands::row_bytes);
+                                ds[sb][ob] = smfmac_f16(band, rows, ds[sb][ob], sb ? sp_index ^ 0xAAAA : sp_index);
+                            }
                         });
                     });
                 });
@@ -825,7 +825,7 @@ hipError_t launch_chain3(const Problem &p, const void *q, const void *k, const v
                          const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk,
                          void *dv, void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
     auto kern = bwd_chain3_kernel<D, CQT, TO, WANT>;
-    constexpr int lds = Chain3Lds<D, CQT>::total3;
+    constexpr int lds = ChainLds<D, CQT>::total;
     static_assert(lds <= 160 * 1024, "LDS budget");
     hipError_t e = set_max_lds_once<bwd_chain3_kernel<D, CQT, TO, WANT>>(lds);
     if (e != hipSuccess) return e;
@@ -842,12 +842,9 @@ hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v
                    void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
 #define CALL(CQT) launch_chain3<D, CQT, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s)
     if (p.c_q <= 3) return CALL(3);
-    // (7 and 8 slots apart: a padding tap for 7 costs 2.5 % in the two-role kernel)
-    if constexpr (D <= 64) {
-        if (p.c_q == 7) return CALL(7);
-        if (p.c_q == 8) return CALL(8);
-        if (p.c_q > 8) return CALL(11);
-    }
+    // (7 slots take as many products as 8; at d = 128 with fewer spills in 8: kernel of B4 H16 N4096 7x7 1480 us in 7, 1410 in 8)
+    if (p.c_q > 8) return CALL(11);
+    if (p.c_q > 6) return CALL(8);
     return CALL(6);
 #undef CALL
 }

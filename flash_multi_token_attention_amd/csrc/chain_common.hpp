@@ -1,4 +1,4 @@
-// Shared pieces of the key-stationary backward kernels (bwd_chain_mfma.hip, bwd_chain3_mfma.hip): LDS layout,
+// Pieces of the key-stationary backward kernel (bwd_chain3_mfma.hip): LDS layout,
 // fragment addressing, DPP row windows, Toeplitz bands for the packed operand order, the argument block.
 #pragma once
 #include <type_traits>
@@ -17,13 +17,68 @@ constexpr int NCB = 3;           // C / dP / dC blocks: keys c0-8+16cb
 constexpr int NDB = 2;           // dS blocks: keys c0+16sb
 constexpr int SST = 112;         // bytes per row of the S tile in LDS (48 keys fp16 + 16)
 constexpr int S_RING = 72;       // rows of the S ring: a tile being written, the tile before it and 8 rows more (>= c_q - 1)
-constexpr int kBandTab = 352;    // bytes of a compact band table: 44 slots of 4 fp16 (see band_tab_build)
 constexpr int CST = 112;         // bytes per row of the dC tile (48 keys fp16 + 16)
 constexpr int PST = 72;          // bytes per row of the P and dS tiles (32 keys bf16 + 8)
 static_assert(BKW == kKvKeysPerWg && WK == kChainKeys && BR == kChainRows, "dS workspace layout");
 
-// THREE: the layout of the three-role kernel, whose key waves keep their bands in registers
-template <int D, int CQT, bool THREE = false> struct ChainLds {
+// The bands of the sparse products (two tap slots each, see SparseTaps).  The half of a fragment that belongs to one slot is the same
+// wherever that slot stands: a row of 32 lanes x 16 bytes, and a product whose two slots have neighbouring rows reads its
+// fragment as 1 KB from the first one's row on.  Odd CQT: a row of zeros before slot 0 and after the last (a parity's single slot is a
+// product with one of them).  Even: two more rows for the product of slots 0 and CQT - 1.  `flip`: the transposed convolution, whose
+// rows are counted downwards (row offset e = delta + CQT - 1, tap slot CQT - 1 - slot).
+template <int CQT> using ChainTaps = SparseTaps<CQT, false>;
+template <int CQT> struct ChainBands {
+    using T = ChainTaps<CQT>;
+    static constexpr int rows = CQT + 2, row_bytes = 512;
+    static constexpr int slot(int row) { return T::odd ? row - 1 : row < CQT ? row : row == CQT ? 0 : CQT - 1; }
+    // first row of product i of output parity ob
+    static constexpr int row(int i, int ob) { return T::odd ? 2 * i - ob + 1 : !ob && i == T::products - 1 ? CQT : 2 * i + 1 - ob; }
+    static constexpr bool rows_right() {
+        for (int ob = 0; ob < 2; ++ob)
+            for (int i = 0; i < T::products; ++i)
+                for (int half = 0; half < 2; ++half) {
+                    const int want = T::slot(T::tuple(i, ob), half, ob), have = slot(row(i, ob) + half);
+                    if (want != have && !(want == CQT && (have < 0 || have >= CQT))) return false;
+                }
+        return true;
+    }
+    static_assert(rows_right(), "rows of the products");
+    // this lane's 16 bytes of a row
+    static __device__ __forceinline__ f16x8 frag(int row, const float *__restrict__ w_head, int c_q, int c_k, int pk, int g, int n,
+                                                 bool flip, float mul) {
+        int t = slot(row);
+        const bool none = t < 0 || t >= CQT;
+        if (flip) t = CQT - 1 - t;
+        const int a = t - (CQT - c_q);
+        // (unconditional loads from clamped indices: the eight of a fragment are in flight together)
+        const float *w = w_head + min(max(a, 0), c_q - 1) * c_k;
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int kappa = sparse_key(g, q), off = kappa + e + (kappa + 1 > n ? 0 : 16) - kKeyHalo - n;
+                const int bb = flip ? pk - off : pk + off;
+                v[2 * q + e] = w[min(max(bb, 0), c_k - 1)];
+                if (none || a < 0 || bb < 0 || bb >= c_k) v[2 * q + e] = 0.f;
+            }
+        f16x8 f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = (_Float16)(v[e] * mul);
+        return f;
+    }
+    // the rows from `first` on to LDS, dealt out in pairs to `n_waves` waves
+    static __device__ __forceinline__ void build(unsigned char *tab, int first, const float *__restrict__ w_head, int c_q, int c_k, int pk,
+                                                 bool flip, float mul, int wave, int n_waves, int g, int n) {
+        for (int r0 = first + 2 * wave; r0 < rows; r0 += 2 * n_waves) {
+            const int r = r0 + (g >> 1);
+            const f16x8 f = frag(r, w_head, c_q, c_k, pk, g, n, flip, mul);
+            if (r < rows) *reinterpret_cast<f16x8 *>(tab + (r - first) * row_bytes + ((g & 1) * 16 + n) * 16) = f;
+        }
+    }
+};
+
+template <int D, int CQT> struct ChainLds {
     // Q / dO tiles are filled by buffer loads with the LDS modifier (64 lanes = 1 KB of consecutive
     // LDS), which rules out padded rows.  A tile of 32 rows is kept as [k-step ks][row parity f]
     // [row pair n][64 bytes]: the 4 chunks of 16 bytes that row 2n + f holds of head-dim columns
@@ -36,22 +91,27 @@ template <int D, int CQT, bool THREE = false> struct ChainLds {
     static constexpr int g_off = q_off + q_slots * tile_bytes, g_slots = 3;  // tiles it-1 .. it+1
     static constexpr int stat_off = g_off + g_slots * tile_bytes;   // LSE and D of a tile: two slots
     static constexpr int stat_bytes = 2 * (2 * BR * 4);
-    // bands, then flipped bands: one KB of ready-made fragments per tap slot, or (windows of more than 8
-    // query taps, where those do not fit) one compact table per tap slot that the lanes read their fragments from;
-    // THREE: one KB per sparse product of two slots and output parity, the direct ones only
-    static constexpr bool compact_bands = !THREE && CQT > 8 && D > 64;
-    static constexpr int band_slot = compact_bands ? kBandTab : 1024;
+    // the bands of the convolution, then those of the transposed one that the key waves do not keep in registers: those
+    // from product key_regs on (up to d = 64 and up to 6 slots none; 8 slots at d = 128 all, 11 what leaves room for the S ring)
+    using Bands = ChainBands<CQT>;
+    static constexpr int key_regs = D <= 64 || CQT <= 6 ? Bands::T::products : CQT <= 8 ? 0 : 2;
+    static constexpr int key_row = 2 * key_regs;   // first row of the transposed bands in LDS
+    static constexpr int key_rows = key_regs < Bands::T::products ? Bands::rows - key_row : 0;
     static constexpr int band_off = stat_off + stat_bytes;
-    static constexpr int band_bytes = THREE ? (CQT + 1) / 2 * 2048 : 2 * CQT * band_slot;
+    static constexpr int key_band_off = band_off + Bands::rows * Bands::row_bytes;
+    static constexpr int band_bytes = (Bands::rows + key_rows) * Bands::row_bytes;
+    static_assert(key_regs == 0 || key_regs == Bands::T::products || Bands::T::odd, "rows of product i from 2 i on");
     static constexpr int pair_off = band_off + band_bytes;
-    static constexpr int ring_rows = CQT > 9 ? S_RING + 4 : S_RING;   // >= 64 + CQT - 1
+    static constexpr int ring_rows = CQT > 9 ? S_RING + 2 : S_RING;   // >= 64 + CQT - 1
     static constexpr int s_bytes = ring_rows * SST;
     static constexpr int c_bytes = 2 * BR * CST;
     static constexpr int p_bytes = 2 * BR * PST;
     static constexpr int ds_bytes = BR * PST;
     static constexpr int pair_bytes = s_bytes + c_bytes + p_bytes + ds_bytes;
-    static constexpr int total = pair_off + NP * pair_bytes;
-    static_assert((THREE ? 1 : 2) * CQT * 2 * 1024 <= NP * pair_bytes, "room for the dW accumulators (they take the place of the pairs' tiles)");
+    // V fragments of the block after the workgroup's keys (16 rows; the wave that computes it has no registers to keep them in)
+    static constexpr int e_off = pair_off + NP * pair_bytes;
+    static constexpr int total = e_off + 16 * D * 2;
+    static_assert(CQT * 2 * 1024 <= NP * pair_bytes, "room for the dW accumulators (they take the place of the pairs' tiles)");
 };
 
 // A lane-dependent LDS offset the compiler may not fold or hoist: what is added to it afterwards
@@ -113,91 +173,6 @@ __device__ __forceinline__ unsigned int win_down(unsigned int a, unsigned int b)
 
 __device__ __forceinline__ unsigned int pack_f16_rtz(float a, float b) {
     return __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(a, b));
-}
-
-// Toeplitz bands for the packed operand order: k slot 8g+e of a 32-key window is key 4g+e of its
-// first 16-key block for e < 4 and key 4g+e-4 of its second for e >= 4; the output block starts 8
-// keys into the window.  Tap slot t stands for query tap a = t - (CQT - c_q) (zero taps in front).
-// `flip` builds the bands of the transposed convolution.
-template <int CQT>
-__device__ __forceinline__ f16x8 band_frag(int t, const float *__restrict__ w_head, int c_q, int c_k, int pk,
-                                           int g, int n, bool flip, float mul) {
-    const int a = t - (CQT - c_q);
-    // (unconditional loads from clamped indices: the eight of a fragment are in flight together)
-    const float *row = w_head + max(a, 0) * c_k;
-    float v[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int kappa = e < 4 ? 4 * g + e : 16 + 4 * g + e - 4;
-        const int off = kappa - kKeyHalo - n;
-        const int bb = flip ? pk - off : pk + off;
-        v[e] = row[min(max(bb, 0), c_k - 1)];
-        if (a < 0 || bb < 0 || bb >= c_k) v[e] = 0.f;
-    }
-    f16x8 f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = (_Float16)(v[e] * mul);
-    return f;
-}
-
-// The bands of the sparse products (two tap slots each, see SparseTaps) for the same operand order: fragment `idx` = product i of
-// output parity ob at idx = ob * products + i.  `flip`: the transposed convolution, whose rows are counted downwards (row offset
-// e = delta + CQT - 1, tap slot CQT - 1 - slot).
-template <int CQT> using ChainTaps = SparseTaps<CQT, false>;
-template <int CQT>
-__device__ __forceinline__ f16x8 sparse_band_frag(int idx, const float *__restrict__ w_head, int c_q, int c_k, int pk,
-                                                  int g, int n, bool flip, float mul) {
-    using T = ChainTaps<CQT>;
-    const int ob = idx >= T::products ? 1 : 0, i = idx - ob * T::products;
-    int t = T::slot(T::tuple(i, ob), g >> 1, ob);
-    const bool none = t == CQT;
-    if (flip) t = CQT - 1 - t;
-    const int a = t - (CQT - c_q);
-    // (unconditional loads from clamped indices: the eight of a fragment are in flight together)
-    const float *row = w_head + min(max(a, 0), c_q - 1) * c_k;
-    float v[8];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int kappa = sparse_key(g, q), off = kappa + e + (kappa + 1 > n ? 0 : 16) - kKeyHalo - n;
-            const int bb = flip ? pk - off : pk + off;
-            v[2 * q + e] = row[min(max(bb, 0), c_k - 1)];
-            if (none || a < 0 || bb < 0 || bb >= c_k) v[2 * q + e] = 0.f;
-        }
-    f16x8 f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = (_Float16)(v[e] * mul);
-    return f;
-}
-
-// The same bands as compact tables.  A fragment is Toeplitz in (slot, lane): its value at k slot e of lane
-// (g, n) is T[x] with x = kappa(e, g) - n in [-15, 31], T[x] = w[a][pk +- (x - 8)] (zero outside the window),
-// and the eight k slots of a lane are x0 .. x0+3 and x0+16 .. x0+19 with x0 = 4g - n.  A table holds T as 44
-// slots of 4 fp16: slot 4k + r (k = 0..10, r = 0..3) = T[4k + r - 15 .. 4k + r - 12], so that lane (g, n) finds
-// its two groups at the slots 4k + r and 4(k + 4) + r with k = g - n/4 + 3, r = 3 - n%4: two aligned 8-byte
-// reads, 128 bytes apart, and the 28 distinct addresses of a wave fall into distinct banks.
-__device__ __forceinline__ unsigned int band_tab_lane_off(int g, int n) {
-    return (unsigned int)(((g - (n >> 2) + 3) * 4 + 3 - (n & 3)) * 8);
-}
-__device__ __forceinline__ f16x8 band_tab_read(const unsigned char *lane_ptr) {
-    const u32x2 lo = *reinterpret_cast<const u32x2 *>(lane_ptr), hi = *reinterpret_cast<const u32x2 *>(lane_ptr + 128);
-    return __builtin_bit_cast(f16x8, (u32x4){lo[0], lo[1], hi[0], hi[1]});
-}
-// Tables of all tap slots: CQT direct ones (times mul_direct), then CQT flipped ones (times mul_flipped), built
-// by all `nthreads` threads of the workgroup; a barrier has to follow before they are read.
-template <int CQT>
-__device__ __forceinline__ void band_tab_build(unsigned char *tabs, const float *__restrict__ w_head, int c_q, int c_k,
-                                               int pk, float mul_direct, float mul_flipped, int tid, int nthreads) {
-    constexpr int PER = kBandTab / 2;   // fp16 entries per table
-    for (int i = tid; i < 2 * CQT * PER; i += nthreads) {
-        const int td = i / PER, q = i - td * PER, flip = td >= CQT, t = td - flip * CQT;
-        const int a = t - (CQT - c_q), x = q - (q >> 2) * 3 - 15;   // entry e of slot s: x = s + e - 15
-        const int bb = flip ? pk - (x - kKeyHalo) : pk + (x - kKeyHalo);
-        float v = 0.f;
-        if (a >= 0 && bb >= 0 && bb < c_k) v = w_head[a * c_k + bb] * (flip ? mul_flipped : mul_direct);
-        reinterpret_cast<_Float16 *>(tabs)[i] = (_Float16)v;
-    }
 }
 
 // Kernel arguments as one block: each role reads them from the kernel argument segment with

@@ -193,22 +193,6 @@ __device__ __forceinline__ u32x2 pack_scores_f16(f32x4 s) {
                    __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(s[2], s[3]))};
 }
 
-// Toeplitz fragment of query tap `a` for this lane: element e is
-// W[a][b], b = (8g + e) - 8 - n + pk, zero outside the window.  `flip` builds the
-// transposed-convolution band instead (b -> c_k - 1 - b).
-__device__ __forceinline__ f16x8 toeplitz_frag(const float *__restrict__ w_row, int c_k, int pk,
-                                               int g, int n, bool flip) {
-    f16x8 t;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        int b = 8 * g + e - kKeyHalo - n + pk;
-        float v = 0.f;
-        if (b >= 0 && b < c_k) v = w_row[flip ? (c_k - 1 - b) : b];
-        t[e] = (_Float16)v;
-    }
-    return t;
-}
-
 // Bands for a compile-time tap count CQT >= c_q: the window is padded with zero
 // taps in FRONT (older query rows), so tap slot t stands for tap a = t - (CQT - c_q)
 // and reads score row  i + t - (CQT - 1); the padded slots read rows that exist
@@ -363,7 +347,7 @@ hipError_t mfma_bwd_dq_dw(const Problem &p, int out_dt, const void *q, const voi
                           const void *d_o, const float *Dl, const float *lse, const float *w, void *dq,
                           float *dw_part, hipStream_t s);
 
-// ---- whole backward with the score chain in registers (bwd_chain_mfma.hip, bwd_chain3_mfma.hip, bwd_dq_rows.hip) ----
+// ---- whole backward with the score chain in registers (bwd_chain3_mfma.hip, bwd_dq_rows.hip) ----
 constexpr int kKvKeysPerWg = 128;
 inline int mfma_kv_tiles(const Problem &p) { return (p.Nk + 8 + kKvKeysPerWg - 1) / kKvKeysPerWg; }
 // The key-stationary kernel's workgroups cover 128 keys each (+ 8:
@@ -442,34 +426,19 @@ hipError_t bwd_prepare(const Problem &p, int out_dt, const void *o, const void *
     hipError_t name(const Problem &p, int out_dt, const void *q, const void *k, const void *v, const void *d_o, \
                     const float *Dl, const float *lse, const float *w, const float *dc_scale, void *dk, void *dv, \
                     void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s)
-CHAIN_DECL(mfma_bwd_chain_kv);
-CHAIN_DECL(mfma_bwd_chain_qw);
-CHAIN_DECL(mfma_bwd_chain_all);
-CHAIN_DECL(mfma_bwd_chain_split);   // everything, with share > 0
-// the same with three waves per SIMD (bwd_chain3_mfma.hip)
 CHAIN_DECL(mfma_bwd_chain3_kv);
 CHAIN_DECL(mfma_bwd_chain3_qw);
 CHAIN_DECL(mfma_bwd_chain3_all);
-CHAIN_DECL(mfma_bwd_chain3_split);
+CHAIN_DECL(mfma_bwd_chain3_split);   // everything, with share > 0
 #undef CHAIN_DECL
 inline hipError_t mfma_bwd_chain(const Problem &p, int out_dt, int want, const void *q, const void *k, const void *v,
                                  const void *d_o, const float *Dl, const float *lse, const float *w,
                                  const float *dc_scale, void *dk, void *dv, void *ds_ws, float *dw_part,
                                  hipStream_t s, int share = 0, float *kv_part = nullptr) {
-    // Three waves of 168 registers per SIMD hold any window's roles up to d = 64 (the second kernel computes a third C block per 32
-    // keys, which a neighbour has anyway); beyond 6 query taps the dV and dW accumulators of d = 128 do not fit.  Forward + backward, us, two
-    // waves in 8 or 12 slots and three in 7 or 11: B4 H16 N4096 11x11 d64 2406 and 2216, d32 2225 and 2032, 7x7 d64 1898 and 1797,
-    // d32 1742 and 1581, B2 H8 N1531 d64 11x11 168 and 156.
-    if (p.c_q <= 6 || p.d <= 64) {
-        if (want == 1) return mfma_bwd_chain3_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-        if (want == 2) return mfma_bwd_chain3_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-        if (share) return mfma_bwd_chain3_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-        return mfma_bwd_chain3_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    }
-    if (want == 1) return mfma_bwd_chain_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    if (want == 2) return mfma_bwd_chain_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    if (share) return mfma_bwd_chain_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
-    return mfma_bwd_chain_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    if (want == 1) return mfma_bwd_chain3_kv(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    if (want == 2) return mfma_bwd_chain3_qw(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    if (share) return mfma_bwd_chain3_split(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
+    return mfma_bwd_chain3_all(p, out_dt, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s);
 }
 // What follows the key-stationary kernel: dQ, the sum of the n_wg dW partials per (batch, head) and, with share > 0, dK and dV from
 // their parts.  One launch where dQ's waves share keys (small problems), else one each.

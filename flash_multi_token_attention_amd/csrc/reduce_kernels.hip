@@ -175,6 +175,48 @@ __global__ __launch_bounds__(256) void combine_kernel(int n_splits, int d, const
     if (tid == 0 && blockIdx.y == 0) { M[bh] = m; L[bh] = l; }
 }
 
+// amax|dO| and amax|V| of one (batch, head) -> {s, log2 s}, s the power of two that brings
+// sqrt(d) * amax|dO| * amax|V| (a few times a typical |dP|) to about 2^12.  Two steps: kScaleChunks
+// workgroups per (batch, head) leave their maxima in `part`, one thread per (batch, head) finishes.
+__global__ __launch_bounds__(256) void dc_scale_partial_kernel(int Nq, int Nk, int d, const bf16_t *__restrict__ dO,
+                                                               const bf16_t *__restrict__ V, float *__restrict__ part) {
+    const size_t bh = (size_t)blockIdx.z * gridDim.y + blockIdx.y;   // y = head, z = batch
+    __shared__ float red[2][4];
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+        const size_t cnt = (size_t)(which ? Nk : Nq) * d / 8;   // 16-byte pieces of the slab
+        const size_t per = (cnt + kScaleChunks - 1) / kScaleChunks;
+        const size_t lo = blockIdx.x * per, hi = lo + per < cnt ? lo + per : cnt;
+        const u32x4 *src = reinterpret_cast<const u32x4 *>((which ? V : dO) + bh * (which ? Nk : Nq) * (size_t)d);
+        unsigned int m = 0;
+        for (size_t i = lo + threadIdx.x; i < hi; i += 256) {
+            const u32x4 v = src[i];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                m = max(m, (v[j] << 16) & 0x7fffffffu);
+                m = max(m, v[j] & 0x7fff0000u);
+            }
+        }
+        // NaN / Inf inputs (exponent all ones) are left out of the maximum: they poison the results anyway
+        const float mx = wave_max(m < 0x7f800000u ? __uint_as_float(m) : 0.f);
+        if ((threadIdx.x & 63) == 0) red[which][threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        part[(bh * kScaleChunks + blockIdx.x) * 2 + threadIdx.x] =
+            fmaxf(fmaxf(red[threadIdx.x][0], red[threadIdx.x][1]), fmaxf(red[threadIdx.x][2], red[threadIdx.x][3]));
+}
+__global__ void dc_scale_finish_kernel(int n_bh, int d, const float *__restrict__ part, float *__restrict__ out) {
+    const int bh = blockIdx.x * blockDim.x + threadIdx.x;
+    if (bh >= n_bh) return;
+    float a = 0.f, v = 0.f;
+    for (int c = 0; c < kScaleChunks; ++c) {
+        a = fmaxf(a, part[((size_t)bh * kScaleChunks + c) * 2]);
+        v = fmaxf(v, part[((size_t)bh * kScaleChunks + c) * 2 + 1]);
+    }
+    write_dc_scale(d, a, v, out + 2 * bh);
+}
+
 }  // namespace
 
 hipError_t bwd_preprocess(const Problem &p, int in_dt, int out_dt, const void *o, const void *d_o,
@@ -295,6 +337,19 @@ hipError_t chain_reduce(const Problem &p, int out_dt, int share, const float *pa
         chain_reduce_kernel<bf16_t><<<grid, 256, 0, s>>>(p, share, n_wg, part, (bf16_t *)dk, (bf16_t *)dv);
     else
         chain_reduce_kernel<float><<<grid, 256, 0, s>>>(p, share, n_wg, part, (float *)dk, (float *)dv);
+    return hipGetLastError();
+}
+
+hipError_t mfma_dc_scale(const Problem &p, const void *d_o, const void *v, float *dc_scale, hipStream_t s) {
+    // dc_scale holds {s, log2 s} per (batch, head), then the partial maxima
+    float *part = dc_scale + (size_t)p.B * p.H * 2;
+    dc_scale_partial_kernel<<<dim3(kScaleChunks, p.H, p.B), 256, 0, s>>>(p.Nq, p.Nk, p.d, (const bf16_t *)d_o,
+                                                                          (const bf16_t *)v, part);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? dc_scale_finish(p, dc_scale, s) : e;
+}
+hipError_t dc_scale_finish(const Problem &p, float *dc_scale, hipStream_t s) {
+    dc_scale_finish_kernel<<<dim3((p.B * p.H + 255) / 256), 256, 0, s>>>(p.B * p.H, p.d, dc_scale + (size_t)p.B * p.H * 2, dc_scale);
     return hipGetLastError();
 }
 

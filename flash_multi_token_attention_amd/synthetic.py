@@ -95,37 +95,38 @@ def useful_flops(wl: Workload) -> Dict[str, float]:
 def executed_mfma_flops(wl: Workload, two_pass: bool = False) -> Dict[str, object]:
     """FLOPs the bf16 MFMA kernels execute on the matrix cores for one step of a causal workload
     with d in {64, 128} and at most 6 query taps, counted from their tiles (every MFMA is
-    16 x 16 x 32 = 16384 FLOP), next to the useful ones; the difference is halo, convolution, dW and
+    16 x 16 x 32 = 16384 FLOP; a sparse 16 x 16 x 64 one, which takes two tap slots of a convolution in
+    the same time, counts the same), next to the useful ones; the difference is halo, convolution, dW and
     recompute.  Per kernel:
 
     forward: a wave owns 33 - T output rows (T = 3 or 6 tap slots) of a 32-row score tile and walks
       the keys in 32-key steps up to its last row + 16: per step S^T 2 (row fragments) x 2 (key
-      blocks) x d/32, convolution 4 T, P V 2 x d/16 MFMAs.
+      blocks) x d/32, convolution 4 C (C = 2 or 3 products for the T slots), P V 2 x d/16 MFMAs.
     key-stationary backward: a wave triple owns 32 keys and walks 32-row tiles from the first row that
-      sees its keys: per tile S^T 6 d/32 (48 keys for 32 owned), convolution 4 T (32 keys), dP 4 d/32,
-      transposed convolution 4 T, dV and dK 2 d/16 each, dW 4 T MFMAs; for the last of a workgroup's
+      sees its keys: per tile S^T 6 d/32 (48 keys for 32 owned), convolution 4 C (32 keys), dP 4 d/32,
+      transposed convolution 4 C, dV and dK 2 d/16 each, dW 4 T MFMAs; for the last of a workgroup's
       four triples a second score chain computes the 16 keys after its own (S^T 4 d/32 for the two
-      16-key blocks around them, convolution 2 T, dP 2 d/32).
+      16-key blocks around them, convolution 2 C, dP 2 d/32).
     dQ = dS K: 2 x d/16 per 32 rows x 32 keys below the diagonal (nothing wasted but the diagonal
       blocks' upper halves).
     """
     assert wl.causal and wl.Nq == wl.Nk
     N, d, T, bh = wl.Nq, wl.d, (3 if wl.c_q <= 3 else 6), wl.B * wl.H
-    mf = 16.0 * 16 * 32 * 2
+    mf, C = 16.0 * 16 * 32 * 2, (T + 1) // 2
     rows = 33 - T
     fwd = 0
     for w0 in range(0, N, rows):                       # one wave per `rows` output rows
         wg_end = min(N, (w0 // (4 * rows) + 1) * 4 * rows)          # its workgroup's last row + 1
         steps = min((w0 + rows + 15) // 32 + 1, (wg_end + 16 + 31) // 32)
-        fwd += steps * (4 * d // 32 + 4 * T + 2 * d // 16)
-    consumer = 4 * T + 4 * d // 16 + 4 * T             # transposed convolution, dV and dK, dW
-    light = 6 * d // 32 + 4 * T + 4 * d // 32
-    extra = 4 * d // 32 + 2 * T + 2 * d // 32           # the score chain of the block after the workgroup's keys
+        fwd += steps * (4 * d // 32 + 4 * C + 2 * d // 16)
+    consumer = 4 * C + 4 * d // 16 + 4 * T             # transposed convolution, dV and dK, dW
+    light = 6 * d // 32 + 4 * C + 4 * d // 32
+    extra = 4 * d // 32 + 2 * C + 2 * d // 32           # the score chain of the block after the workgroup's keys
     heavy = light + extra
     full = kv = qw = s_only = 0
-    for c0 in range(0, (N + 8 + 127) // 128 * 128, 32):   # one wave pair per 32 keys
+    for c0 in range(0, (N + 8 + 127) // 128 * 128, 32):   # one wave triple per 32 keys
         k0 = c0 // 128 * 128
-        last = c0 - k0 == 96                            # the last pair of its workgroup
+        last = c0 - k0 == 96                            # the last triple of its workgroup
         r_begin = max(0, k0 - 8) // 32 * 32
         n_t = max(0, (N - r_begin + 31) // 32)
         skipped = sum(1 for t in range(n_t) if r_begin + 32 * t + 31 < c0 - 8)   # scores only

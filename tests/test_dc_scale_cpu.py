@@ -1,7 +1,7 @@
 """CPU emulation of the quantisation step of the backward's dC tiles: dC = P (dP - D) is stored as
 fp16 times a power of two s per (batch, head).  Without s, dC underflows fp16 for small upstream
 gradients; with s taken from amax|D| (csrc/mfma_common.hpp: dc_scale_log2_from_d) or from
-amax|dO| amax|V| (csrc/bwd_chain_mfma.hip: dc_scale_finish_kernel) the relative error of the
+amax|dO| amax|V| (csrc/reduce_kernels.hip: dc_scale_finish_kernel) the relative error of the
 quantised dC does not depend on the magnitude of dO."""
 import math
 
