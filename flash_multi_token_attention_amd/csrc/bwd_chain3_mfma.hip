@@ -33,19 +33,15 @@ namespace {
 using namespace chain;
 
 constexpr int NT3 = 3 * NP * 64;  // 768 threads
-// Wave priorities (s_setprio): the wave of a SIMD that has the least slack before the barrier issues first.
-#ifndef C3_PRIO_SCORE
-#define C3_PRIO_SCORE 1   // score waves, MFMA phases (0 in the P / dC arithmetic)
-#endif
-#ifndef C3_PRIO_EXTRA
-#define C3_PRIO_EXTRA 3   // the value wave that also computes the block after the workgroup's keys
-#endif
-#ifndef C3_PRIO_VALUE
-#define C3_PRIO_VALUE 1   // value waves
-#endif
-#ifndef C3_PRIO_KEY
-#define C3_PRIO_KEY 0     // key waves
-#endif
+// Wave priorities (s_setprio): the score and the key waves' chains are the longest, and the value wave that also computes the block
+// after the workgroup's keys has the least slack before the barrier.  Kernel of B4 H16 N4096, us, against 1 for score and value waves and 0
+// for key waves: d 128 6x11 1340 -> 1310, d 64 6x11 1025 -> 970, 11x11 1350 -> 1265; key waves first of all, or value waves at 0 or the
+// arithmetic of P and dC above 0, are slower or the same.
+constexpr int kPrioScore = 2;   // score waves, MFMA phases (0 in the P / dC arithmetic)
+constexpr int kPrioExtra = 3;   // the value wave that also computes the block after the workgroup's keys
+constexpr int kPrioValue = 1;   // value waves
+constexpr int kPrioKey = 2;     // key waves
+
 // One role of the workgroup: ROLE 0 = score waves, 1 = value waves (dV, dW, the block after the
 // workgroup's keys), 2 = key waves (dS, dK).  WANT: bit 0 = dK and dV, bit 1 = dS (for dQ) and dW.
 template <int D, int CQT, typename TO, int ROLE, int WANT>
@@ -306,7 +302,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 constexpr bool FULL = decltype(full_tag)::value;
                 const unsigned char *Qs = smem + opaque((unsigned int)(q_slot(it) - smem) + row_frag_off());
                 const unsigned char *Gs = smem + opaque((unsigned int)(g_slot(it) - smem) + row_frag_off());
-                __builtin_amdgcn_s_setprio(VLDS ? C3_PRIO_EXTRA : C3_PRIO_SCORE);
+                __builtin_amdgcn_s_setprio(VLDS ? kPrioExtra : kPrioScore);
                 f32x4 dp[NCBL][2];
                 float2 l2 = {0.f, 0.f};
                 if constexpr (FULL) l2 = *reinterpret_cast<const float2 *>(stat_slot(it) + 2 * n);
@@ -385,7 +381,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                     if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
                     static_for<NCBL>([&](auto CB) {
                         constexpr int cb = decltype(CB)::value, cba = CB0 + cb;
-                        __builtin_amdgcn_s_setprio(VLDS ? C3_PRIO_EXTRA : 0);
+                        __builtin_amdgcn_s_setprio(VLDS ? kPrioExtra : 0);
 #pragma unroll
                         for (int ob = 0; ob < 2; ++ob) {
                             f32x4 prob, dc;
@@ -524,7 +520,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                     __syncthreads();
                     if (it + 1 < n_scored) fetch_tile(it + 1);
                     const int u = it - 1;
-                    if (WANT_KV && it >= 1 && u < n_tiles && !is_skipped(r_begin + u * BR)) dv_phase(u, std::integral_constant<int, C3_PRIO_EXTRA>{});
+                    if (WANT_KV && it >= 1 && u < n_tiles && !is_skipped(r_begin + u * BR)) dv_phase(u, std::integral_constant<int, kPrioExtra>{});
                     __builtin_amdgcn_sched_barrier(0);
                     tile(it);
                 }
@@ -545,7 +541,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 if (it + 1 < n_scored) fetch_tile(it + 1);
                 const int u = it - 1;
                 const bool u_in = it >= 1 && u < n_tiles;
-                if (WANT_KV && u_in && !is_skipped(r_begin + u * BR)) dv_phase(u, std::integral_constant<int, C3_PRIO_VALUE>{});
+                if (WANT_KV && u_in && !is_skipped(r_begin + u * BR)) dv_phase(u, std::integral_constant<int, kPrioValue>{});
                 // ---- dW, key blocks jb = 0..7 (block jb = dC block jb & 1 of triple jb / 2, keys k0 - 8 + 16 jb ..):
                 // G_t[j][j'] += sum_rows dC[row][j] S[row + t - (CQT-1)][j'] with j' in the score block
                 // 8 keys before the dC block (x = 0) and the one 8 keys after it (x = 1).
@@ -683,7 +679,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
             }
             if (v_ok) {
                 bf16_t *ds_blk = ds_pair + (size_t)(r0v / BR) * (WK * BR);
-                __builtin_amdgcn_s_setprio(C3_PRIO_KEY);
+                __builtin_amdgcn_s_setprio(kPrioKey);
                 // ---- dS^T of tile v: rows below it come from tile v+1.  Operand of row offset
                 // e = parity + (CQT-1 - tap slot): fragment e & 1 shifted e >> 1 lanes up; two tap slots per product. ----
                 f32x4 ds[NDB][2];
