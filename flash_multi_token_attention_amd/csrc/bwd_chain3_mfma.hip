@@ -20,9 +20,11 @@
 // other roles' work left out), the other roles as much without it, and together they share the LDS (two thirds busy), the matrix
 // pipe and the vector ALUs.  So both convolutions take two tap slots per sparse product (SparseTaps in mfma_common.hpp), the key
 // waves keep their bands in registers, and dW's operands of neighbouring taps share their transpose reads (43 per wave and tile for
-// 56 at 6 slots, 61 for 112 at 11).  Kernel alone, B4 H16 N4096 causal, before -> after, us, in turn on one card: d 128 6x11 1409 -> 1310,
-// d 64 6x11 1097 -> 1048, 11x11 1442 -> 1283, 3x3 833 -> 804; at d 128 with more than 6 taps, in the place of a kernel of two waves per
-// SIMD and 256 registers, 7x7 1510 -> 1424, 11x11 1960 -> 1565 (B1 H8 N1500 61 -> 49).
+// 56 at 6 slots, 61 for 112 at 11).  Rows of S and dC of 104 bytes (112 before: an 8-byte store of 16 rows two apart took 17 clocks of
+// the LDS, now 9) and the offset of the odd rows of Q and dO (transpose reads 5 -> 3) left 34 % of the LDS's busy clocks to conflicts at d = 128,
+// 42 before; the rest, row fragments and the stores, gained nothing when taken out at the price of registers.  Kernel alone,
+// B4 H16 N4096 causal, before -> after, us: d 128 6x11 1409 -> 1270, d 64 6x11 1097 -> 930, 11x11 1442 -> 1243, 3x3 833 -> 770; at d 128 with more than 6 taps, in the place of a kernel of two waves per
+// SIMD and 256 registers, 7x7 1510 -> 1350, 11x11 1960 -> 1520 (B1 H8 N1500 61 -> 49).
 #include <type_traits>
 
 #include "chain_common.hpp"
@@ -120,8 +122,8 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
     // and key waves (the score waves start on the tile right after the barrier).  A tile is 2 KBT units
     // of 1 KB (KBT of Q, then KBT of dO; unit 2 ks + f = the 16 row pairs of one k-step and parity).
     typedef int i32x4 __attribute__((ext_vector_type(4)));
-    constexpr int KBT = Lds::tile_bytes / 1024;
-    static_assert(KBT == 2 * KS && ((2 * KBT) % (2 * NP) == 0 || 2 * KBT < 2 * NP), "whole units per loading wave");
+    constexpr int KBT = 2 * KS;
+    static_assert(((2 * KBT) % (2 * NP) == 0 || 2 * KBT < 2 * NP), "whole units per loading wave");
     auto dma_rsrc = [&](const bf16_t *ptr) {
         const unsigned long long a = reinterpret_cast<unsigned long long>(ptr);
         return (i32x4){(int)(unsigned int)a, (int)(unsigned int)(a >> 32), p.Nq * D * 2, 0x00020000};
@@ -137,7 +139,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 if (j >= 2 * KBT) break;   // (head dimension 32: four units for eight waves)
                 const int row = 2 * (ln >> 2) + (kb & 1), chunk = (kb >> 1) * 4 + ((ln & 3) ^ ((ln >> 4) & 3));
                 const int voff = ((r_begin + t * BR + row) * D + chunk * 8) * 2;
-                const unsigned int dst = lds0 + (m ? Lds::g_off + (t % 3) * Lds::tile_bytes : Lds::q_off + (t & 3) * Lds::tile_bytes) + kb * 1024;
+                const unsigned int dst = lds0 + (m ? Lds::g_off + (t % 3) * Lds::tile_bytes : Lds::q_off + (t & 3) * Lds::tile_bytes) + kb * Lds::plane;
                 const i32x4 rsrc = m ? g_dma : q_dma;
                 // (M0 is written here and read by the load that follows; nothing else of this kernel uses it)
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
@@ -181,11 +183,11 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
     // Lane parts of the fragment addresses inside a tile (see ChainLds).
     auto row_frag_off = [&] { return (unsigned int)(n * 64 + ((g ^ ((n >> 2) & 3)) << 4)); };
     auto tr_frag_off = [&] {
-        return (unsigned int)(((n >> 2) & 1) * 1024 + (2 * g + (n >> 3)) * 64 + ((((n >> 1) & 1) ^ (g >> 1)) << 4) + (n & 1) * 8);
+        return (unsigned int)(((n >> 2) & 1) * Lds::plane + (2 * g + (n >> 3)) * 64 + ((((n >> 1) & 1) ^ (g >> 1)) << 4) + (n & 1) * 8);
     };
     auto read_tr_t = [&](const unsigned char *lane_ptr, int db) {   // (db: a constant after unrolling)
-        bf16x4 lo = lds_tr64(lane_ptr + (db >> 1) * 2048 + ((db & 1) << 5));
-        bf16x4 hi = lds_tr64(lane_ptr + (db >> 1) * 2048 + (((db & 1) ^ 1) << 5) + 512);
+        bf16x4 lo = lds_tr64(lane_ptr + (db >> 1) * 2 * Lds::plane + ((db & 1) << 5));
+        bf16x4 hi = lds_tr64(lane_ptr + (db >> 1) * 2 * Lds::plane + (((db & 1) ^ 1) << 5) + 512);
         return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     };
 
@@ -309,7 +311,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 // ---- S^T ----
                 unsigned int pd[NKB][2][2];
                 s_phase(r0, it + 1, pd, edge_tag, [&](int f, int ks) {
-                    return *reinterpret_cast<const bf16x8 *>(Qs + f * 1024 + ks * 2048);
+                    return *reinterpret_cast<const bf16x8 *>(Qs + (2 * ks + f) * Lds::plane);
                 });
                 // (the instance beside the dV accumulators has no registers for phases that overlap)
                 if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
@@ -337,7 +339,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                             bf16x8 gf[2];
 #pragma unroll
                             for (int f = 0; f < 2; ++f)
-                                gf[f] = *reinterpret_cast<const bf16x8 *>(Gs + f * 1024 + ks * 2048);
+                                gf[f] = *reinterpret_cast<const bf16x8 *>(Gs + (2 * ks + f) * Lds::plane);
 #pragma unroll
                             for (int cb = 0; cb < NCBL; ++cb) {
                                 bf16x8 vk = vf[cb][ks];
@@ -547,7 +549,7 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 // 8 keys before the dC block (x = 0) and the one 8 keys after it (x = 1).
                 // A transpose read takes four rows from wherever its lanes point: k slot 4 m + r of a lane group is row
                 // 8 g + 2 r + m, so that a read of the rows one further down is the second half of one tap's operand and the
-                // first of the next one's: TW + 1 reads for TW taps.  (Eight such rows of 112 bytes cover every bank once.) ----
+                // first of the next one's: TW + 1 reads for TW taps. ----
                 if (WANT_QW && u_in) {
                     const int wbase = ((u + 1) * BR - (CQT - 1) + Lds::ring_rows) % Lds::ring_rows;
                     const unsigned int row = 8 * g + 2 * (n >> 2), col = 4 * (n & 3) * 2;

@@ -15,9 +15,9 @@ constexpr int BR = 32;           // query rows per tile
 constexpr int NSB = 4;           // S^T blocks of a pair: keys c0-16+16kb
 constexpr int NCB = 3;           // C / dP / dC blocks: keys c0-8+16cb
 constexpr int NDB = 2;           // dS blocks: keys c0+16sb
-constexpr int SST = 112;         // bytes per row of the S tile in LDS (48 keys fp16 + 16)
+constexpr int SST = 104;         // bytes per row of the S tile in LDS (48 keys fp16 + 8)
 constexpr int S_RING = 72;       // rows of the S ring: a tile being written, the tile before it and 8 rows more (>= c_q - 1)
-constexpr int CST = 112;         // bytes per row of the dC tile (48 keys fp16 + 16)
+constexpr int CST = 104;         // bytes per row of the dC tile (48 keys fp16 + 8)
 constexpr int PST = 72;          // bytes per row of the P and dS tiles (32 keys bf16 + 8)
 static_assert(BKW == kKvKeysPerWg && WK == kChainKeys && BR == kChainRows, "dS workspace layout");
 
@@ -86,7 +86,8 @@ template <int D, int CQT> struct ChainLds {
     // 2n + f) and transposed fragments then touch every bank equally often, and k-step, parity and
     // head-dim block are constant offsets from one lane address.
     static constexpr int RST = D * 2;                               // bytes per Q / dO row
-    static constexpr int tile_bytes = BR * RST;
+    // (a plane of one parity is 32 bytes longer than its rows: the transpose reads take two rows of either parity at a time)
+    static constexpr int plane = 1024 + 32, tile_bytes = RST / 32 * plane;
     static constexpr int q_off = 0, q_slots = 4;                    // tiles it-2 .. it+1
     static constexpr int g_off = q_off + q_slots * tile_bytes, g_slots = 3;  // tiles it-1 .. it+1
     static constexpr int stat_off = g_off + g_slots * tile_bytes;   // LSE and D of a tile: two slots
