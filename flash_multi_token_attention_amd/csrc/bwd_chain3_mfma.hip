@@ -205,12 +205,13 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
         const bf16_t *Kb = K + bh * p.Nk * D;
         const bf16_t *Vb = V + bh * p.Nk * D;
         const unsigned char *bands = smem + opaque((unsigned int)Lds::band_off + lane * 16);
-        // (the score waves keep their V fragments in registers; the value wave that computes the block after
-        // the workgroup's keys parks them in LDS, in fragment order: one conflict-free 16-byte read per k-step)
+        // (the score waves keep their K and V fragments in registers; the value wave that computes the block after
+        // the workgroup's keys parks V's and half of K's in LDS, in fragment order: one conflict-free 16-byte read per k-step)
         constexpr bool VLDS = KB0 != 0;
         static_assert(!VLDS || NCBL == 1, "LDS room for one block of V fragments");
         bf16x8 kf[NKB][KS], vf[NCBL][KS];
         unsigned char *v_park = smem + opaque((unsigned int)Lds::e_off + lane * 16);
+        constexpr bool KLDS = VLDS && Lds::k_park;   // the K fragments of its last block as well
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
@@ -223,7 +224,10 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                 vf[cb][ks] = __builtin_bit_cast(bf16x8, load_row16_nb<D>(Vb, c0 - 8 + (CB0 + cb) * 16 + n, p.Nk, ks * 32 + g * 8));
         if constexpr (VLDS) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) *reinterpret_cast<bf16x8 *>(v_park + ks * 1024) = vf[0][ks];
+            for (int ks = 0; ks < KS; ++ks) {
+                *reinterpret_cast<bf16x8 *>(v_park + ks * 1024) = vf[0][ks];
+                if constexpr (KLDS) *reinterpret_cast<bf16x8 *>(v_park + (KS + ks) * 1024) = kf[NKB - 1][ks];
+            }
         }
         // Q rows of the 32 rows above the first tile
         bf16x8 q_above[2][KS];
@@ -250,9 +254,12 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
 #pragma unroll
                 for (int f = 0; f < 2; ++f) qf[f] = load_qf(f, ks);
 #pragma unroll
-                for (int kb = 0; kb < NKB; ++kb)
+                for (int kb = 0; kb < NKB; ++kb) {
+                    bf16x8 kk = kf[kb][ks];
+                    if (KLDS && kb == NKB - 1) kk = *reinterpret_cast<const bf16x8 *>(v_park + (KS + ks) * 1024);
 #pragma unroll
-                    for (int f = 0; f < 2; ++f) acc[kb][f] = mfma_bf16(kf[kb][ks], qf[f], acc[kb][f]);
+                    for (int f = 0; f < 2; ++f) acc[kb][f] = mfma_bf16(kk, qf[f], acc[kb][f]);
+                }
             }
             const int rbase = (tp * BR) % Lds::ring_rows;
 #pragma unroll

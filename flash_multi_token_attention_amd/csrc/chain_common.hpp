@@ -109,9 +109,12 @@ template <int D, int CQT> struct ChainLds {
     static constexpr int p_bytes = 2 * BR * PST;
     static constexpr int ds_bytes = BR * PST;
     static constexpr int pair_bytes = s_bytes + c_bytes + p_bytes + ds_bytes;
-    // V fragments of the block after the workgroup's keys (16 rows; the wave that computes it has no registers to keep them in)
+    // V and, where there is room, K fragments of the block after the workgroup's keys (16 rows each): the wave that computes it has no
+    // registers to keep them in (with K in registers 12 and 24 spilled at d = 128, 6 and 8 slots, now 0 and 2; kernel of B4 H16 N4096 1254 ->
+    // 1253 and 1384 -> 1352 us, of B1 H32 N16384 6x11 9075 -> 9009)
     static constexpr int e_off = pair_off + NP * pair_bytes;
-    static constexpr int total = e_off + 16 * D * 2;
+    static constexpr bool k_park = D == 128 && CQT <= 8;   // (11 slots: no room)
+    static constexpr int total = e_off + 16 * D * 2 * (k_park ? 2 : 1);
     static_assert(CQT * 2 * 1024 <= NP * pair_bytes, "room for the dW accumulators (they take the place of the pairs' tiles)");
 };
 
