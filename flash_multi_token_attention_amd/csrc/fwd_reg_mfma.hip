@@ -429,7 +429,7 @@ __global__ __launch_bounds__(NW * 64, fwd_waves(D, CQT)) void fwd_reg_mfma_kerne
                 const float alpha = fast_exp2(m_ref[ob] - new_use);
                 const float delta = new_use - old_use;
                 m_ref[ob] = m_new;
-                m_rel[ob] -= delta;
+                if (new_use < -kNegInf) m_rel[ob] -= delta;   // (under a base of +inf it stays +inf: inf - inf is no maximum)
                 slack[ob] = (m_new == kNegInf) ? kNegInf : kMaxSlack;
                 neg_base[ob] = (f32x4){-new_use, -new_use, -new_use, -new_use};
                 l_run[ob] *= alpha;

@@ -1,0 +1,33 @@
+"""Window forward of rows that see an infinite score: their maximum is +inf, and every other row is what it is without."""
+import pytest
+import torch
+
+from flash_multi_token_attention_amd.conv_attn import ops
+from tests.util import TOL_BF16, max_abs, oracle_fwd, rand_case, scale_of
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# sparse and dense windows, odd and even tap slots, keys of a row tile in one workgroup and in several (N >= 1000)
+@pytest.mark.parametrize("N,d,c_q,c_k,causal", [
+    (200, 64, 6, 11, True), (200, 128, 8, 15, False), (200, 32, 7, 17, False), (1100, 64, 3, 3, True), (1100, 128, 6, 17, True),
+])
+def test_maximum_is_infinite(N, d, c_q, c_k, causal):
+    Q, K, V, _, W = rand_case(1, 2, N, N, d, c_q, c_k, torch.bfloat16, seed=N + d)
+    W = W.abs() + 0.05              # (one sign: no row adds +inf and -inf)
+    key = 37
+    Q[..., 0] = Q[..., 0].abs() + 0.5
+    K[0, 0, key, 0] = 1.0           # the finite case, then infinite scores of this key in head 0
+    args = (W.to(DEV), scale_of(d), c_q - 1, (c_k - 1) // 2, causal)
+    _, M_fin, L_fin = ops.forward(Q.to(DEV), K.to(DEV), V.to(DEV), *args, out_dtype=torch.float32)
+    _, M_ref, _ = oracle_fwd(Q, K, V, W, causal)
+    assert max_abs(M_fin, M_ref) <= TOL_BF16
+    K[0, 0, key, 0] = float("inf")
+    _, M, L = ops.forward(Q.to(DEV), K.to(DEV), V.to(DEV), *args, out_dtype=torch.float32)
+    # (the rows before the first have zeros for Q, whose product with the infinity is NaN: without the mask the first rows see one)
+    first = key if causal else c_q - 1
+    assert bool((M[0, 0, first:] == float("inf")).all()) and bool(L[0, 0, first:].isnan().all())
+    assert torch.equal(M[0, 1], M_fin[0, 1]) and torch.equal(L[0, 1], L_fin[0, 1])
+    if causal:
+        assert max_abs(M[0, 0, :key], M_ref[0, 0, :key]) <= TOL_BF16 and bool(L[0, 0, :key].isfinite().all())
