@@ -372,6 +372,12 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                         static_for<NCBL>([&](auto CB) {
                             constexpr int cb = decltype(CB)::value;
                             if constexpr (cb > 0) put(std::integral_constant<int, CB0 - KB0 + cb + 1>{}, std::integral_constant<int, (cb + 1) % 2>{});
+                            static_for<2>([&](auto OB) {
+                                constexpr int ob = decltype(OB)::value;
+                                if constexpr (Taps::odd && Taps::single_tuple(ob) == j)
+                                    c[cb][ob] = Lds::Bands::single(*reinterpret_cast<const f16x8 *>(bands + Lds::Bands::single_row(ob) * Lds::Bands::row_bytes), ob,
+                                                                   cb % 2 != 0, rows, c[cb][ob]);
+                            });
                             static_for<2 * Taps::products>([&](auto X) {
                                 constexpr int ob = decltype(X)::value / Taps::products, i = decltype(X)::value % Taps::products;
                                 if constexpr (Taps::tuple(i, ob) == j)
@@ -631,11 +637,15 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
         using Taps = ChainTaps<CQT>;
         const int sp_index = sparse_index(g, n, false);
         constexpr int KR = Lds::key_regs;
-        f16x8 band_regs[KR > 0 ? KR : 1][2];
+        f16x8 band_regs[KR > 0 ? KR : 1][2], single_regs[2];
 #pragma unroll
         for (int i = 0; i < KR; ++i)
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) band_regs[i][ob] = Lds::Bands::frag(Lds::Bands::row(i, ob) + (g >> 1), w_head, cq, ck, pk, g, n, true, p.scale);
+        constexpr bool SINGLE_REGS = Taps::odd && KR == Taps::products;
+#pragma unroll
+        for (int ob = 0; ob < 2; ++ob)
+            if constexpr (SINGLE_REGS) single_regs[ob] = Lds::Bands::frag(Lds::Bands::single_row(ob) + (g >> 1), w_head, cq, ck, pk, g, n, true, p.scale);
         const unsigned char *bands = smem + opaque((unsigned int)Lds::key_band_off + lane * 16);
         if constexpr (KR < Taps::products)
             Lds::Bands::build(smem + Lds::key_band_off, Lds::key_row, w_head, cq, ck, pk, true, p.scale, pr, NP, g, n);
@@ -710,6 +720,15 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                     static_for<NDB>([&](auto SB) {
                         constexpr int sb = decltype(SB)::value;
                         if constexpr (sb > 0) put(std::integral_constant<int, sb + 1>{}, std::integral_constant<int, (sb + 1) % 2>{});
+                        static_for<2>([&](auto OB) {
+                            constexpr int ob = decltype(OB)::value;
+                            if constexpr (Taps::odd && Taps::single_tuple(ob) == j) {
+                                f16x8 band = single_regs[ob];
+                                if constexpr (!SINGLE_REGS)
+                                    band = *reinterpret_cast<const f16x8 *>(bands + (Lds::Bands::single_row(ob) - Lds::key_row) * Lds::Bands::row_bytes);
+                                ds[sb][ob] = Lds::Bands::single(band, ob, sb % 2 != 0, rows, ds[sb][ob]);
+                            }
+                        });
                         static_for<2 * Taps::products>([&](auto X) {
                             constexpr int ob = decltype(X)::value / Taps::products, i = decltype(X)::value % Taps::products;
                             if constexpr (Taps::tuple(i, ob) == j) {

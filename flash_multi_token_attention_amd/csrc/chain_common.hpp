@@ -23,33 +23,32 @@ static_assert(BKW == kKvKeysPerWg && WK == kChainKeys && BR == kChainRows, "dS w
 
 // The bands of the sparse products (two tap slots each, see SparseTaps).  The half of a fragment that belongs to one slot is the same
 // wherever that slot stands: a row of 32 lanes x 16 bytes, and a product whose two slots have neighbouring rows reads its
-// fragment as 1 KB from the first one's row on.  Odd CQT: a row of zeros before slot 0 and after the last (a parity's single slot is a
-// product with one of them).  Even: two more rows for the product of slots 0 and CQT - 1.  `flip`: the transposed convolution, whose
-// rows are counted downwards (row offset e = delta + CQT - 1, tap slot CQT - 1 - slot).
-template <int CQT> using ChainTaps = SparseTaps<CQT, false>;
+// fragment as 1 KB from the first one's row on.  Even CQT: two more rows for the product of slots 0 and CQT - 1.  Odd: two more for each
+// parity's single slot, the operand of a dense product (64 lanes x 16 bytes, the window's first block in the even dwords).  `flip`: the
+// transposed convolution, whose rows are counted downwards (row offset e = delta + CQT - 1, tap slot CQT - 1 - slot).
+template <int CQT> using ChainTaps = SparseTaps<CQT>;
 template <int CQT> struct ChainBands {
     using T = ChainTaps<CQT>;
-    static constexpr int rows = CQT + 2, row_bytes = 512;
-    static constexpr int slot(int row) { return T::odd ? row - 1 : row < CQT ? row : row == CQT ? 0 : CQT - 1; }
-    // first row of product i of output parity ob
-    static constexpr int row(int i, int ob) { return T::odd ? 2 * i - ob + 1 : !ob && i == T::products - 1 ? CQT : 2 * i + 1 - ob; }
+    static constexpr int rows = CQT + (T::odd ? 4 : 2), row_bytes = 512;
+    static constexpr int slot(int row) {
+        return row < CQT ? row : T::odd ? T::single_slot(row >= CQT + 2) : row == CQT ? 0 : CQT - 1;
+    }
+    // first row of product i of output parity ob, and of its single slot
+    static constexpr int row(int i, int ob) { return T::odd ? 2 * i + ob : !ob && i == T::products - 1 ? CQT : 2 * i + 1 - ob; }
+    static constexpr int single_row(int ob) { return CQT + 2 * ob; }
     static constexpr bool rows_right() {
         for (int ob = 0; ob < 2; ++ob)
             for (int i = 0; i < T::products; ++i)
-                for (int half = 0; half < 2; ++half) {
-                    const int want = T::slot(T::tuple(i, ob), half, ob), have = slot(row(i, ob) + half);
-                    if (want != have && !(want == CQT && (have < 0 || have >= CQT))) return false;
-                }
+                for (int half = 0; half < 2; ++half)
+                    if (T::slot(T::tuple(i, ob), half, ob) != slot(row(i, ob) + half)) return false;
         return true;
     }
-    static_assert(rows_right(), "rows of the products");
+    static_assert(T::every_slot_once() && rows_right(), "rows of the products");
     // this lane's 16 bytes of a row
     static __device__ __forceinline__ f16x8 frag(int row, const float *__restrict__ w_head, int c_q, int c_k, int pk, int g, int n,
                                                  bool flip, float mul) {
-        int t = slot(row);
-        const bool none = t < 0 || t >= CQT;
-        if (flip) t = CQT - 1 - t;
-        const int a = t - (CQT - c_q);
+        const int t = flip ? CQT - 1 - slot(row) : slot(row), a = t - (CQT - c_q);
+        const bool single = T::odd && row >= CQT;
         // (unconditional loads from clamped indices: the eight of a fragment are in flight together)
         const float *w = w_head + min(max(a, 0), c_q - 1) * c_k;
         float v[8];
@@ -57,15 +56,21 @@ template <int CQT> struct ChainBands {
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const int kappa = sparse_key(g, q), off = kappa + e + (kappa + 1 > n ? 0 : 16) - kKeyHalo - n;
+                const int kappa = single ? 8 * ((row - CQT) & 1) + 4 * (g & 1) + 2 * (q >> 1) : sparse_key(g, q);
+                const int off = kappa + e + ((single ? (q & 1) == 0 : kappa + 1 > n) ? 0 : 16) - kKeyHalo - n;
                 const int bb = flip ? pk - off : pk + off;
                 v[2 * q + e] = w[min(max(bb, 0), c_k - 1)];
-                if (none || a < 0 || bb < 0 || bb >= c_k) v[2 * q + e] = 0.f;
+                if (a < 0 || bb < 0 || bb >= c_k) v[2 * q + e] = 0.f;
             }
         f16x8 f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) f[e] = (_Float16)(v[e] * mul);
         return f;
+    }
+    // c + the single slot of parity ob, from the tuple it is in (`swapped`: the window's first block in the odd dwords)
+    static __device__ __forceinline__ f32x4 single(f16x8 band, int ob, bool swapped, u32x8 rows, f32x4 c) {
+        const u32x4 v = ob ? (u32x4){rows[4], rows[5], rows[6], rows[7]} : (u32x4){rows[0], rows[1], rows[2], rows[3]};
+        return mfma_f16(band, __builtin_bit_cast(f16x8, swapped ? (u32x4){v[1], v[0], v[3], v[2]} : v), c);
     }
     // the rows from `first` on to LDS, dealt out in pairs to `n_waves` waves
     static __device__ __forceinline__ void build(unsigned char *tab, int first, const float *__restrict__ w_head, int c_q, int c_k, int pk,

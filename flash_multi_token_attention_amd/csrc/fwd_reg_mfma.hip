@@ -141,11 +141,9 @@ __global__ __launch_bounds__(NW * 64, fwd_waves(D, CQT)) void fwd_reg_mfma_kerne
 
     // Toeplitz bands of this head, pre-multiplied by scale * log2(e): the convolved scores come out in log2 units.  WIDE: k slot
     // 8g+e of a window is key 4g+e of its first 16-key block for e < 4, key 4g+e-4 of its second for e >= 4.
-    // (11 slots at d = 128 have no registers for the dense operands of the single slots)
-    constexpr bool DENSE_SINGLE = CQT <= 7 || D <= 64;
-    using Taps = SparseTaps<CQT, DENSE_SINGLE>;
+    using Taps = SparseTaps<CQT>;
     f16x8 tf[WIDE ? CQT : 1];
-    SparseBands<CQT, DENSE_SINGLE> bands;
+    SparseBands<CQT, (CQT <= 7 || D <= 64)> bands;   // (11 slots at d = 128 have no registers for both orders of the single slots' blocks)
     int index[2] = {0, 0};   // of the windows that end with a step's first and second score block
     {
         // (the table lies in the K / V buffer that the first step does not use)
@@ -311,7 +309,7 @@ __global__ __launch_bounds__(NW * 64, fwd_waves(D, CQT)) void fwd_reg_mfma_kerne
             if constexpr (blk == 0) {
                 load_kf(1);
                 SCHED_DS_READ(KS);
-                SCHED_MFMA(WIDE ? 2 * CQT : 2 * (Taps::products + Taps::ONE));
+                SCHED_MFMA(WIDE ? 2 * CQT : 2 * (Taps::products + Taps::odd));
             }
             const int key0 = jk + blk * 16 + 4 * g;
 #pragma unroll
@@ -336,19 +334,18 @@ __global__ __launch_bounds__(NW * 64, fwd_waves(D, CQT)) void fwd_reg_mfma_kerne
 #pragma unroll
             for (int ob = 0; ob < 2; ++ob) c[ob][blk] = neg_base[ob];
             if constexpr (!WIDE) {
-                auto single = [&](auto OB) {   // (the first product of its parity)
-                    constexpr int ob = decltype(OB)::value, j = Taps::single_tuple(ob);
-                    const u32x4 bv = {rows[j][4 * ob], rows[j][4 * ob + 1], rows[j][4 * ob + 2], rows[j][4 * ob + 3]};
-                    c[ob][blk] = mfma_f16(bands.one[Taps::ONE ? blk : 0][ob], __builtin_bit_cast(f16x8, bv), c[ob][blk]);
+                auto single = [&](auto OB) {   // (the first product of its parity, which brings the chain's starting value with it)
+                    constexpr int ob = decltype(OB)::value;
+                    c[ob][blk] = bands.single(1 - blk, ob, rows[Taps::single_tuple(ob)], c[ob][blk]);
                 };
-                if constexpr (Taps::ONE) {
+                if constexpr (Taps::odd) {
                     put_rows(std::integral_constant<int, Taps::tuples - 1>{}, BL, pd[blk]);
                     single(std::integral_constant<int, 0>{});
                 }
                 static_for<Taps::tuples>([&](auto J) {
                     constexpr int j = decltype(J)::value;
-                    if constexpr (!Taps::ONE || j < Taps::tuples - 1) put_rows(J, BL, pd[blk]);
-                    if constexpr (Taps::ONE && j == 0) single(std::integral_constant<int, 1>{});
+                    if constexpr (!Taps::odd || j < Taps::tuples - 1) put_rows(J, BL, pd[blk]);
+                    if constexpr (Taps::odd && j == 0) single(std::integral_constant<int, 1>{});
                     static_for<2>([&](auto OB) {
                         constexpr int ob = decltype(OB)::value;
                         static_for<Taps::products>([&](auto I) {

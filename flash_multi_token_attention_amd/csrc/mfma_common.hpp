@@ -79,54 +79,72 @@ __device__ __forceinline__ int sparse_index(int g, int n, bool swapped) {
 }
 // Which taps share a product.  A window of CQT tap slots needs, for output rows of parity ob = 0 and 1, the score rows at
 // offsets delta = slot - (CQT - 1) + ob, CQT + 1 of them.  Operand tuple j holds the offsets delta(j, 0) and delta(j, 1).  For an odd
-// CQT the tuples hold all offsets in pairs, and one slot of each parity stays single: a dense product of four dwords of a tuple,
-// which also brings the chain's starting value with it (ONE), or half of a sparse one (16 registers less).  For an even CQT they hold
-// the offsets of parity 1, and parity 0 has, for its first and its last slot, a tuple of its own in the place of the last one.
-template <int CQT, bool DENSE_SINGLE> struct SparseTaps {
-    static constexpr bool odd = CQT % 2 != 0, ONE = odd && DENSE_SINGLE;
-    static constexpr int tuples = odd ? (CQT + 1) / 2 : CQT / 2 + 1;        // operand tuples
-    static constexpr int products = odd && !ONE ? (CQT + 1) / 2 : CQT / 2;  // sparse products per output parity
+// CQT the tuples hold all offsets in pairs, and one slot of each parity stays single: a dense product of four dwords of a tuple.  (Not
+// a sparse one with zero weights for the other four: those are a row outside the window, whose infinities and NaN would get into the
+// output row.  Nor the sparse 16x16x32: where the 16x16x64 one follows it on the same accumulators, the compiler's waits are too short.)
+// For an even CQT they hold the offsets of parity 1, and parity 0 has, for its first and its last slot, a tuple of its own in the place
+// of the last one.
+template <int CQT> struct SparseTaps {
+    static constexpr bool odd = CQT % 2 != 0;
+    static constexpr int tuples = CQT / 2 + 1;   // operand tuples
+    static constexpr int products = CQT / 2;     // sparse products per output parity
     static constexpr int delta(int j, int half) {
         return !odd && j == CQT / 2 ? (half ? 0 : -(CQT - 1)) : -(CQT - (odd ? 1 : 2)) + 2 * j + half;
     }
     // tuple of product i of parity ob
-    static constexpr int tuple(int i, int ob) { return odd ? (ONE ? i + ob : i) : !ob && i == CQT / 2 - 1 ? CQT / 2 : i; }
-    // tap slot of a half of tuple j for parity ob; the table's row CQT (zeros) where it has none
-    static constexpr int slot(int j, int half, int ob) {
-        const int t = delta(j, half) + CQT - 1 - ob;
-        return t < 0 || t >= CQT ? CQT : t;
-    }
-    // the single slot of a parity (ONE): half ob of this tuple
+    static constexpr int tuple(int i, int ob) { return odd ? i + ob : !ob && i == CQT / 2 - 1 ? CQT / 2 : i; }
+    // tap slot of a half of tuple j for parity ob
+    static constexpr int slot(int j, int half, int ob) { return delta(j, half) + CQT - 1 - ob; }
+    // the single slot of a parity (odd CQT): half ob of this tuple
     static constexpr int single_tuple(int ob) { return ob ? 0 : tuples - 1; }
     static constexpr int single_slot(int ob) { return slot(single_tuple(ob), ob, ob); }
+    static constexpr bool every_slot_once() {
+        for (int ob = 0; ob < 2; ++ob) {
+            int seen = odd ? 1 << single_slot(ob) : 0;
+            for (int x = 0; x < 2 * products; ++x) {
+                const int t = slot(tuple(x / 2, ob), x % 2, ob);
+                if (t < 0 || t >= CQT || (seen >> t & 1)) return false;
+                seen |= 1 << t;
+            }
+            if (seen != (1 << CQT) - 1) return false;
+        }
+        return true;
+    }
 };
 // The bands of a head as a table in LDS: dword x + 16 of tap slot t's 48 holds the weights of two neighbouring keys, T[x] and T[x + 1]
 // with T[x] = w[a][pk + x - 8] * mul (`flip`: pk - (x - 8); zero outside the window), x = the key's place in the window less the output
-// key's; slot t stands for tap a = t - (CQT - c_q), and one more slot of zeros follows.  A lane finds the pairs of its operands there with
+// key's; slot t stands for tap a = t - (CQT - c_q).  A lane finds the pairs of its operands there with
 // 4-byte reads: one or two loads of W per thread instead of the 48 to 88 gathers of every lane.
 constexpr int kBandRow = 48;
-template <int CQT> constexpr int band_table_bytes() { return (CQT + 1) * kBandRow * 4; }
+template <int CQT> constexpr int band_table_bytes() { return CQT * kBandRow * 4; }
 template <int CQT>
 __device__ __forceinline__ void band_table_build(unsigned int *tab, const float *__restrict__ w_head, int c_q, int c_k, int pk, bool flip,
                                                  float mul, int tid, int nthreads) {
-    for (int i = tid; i < (CQT + 1) * kBandRow; i += nthreads) {
+    for (int i = tid; i < CQT * kBandRow; i += nthreads) {
         const int t = i / kBandRow, a = t - (CQT - c_q), off = i - t * kBandRow - 16 - kKeyHalo;
         float v[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const int b = flip ? pk - off - e : pk + off + e;
             v[e] = w_head[min(max(a, 0), c_q - 1) * c_k + min(max(b, 0), c_k - 1)];
-            v[e] = t < CQT && a >= 0 && b >= 0 && b < c_k ? v[e] * mul : 0.f;
+            v[e] = a >= 0 && b >= 0 && b < c_k ? v[e] * mul : 0.f;
         }
         const f16x2 two = {(_Float16)v[0], (_Float16)v[1]};
         tab[i] = __builtin_bit_cast(unsigned int, two);
     }
 }
-// The A operands of both parities: band[ob][i] of product i, one[w][ob] of the single slot where the window's first block has the
-// odd (w = 0) or the even (w = 1) dwords.
-template <int CQT, bool DENSE_SINGLE> struct SparseBands {
-    using T = SparseTaps<CQT, DENSE_SINGLE>;
-    f16x8 band[2][T::products], one[T::ONE ? 2 : 1][2];
+// The A operands of both parities: band[ob][i] of product i, and of the single slot one[w][ob] where the window's first block has the
+// even (w = 0) or, BOTH, the odd (w = 1) dwords.
+template <int CQT, bool BOTH> struct SparseBands {
+    using T = SparseTaps<CQT>;
+    static_assert(T::every_slot_once(), "the slots of the products");
+    f16x8 band[2][T::products], one[BOTH ? 2 : 1][2];
+    // c + the single slot of parity ob, from the tuple it is in
+    __device__ __forceinline__ f32x4 single(int w, int ob, u32x8 rows, f32x4 c) const {
+        const u32x4 v = ob ? (u32x4){rows[4], rows[5], rows[6], rows[7]} : (u32x4){rows[0], rows[1], rows[2], rows[3]};
+        if (!BOTH && w) return mfma_f16(one[0][ob], __builtin_bit_cast(f16x8, (u32x4){v[1], v[0], v[3], v[2]}), c);
+        return mfma_f16(one[w][ob], __builtin_bit_cast(f16x8, v), c);
+    }
     __device__ __forceinline__ void read(const unsigned int *tab, int g, int n) {
 #pragma unroll
         for (int ob = 0; ob < 2; ++ob) {
@@ -141,13 +159,13 @@ template <int CQT, bool DENSE_SINGLE> struct SparseBands {
                 }
                 band[ob][i] = __builtin_bit_cast(f16x8, v);
             }
-            if constexpr (T::ONE)
+            if constexpr (T::odd)
 #pragma unroll
-                for (int w = 0; w < 2; ++w) {
+                for (int w = 0; w < (BOTH ? 2 : 1); ++w) {
                     u32x4 v;
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
-                        v[q] = tab[T::single_slot(ob) * kBandRow + 4 * g + 2 * (q >> 1) + ((q & 1) == w ? 16 : 0) - n + 16];
+                        v[q] = tab[T::single_slot(ob) * kBandRow + 4 * g + 2 * (q >> 1) + ((q & 1) != w ? 16 : 0) - n + 16];
                     one[w][ob] = __builtin_bit_cast(f16x8, v);
                 }
         }
