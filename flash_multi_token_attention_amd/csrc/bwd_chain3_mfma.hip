@@ -866,8 +866,12 @@ hipError_t pick_cq(const Problem &p, const void *q, const void *k, const void *v
                    void *ds_ws, float *dw_part, int share, float *kv_part, hipStream_t s) {
 #define CALL(CQT) launch_chain3<D, CQT, TO, WANT>(p, q, k, v, d_o, Dl, lse, w, dc_scale, dk, dv, ds_ws, dw_part, share, kv_part, s)
     if (p.c_q <= 3) return CALL(3);
-    // (7 slots take as many products as 8; at d = 128 with fewer spills in 8: kernel of B4 H16 N4096 7x7 1480 us in 7, 1410 in 8)
     if (p.c_q > 8) return CALL(11);
+    // (7 taps in 8 slots have a zero weight for a row outside the window, whose infinities and NaN then reach dQ, and a fifth operand tuple:
+    // whole backward of B4 H16 N4096 7x7 in 8 and in 7, us: d64 1315 and 1291, d32 1139 and 1132, B2 H8 N1531 d32 80 and 77.  At d = 128
+    // 7 slots spill more: the kernel 1410 and 1480)
+    if constexpr (D <= 64)
+        if (p.c_q == 7) return CALL(7);
     if (p.c_q > 6) return CALL(8);
     return CALL(6);
 #undef CALL

@@ -64,3 +64,10 @@ def test_backward_rows_outside_the_window(c_q, c_k, d, causal, row):
     for one_pass in (False, True):
         got = _run_bwd(*[t.to(DEV) for t in (Q, K, V, dO, W)], causal, torch.float32, one_pass)[0]
         assert max_abs(got[:, :, rows], want[:, :, rows]) <= TOL_BF16
+
+
+# 7 taps have slots of their own up to d = 64
+@pytest.mark.parametrize("d,causal", [(32, True), (32, False), (64, True), (64, False)])
+@pytest.mark.parametrize("row", [100, 101])
+def test_backward_rows_outside_a_window_of_seven(d, causal, row):
+    test_backward_rows_outside_the_window(7, 7, d, causal, row)
