@@ -390,7 +390,9 @@ __device__ __forceinline__ void chain3_role(const CHAIN_CONST_AS ChainArgs *args
                     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                         for (int f = 0; f < 2; ++f) { prev_pd[kb][f][0] = pd[kb][f][0]; prev_pd[kb][f][1] = pd[kb][f][1]; }
-                    if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
+                    // (3 slots at d = 128: moved into their short convolution, dP's loads spilled 9 registers of the score waves; B4 H16 N2048 3x3
+                    // whole backward 413 -> 382 us, not causal 772 -> 732, B2 H8 N1531 not causal, split, 144 -> 135)
+                    if constexpr (VLDS || (D == 128 && CQT <= 3)) __builtin_amdgcn_sched_barrier(0);
                     dp_phase();
                     // ---- P = exp2(C - LSE) (times the dC scale), dC = P dP ----
                     if constexpr (VLDS) __builtin_amdgcn_sched_barrier(0);
