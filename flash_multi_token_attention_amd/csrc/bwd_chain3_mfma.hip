@@ -13,18 +13,20 @@
 //   key wave (waves 8-11), tile it-2: dS^T by flipped-band MFMAs over the packed dC^T of tiles it-2
 //       and it-1, dS -> workspace and -> LDS, dK^T += Q^T dS.  The value and key waves issue the
 //       loads of the Q / dO tile it+1 (global memory -> LDS); the last key wave stages LSE / D.
-// One workgroup barrier per tile.  With 168 registers per wave every role keeps its operands and
-// accumulators in registers, and a SIMD always has two other waves to issue from while one waits
-// for LDS data, the matrix pipe or the barrier.
+// One workgroup barrier per tile.  A SIMD always has two other waves to issue from while one waits
+// for LDS data, the matrix pipe or the barrier.  168 registers per wave hold the operands and accumulators of every role up to d = 64
+// (8 slots spill 0 to 8 registers, 11 0 to 8) and of 6 slots at d = 128; there 3 slots spill none (in parts 8), 8 slots 2 to 4 (in parts 16)
+// and 11 slots 32 to 36, and of the key waves' bands 8 slots have all and 11 slots three fifths in LDS (ChainLds).
 // What bounds it: a score wave's chain per tile alone takes two thirds of the kernel's time (d = 64, 6 taps: 680 of 1020 us with the
 // other roles' work left out), the other roles as much without it, and together they share the LDS (two thirds busy), the matrix
 // pipe and the vector ALUs.  So both convolutions take two tap slots per sparse product (SparseTaps in mfma_common.hpp), the key
-// waves keep their bands in registers, and dW's operands of neighbouring taps share their transpose reads (43 per wave and tile for
+// waves keep their bands in registers where those suffice, and dW's operands of neighbouring taps share their transpose reads (43 per wave and tile for
 // 56 at 6 slots, 61 for 112 at 11).  Rows of S and dC of 104 bytes (112 before: an 8-byte store of 16 rows two apart took 17 clocks of
-// the LDS, now 9) and the offset of the odd rows of Q and dO (transpose reads 5 -> 3) left 34 % of the LDS's busy clocks to conflicts at d = 128,
-// 42 before; the rest, row fragments and the stores, gained nothing when taken out at the price of registers.  Kernel alone,
-// B4 H16 N4096 causal, before -> after, us: d 128 6x11 1409 -> 1270, d 64 6x11 1097 -> 930, 11x11 1442 -> 1243, 3x3 833 -> 770; at d 128 with more than 6 taps, in the place of a kernel of two waves per
-// SIMD and 256 registers, 7x7 1510 -> 1350, 11x11 1960 -> 1520 (B1 H8 N1500 61 -> 49).
+// the LDS, now 9) and the offset of the odd rows of Q and dO (transpose reads 5 -> 3) left 42 % of the clocks in which the LDS is active to
+// conflicts at d = 128, 53 before; the rest, row fragments and the stores, gained nothing when taken out at the price of registers.
+// Kernel alone, B4 H16 N4096 causal, before -> after, us: d 128 6x11 1409 -> 1270, d 64 6x11 1097 -> 930, 11x11 1442 -> 1243, 3x3 833 -> 770; at
+// d 128 with more than 6 taps, in the place of a kernel of two waves per SIMD and 256 registers, 7x7 1510 -> 1350, 11x11 1960 -> 1520 (B1 H8 N1500
+// 61 -> 49).  The single slots of odd counts are dense products since (SparseTaps): 11x11 2 to 5 % more, 3x3 at d 128 with its fence 6 % less.
 #include <type_traits>
 
 #include "chain_common.hpp"

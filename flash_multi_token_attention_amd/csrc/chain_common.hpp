@@ -8,11 +8,10 @@
 namespace convattn {
 namespace chain {
 
-constexpr int NP = 4;            // wave pairs = 32-key ranges per workgroup
-constexpr int WK = 32;           // own keys per pair
+constexpr int NP = 4;            // wave triples = 32-key ranges per workgroup
+constexpr int WK = 32;           // own keys per triple
 constexpr int BKW = NP * WK;     // 128 keys per workgroup
 constexpr int BR = 32;           // query rows per tile
-constexpr int NSB = 4;           // S^T blocks of a pair: keys c0-16+16kb
 constexpr int NCB = 3;           // C / dP / dC blocks: keys c0-8+16cb
 constexpr int NDB = 2;           // dS blocks: keys c0+16sb
 constexpr int SST = 104;         // bytes per row of the S tile in LDS (48 keys fp16 + 8)
@@ -115,7 +114,7 @@ template <int D, int CQT> struct ChainLds {
     static constexpr int ds_bytes = BR * PST;
     static constexpr int pair_bytes = s_bytes + c_bytes + p_bytes + ds_bytes;
     // V and, where there is room, K fragments of the block after the workgroup's keys (16 rows each): the wave that computes it has no
-    // registers to keep them in (with K in registers 12 and 24 spilled at d = 128, 6 and 8 slots, now 0 and 2; kernel of B4 H16 N4096 1254 ->
+    // registers to keep them in (with K in registers 12 and 24 spilled at d = 128, 6 and 8 slots, now 0 and 2, in parts 0 and 16; kernel of B4 H16 N4096 1254 ->
     // 1253 and 1384 -> 1352 us, of B1 H32 N16384 6x11 9075 -> 9009)
     static constexpr int e_off = pair_off + NP * pair_bytes;
     static constexpr bool k_park = D == 128 && CQT <= 8;   // (11 slots: no room)

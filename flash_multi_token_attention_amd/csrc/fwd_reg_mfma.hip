@@ -92,7 +92,8 @@ template <int BQ> inline int fwd_wgs(const Problem &p, int share) {
 }
 
 // Waves per SIMD that the registers have to leave room for: windows of up to 6 slots fit three (168 registers) up to d = 64.  Forced to
-// three, 7 and 8 slots spill 8 to 15 registers (B4 H16 N4096 d64 7x7 299 -> 350 us, 8x9 324 -> 354); four at d = 32 with 3 slots: 19.0 -> 19.4.
+// three, 7 and 8 slots spill (B4 H16 N4096 d64 7x7 324 -> 402 us, 8x11 340 -> 380, B2 H12 N3000 7x7 79 -> 109); four at d = 32 with 3 slots:
+// the same (B4 H16 N4096 154 and 156).
 constexpr int fwd_waves(int d, int cqt) { return d <= 64 && cqt <= 6 ? 3 : 2; }
 // (SPLIT: an instance of its own, the other one is a percent slower with the parts' bounds at run time)
 // LONG: the tiles from split.first_long on run at a higher wave priority (long_tiles_first)
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(NW * 64, fwd_waves(D, CQT)) void fwd_reg_mfma_kerne
         // (the table lies in the K / V buffer that the first step does not use)
         static_assert(band_table_bytes<CQT>() <= Lds::buf_bytes, "room for the table");
         unsigned int *tab = reinterpret_cast<unsigned int *>(smem + ((u_first & 1) ^ 1) * Lds::buf_bytes);
-        band_table_build<CQT>(tab, W + (size_t)h * cq * p.c_k, cq, p.c_k, pk, false, p.scale * kLog2e, tid, NW * 64);
+        band_table_build<CQT>(tab, W + (size_t)h * cq * p.c_k, cq, p.c_k, pk, p.scale * kLog2e, tid, NW * 64);
         __syncthreads();
         if constexpr (WIDE) {
 #pragma unroll
@@ -615,16 +616,18 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(Problem p, FwdSplit spli
 // Steps per workgroup, or 0: one workgroup per query tile.  In units of a key step of a workgroup that has a CU to itself:
 // a workgroup costs its steps and about 4 (5 where it is a part); with two per CU each runs at 0.6 of that; the merge
 // kernel about 8.  Few (batch, head) pairs or rows leave the launch as long as its longest tile
-// (B1 H8 N2048 d64 7x7: 49 -> 30 + 7 us, B1 H8 N1000 d128 6x11: 30 -> 16 + 6).
+// (B1 H8 N2048 d64 7x7: 41 -> 34 us with the merge, B1 H8 N1000 d128 6x11: 28 -> 25).
 // What this leaves out is the traffic of the parts, D + 4 floats per row and part: with many unsplit workgroups for their length
-// the split form is slower (B2 H16 N2048 6x11: d64 57 us unsplit, 65 in parts, d128 70 and 91; 3x3 d128 59 and 81), so it is
-// taken up to `fill` of them only.  The line is measured: of 753 shapes of 1 to 64 heads and 1000 to 8000 rows (3x3 to 11x11 taps,
-// d 32 to 128) that the estimate splits, 6 are up to 4 % slower than unsplit with it (105, up to 38 %, without), 8 would be 3 to
-// 8 % faster.
-// Sequences of less than 32 steps would gain too (B1 H8 N640 d64 6x11 18.5 -> 16.2 us); their calls are bound by the host.  Beyond 64
-// heads no cut gains (13 to 55 % slower at 80 to 256 heads of 1024 to 4096 rows).  From 8192 rows on nothing is split, whatever
+// the split form is slower (B2 H16 N2048 6x11: d64 54 us unsplit, 60 in parts, d128 69 and 87; 3x3 d128 61 and 81), so it is
+// taken up to `fill` of them only.  The line was drawn with one dense product per tap: of 753 shapes of 1 to 64 heads and 1000 to 8000
+// rows (3x3 to 11x11 taps, d 32 to 128) that the estimate splits, 6 were up to 4 % slower than unsplit with it (105, up to 38 %, without).
+// With the present steps, 11 to 23 % shorter, of 150 other such shapes 73 run in parts, in 0.75 of the unsplit time on average, 12 of them
+// 3 to 8 % slower than unsplit; 7 unsplit ones would gain more than 3 %.  The cut taken is 2.8 % over the best of up to six parts on
+// average (unsplit: 25 %), single ones up to 27 % (B1 H2 N7781 d128 8x15 109 us, in five parts 86).
+// Sequences of less than 32 steps would gain too (B1 H8 N640 d64 6x11 16.0 -> 15.1 us); their calls are bound by the host.  Beyond 64
+// heads no cut gained (13 to 55 % slower at 80 to 256 heads of 1024 to 4096 rows, dense products).  From 8192 rows on nothing is split, whatever
 // the number of heads is, so that a head's results do not depend on how many others there are; up to four heads would gain
-// (B1 H1 N16384 d128 386 -> 201 us, B1 H4 N8192 209 -> 175), more would not (B1 H8 N8192 252 -> 284).
+// (B1 H1 N16384 d128 349 -> 156 us, B1 H4 N8192 190 -> 152), more would not (B1 H8 N8192 237 -> 259).
 template <int BQ> int fwd_share(const Problem &p) {
     const int n_qt = (p.Nq + BQ - 1) / BQ, most = fwd_steps<BQ>(p, n_qt - 1);
     if (most < 32 || p.Nq >= 8192 || p.Nk >= 8192 || p.B * (long long)p.H > 64) return 0;
@@ -659,14 +662,15 @@ template <int BQ> int fwd_share(const Problem &p) {
 // Causal launches of 1.4 to 2 rounds of workgroups end with their longest tiles: a CU has three workgroups, a slot's tiles are shorter
 // together than the longest one alone (65 and 55 steps at B4 H16 N2048 d64 6x11), and that one runs at a third of the CU until the others
 // leave.  There the longer half of the tiles gets the issue slots first; us without and with it at B4 H16 N2048 (1.6 rounds): d64 6x11
-// 95 / 90, 3x3 82 / 78, d32 6x11 77 / 74.
-// Below 1.4 and beyond 2 rounds the two waves of a SIMD had better take turns by phase (d64): B2 H12 6x11 of 1.25 rounds 139 / 148, 1.31 149 / 159,
-// 1.38 168 / 171, 1.41 178 / 176, 1.5 207 / 195; N8000 (2.3) 443 / 452, B4 H16 N4096 (3.2) 320 / 342.
-// The fewer tiles a head has, the less there is to put in order, and the earlier that ends: with 47 tiles (B1 H32 N5000) 1.96 rounds 256 / 245, with
-// 24 (B4 H16 N2581) 2.0 rounds 137 / 144, 22 tiles 1.83 rounds 119 / 116; 16 tiles 2.0 rounds 98 / 98, 14 1.75 80 / 79; 12 2.0 75 / 76, 12 1.5
-// 63 / 61; 7 (B12 H16 N745) 1.75 48.4 / 49.0, 6 2.0 49.3 / 50.4, 6 1.5 40.2 / 39.6; 3 1.5 25.3 / 25.6.  144 launches of 64 to 384 heads.
-// The instances that have three workgroups per CU; with two it costs up to 10 % in this band (B1 H32 N2500 d64 7x7 82 / 90, d128 6x11 101 / 110), with
-// four 1 to 3 %.
+// 86 / 80, 3x3 70 / 65, d32 6x11 66 / 63.
+// Below 1.4 and beyond 2 rounds the two waves of a SIMD had better take turns by phase (d64): 6x11 of 1.17 rounds (32 heads) 82.6 / 85.1, d32 of 1.41
+// (24 heads) 115 / 122; 2.17 130 / 131, 2.4 397 / 399, B4 H16 N4096 (3.2) 264 / 269.
+// The fewer tiles a head has, the less there is to put in order, and the earlier that ends: with 47 tiles (B1 H32 N5000) 1.96 rounds 213 / 204, 22
+// tiles 1.83 rounds 101 / 96; 10 tiles 1.67 rounds 49.5 / 48.2.  That end was drawn with one dense product per tap (144 launches of 64 to 384 heads;
+// 24 tiles (B4 H16 N2581) 2.0 rounds 137 / 144, 7 tiles (B12 H16 N745) 1.75 48.4 / 49.0); now these would gain as well (118 / 112, 41.9 / 40.0), and so
+// would 7 and 8 slots at d = 32, which have three workgroups per CU since (B4 H16 N2048 7x7 71 / 65, 8x15 80 / 74).
+// The instances that had three workgroups per CU then; with two it costs up to 10 % in this band (B1 H32 N2500 d64 7x7 64 / 71), with four (d32 3x3)
+// 1 to 4 %.
 constexpr bool has_long(int d, int cqt) { return (d == 64 && cqt <= 6) || (d == 32 && cqt == 6); }
 template <int BQ> bool long_tiles_first(const Problem &p) {
     const long long tiles = (p.Nq + BQ - 1) / BQ, wgs = p.B * p.H * tiles, round = 3 * 256;
@@ -702,7 +706,7 @@ hipError_t pick_cq(const Problem &p, float *part, const void *q, const void *k, 
                    void *o, float *m, float *l, hipStream_t s) {
     if (p.c_q <= 3) return launch_fwd<D, 3, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
     if (p.c_q <= 6) return launch_fwd<D, 6, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
-    // (7 taps in 8 slots: B2 H12 N4691 d128 7x7 281 us, in 7 266)
+    // (7 taps in 8 slots, B2 H12 N4691: d128 231 us, in 7 225, d64 170 and 157)
     if (p.c_q <= 7) return launch_fwd<D, 7, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
     if (p.c_q <= 8) return launch_fwd<D, 8, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);
     return launch_fwd<D, 11, TO, WIDE>(p, part, q, k, v, w, o, m, l, s);

@@ -112,20 +112,20 @@ template <int CQT> struct SparseTaps {
     }
 };
 // The bands of a head as a table in LDS: dword x + 16 of tap slot t's 48 holds the weights of two neighbouring keys, T[x] and T[x + 1]
-// with T[x] = w[a][pk + x - 8] * mul (`flip`: pk - (x - 8); zero outside the window), x = the key's place in the window less the output
+// with T[x] = w[a][pk + x - 8] * mul (zero outside the window), x = the key's place in the window less the output
 // key's; slot t stands for tap a = t - (CQT - c_q).  A lane finds the pairs of its operands there with
 // 4-byte reads: one or two loads of W per thread instead of the 48 to 88 gathers of every lane.
 constexpr int kBandRow = 48;
 template <int CQT> constexpr int band_table_bytes() { return CQT * kBandRow * 4; }
 template <int CQT>
-__device__ __forceinline__ void band_table_build(unsigned int *tab, const float *__restrict__ w_head, int c_q, int c_k, int pk, bool flip,
-                                                 float mul, int tid, int nthreads) {
+__device__ __forceinline__ void band_table_build(unsigned int *tab, const float *__restrict__ w_head, int c_q, int c_k, int pk, float mul,
+                                                 int tid, int nthreads) {
     for (int i = tid; i < CQT * kBandRow; i += nthreads) {
         const int t = i / kBandRow, a = t - (CQT - c_q), off = i - t * kBandRow - 16 - kKeyHalo;
         float v[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const int b = flip ? pk - off - e : pk + off + e;
+            const int b = pk + off + e;
             v[e] = w_head[min(max(a, 0), c_q - 1) * c_k + min(max(b, 0), c_k - 1)];
             v[e] = a >= 0 && b >= 0 && b < c_k ? v[e] * mul : 0.f;
         }
@@ -177,12 +177,10 @@ template <int CQT, bool BOTH> struct SparseBands {
 // of stage s" so that fragment reads stay one stage ahead instead of sinking next to their use.
 #define SCHED_DS_READ(n) __builtin_amdgcn_sched_group_barrier(0x100, (n), 0)
 #define SCHED_MFMA(n) __builtin_amdgcn_sched_group_barrier(0x008, (n), 0)
-#define SCHED_VALU(n) __builtin_amdgcn_sched_group_barrier(0x002, (n), 0)
 // The same with an explicit pipeline id: groups are only ordered against groups of their own id,
 // and the backend places long pipelines badly, so every row block of a phase gets its own.
 #define SCHED_DS_READ_ID(n, id) __builtin_amdgcn_sched_group_barrier(0x100, (n), (id))
 #define SCHED_MFMA_ID(n, id) __builtin_amdgcn_sched_group_barrier(0x008, (n), (id))
-#define SCHED_VALU_ID(n, id) __builtin_amdgcn_sched_group_barrier(0x002, (n), (id))
 
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>): a loop whose index is a
 // constant expression in the body (the scheduling-group builtins need one).
@@ -192,12 +190,6 @@ __device__ __forceinline__ void static_for(F &&f) {
         static_for<N - 1>(f);
         f(std::integral_constant<int, N - 1>{});
     }
-}
-
-// Lane n of every 16-lane row gets the value lane n+1 of that row holds (lane 15 gets 0):
-// DPP row_shl:1.
-__device__ __forceinline__ unsigned int lane_from_next(unsigned int v) {
-    return (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, 0x101, 0xf, 0xf, true);
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

@@ -290,16 +290,17 @@ class Schedule {
 // Row tiles per workgroup of the split backward, or 0: one workgroup per key block.  The launch is laid out on 256 CUs for each
 // cut of the longest key block, from 1 1/4 to 8 parts; in units of a row tile a workgroup costs its tiles, 10 for set-up and wind-down and
 // 1 more where its range ends inside the key block (windows of 7 to 11 query taps, whose tiles take longer: 4 and 1 up to d = 64, 6 and
-// 2 at 128); what the reduction takes is in the margin over the unsplit launch.  Against every cut for 2 to 64 heads of 640 to
-// 8000 rows (482 shapes of 3x3 to 11x11 taps, d 32 to 128, a quarter of the last 221 not causal): 0.3 to 0.8 % over the best on
-// average (with cuts into 2, 3, 4, 6 and 8 parts only 1.9 to 2.5 %).  (B2 H8 N1531 d64 11x11, us, whole backward without D: unsplit 163,
-// into 3 parts 125, 1 1/2 parts 117; B1 H8 N2048 d64 7x7 164, 108 and, into 3 parts, 92; with more than two rounds of workgroups a split loses:
-// B1 H8 N8000 d128 6x11 774 us unsplit, 933 in parts, B1 H12 N5000 491 and 594.)
-// The limits: 12 to 19 row tiles would gain too (B1 H8 N512 d64 6x11 the whole backward 47 -> 31 us), which such calls, bound by
-// the host (75 us for a step), show in a captured graph only.  Beyond 64 heads no cut gains (5 to 45 % slower at 80 to
-// 256 heads of 640 to 4096 rows).  From 8192 rows on nothing is split, whatever the number of heads is, so that a head's results
-// do not depend on how many others there are; up to four heads would gain (B1 H1 N16384 d128 1323 -> 771 us, B1 H4 N8192 682 -> 587),
-// more would not (B1 H8 N8192 790 -> 946).
+// 2 at 128); what the reduction takes is in the margin over the unsplit launch.  The constants were fitted with one dense product per tap, against
+// every cut for 2 to 64 heads of 640 to 8000 rows (482 shapes of 3x3 to 11x11 taps, d 32 to 128, a quarter of the last 221 not causal): 0.3 to
+// 0.8 % over the best on average.  With two taps per product, 110 other such shapes: 1.7 % over the best of twelve cuts on average (unsplit
+// 38 %), single ones up to 15 % (B1 H12 N2023 d32 7x7 105 us, into 1 3/4 parts 91), 8 of the 73 in parts 2 to 6 % slower than unsplit.
+// (B2 H8 N1531 d64 11x11, us, whole backward without D: unsplit 133, into 3 parts 116, 1 1/2 parts 101; B1 H8 N2048 d64 7x7 137, 84, 100; with more
+// than two rounds of workgroups a split loses: B1 H8 N8000 d128 6x11 771 us unsplit, 889 in 2 parts, B1 H12 N5000 486 and 563.)
+// The limits: 12 to 19 row tiles would gain too (B1 H8 N512 d64 6x11 the whole backward 44 -> 30 us), which such calls, bound by
+// the host (75 us for a step), show in a captured graph only.  Beyond 64 heads no cut gained (5 to 45 % slower at 80 to
+// 256 heads of 640 to 4096 rows, dense products).  From 8192 rows on nothing is split, whatever the number of heads is, so that a head's results
+// do not depend on how many others there are; up to four heads would gain (B1 H1 N16384 d128 1180 -> 632 us, B1 H4 N8192 614 -> 501),
+// more would not (B1 H8 N8192 732 -> 749).
 int chain_share(const Problem &p) {
     const int n_rt = chain_row_tiles(p), n_kb = mfma_kv_tiles(p);
     const long long heads = (long long)p.B * p.H;
